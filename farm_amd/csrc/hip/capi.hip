@@ -18,20 +18,23 @@
 
 namespace farm {
 __global__ void k_filter(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *, int, int, const uint8_t *,
-                         uint32_t *, const uint32_t *, PixPair *, uint64_t, uint32_t *, unsigned long long *);
+                         uint32_t *, const uint32_t *, PixPair *, uint64_t, uint32_t *, const unsigned long long *,
+                         unsigned long long *);
 __global__ void k_scan_sums(const uint32_t *, const unsigned long long *, uint64_t, uint32_t *);
-__global__ void k_scan_parts(uint32_t *, const unsigned long long *, uint64_t, uint32_t *);
+__global__ void k_scan_parts(uint32_t *, const unsigned long long *, uint64_t, uint32_t *, unsigned long long *,
+                             unsigned long long *, int);
 __global__ void k_scan_apply(const uint32_t *, const unsigned long long *, uint64_t, const uint32_t *, uint32_t *);
-__global__ void k_set_desc(IsxDesc *, unsigned long long, unsigned long long, uint8_t *, uint32_t *);
+__global__ void k_set_desc(IsxDesc *, unsigned long long, unsigned long long, uint8_t *, uint32_t *, uint32_t *);
 __global__ void k_bucket_hist(DevSet, const uint32_t *, const IsxDesc *, const PixPair *, const unsigned long long *,
                               uint64_t, const float *, uint8_t *, uint32_t *);
 __global__ void k_bucket_scan(uint32_t *, uint32_t *);
 __global__ void k_bucket_scatter(const uint8_t *, const unsigned long long *, uint64_t, uint32_t *, uint32_t *);
 template <int E>
-__global__ void k_tiles(const PixPair *, const uint32_t *, unsigned long long *, uint64_t, uint32_t *);
+__global__ void k_tiles(const PixPair *, const uint32_t *, const unsigned long long *, unsigned long long *, uint64_t,
+                        uint32_t *);
 template <int E, int C>
 __global__ void k_refine(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *, const TileDesc *, uint64_t,
-                         uint64_t, uint32_t *, uint32_t *, unsigned long long *, int);
+                         uint64_t, uint32_t *, uint32_t *, const unsigned long long *, unsigned long long *, int);
 __global__ void k_tile_map(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *, const PixPair *,
                            const uint32_t *, const uint32_t *, const unsigned long long *, uint64_t, uint64_t,
                            TileDesc *);
@@ -39,8 +42,8 @@ __global__ void k_plain(DevSet, const uint32_t *, const uint32_t *, uint32_t, ui
 __global__ void k_pixedges(DevSet, int64_t, uint32_t *);
 __global__ void k_vdiff(const float *, const float *, uint64_t, float4 *);
 __global__ void k_chunk_count(DevSet, int64_t, uint32_t, uint32_t *);
-__global__ void k_chunk_box(DevSet, int64_t, uint32_t, const uint32_t *, float4 *);
-__global__ void k_finalize(const uint32_t *, const IsxDesc *, unsigned long long *);
+__global__ void k_chunk_box(DevSet, int64_t, uint32_t, const uint32_t *, float4 *, uint2 *);
+__global__ void k_finalize(const uint32_t *, const IsxDesc *, unsigned long long *, unsigned long long *);
 }  // namespace farm
 
 extern "C" int farm_mlp_predict_pairs(farm_handle h, uint64_t begin, uint64_t end, float *out);
@@ -97,12 +100,14 @@ int exclusive_scan(farm_handle h, const T *in, T *out, uint64_t n) {
 }
 
 // Exclusive scan on the device of n = bounded_count(nsrc, cap) values,
-// out[n] = total (no host round trip, no temporaries beyond W.part).
+// out[n] = total (no host round trip, no temporaries beyond W.part); the
+// shards of counter `slot` are folded on the way.
 int scan_dev(farm_handle h, const IsxWork &W, const uint32_t *in, const unsigned long long *nsrc, uint64_t cap,
-             uint32_t *out) {
+             uint32_t *out, int slot) {
     hipLaunchKernelGGL(k_scan_sums, dim3(kScanParts), dim3(256), 0, h->stream, in, nsrc, cap, W.part);
     HIPCHK(h, hipGetLastError());
-    hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kScanParts), 0, h->stream, W.part, nsrc, cap, out);
+    hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kScanParts), 0, h->stream, W.part, nsrc, cap, out, W.ctr,
+                       W.shards, slot);
     HIPCHK(h, hipGetLastError());
     hipLaunchKernelGGL(k_scan_apply, dim3(kScanParts), dim3(256), 0, h->stream, in, nsrc, cap,
                        (const uint32_t *)W.part, out);
@@ -134,51 +139,51 @@ static_assert(sizeof(IsxCfg) <= sizeof(((farm_handle_s::IsxGraph *)nullptr)->key
 int isx_front(farm_handle h, const DevSet &S, const IsxWork &W, const IsxCfg &c) {
     int rc;
     const unsigned g = (unsigned)c.grid;
-    if ((rc = fill_u32(h, W.ctr, 2 * kCtrSlots, 0))) return rc;
     hipLaunchKernelGGL(k_filter, dim3(g), dim3(256), 0, h->stream, S, c.pa, c.pb, (const IsxDesc *)W.desc, 0,
                        c.approx, c.skip, W.npp, (const uint32_t *)nullptr, (PixPair *)nullptr, W.cap_pp, W.result,
-                       W.ctr);
+                       (const unsigned long long *)W.ctr, W.shards);
     HIPCHK(h, hipGetLastError());
     if (c.approx) return FARM_OK;
-    if ((rc = scan_dev(h, W, W.npp, &W.desc->n, W.cap_pairs, W.pp_off))) return rc;
+    if ((rc = scan_dev(h, W, W.npp, &W.desc->n, W.cap_pairs, W.pp_off, kCtrPixPairs))) return rc;
     hipLaunchKernelGGL(k_filter, dim3(g), dim3(256), 0, h->stream, S, c.pa, c.pb, (const IsxDesc *)W.desc, 1, 0,
-                       c.skip, W.npp, (const uint32_t *)W.pp_off, W.pps, W.cap_pp, W.result, W.ctr);
+                       c.skip, W.npp, (const uint32_t *)W.pp_off, W.pps, W.cap_pp, W.result,
+                       (const unsigned long long *)W.ctr, W.shards);
     HIPCHK(h, hipGetLastError());
-    if ((rc = fill_u32(h, W.hist, 64, 0))) return rc;
-    hipLaunchKernelGGL(k_bucket_hist, dim3(g), dim3(256), 0, h->stream, S, c.pb, (const IsxDesc *)W.desc,
+    // (a quarter of the blocks: each adds its non-empty buckets to one histogram)
+    hipLaunchKernelGGL(k_bucket_hist, dim3(g / 4), dim3(256), 0, h->stream, S, c.pb, (const IsxDesc *)W.desc,
                        (const PixPair *)W.pps, (const unsigned long long *)W.ctr, W.cap_pp, c.pred_cost, W.bucket,
                        W.hist);
     HIPCHK(h, hipGetLastError());
     hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(64), 0, h->stream, W.hist, W.cursor);
     HIPCHK(h, hipGetLastError());
-    hipLaunchKernelGGL(k_bucket_scatter, dim3(g), dim3(256), 0, h->stream, (const uint8_t *)W.bucket,
+    hipLaunchKernelGGL(k_bucket_scatter, dim3(g / 4), dim3(256), 0, h->stream, (const uint8_t *)W.bucket,
                        (const unsigned long long *)W.ctr, W.cap_pp, W.cursor, W.order);
     HIPCHK(h, hipGetLastError());
+    auto count_tiles = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(g), dim3(256), 0, h->stream, (const PixPair *)W.pps,
+                           (const uint32_t *)W.order, (const unsigned long long *)W.ctr, W.shards, W.cap_pp, W.tiles);
+    };
     switch (c.tile) {
         case 1:
-            hipLaunchKernelGGL(k_tiles<1>, dim3(g), dim3(256), 0, h->stream, (const PixPair *)W.pps,
-                               (const uint32_t *)W.order, W.ctr, W.cap_pp, W.tiles);
+            count_tiles(k_tiles<1>);
             break;
         case 2:
-            hipLaunchKernelGGL(k_tiles<2>, dim3(g), dim3(256), 0, h->stream, (const PixPair *)W.pps,
-                               (const uint32_t *)W.order, W.ctr, W.cap_pp, W.tiles);
+            count_tiles(k_tiles<2>);
             break;
         case 4:
-            hipLaunchKernelGGL(k_tiles<4>, dim3(g), dim3(256), 0, h->stream, (const PixPair *)W.pps,
-                               (const uint32_t *)W.order, W.ctr, W.cap_pp, W.tiles);
+            count_tiles(k_tiles<4>);
             break;
         default:
-            hipLaunchKernelGGL(k_tiles<8>, dim3(g), dim3(256), 0, h->stream, (const PixPair *)W.pps,
-                               (const uint32_t *)W.order, W.ctr, W.cap_pp, W.tiles);
+            count_tiles(k_tiles<8>);
             break;
     }
     HIPCHK(h, hipGetLastError());
-    if ((rc = scan_dev(h, W, W.tiles, &W.ctr[kCtrPixPairs], W.cap_pp, W.tile_off))) return rc;
+    if ((rc = scan_dev(h, W, W.tiles, &W.ctr[kCtrPixPairs], W.cap_pp, W.tile_off, kCtrTiles))) return rc;
     hipLaunchKernelGGL(k_tile_map, dim3(g), dim3(256), 0, h->stream, S, c.pa, c.pb, (const IsxDesc *)W.desc,
                        (const PixPair *)W.pps, (const uint32_t *)W.order, (const uint32_t *)W.tile_off,
                        (const unsigned long long *)W.ctr, W.cap_pp, W.cap_tiles, W.tile_map);
     HIPCHK(h, hipGetLastError());
-    return fill_u32(h, W.cursor + 63, 1, 0);  // the refinement's tile cursor
+    return FARM_OK;
 }
 
 // The persistent refinement with the tile width and chunk size of the call.
@@ -186,8 +191,8 @@ template <int E, int C>
 void launch_refine(farm_handle h, const DevSet &S, const IsxWork &W, const IsxCfg &c) {
     const dim3 grid((unsigned)(h->num_cus * c.bpc)), blk(256);
     hipLaunchKernelGGL((k_refine<E, C>), grid, blk, 0, h->stream, S, c.pa, c.pb, (const IsxDesc *)W.desc,
-                       (const TileDesc *)W.tile_map, W.cap_pp, W.cap_tiles, W.cursor + 63, W.result, W.ctr,
-                       c.prune);
+                       (const TileDesc *)W.tile_map, W.cap_pp, W.cap_tiles, W.tcur, W.result,
+                       (const unsigned long long *)W.ctr, W.shards, c.prune);
 }
 
 template <int E>
@@ -301,6 +306,13 @@ namespace farm {
 
 int build_chunk_boxes(farm_handle h, uint32_t C);
 
+// Mean edges per BORDER pixel below which the default tile is 1 edge per lane
+// (2 below twice that, 4 below four times).  Measured, k_refine at 1 / 4 / 8
+// edges per lane: 23 edges per pixel (jagged rings, -v 10, 8 sequences a
+// pixel) 2.5 / 3.2 / 4.6 ms; 560 to 740 (complex x lakes, -v 256) 22.4 / 14.6
+// / 13.9 ms.
+constexpr double kTileEdges = 48.0;
+
 // Sum and count of the nonzero per-pixel edge counts (BORDER pixels).
 __global__ __launch_bounds__(256) void k_shape_stats(const uint32_t *__restrict__ pixedges, uint64_t n,
                                                      uint64_t *__restrict__ out) {
@@ -365,6 +377,12 @@ int finish_set(farm_handle h) {
         h->tuned_tile = it->second.tile_a;
         h->tuned_chunk = it->second.chunk;
         h->tuned_bpc = it->second.blocks_per_cu;
+    } else if (!h->tile_chosen) {
+        // nothing tuned or set: the narrowest tile whose 64 lanes hold a mean
+        // pixel's edges (short edge sequences add a slot each, so the lines
+        // lie below 64, 128 and 256)
+        const double e = hs[1] ? (double)hs[0] / (double)hs[1] : 0.0;
+        h->tuned_tile = e < kTileEdges ? 1 : e < 2 * kTileEdges ? 2 : e < 4 * kTileEdges ? 4 : 8;
     }
     return build_chunk_boxes(h, (uint32_t)h->tuned_chunk);
 }
@@ -389,9 +407,10 @@ int build_chunk_boxes(farm_handle h, uint32_t C) {
     HIPCHK(h, hipMemcpyAsync(&nchunks, P<uint32_t>(h->choff) + nseqs, 4, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     if ((rc = ensure(h, h->chbox, 16ull * (nchunks + kRefScreen)))) return rc;
+    if ((rc = ensure(h, h->chseg, 8ull * (nchunks + kRefScreen)))) return rc;
     if (h->npolys > 0) {
         hipLaunchKernelGGL(k_chunk_box, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys, C,
-                           (const uint32_t *)P<uint32_t>(h->choff), P<float4>(h->chbox));
+                           (const uint32_t *)P<uint32_t>(h->choff), P<float4>(h->chbox), P<uint2>(h->chseg));
         HIPCHK(h, hipGetLastError());
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -420,7 +439,8 @@ int build_ix_boxes(farm_handle h) {
     if ((rc = ensure(h, h->ixbox, 16ull * (nchunks + 1)))) return rc;
     if (h->npolys > 0) {
         hipLaunchKernelGGL(k_chunk_box, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys,
-                           kIxChunk, (const uint32_t *)P<uint32_t>(h->ixoff), P<float4>(h->ixbox));
+                           kIxChunk, (const uint32_t *)P<uint32_t>(h->ixoff), P<float4>(h->ixbox),
+                           (uint2 *)nullptr);
         HIPCHK(h, hipGetLastError());
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -472,6 +492,7 @@ static bool valid_tuning(const farm_tuning &t) {
 // Make t the default configuration and the entry of the set's bucket.
 static int apply_tuning(farm_handle h, const farm_tuning &t) {
     h->tuned_tile = t.tile_a;
+    h->tile_chosen = true;
     h->tuned_chunk = t.chunk;
     h->tuned_bpc = t.blocks_per_cu;
     farm_tuning e = t;
@@ -548,6 +569,7 @@ int farm_set_tile(farm_handle h, int tile) {
     if (!h) return FARM_EINVAL;
     if (tile != 1 && tile != 2 && tile != 4 && tile != 8) return fail(h, FARM_EINVAL, "tile must be 1, 2, 4 or 8");
     h->tuned_tile = tile;
+    h->tile_chosen = true;
     return FARM_OK;
 }
 
@@ -681,7 +703,7 @@ int farm_close(farm_handle h) {
         if (h->stage[k]) (void)hipHostFree(h->stage[k]);
         if (h->stage_ev[k]) (void)hipEventDestroy(h->stage_ev[k]);
     }
-    DevBuf *bufs[] = {&h->hdr,    &h->status,  &h->pixoff, &h->seqs,   &h->x,      &h->y,        &h->xyd,      &h->fill,     &h->choff,  &h->chcnt,  &h->chbox,  &h->ixcnt, &h->ixoff, &h->ixbox, &h->voff,
+    DevBuf *bufs[] = {&h->hdr,    &h->status,  &h->pixoff, &h->seqs,   &h->x,      &h->y,        &h->xyd,      &h->fill,     &h->choff,  &h->chcnt,  &h->chbox,  &h->chseg,  &h->ixcnt, &h->ixoff, &h->ixbox, &h->voff,
                       &h->vnodes, &h->pixedges, &h->shape_ctr, &h->pa, &h->pb, &h->isx,
                       &h->scan_tmp, &h->pair_tests, &h->mlp_w, &h->mlp_m, &h->mlp_v, &h->mlp_g,
                       &h->mlp_norm, &h->mlp_x, &h->mlp_h1, &h->mlp_h2, &h->mlp_z3, &h->mlp_d3, &h->mlp_dh2,
@@ -855,12 +877,11 @@ static int run_intersect(farm_handle h, uint64_t begin, uint64_t end, const farm
         if (fixed) W = isx_carve(h->scratch, kNaPairs, kNaPixPairs, kNaTiles);
         else if ((rc = isx_reserve(h, n, &W))) return rc;
         uint8_t *outp = out_kind == OUT_DEV ? out : (out_kind == OUT_HOST ? W.bits : nullptr);
-        hipLaunchKernelGGL(k_set_desc, dim3(1), dim3(64), 0, h->stream, W.desc, (unsigned long long)begin,
-                           (unsigned long long)n, outp, pair_tests);
+        hipLaunchKernelGGL(k_set_desc, dim3(blocks_for(kIsxClear)), dim3(256), 0, h->stream, W.desc,
+                           (unsigned long long)begin, (unsigned long long)n, outp, pair_tests, (uint32_t *)W.ctr);
         HIPCHK(h, hipGetLastError());
         HIPCHK(h, hipEventRecord(h->ev[0], h->stream));
         if (mode == FARM_MODE_EXACT_PLAIN) {
-            if ((rc = fill_u32(h, W.ctr, 2 * kCtrSlots, 0))) return rc;
             if ((rc = fill_u32(h, W.result, n, 0))) return rc;
             if (pair_tests && (rc = fill_u32(h, pair_tests, n, 0))) return rc;
             HIPCHK(h, hipEventRecord(h->ev[1], h->stream));
@@ -909,8 +930,10 @@ static int run_intersect(farm_handle h, uint64_t begin, uint64_t end, const farm
             if (!approx && (rc = isx_refine(h, S, W, cfg))) return rc;
         }
         HIPCHK(h, hipEventRecord(h->ev[3], h->stream));
-        hipLaunchKernelGGL(k_finalize, dim3(h->num_cus * 4), dim3(256), 0, h->stream, (const uint32_t *)W.result,
-                           (const IsxDesc *)W.desc, W.ctr);
+        // (few blocks: each adds its count of true pairs to one counter)
+        const unsigned fb = std::min(std::max(blocks_for(n, 4096), 1u), (unsigned)h->num_cus);
+        hipLaunchKernelGGL(k_finalize, dim3(fb), dim3(256), 0, h->stream, (const uint32_t *)W.result,
+                           (const IsxDesc *)W.desc, W.ctr, W.shards);
         HIPCHK(h, hipGetLastError());
         HIPCHK(h, hipMemcpyAsync(c, W.ctr, sizeof c, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));

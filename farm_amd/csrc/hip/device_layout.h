@@ -22,9 +22,11 @@ struct DevSet {
     // 16-byte load per target step)
     const float4 *xyd;
     // per edge sequence: index of its first C-step chunk box; the boxes
-    // (centre x, y, half extents x, y), refinement only
+    // (centre x, y, half extents x, y) and each chunk's first vertex and
+    // segment count, refinement only
     const uint32_t *choff;
     const float4 *chbox;
+    const uint2 *chseg;
     // the same for chunks of kIxChunk segments, for the intersection's chunk
     // skip (the refinement's arrays when C == kIxChunk; null: no skip)
     const uint32_t *ixoff;
@@ -44,8 +46,8 @@ struct DevSet {
 
 // The refinement walks a target edge sequence in chunks of C steps (8, 16 or
 // 32; kRefChunkDefault until the autotuner or the caller picks another) and
-// screens kRefScreen chunk boxes per scalar load (the box array keeps
-// kRefScreen spare entries past its end).
+// screens kRefScreen chunk boxes per scalar load (the box and chunk arrays keep
+// kRefScreen spare entries past their end).
 constexpr uint32_t kRefChunkDefault = 16;
 // target segments per chunk of the intersection's collection screen
 constexpr uint32_t kIxChunk = 16;

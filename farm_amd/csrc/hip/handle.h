@@ -43,7 +43,7 @@ struct farm_handle_s {
     int64_t npolys = 0;
     farm::DevBuf fill;    // -w fill classes (when the set has them)
     int cc = FARM_CATEGORY_COUNT;
-    farm::DevBuf hdr, status, pixoff, seqs, x, y, xyd, choff, chcnt, chbox, voff, vnodes, pixedges, shape_ctr;
+    farm::DevBuf hdr, status, pixoff, seqs, x, y, xyd, choff, chcnt, chbox, chseg, voff, vnodes, pixedges, shape_ctr;
     // 16-segment chunk boxes for the intersection's chunk skip when the
     // refinement's boxes are of another size (built for set generation ix_gen)
     farm::DevBuf ixcnt, ixoff, ixbox;
@@ -76,6 +76,7 @@ struct farm_handle_s {
     // set's boxes are built for, and `tunings` holds the autotuner's choice
     // per shape bucket (farm_tuning_save / farm_tuning_load persist it)
     int tuned_tile = 4;
+    bool tile_chosen = false;  // the caller (or the autotuner) named the tile width
     int tuned_chunk = 16;
     int tuned_bpc = 8;
     uint32_t chunk = 16;
@@ -168,6 +169,7 @@ inline DevSet devset(farm_handle h) {
     S.cc = h->cc;
     S.choff = P<uint32_t>(h->choff);
     S.chbox = P<float4>(h->chbox);
+    S.chseg = P<uint2>(h->chseg);
     if (h->chunk == kIxChunk) {
         S.ixoff = S.choff;
         S.ixbox = S.chbox;

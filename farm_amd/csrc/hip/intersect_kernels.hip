@@ -20,7 +20,8 @@ namespace farm {
 // Raster filter: one lane per candidate pair (grid-stride over the window).
 // pass 0: count BORDER x BORDER pixel pairs, decide IN hits (and the
 //         reference -a heuristic when approx != 0); the 64-bit total of the
-//         pixel pairs goes to ctr[kCtrPixPairs]
+//         pixel pairs goes to the shards of kCtrPixPairs (the scan's second
+//         kernel folds them into ctr)
 // pass 1: emit the pixel pairs at the offsets of an exclusive scan; it does
 //         nothing when that total exceeds cap_pp (the buffer's capacity: the
 //         host grows it or fails the call, and no offset has wrapped).
@@ -36,7 +37,8 @@ __global__ __launch_bounds__(256) void k_filter(DevSet S, const uint32_t *__rest
                                                  const uint8_t *__restrict__ skip, uint32_t *__restrict__ npp,
                                                  const uint32_t *__restrict__ pp_off, PixPair *__restrict__ pps,
                                                  uint64_t cap_pp, uint32_t *__restrict__ result,
-                                                 unsigned long long *__restrict__ ctr) {
+                                                 const unsigned long long *__restrict__ ctr,
+                                                 unsigned long long *__restrict__ shards) {
     if (pass == 1 && ctr[kCtrPixPairs] > cap_pp) return;
     const uint64_t n = desc->n;
     const uint32_t *pa_ids = pa_all + desc->begin;
@@ -125,9 +127,10 @@ __global__ __launch_bounds__(256) void k_filter(DevSet S, const uint32_t *__rest
             bb += __shfl_xor(bb, o);
         }
         if ((threadIdx.x & 63) == 0) {
-            if (bytes) atomicAdd(&ctr[kCtrFilterBytes], bytes);
-            if (inhit) atomicAdd(&ctr[kCtrInHits], inhit);
-            if (bb) atomicAdd(&ctr[kCtrPixPairs], bb);
+            unsigned long long *sh = ctr_shard(shards, blockIdx.x * 4u + (threadIdx.x >> 6));
+            if (bytes) atomicAdd(&sh[kCtrFilterBytes], bytes);
+            if (inhit) atomicAdd(&sh[kCtrInHits], inhit);
+            if (bb) atomicAdd(&sh[kCtrPixPairs], bb);
         }
     }
 }
@@ -165,10 +168,17 @@ __global__ __launch_bounds__(256) void k_scan_sums(const uint32_t *__restrict__ 
     if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// one block of kScanParts lanes
+// one block of kScanParts lanes; it also folds the shards of counter `slot`,
+// whose total the kernels after the scan read
 __global__ __launch_bounds__(kScanParts) void k_scan_parts(uint32_t *__restrict__ part,
                                                             const unsigned long long *__restrict__ nsrc,
-                                                            uint64_t cap, uint32_t *__restrict__ out) {
+                                                            uint64_t cap, uint32_t *__restrict__ out,
+                                                            unsigned long long *__restrict__ ctr,
+                                                            unsigned long long *__restrict__ shards, int slot) {
+    if (threadIdx.x < 64) {
+        const unsigned long long v = fold_shards(shards, slot, threadIdx.x, true);
+        if (threadIdx.x == 0) ctr[slot] = v;
+    }
     __shared__ uint32_t wsum[kScanParts / 64];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const uint32_t v = part[t];
@@ -223,9 +233,12 @@ __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t *__restrict__
     }
 }
 
-__global__ void k_set_desc(IsxDesc *d, unsigned long long begin, unsigned long long n, uint8_t *out,
-                           uint32_t *pair_tests) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
+// the call's window, and its counters cleared
+__global__ __launch_bounds__(256) void k_set_desc(IsxDesc *d, unsigned long long begin, unsigned long long n,
+                                                  uint8_t *out, uint32_t *pair_tests, uint32_t *__restrict__ clear) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < kIsxClear) clear[i] = 0;
+    if (i == 0) {
         d->begin = begin;
         d->n = n;
         d->out = out;
@@ -292,32 +305,41 @@ __global__ void k_bucket_scan(uint32_t *__restrict__ hist, uint32_t *__restrict_
 __global__ __launch_bounds__(256) void k_bucket_scatter(const uint8_t *__restrict__ bucket,
                                                          const unsigned long long *__restrict__ ctr, uint64_t cap_pp,
                                                          uint32_t *__restrict__ cursor, uint32_t *__restrict__ order) {
+    constexpr int kPer = 8;  // items per lane and round: a global atomic per bucket serves 2,048 items
     __shared__ uint32_t cnt[kBuckets], base[kBuckets];
     const uint64_t n = bounded_count(&ctr[kCtrPixPairs], cap_pp);
-    for (uint64_t b0 = (uint64_t)blockIdx.x * blockDim.x; b0 < n; b0 += (uint64_t)gridDim.x * blockDim.x) {
+    for (uint64_t b0 = (uint64_t)blockIdx.x * 256 * kPer; b0 < n; b0 += (uint64_t)gridDim.x * 256 * kPer) {
         for (int j = threadIdx.x; j < kBuckets; j += blockDim.x) cnt[j] = 0;
         __syncthreads();
-        const uint64_t i = b0 + threadIdx.x;
-        int b = 0;
-        uint32_t local = 0;
-        if (i < n) {
-            b = bucket[i];
-            local = atomicAdd(&cnt[b], 1u);
+        int b[kPer];
+        uint32_t local[kPer];
+#pragma unroll
+        for (int q = 0; q < kPer; q++) {
+            const uint64_t i = b0 + (uint64_t)q * 256 + threadIdx.x;
+            b[q] = i < n ? bucket[i] : 0;
         }
+#pragma unroll
+        for (int q = 0; q < kPer; q++)
+            if (b0 + (uint64_t)q * 256 + threadIdx.x < n) local[q] = atomicAdd(&cnt[b[q]], 1u);
         __syncthreads();
         for (int j = threadIdx.x; j < kBuckets; j += blockDim.x)
             if (cnt[j]) base[j] = atomicAdd(&cursor[j], cnt[j]);
         __syncthreads();
-        if (i < n) order[base[b] + local] = (uint32_t)i;
+#pragma unroll
+        for (int q = 0; q < kPer; q++) {
+            const uint64_t i = b0 + (uint64_t)q * 256 + threadIdx.x;
+            if (i < n) order[base[b[q]] + local[q]] = (uint32_t)i;
+        }
         __syncthreads();
     }
 }
 
 // tiles per ordered pixel pair (written at position i, scanned afterwards);
-// the 64-bit total goes to ctr[kCtrTiles]
+// the 64-bit total goes to the shards of kCtrTiles
 template <int E>
 __global__ __launch_bounds__(256) void k_tiles(const PixPair *__restrict__ pps, const uint32_t *__restrict__ order,
-                                                unsigned long long *__restrict__ ctr, uint64_t cap_pp,
+                                                const unsigned long long *__restrict__ ctr,
+                                                unsigned long long *__restrict__ shards, uint64_t cap_pp,
                                                 uint32_t *__restrict__ tiles) {
     const uint64_t n = bounded_count(&ctr[kCtrPixPairs], cap_pp);
     unsigned long long t = 0;
@@ -329,7 +351,8 @@ __global__ __launch_bounds__(256) void k_tiles(const PixPair *__restrict__ pps, 
         t += ti;
     }
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
-    if ((threadIdx.x & 63) == 0 && t) atomicAdd(&ctr[kCtrTiles], t);
+    if ((threadIdx.x & 63) == 0 && t)
+        atomicAdd(&ctr_shard(shards, blockIdx.x * 4u + (threadIdx.x >> 6))[kCtrTiles], t);
 }
 
 // The descriptor of every tile (its ordered pixel pair, the tile within it,
@@ -356,12 +379,14 @@ __global__ __launch_bounds__(256) void k_tile_map(DevSet S, const uint32_t *__re
         d.pair = P.pair;
         d.a_s0 = A.seq_start + S.pixoff[A.pixoff_start + P.pa];
         d.a_s1 = A.seq_start + S.pixoff[A.pixoff_start + P.pa + 1];
-        d.b_s0 = B.seq_start + S.pixoff[B.pixoff_start + P.pb];
-        d.b_s1 = B.seq_start + S.pixoff[B.pixoff_start + P.pb + 1];
+        const uint32_t b_s0 = B.seq_start + S.pixoff[B.pixoff_start + P.pb];
+        const uint32_t b_s1 = B.seq_start + S.pixoff[B.pixoff_start + P.pb + 1];
+        d.b_c0 = S.choff[b_s0];
+        d.b_c1 = S.choff[b_s1];
         d.a_vert = A.vert_start;
         d.b_vert = B.vert_start;
         // the target pixel's sequences once: offsets, sequence entries, vertices
-        const uint32_t nb = d.b_s1 - d.b_s0;
+        const uint32_t nb = b_s1 - b_s0;
         d.rbytes = 16 + 8u * nb + 8u * (S.pixedges[B.pix_start + P.pb] + nb);
         d.pad[0] = d.pad[1] = d.pad[2] = 0;
         for (uint32_t t = t0; t < t1; t++) {
@@ -372,11 +397,15 @@ __global__ __launch_bounds__(256) void k_tile_map(DevSet S, const uint32_t *__re
 }
 
 // ------------------------------------------------------------------------
-// Persistent refinement.  Each wave takes the next tile from a global
-// cursor.  A tile is 64 lanes x W consecutive edge slots of one source
+// Persistent refinement over the tiles of the window.  A tile is 64 lanes x W consecutive edge slots of one source
 // pixel's sequences (consecutive lanes share one vertex), refined against
 // the edge sequences of one target pixel, walked in chunks of C segments
-// (C = 8, 16 or 32, chosen per call; the autotuner picks it).
+// (C = 8, 16 or 32, chosen per call; the autotuner picks it).  The chunks of
+// all the pixel's sequences are one consecutive range of the box and chunk
+// arrays, so kRefScreen of them are screened per round whatever sequences
+// they belong to: at 10 vertices per pixel a pixel of a jagged ring holds 8
+// sequences of 3 edges, and walking them one by one (a dependent chain of
+// sequence, chunk offset and box loads each) took most of the kernel.
 // Per chunk every lane first tests its W edges against the chunk's box (an
 // exact prune: no edge whose line keeps the whole box at a safe distance can
 // meet a segment of the chunk under the reference predicate); the (lane,
@@ -406,7 +435,8 @@ __global__ __launch_bounds__(256) void k_chunk_count(DevSet S, int64_t npolys, u
 }
 
 __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uint32_t C,
-                                                   const uint32_t *__restrict__ choff, float4 *__restrict__ box) {
+                                                   const uint32_t *__restrict__ choff, float4 *__restrict__ box,
+                                                   uint2 *__restrict__ seg) {
     const int64_t p = blockIdx.x;
     if (p >= npolys) return;
     const farm_raster_hdr H = S.hdr[p];
@@ -437,6 +467,7 @@ __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uin
             const float big = 0x1p40f;
             if (!(open && fabsf(cx) + hx < big && fabsf(cy) + hy < big)) hx = hy = INFINITY;
             box[o] = make_float4(cx, cy, hx, hy);
+            if (seg) seg[o] = make_uint2(sq.x + base - 1, n);
         }
     }
 }
@@ -444,6 +475,7 @@ __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uin
 // Chunk boxes read through the constant address space: they do not change
 // during a launch, and uniform addresses then become scalar loads.
 typedef __attribute__((address_space(4))) const float cfloat;
+typedef __attribute__((address_space(4))) const uint32_t cuint;
 
 constexpr uint32_t kRefQueue = 512;  // queued items per wave: a power of 2 above 63 + 64 kRefScreen
 
@@ -453,8 +485,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                                  const IsxDesc *__restrict__ desc,
                                                  const TileDesc *__restrict__ tile_map, uint64_t cap_pp,
                                                  uint64_t cap_tiles, uint32_t *__restrict__ cursor,
-                                                 uint32_t *__restrict__ result, unsigned long long *__restrict__ ctr,
-                                                 int prune) {
+                                                 uint32_t *__restrict__ result,
+                                                 const unsigned long long *__restrict__ ctr,
+                                                 unsigned long long *__restrict__ shards, int prune) {
     // the tile total, unless a buffer of an earlier phase overflowed (the
     // host then grows the workspace and repeats the call, or fails it)
     if (ctr[kCtrPixPairs] > cap_pp || ctr[kCtrTiles] > cap_tiles) return;
@@ -471,34 +504,74 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     float(*src)[2 * (W + 1)] = s_src[wv];
     uint32_t *sev = s_ev[wv];
     uint2 *ring = s_ring[wv];
-    // work counters: per tile in 32-bit lane registers, summed over the wave
-    // at the end of the tile into this wave's 64-bit totals in LDS (64-bit
-    // lane totals live across the whole loop and push the kernel past its
-    // register budget)
-    __shared__ unsigned long long s_acc[4][3];  // tests, refine bytes, pruned tests
-    if (lane < 3) s_acc[wv][lane] = 0;
-    unsigned long long items = 0;
+    // work counters: per tile in 32-bit lane registers, added at its end to
+    // the lane's own 64-bit totals in LDS (64-bit lane totals in registers
+    // push the kernel past its register budget; summing them over the wave
+    // per tile took 36 shuffles); the refine bytes are wave-uniform
+    __shared__ unsigned long long s_acc[4][2][64];  // tests, pruned tests
+    s_acc[wv][0][lane] = s_acc[wv][1][lane] = 0;
+    unsigned long long items = 0, rbytes = 0;
+    // A wave takes `grab` consecutive tiles at a time, whose pairs' flags are
+    // looked up together, one per lane (on jagged small polygons 70 % of the
+    // tiles belong to pairs already decided; a descriptor and a flag load for
+    // each, one tile after the other, was most of their time).  Grab k of
+    // cursor c covers tiles (k * kCtrShards + c) * grab onwards, so every
+    // cursor runs through the cost order.  A wave stays with its own cursor
+    // until that has run out, then looks at all of them (one load) and moves
+    // on to the next that has not.  One cursor for all waves took 0.6 ms to
+    // hand out the 26,000 tiles of a 4,000-pair call; handing tiles out by
+    // position alone left waves idle (a call of 1.3e6 tiles of uneven cost
+    // took 17.5 ms instead of 13.9).
+    const uint32_t nwaves = gridDim.x * 4u, wid = blockIdx.x * 4u + (uint32_t)wv;
+    const uint32_t grab = min(max(total / (nwaves * 16u), 1u), 16u);
+    uint32_t home = wid & (kCtrShards - 1);
+    uint32_t tbase = 0;
+    unsigned long long live = 0;  // the batch's tiles still to run
     for (;;) {
-        uint32_t tests = 0, rbytes = 0, pruned = 0;
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(cursor, 1u);
-        t = __builtin_amdgcn_readfirstlane(__shfl(t, 0));
-        if (t >= total) break;
+        if (!live) {
+            // (an opaque copy of the lane: the addresses below are computed
+            // here, not kept in registers across the tiles)
+            uint32_t ln = (uint32_t)lane;
+            asm volatile("" : "+v"(ln));
+            uint32_t c = 0;
+            if (ln == 0) c = atomicAdd(&cursor[home * kCursorStride], 1u);
+            c = __builtin_amdgcn_readfirstlane(c);
+            const uint64_t b = ((uint64_t)c * kCtrShards + home) * grab;
+            if (b >= total) {
+                const uint32_t at = __hip_atomic_load(&cursor[ln * kCursorStride], __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned long long left =
+                    __ballot(((uint64_t)at * kCtrShards + ln) * grab < total);
+                if (!left) break;  // every cursor has run out
+                // the first cursor after home with tiles left
+                const unsigned long long after = home < 63u ? left >> (home + 1u) << (home + 1u) : 0ull;
+                home = (uint32_t)__ffsll(after ? after : left) - 1u;
+                continue;
+            }
+            tbase = (uint32_t)b;
+            bool open = false;
+            if (ln < grab && tbase + (uint64_t)ln < total)
+                open = !__hip_atomic_load(&result[tile_map[tbase + ln].pair], __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+            live = __ballot(open);
+            continue;
+        }
+        const uint32_t t = tbase + (uint32_t)__ffsll(live) - 1u;
+        live &= live - 1;
+        uint32_t tests = 0, pruned = 0;
         // the tile's descriptor (one uniform load), then its pair's flag
+        // again (an earlier tile of the grab may have decided it)
         const TileDesc td = tile_map[t];
-        const uint32_t pair = __builtin_amdgcn_readfirstlane(td.pair);
-        const uint32_t tile = __builtin_amdgcn_readfirstlane(td.tile);
+        const uint32_t pair = uni(td.pair), tile = uni(td.tile);
         if (__hip_atomic_load(&result[pair], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) continue;
         items++;
         const uint2 *sqa = S.seqs;  // absolute sequence indices
-        const uint2 *sqb = S.seqs;
-        const float *ax_ = S.x + __builtin_amdgcn_readfirstlane(td.a_vert);
-        const float *ay_ = S.y + __builtin_amdgcn_readfirstlane(td.a_vert);
-        const float4 *bq_ = S.xyd + __builtin_amdgcn_readfirstlane(td.b_vert);
-        const uint32_t *bchoff = S.choff;
-        const uint32_t a_s0 = __builtin_amdgcn_readfirstlane(td.a_s0), a_s1 = __builtin_amdgcn_readfirstlane(td.a_s1);
-        const uint32_t b_s0 = __builtin_amdgcn_readfirstlane(td.b_s0);
-        const uint32_t b_s1 = __builtin_amdgcn_readfirstlane(td.b_s1);
+        const uint32_t a_s0 = uni(td.a_s0), a_s1 = uni(td.a_s1);
+        const uint32_t b_c0 = uni(td.b_c0), b_c1 = uni(td.b_c1);
+        const float *ax_ = S.x + uni(td.a_vert);
+        const float *ay_ = S.y + uni(td.a_vert);
+        const float4 *bq_ = S.xyd + uni(td.b_vert);
+        const uint32_t td_rbytes = uni(td.rbytes);
         // the tile's body, invoked once below (as a lambda it is allocated
         // to fewer registers than as a plain block: 128 against 155 VGPRs at
         // W = 8, four waves per SIMD instead of three)
@@ -703,15 +776,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     stop = true;
             };
 
-            for (uint32_t j = b_s0; j < b_s1 && !stop; j++) {
-                const uint2 sq = sqb[j];
-                const uint32_t v0 = __builtin_amdgcn_readfirstlane(sq.x);
-                const uint32_t L = __builtin_amdgcn_readfirstlane(sq.y);
-                const cfloat *cbox = (const cfloat *)(S.chbox + __builtin_amdgcn_readfirstlane(bchoff[j]));
-                const uint32_t nch = (L + C - 1) / C;
+            {
+                const cfloat *cbox = (const cfloat *)(S.chbox + b_c0);
+                const cuint *cseg = (const cuint *)(S.chseg + b_c0);
+                const uint32_t nch = b_c1 - b_c0;
                 for (uint32_t g = 0; g < nch && !stop; g += kRefScreen) {
                     // Exact prune of this lane's edges against kRefScreen chunks
-                    // (their boxes are scalar loads; boxes past the sequence's
+                    // (their boxes are scalar loads; boxes past the pixel's
                     // last chunk are read, the array keeps spare entries, but not
                     // used).  q >= Q, the L1 reach from any vertex of the lane's
                     // edges to the chunk box, is taken from the box of those
@@ -736,10 +807,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     // over.  (A chunk with a segment of length 0 has an
                     // infinite box and is never pruned.)
                     // this lane's slots again, from LDS (not kept in registers
-                    // across the evaluation of queued items)
+                    // across the evaluation of queued items: the lane's index
+                    // is made opaque, or the loads would move out of the loop)
+                    uint32_t sln = (uint32_t)lane;
+                    asm volatile("" : "+v"(sln));
                     float sbx[E], sby[E], scc[E];
                     float lxl, lxh, lyl, lyh;  // box of the lane's slot vertices
-                    const float ox = src[lane][0], oy = src[lane][E + 1];
+                    const float ox = src[sln][0], oy = src[sln][E + 1];
                     {
                         float nx = ox, ny = oy;
                         lxl = lxh = nx;
@@ -747,8 +821,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 #pragma unroll
                         for (int e = 0; e < E; e++) {
                             const float ax = nx, ay = ny;
-                            nx = src[lane][e + 1];
-                            ny = src[lane][E + 2 + e];
+                            nx = src[sln][e + 1];
+                            ny = src[sln][E + 2 + e];
                             lxl = fminf(lxl, nx);
                             lxh = fmaxf(lxh, nx);
                             lyl = fminf(lyl, ny);
@@ -799,7 +873,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     for (int i = 0; i < (int)kRefScreen; i++) {
                         const uint32_t c = g + i;
                         if (c >= nch) break;
-                        const uint32_t nstep = min((uint32_t)C, L - c * C);
+                        const uint32_t v0 = cseg[2 * c], nstep = cseg[2 * c + 1];
                         scr_steps += nstep;
                         const unsigned long long bm = __ballot(need[i]);
                         if (bm) {
@@ -808,7 +882,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                 (uint32_t)(bm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u));
                             if (need[i]) {
                                 ring[(qhead + qn + below) & (kRefQueue - 1)] =
-                                    make_uint2(v0 + c * C, (uint32_t)lane | (nstep << 8));
+                                    make_uint2(v0, (uint32_t)lane | (nstep << 8));
                                 queued_steps += nstep;
                             }
                             qn += (uint32_t)__popcll(bm);
@@ -833,34 +907,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 
             // algorithmic refine bytes of this tile: its source vertices plus
             // the target pixel's sequences once
-            if (lane == 0) rbytes += __builtin_amdgcn_readfirstlane(td.rbytes);
-            rbytes += (uint32_t)nvalid * 8u;
+            uint32_t edges = 0;
+#pragma unroll
+            for (int e = 0; e < E; e++) edges += (uint32_t)__popcll(__ballot((evb >> e) & 1u));
+            rbytes += td_rbytes + edges * 8u;
             // tests of this lane's edges the prune skipped: every screened step
             // that was not queued
             pruned += (uint32_t)nvalid * (scr_steps - queued_steps);
         };
         run(std::integral_constant<int, W>());
-        // the tile's totals (a tile holds at most 512 edges against one target
-        // pixel's: its sums stay far below 2^64 and each lane's below 2^32)
-        unsigned long long t64 = tests, b64 = rbytes, p64 = pruned;
-        for (int o = 32; o > 0; o >>= 1) {
-            t64 += __shfl_xor(t64, o);
-            b64 += __shfl_xor(b64, o);
-            p64 += __shfl_xor(p64, o);
-        }
-        if (lane == 0) {
-            s_acc[wv][0] += t64;
-            s_acc[wv][1] += b64;
-            s_acc[wv][2] += p64;
+        s_acc[wv][0][lane] += tests;
+        s_acc[wv][1][lane] += pruned;
+        if (pair_tests) {
             // executed tests of this tile, for the cost labels
-            if (pair_tests) atomicAdd(&pair_tests[pair], (uint32_t)min(t64, 0xffffffffull));
+            unsigned long long t64 = tests;
+            for (int o = 32; o > 0; o >>= 1) t64 += __shfl_xor(t64, o);
+            if (lane == 0) atomicAdd(&pair_tests[pair], (uint32_t)min(t64, 0xffffffffull));
         }
     }
-    if (lane == 0) {
-        atomicAdd(&ctr[kCtrTests], s_acc[wv][0]);
-        atomicAdd(&ctr[kCtrItems], items);
-        atomicAdd(&ctr[kCtrRefineBytes], s_acc[wv][1]);
-        atomicAdd(&ctr[kCtrPruned], s_acc[wv][2]);
+    unsigned long long t64 = s_acc[wv][0][lane], p64 = s_acc[wv][1][lane];
+    for (int o = 32; o > 0; o >>= 1) {
+        t64 += __shfl_xor(t64, o);
+        p64 += __shfl_xor(p64, o);
+    }
+    if (lane == 0 && items) {
+        unsigned long long *sh = ctr_shard(shards, wid);
+        atomicAdd(&sh[kCtrTests], t64);
+        atomicAdd(&sh[kCtrItems], items);
+        atomicAdd(&sh[kCtrRefineBytes], rbytes);
+        atomicAdd(&sh[kCtrPruned], p64);
     }
 }
 
@@ -1053,26 +1128,35 @@ __global__ __launch_bounds__(256) void k_pixedges(DevSet S, int64_t npolys, uint
 
 __global__ __launch_bounds__(256) void k_finalize(const uint32_t *__restrict__ result,
                                                    const IsxDesc *__restrict__ desc,
-                                                   unsigned long long *__restrict__ ctr) {
+                                                   unsigned long long *__restrict__ ctr,
+                                                   unsigned long long *__restrict__ shards) {
+    __shared__ uint32_t lds[4];
     const uint64_t n = desc->n;
     uint8_t *out = desc->out;
-    unsigned long long f = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        // what the earlier kernels counted
+        for (int s = 0; s < kCtrSlots; s++) {
+            const unsigned long long v = fold_shards(shards, s, threadIdx.x, false);
+            if (threadIdx.x == 0 && v) atomicAdd(&ctr[s], v);
+        }
+    }
+    uint32_t f = 0;  // a block's part of at most 2^31 pairs
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t r = result[i] ? 1u : 0u;
         if (out) out[i] = (uint8_t)r;
         f += r;
     }
-    for (int o = 32; o > 0; o >>= 1) f += __shfl_xor(f, o);
-    if ((threadIdx.x & 63) == 0 && f) atomicAdd(&ctr[kCtrFound], f);
+    f = block_sum256(f, lds);
+    if (threadIdx.x == 0 && f) atomicAdd(&ctr[kCtrFound], (unsigned long long)f);
 }
 
 #define FARM_TILES_INST(EE)                                                                                    \
-    template __global__ void k_tiles<EE>(const PixPair *, const uint32_t *, unsigned long long *, uint64_t,      \
-                                         uint32_t *);
+    template __global__ void k_tiles<EE>(const PixPair *, const uint32_t *, const unsigned long long *,          \
+                                         unsigned long long *, uint64_t, uint32_t *);
 #define FARM_REFINE_INST(EE, CC)                                                                               \
     template __global__ void k_refine<EE, CC>(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *,      \
                                               const TileDesc *, uint64_t, uint64_t, uint32_t *, uint32_t *,     \
-                                              unsigned long long *, int);
+                                              const unsigned long long *, unsigned long long *, int);
 FARM_TILES_INST(1)
 FARM_TILES_INST(2)
 FARM_TILES_INST(4)

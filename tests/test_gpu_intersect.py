@@ -180,3 +180,36 @@ def test_category_bits(device, bits):
         assert not np.array_equal(heur, heur16) or bits == 4  # the category count matters to -a
     finally:
         w.both.set_categories(4)
+
+
+def _comb(n, up, shift, tip=None):
+    """A comb of n long teeth (from below, or from above), 1,200 high; tooth
+    n / 2 reaches to y = tip."""
+    pts = [(0.0, -60.0 if up else 1260.0), (4.0 * n, -60.0 if up else 1260.0)]
+    y0, y1 = (0.0, 1080.0) if up else (1200.0, 120.0)
+    for i in range(n - 1, -1, -1):
+        x = 4.0 * i + shift
+        yt = tip if (tip is not None and i == n // 2) else y1
+        pts += [(x + 1.0, y0), (x + 0.8, yt), (x + 0.2, yt), (x, y0)]
+    return np.array(pts if up else pts[1::-1] + pts[:1:-1])
+
+
+@pytest.mark.parametrize("npairs", [1, 7, 64, 65, 1000])
+@pytest.mark.parametrize("tile", [1, 8])
+def test_window_sizes(device, npairs, tile):
+    # from fewer tiles than cursors to several tiles per wave, and pixels of
+    # more than 64 edge sequences of one edge (their chunks screened across
+    # sequences): interlocked combs, apart or with one tooth through a spine
+    combs = Workload(rings_from_list([_comb(300, True, 0.0)]),
+                     rings_from_list([_comb(300, False, 2.0), _comb(300, False, 2.0, -80.0)]), vpr=48)
+    assert max(np.diff(combs.both.layout()["pixoff"].astype(np.int64))) > 64
+    assert combs.oracle(0)[0].tolist() == [0, 1]
+    for w in (star_pairs(31, n=600), combs):
+        want, _ = w.oracle(0)
+        w.upload(device)
+        n = len(w.pa)
+        for b in range(0, n, max(npairs, n // 3)):
+            e = min(b + npairs, n)
+            print(f"  window {b}..{e} of {n} tile={tile}", flush=True)
+            got = device.intersect(b, e, mode=capi.MODE_EXACT_BATCHED, tile_a=tile)
+            assert np.array_equal(got.bits, (want[b:e] == 1).astype(np.uint8))
