@@ -86,7 +86,8 @@ struct farm_handle_s {
     bool mlp_ready = false;
     farm::DevBuf mlp_w, mlp_m, mlp_v, mlp_g;  // f32 master params, Adam moments, grads
     farm::DevBuf mlp_norm;                    // per feature: mean, 1/std (2 * kNFeat)
-    farm::DevBuf mlp_x, mlp_h1, mlp_h2, mlp_z3, mlp_d3, mlp_dh2, mlp_dh1, mlp_y, mlp_c, mlp_loss;
+    farm::DevBuf mlp_wb;                      // bf16 copies of the weights
+    farm::DevBuf mlp_x, mlp_z3, mlp_y, mlp_c, mlp_loss, mlp_part, mlp_lpart;
     farm::DevBuf feat, decided, pred;  // per-pair features / decided flags / predictions
     farm::DevBuf skipbuf;              // pairs decided before the exact filter
     uint64_t adam_t = 0;

@@ -1,13 +1,13 @@
 // The learned part: pair features and an 80-128-128-2 MLP (intersect logit,
 // log refinement cost) trained and evaluated on the GPU.
 //
-// GEMMs run on MFMA (v_mfma_f32_16x16x16_bf16): operands are rounded to
-// bf16 when staged into LDS (round to nearest even), products accumulate in
-// fp32.  One generic kernel covers the forward products, the transposed
-// backward products and the batch reductions of the weight gradients
-// (split-K with atomic accumulation).  The reference has no learned
-// component; the features come from the same raster windows as the filter
-// (Ideal::intersect, Ideal.cpp:1329-1357).
+// The products run on MFMA (v_mfma_f32_16x16x16_bf16): operands are rounded
+// to bf16 when staged (round to nearest even), products accumulate in fp32.
+// Inference is one kernel (k_mlp_infer); a training step is two: k_mlp_grad
+// (forward, loss and every gradient of 32 rows at a time, the activations
+// never leaving LDS) and k_mlp_step (the sum of the workgroups' gradients and
+// Adam).  The reference has no learned component; the features come from the
+// same raster windows as the filter (Ideal::intersect, Ideal.cpp:1329-1357).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -111,80 +111,13 @@ __global__ __launch_bounds__(128) void k_features(DevSet S, const uint32_t *__re
     decided[k] = n_in ? 1 : (n_bb ? -1 : 0);
 }
 
-// x[i, :] = (x[i, :] - mean) * inv_std
-__global__ __launch_bounds__(256) void k_normalize(float *__restrict__ x, uint64_t n, const float *__restrict__ norm) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n * kNFeat) return;
-    const int c = (int)(i % kNFeat);
-    x[i] = (x[i] - norm[c]) * norm[kNFeat + c];
-}
-
-// ------------------------------------------------------------------------
-// C (M x N, row stride ldc) = op(A) op(B) [+ bias] [relu], or accumulated
-// atomically (split-K over blockIdx.z).  A(m, k) = A[m*sam + k*sak],
-// B(k, n) = B[k*sbk + n*sbn].  Block tile 64 x 64, 4 waves x (16 rows x 4
-// MFMA tiles of 16 x 16), K step 16.
-// MFMA 16x16x16 operand layout (lane l): A row l%16, k 4*(l/16)+j;
-// B col l%16, k 4*(l/16)+j; D row 4*(l/16)+j, col l%16.
-// ------------------------------------------------------------------------
-enum { GEMM_BIAS = 1, GEMM_RELU = 2, GEMM_ATOMIC = 4 };
-
-__global__ __launch_bounds__(256) void k_gemm(const float *__restrict__ A, int64_t sam, int64_t sak,
-                                               const float *__restrict__ B, int64_t sbk, int64_t sbn,
-                                               float *__restrict__ C, int64_t ldc, int M, int N, int K, int kchunk,
-                                               const float *__restrict__ bias, int flags) {
-    __shared__ short As[64][20];
-    __shared__ short Bs[16][68];
-    const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-    const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
-    f32x4 acc[4];
-    for (int i = 0; i < 4; i++) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kb; k0 < ke; k0 += 16) {
-        for (int i = 0; i < 4; i++) {
-            const int idx = t + 256 * i;
-            const int r = idx >> 4, c = idx & 15;
-            const int gm = m0 + r, gk = k0 + c;
-            As[r][c] = (gm < M && gk < ke) ? f2bf(A[(int64_t)gm * sam + (int64_t)gk * sak]) : (short)0;
-            const int rb = idx >> 6, cb = idx & 63;
-            const int bk = k0 + rb, bn = n0 + cb;
-            Bs[rb][cb] = (bk < ke && bn < N) ? f2bf(B[(int64_t)bk * sbk + (int64_t)bn * sbn]) : (short)0;
-        }
-        __syncthreads();
-        bf16x4 a;
-        const int ar = 16 * w + (l & 15), ak = 4 * (l >> 4);
-        for (int j = 0; j < 4; j++) a[j] = As[ar][ak + j];
-        for (int tt = 0; tt < 4; tt++) {
-            bf16x4 b;
-            for (int j = 0; j < 4; j++) b[j] = Bs[ak + j][16 * tt + (l & 15)];
-            acc[tt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[tt], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    for (int tt = 0; tt < 4; tt++) {
-        for (int j = 0; j < 4; j++) {
-            const int row = m0 + 16 * w + 4 * (l >> 4) + j;
-            const int col = n0 + 16 * tt + (l & 15);
-            if (row >= M || col >= N) continue;
-            float v = acc[tt][j];
-            float *dst = C + (int64_t)row * ldc + col;
-            if (flags & GEMM_ATOMIC) {
-                atomicAdd(dst, v);
-            } else {
-                if (flags & GEMM_BIAS) v += bias[col];
-                if (flags & GEMM_RELU) v = fmaxf(v, 0.f);
-                *dst = v;
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------------------------
 // Inference in one pass: normalisation and the three layers of 64 pairs at a
 // time, the weights staged in LDS once per workgroup, the activations never
-// leaving it.  The operands are rounded to bf16 exactly where k_gemm rounds
-// them and every output takes the same MFMA sequence over K (16 at a time,
-// ascending), so the logits equal the three-launch path's bit for bit.
+// leaving it.  norm may be null (rows that are normalised already).  Every
+// output takes one MFMA sequence over K (16 at a time, ascending).
+// MFMA 16x16x16 operand layout (lane l): A row l%16, k 4*(l/16)+j;
+// B col l%16, k 4*(l/16)+j; D row 4*(l/16)+j, col l%16.
 // Wave w owns rows 16w .. 16w + 15 of the tile.
 // ------------------------------------------------------------------------
 constexpr int kInferRows = 64;
@@ -247,7 +180,10 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float *__restrict__ fea
         for (int i = t; i < kInferRows * kNFeat; i += 256) {
             const int r = i / kNFeat, c = i % kNFeat;
             float v = 0.f;
-            if (r0 + r < n) v = (feat[(r0 + r) * kNFeat + c] - norm[c]) * norm[kNFeat + c];
+            if (r0 + r < n) {
+                v = feat[(r0 + r) * kNFeat + c];
+                if (norm) v = (v - norm[c]) * norm[kNFeat + c];
+            }
             sX[r][c] = f2bf(v);
         }
         __syncthreads();
@@ -277,66 +213,326 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float *__restrict__ fea
     }
 }
 
-// loss = mean(BCE-with-logits(z0, y)) + lambda * mean((z1 - c)^2), and dL/dz
-__global__ __launch_bounds__(256) void k_loss(const float *__restrict__ z, const float *__restrict__ y,
-                                               const float *__restrict__ c, int M, float lambda,
-                                               float *__restrict__ dz, float *__restrict__ loss) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    float L = 0.f;
-    if (i < M) {
-        const float z0 = z[2 * i], z1 = z[2 * i + 1];
-        const float s = 1.f / (1.f + expf(-z0));
-        dz[2 * i] = (s - y[i]) / M;
-        dz[2 * i + 1] = 2.f * lambda * (z1 - c[i]) / M;
-        L = (fmaxf(z0, 0.f) - z0 * y[i] + log1pf(expf(-fabsf(z0)))) / M + lambda * (z1 - c[i]) * (z1 - c[i]) / M;
+// ------------------------------------------------------------------------
+// Training.  loss = mean(BCE-with-logits(z0, y)) + lambda * mean((z1 - c)^2).
+//
+// k_mlp_grad: one workgroup takes kGradRows rows at a time through the
+// forward pass, the loss and the backward pass, and keeps its part of every
+// weight gradient in MFMA accumulators until its last tile.  Each activation
+// and each dL/dactivation is staged in LDS as bf16 twice: row-major (the A
+// operand of the next product) and transposed (an operand of a weight
+// gradient, whose inner dimension is the rows), padded so that the 8-byte
+// fragment reads of a wave fall two to a bank.  The weights come as bf16 from
+// L2, in the layout each product reads with one 8-byte load per fragment
+// (MlpPacked).  A step of 2,048 rows is bound by latency (64 workgroups, one
+// chain of seven dependent products); with a launch per product, bias and
+// ReLU (20 launches, two 64-row blocks of work per product, a host wait per
+// step) it took 560 us, 165 us of it in each of the two large weight
+// gradients; the two kernels of a step together take 27 us.
+// ------------------------------------------------------------------------
+constexpr int kGradRows = 32;
+constexpr int kTPad = kGradRows + 4;
+constexpr int kGradBlocks = 256;  // most workgroups of one step
+
+// bf16 copies of the weights: W1^T, W2^T, W2, W3^T (16 rows, 2 used), W3
+struct MlpPacked {
+    short w1t[kHidden * kNFeat];
+    short w2t[kHidden * kHidden];
+    short w2[kHidden * kHidden];
+    short w3t[16 * kHidden];
+    short w3[kHidden * kOut];
+};
+
+// parameter i's copies
+__device__ __forceinline__ void pack_param(MlpPacked *__restrict__ P, int i, float v) {
+    const short b = f2bf(v);
+    if (i < kOffB1) {
+        P->w1t[(i % kHidden) * kNFeat + i / kHidden] = b;
+    } else if (i >= kOffW2 && i < kOffB2) {
+        const int k = (i - kOffW2) / kHidden, n = (i - kOffW2) % kHidden;
+        P->w2t[n * kHidden + k] = b;
+        P->w2[k * kHidden + n] = b;
+    } else if (i >= kOffW3 && i < kOffB3) {
+        const int k = (i - kOffW3) / kOut, o = (i - kOffW3) % kOut;
+        P->w3t[o * kHidden + k] = b;
+        P->w3[k * kOut + o] = b;
     }
-    for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
-    if ((threadIdx.x & 63) == 0) atomicAdd(loss, L);
 }
 
-// d[i] *= (h[i] > 0)   (ReLU backward through the stored activation)
-__global__ __launch_bounds__(256) void k_relu_back(float *__restrict__ d, const float *__restrict__ h, uint64_t n) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !(h[i] > 0.f)) d[i] = 0.f;
-}
-
-// out[c] += sum_r d[r * N + c]
-__global__ __launch_bounds__(256) void k_colsum(const float *__restrict__ d, int M, int N, float *__restrict__ out) {
-    const int c = blockIdx.x;
-    float s = 0.f;
-    for (int r = threadIdx.x; r < M; r += blockDim.x) s += d[(int64_t)r * N + c];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    __shared__ float part[4];
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&out[c], part[0] + part[1] + part[2] + part[3]);
-}
-
-__global__ __launch_bounds__(256) void k_adam(float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m,
-                                               float *__restrict__ v, int n, float lr, float b1, float b2, float eps,
-                                               float c1, float c2) {
+__global__ __launch_bounds__(256) void k_mlp_pack(const float *__restrict__ W, MlpPacked *__restrict__ P) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
+    if (i < kNParams) pack_param(P, i, W[i]);
+    if (i < (16 - kOut) * kHidden) P->w3t[kOut * kHidden + i] = 0;
+}
+
+__device__ __forceinline__ bf16x4 frag(const short *p) { return *reinterpret_cast<const bf16x4 *>(p); }
+__device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+
+// One layer's product for this wave: both 16-row tiles x its two 16-column
+// tiles 2w, 2w + 1; A row-major in LDS (stride SA), B column-major in memory.
+template <int K, int SA>
+__device__ __forceinline__ void tile_product(const short *A, const short *__restrict__ B, int w, int l,
+                                             f32x4 (&acc)[2][2]) {
+    const int c = l & 15, q = 4 * (l >> 4);
+    bf16x4 b[2][K / 16];
+#pragma unroll
+    for (int n = 0; n < 2; n++)
+#pragma unroll
+        for (int k = 0; k < K / 16; k++) b[n][k] = frag(B + (16 * (2 * w + n) + c) * K + 16 * k + q);
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < K / 16; k++)
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const bf16x4 a = frag(A + (16 * m + c) * SA + 16 * k + q);
+#pragma unroll
+            for (int n = 0; n < 2; n++) acc[m][n] = mfma(a, b[n][k], acc[m][n]);
+        }
+}
+
+// rows: the rows' indices into X, y and c (null: rows 0 .. M - 1).  part:
+// kNParams gradients per workgroup; loss_part: one loss per workgroup.
+__global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ X, const uint32_t *__restrict__ rows,
+                                                   const float *__restrict__ y, const float *__restrict__ cst, int M,
+                                                   float lambda, const float *__restrict__ W,
+                                                   const MlpPacked *__restrict__ P, float *__restrict__ part,
+                                                   float *__restrict__ loss_part) {
+    constexpr int SX = kNFeat + 8, SH = kHidden + 8;
+    __shared__ __align__(16) short sX[kGradRows * SX], sXT[kNFeat * kTPad];
+    __shared__ __align__(16) short sH1[kGradRows * SH], sH1T[kHidden * kTPad];
+    __shared__ __align__(16) short sH2[kGradRows * SH], sH2T[kHidden * kTPad];
+    __shared__ __align__(16) short sD2[kGradRows * SH], sD2T[kHidden * kTPad];
+    __shared__ __align__(16) short sD1T[kHidden * kTPad];
+    __shared__ __align__(16) short sDz[kGradRows * 4], sDzT[16 * kTPad];
+    __shared__ uint32_t sRow[kGradRows];
+    __shared__ float sLoss[2], sB3[2][kOut];
+    const int t = threadIdx.x, w = t >> 6, l = t & 63, c = l & 15, q = 4 * (l >> 4);
+    for (int i = t; i < 16 * kTPad; i += 256) sDzT[i] = 0;
+    f32x4 g1[5][2], g2[2][8], g3[2];
+    float gb1[2] = {0.f, 0.f}, gb2[2] = {0.f, 0.f}, gb3 = 0.f, loss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 5; i++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) g1[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+#pragma unroll
+        for (int n = 0; n < 8; n++) g2[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+        g3[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const bf16x4 zero = {0, 0, 0, 0};
+    // this wave's tile of a layer's output: + bias, ReLU, staged both ways
+    auto put = [&](const f32x4 v, int m, int n, short *R, short *T) {
+        const int col = 16 * (2 * w + n) + c;
+        bf16x4 b;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            b[j] = f2bf(v[j]);
+            if (R) R[(16 * m + q + j) * SH + col] = b[j];
+        }
+        *reinterpret_cast<bf16x4 *>(T + col * kTPad + 16 * m + q) = b;
+    };
+    const int tiles = (M + kGradRows - 1) / kGradRows;
+    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const int r0 = tile * kGradRows;
+        __syncthreads();  // the previous tile's reads are done
+        if (t < kGradRows) sRow[t] = r0 + t < M ? (rows ? rows[r0 + t] : (uint32_t)(r0 + t)) : 0xffffffffu;
+        __syncthreads();
+        for (int i = t; i < kGradRows * (kNFeat / 4); i += 256) {
+            const int r = i / (kNFeat / 4), k = 4 * (i % (kNFeat / 4));
+            const uint32_t src = sRow[r];
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (src != 0xffffffffu) v = *reinterpret_cast<const float4 *>(X + (size_t)src * kNFeat + k);
+            const bf16x4 b = {f2bf(v.x), f2bf(v.y), f2bf(v.z), f2bf(v.w)};
+            *reinterpret_cast<bf16x4 *>(sX + r * SX + k) = b;
+#pragma unroll
+            for (int j = 0; j < 4; j++) sXT[(k + j) * kTPad + r] = b[j];
+        }
+        __syncthreads();
+        f32x4 h1[2][2], h2[2][2], d[2][2];
+        auto relu_layer = [&](f32x4(&h)[2][2], const float *bias, short *R, short *T) {
+#pragma unroll
+            for (int m = 0; m < 2; m++)
+#pragma unroll
+                for (int n = 0; n < 2; n++) {
+                    const float b = bias[16 * (2 * w + n) + c];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) h[m][n][j] = fmaxf(h[m][n][j] + b, 0.f);
+                    put(h[m][n], m, n, R, T);
+                }
+        };
+        tile_product<kNFeat, SX>(sX, P->w1t, w, l, h1);
+        relu_layer(h1, W + kOffB1, sH1, sH1T);
+        __syncthreads();
+        tile_product<kHidden, SH>(sH1, P->w2t, w, l, h2);
+        relu_layer(h2, W + kOffB2, sH2, sH2T);
+        __syncthreads();
+        if (w < 2) {
+            // logits of rows 16w ..: lane column 0 the logit, 1 the cost
+            f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < kHidden / 16; k++)
+                z = mfma(frag(sH2 + (16 * w + c) * SH + 16 * k + q), frag(P->w3t + c * kHidden + 16 * k + q), z);
+            bf16x4 dz = zero;
+            if (c < kOut) {
+                const float b = W[kOffB3 + c];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t src = sRow[16 * w + q + j];
+                    if (src == 0xffffffffu) continue;
+                    const float zj = z[j] + b;
+                    float g;
+                    if (c == 0) {
+                        const float yj = y[src];
+                        const float s = 1.f / (1.f + expf(-zj));
+                        g = (s - yj) / M;
+                        loss += (fmaxf(zj, 0.f) - zj * yj + log1pf(expf(-fabsf(zj)))) / M;
+                    } else {
+                        const float e = zj - cst[src];
+                        g = 2.f * lambda * e / M;
+                        loss += lambda * e * e / M;
+                    }
+                    gb3 += g;
+                    dz[j] = f2bf(g);
+                }
+                *reinterpret_cast<bf16x4 *>(sDzT + c * kTPad + 16 * w + q) = dz;
+            }
+            if (c < 4)
+#pragma unroll
+                for (int j = 0; j < 4; j++) sDz[(16 * w + q + j) * 4 + c] = dz[j];
+        }
+        __syncthreads();
+        // dL/dh2 = dz W3^T (two inner terms, the rest of the 16 zero), masked
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            bf16x4 b = zero;
+            if (q == 0) {
+                const short *p = P->w3 + (16 * (2 * w + n) + c) * kOut;
+                b[0] = p[0];
+                b[1] = p[1];
+            }
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                const bf16x4 a = q == 0 ? frag(sDz + (16 * m + c) * 4) : zero;
+                f32x4 v = mfma(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    v[j] = h2[m][n][j] > 0.f ? v[j] : 0.f;
+                    gb2[n] += v[j];
+                }
+                put(v, m, n, sD2, sD2T);
+            }
+        }
+        __syncthreads();
+        tile_product<kHidden, SH>(sD2, P->w2, w, l, d);
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    d[m][n][j] = h1[m][n][j] > 0.f ? d[m][n][j] : 0.f;
+                    gb1[n] += d[m][n][j];
+                }
+                put(d[m][n], m, n, nullptr, sD1T);
+            }
+        // weight gradients of layers 3 and 2 (rows are the inner dimension)
+#pragma unroll
+        for (int k = 0; k < kGradRows / 16; k++) {
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const int m = 2 * w + i;
+                g3[i] = mfma(frag(sH2T + (16 * m + c) * kTPad + 16 * k + q), frag(sDzT + c * kTPad + 16 * k + q),
+                             g3[i]);
+                const bf16x4 a = frag(sH1T + (16 * m + c) * kTPad + 16 * k + q);
+#pragma unroll
+                for (int n = 0; n < 8; n++)
+                    g2[i][n] = mfma(a, frag(sD2T + (16 * n + c) * kTPad + 16 * k + q), g2[i][n]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kGradRows / 16; k++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) {
+                const bf16x4 b = frag(sD1T + (16 * (2 * w + n) + c) * kTPad + 16 * k + q);
+#pragma unroll
+                for (int i = 0; i < 5; i++)
+                    g1[i][n] = mfma(frag(sXT + (16 * i + c) * kTPad + 16 * k + q), b, g1[i][n]);
+            }
+    }
+    float *G = part + (size_t)blockIdx.x * kNParams;
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+        const int col = 16 * (2 * w + n) + c;
+#pragma unroll
+        for (int i = 0; i < 5; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) G[kOffW1 + (16 * i + q + j) * kHidden + col] = g1[i][n][j];
+        float s1 = gb1[n], s2 = gb2[n];
+        s1 += __shfl_xor(s1, 16);
+        s1 += __shfl_xor(s1, 32);
+        s2 += __shfl_xor(s2, 16);
+        s2 += __shfl_xor(s2, 32);
+        if (q == 0) {
+            G[kOffB1 + col] = s1;
+            G[kOffB2 + col] = s2;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int row = 16 * (2 * w + i) + q + j;
+#pragma unroll
+            for (int n = 0; n < 8; n++) G[kOffW2 + row * kHidden + 16 * n + c] = g2[i][n][j];
+            if (c < kOut) G[kOffW3 + row * kOut + c] = g3[i][j];
+        }
+    // waves 0 and 1 hold the losses and the output bias gradients
+    if (w < 2) {
+        for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
+        if (l == 0) sLoss[w] = loss;
+    }
+    gb3 += __shfl_xor(gb3, 16);
+    gb3 += __shfl_xor(gb3, 32);
+    if (w < 2 && l < kOut) sB3[w][l] = gb3;
+    __syncthreads();
+    if (t < kOut) G[kOffB3 + t] = sB3[0][t] + sB3[1][t];
+    if (t == 0) loss_part[blockIdx.x] = sLoss[0] + sLoss[1];
+}
+
+// The step's gradients (the workgroups' parts, summed in order) into g when
+// given, and Adam on w and its bf16 copies when adam != 0; the loss to *loss.
+__global__ __launch_bounds__(256) void k_mlp_step(const float *__restrict__ part, const float *__restrict__ loss_part,
+                                                   int nblocks, float *__restrict__ g, float *__restrict__ loss,
+                                                   int adam, float *__restrict__ w, MlpPacked *__restrict__ P,
+                                                   float *__restrict__ m, float *__restrict__ v, float lr, float b1,
+                                                   float b2, float eps, float c1, float c2) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        float L = 0.f;
+        for (int k = threadIdx.x; k < nblocks; k += 64) L += loss_part[k];
+        for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
+        if (threadIdx.x == 0) *loss = L;
+    }
+    if (i >= kNParams) return;
+    float gi = 0.f;
+#pragma unroll 16
+    for (int k = 0; k < nblocks; k++) gi += part[(size_t)k * kNParams + i];
+    if (g) g[i] = gi;
+    if (!adam) return;
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-__global__ __launch_bounds__(256) void k_gather_rows(const float *__restrict__ src, const uint32_t *__restrict__ idx,
-                                                      int rows, int cols, float *__restrict__ dst) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)rows * cols) return;
-    const int r = (int)(i / cols), c = (int)(i % cols);
-    dst[i] = src[(int64_t)idx[r] * cols + c];
-}
-
-__global__ __launch_bounds__(256) void k_gather_vec(const float *__restrict__ src, const uint32_t *__restrict__ idx,
-                                                     int rows, float *__restrict__ dst) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < rows) dst[i] = src[idx[i]];
+    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    w[i] = wi;
+    pack_param(P, i, wi);
 }
 
 }  // namespace farm
@@ -345,86 +541,40 @@ using namespace farm;
 
 namespace {
 
-int gemm(farm_handle h, const float *A, int64_t sam, int64_t sak, const float *B, int64_t sbk, int64_t sbn, float *C,
-         int64_t ldc, int M, int N, int K, const float *bias, int flags, int ksplit = 1) {
-    if (M <= 0 || N <= 0 || K <= 0) return FARM_OK;
-    int kchunk = K;
-    if (ksplit > 1) kchunk = ((K + ksplit - 1) / ksplit + 15) / 16 * 16;
-    const int kz = (K + kchunk - 1) / kchunk;
-    dim3 grid((M + 63) / 64, (N + 63) / 64, kz);
-    hipLaunchKernelGGL(k_gemm, grid, dim3(256), 0, h->stream, A, sam, sak, B, sbk, sbn, C, ldc, M, N, K, kchunk, bias,
-                       flags);
+// Workgroups of a step of M rows, and the buffers of their gradients.
+int grad_blocks(int M) { return std::min((M + kGradRows - 1) / kGradRows, kGradBlocks); }
+
+int grad_buffers(farm_handle h, int M, uint64_t losses) {
+    int rc;
+    if ((rc = ensure(h, h->mlp_part, 4ull * kNParams * grad_blocks(M)))) return rc;
+    if ((rc = ensure(h, h->mlp_lpart, 4ull * kGradBlocks))) return rc;
+    return ensure(h, h->mlp_loss, 4ull * losses);
+}
+
+// loss (to mlp_loss[slot]) and gradients of M rows of X, y, c (device; rows:
+// their indices, or null), then Adam (step adam_t) or the gradients to mlp_g
+int mlp_step(farm_handle h, const float *X, const uint32_t *rows, const float *y, const float *c, int M, float lambda,
+             uint64_t slot, bool adam, float lr) {
+    const int nb = grad_blocks(M);
+    hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), 0, h->stream, X, rows, y, c, M, lambda,
+                       (const float *)P<float>(h->mlp_w), (const MlpPacked *)P<MlpPacked>(h->mlp_wb),
+                       P<float>(h->mlp_part), P<float>(h->mlp_lpart));
+    HIPCHK(h, hipGetLastError());
+    const float c1 = 1.f - powf(0.9f, (float)h->adam_t), c2 = 1.f - powf(0.999f, (float)h->adam_t);
+    hipLaunchKernelGGL(k_mlp_step, dim3(blocks_for(kNParams)), dim3(256), 0, h->stream,
+                       (const float *)P<float>(h->mlp_part), (const float *)P<float>(h->mlp_lpart), nb,
+                       adam ? (float *)nullptr : P<float>(h->mlp_g), P<float>(h->mlp_loss) + slot, adam ? 1 : 0,
+                       P<float>(h->mlp_w), P<MlpPacked>(h->mlp_wb), P<float>(h->mlp_m), P<float>(h->mlp_v), lr, 0.9f,
+                       0.999f, 1e-8f, c1, c2);
     HIPCHK(h, hipGetLastError());
     return FARM_OK;
 }
 
-int mlp_buffers(farm_handle h, int M) {
-    int rc;
-    if ((rc = ensure(h, h->mlp_x, 4ull * M * kNFeat))) return rc;
-    if ((rc = ensure(h, h->mlp_h1, 4ull * M * kHidden))) return rc;
-    if ((rc = ensure(h, h->mlp_h2, 4ull * M * kHidden))) return rc;
-    if ((rc = ensure(h, h->mlp_z3, 4ull * M * kOut))) return rc;
-    if ((rc = ensure(h, h->mlp_d3, 4ull * M * kOut))) return rc;
-    if ((rc = ensure(h, h->mlp_dh2, 4ull * M * kHidden))) return rc;
-    if ((rc = ensure(h, h->mlp_dh1, 4ull * M * kHidden))) return rc;
-    if ((rc = ensure(h, h->mlp_y, 4ull * M))) return rc;
-    if ((rc = ensure(h, h->mlp_c, 4ull * M))) return rc;
-    if ((rc = ensure(h, h->mlp_loss, 64))) return rc;
-    return FARM_OK;
-}
-
-// forward of M rows of X (device, normalised): h1, h2, z3 in the handle
-int mlp_forward_dev(farm_handle h, const float *X, int M) {
-    int rc;
-    const float *W = P<float>(h->mlp_w);
-    if ((rc = gemm(h, X, kNFeat, 1, W + kOffW1, kHidden, 1, P<float>(h->mlp_h1), kHidden, M, kHidden, kNFeat,
-                   W + kOffB1, GEMM_BIAS | GEMM_RELU)))
-        return rc;
-    if ((rc = gemm(h, P<float>(h->mlp_h1), kHidden, 1, W + kOffW2, kHidden, 1, P<float>(h->mlp_h2), kHidden, M,
-                   kHidden, kHidden, W + kOffB2, GEMM_BIAS | GEMM_RELU)))
-        return rc;
-    return gemm(h, P<float>(h->mlp_h2), kHidden, 1, W + kOffW3, kOut, 1, P<float>(h->mlp_z3), kOut, M, kOut, kHidden,
-                W + kOffB3, GEMM_BIAS);
-}
-
-// loss and gradients (into mlp_g, zeroed here) of M rows; y, c device
-int mlp_backward_dev(farm_handle h, const float *X, const float *y, const float *c, int M, float lambda) {
-    int rc;
-    const float *W = P<float>(h->mlp_w);
-    float *G = P<float>(h->mlp_g);
-    if ((rc = fill_u32(h, h->mlp_g.p, kNParams, 0))) return rc;
-    if ((rc = fill_u32(h, h->mlp_loss.p, 1, 0))) return rc;
-    hipLaunchKernelGGL(k_loss, dim3(blocks_for(M)), dim3(256), 0, h->stream, (const float *)P<float>(h->mlp_z3), y, c,
-                       M, lambda, P<float>(h->mlp_d3), P<float>(h->mlp_loss));
-    HIPCHK(h, hipGetLastError());
-    const int ks = max(1, M / 1024);
-    float *d3 = P<float>(h->mlp_d3), *h2 = P<float>(h->mlp_h2), *h1 = P<float>(h->mlp_h1);
-    float *dh2 = P<float>(h->mlp_dh2), *dh1 = P<float>(h->mlp_dh1);
-    // layer 3: dW3 = H2^T dZ3, db3 = colsum dZ3, dH2 = dZ3 W3^T
-    if ((rc = gemm(h, h2, 1, kHidden, d3, kOut, 1, G + kOffW3, kOut, kHidden, kOut, M, nullptr, GEMM_ATOMIC, ks)))
-        return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(kOut), dim3(256), 0, h->stream, (const float *)d3, M, kOut, G + kOffB3);
-    HIPCHK(h, hipGetLastError());
-    if ((rc = gemm(h, d3, kOut, 1, W + kOffW3, 1, kOut, dh2, kHidden, M, kHidden, kOut, nullptr, 0))) return rc;
-    hipLaunchKernelGGL(k_relu_back, dim3(blocks_for((uint64_t)M * kHidden)), dim3(256), 0, h->stream, dh2,
-                       (const float *)h2, (uint64_t)M * kHidden);
-    HIPCHK(h, hipGetLastError());
-    // layer 2
-    if ((rc = gemm(h, h1, 1, kHidden, dh2, kHidden, 1, G + kOffW2, kHidden, kHidden, kHidden, M, nullptr,
-                   GEMM_ATOMIC, ks)))
-        return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(kHidden), dim3(256), 0, h->stream, (const float *)dh2, M, kHidden, G + kOffB2);
-    HIPCHK(h, hipGetLastError());
-    if ((rc = gemm(h, dh2, kHidden, 1, W + kOffW2, 1, kHidden, dh1, kHidden, M, kHidden, kHidden, nullptr, 0)))
-        return rc;
-    hipLaunchKernelGGL(k_relu_back, dim3(blocks_for((uint64_t)M * kHidden)), dim3(256), 0, h->stream, dh1,
-                       (const float *)h1, (uint64_t)M * kHidden);
-    HIPCHK(h, hipGetLastError());
-    // layer 1
-    if ((rc = gemm(h, X, 1, kNFeat, dh1, kHidden, 1, G + kOffW1, kHidden, kNFeat, kHidden, M, nullptr, GEMM_ATOMIC,
-                   ks)))
-        return rc;
-    hipLaunchKernelGGL(k_colsum, dim3(kHidden), dim3(256), 0, h->stream, (const float *)dh1, M, kHidden, G + kOffB1);
+// the three layers of n rows of X (device, normalised unless norm is given)
+int mlp_infer(farm_handle h, const float *X, const float *norm, uint64_t n, float *out) {
+    const unsigned grid = (unsigned)std::min<uint64_t>((n + kInferRows - 1) / kInferRows, 2ull * h->num_cus);
+    hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(256), 0, h->stream, X, norm, (const float *)P<float>(h->mlp_w), n,
+                       out);
     HIPCHK(h, hipGetLastError());
     return FARM_OK;
 }
@@ -448,6 +598,10 @@ int farm_mlp_set_params(farm_handle h, const float *params, uint64_t n, const fl
     if ((rc = ensure(h, h->mlp_m, 4ull * kNParams))) return rc;
     if ((rc = ensure(h, h->mlp_v, 4ull * kNParams))) return rc;
     if ((rc = ensure(h, h->mlp_g, 4ull * kNParams))) return rc;
+    if ((rc = ensure(h, h->mlp_wb, sizeof(MlpPacked)))) return rc;
+    hipLaunchKernelGGL(k_mlp_pack, dim3(blocks_for(kNParams)), dim3(256), 0, h->stream,
+                       (const float *)P<float>(h->mlp_w), P<MlpPacked>(h->mlp_wb));
+    HIPCHK(h, hipGetLastError());
     if ((rc = fill_u32(h, h->mlp_m.p, kNParams, 0))) return rc;
     if ((rc = fill_u32(h, h->mlp_v.p, kNParams, 0))) return rc;
     std::vector<float> nm(2 * kNFeat);
@@ -477,9 +631,9 @@ int farm_mlp_forward(farm_handle h, const float *X, uint64_t n, float *out) {
     const int chunk = 1 << 16;
     for (uint64_t s = 0; s < n; s += chunk) {
         const int M = (int)std::min<uint64_t>(chunk, n - s);
-        if ((rc = mlp_buffers(h, M))) return rc;
+        if ((rc = ensure(h, h->mlp_z3, 4ull * M * kOut))) return rc;
         if ((rc = upload(h, h->mlp_x, X + s * kNFeat, 4ull * M * kNFeat))) return rc;
-        if ((rc = mlp_forward_dev(h, P<float>(h->mlp_x), M))) return rc;
+        if ((rc = mlp_infer(h, P<float>(h->mlp_x), nullptr, M, P<float>(h->mlp_z3)))) return rc;
         HIPCHK(h, hipMemcpyAsync(out + s * kOut, h->mlp_z3.p, 4ull * M * kOut, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
     }
@@ -493,12 +647,13 @@ int farm_mlp_loss_grad(farm_handle h, const float *X, const float *y, const floa
     if (n == 0 || n > (1u << 24)) return fail(h, FARM_EINVAL, "batch of %llu rows", (unsigned long long)n);
     HIPCHK(h, hipSetDevice(h->device));
     const int M = (int)n;
-    if ((rc = mlp_buffers(h, M))) return rc;
+    if ((rc = grad_buffers(h, M, 1))) return rc;
     if ((rc = upload(h, h->mlp_x, X, 4ull * M * kNFeat))) return rc;
     if ((rc = upload(h, h->mlp_y, y, 4ull * M))) return rc;
     if ((rc = upload(h, h->mlp_c, c, 4ull * M))) return rc;
-    if ((rc = mlp_forward_dev(h, P<float>(h->mlp_x), M))) return rc;
-    if ((rc = mlp_backward_dev(h, P<float>(h->mlp_x), P<float>(h->mlp_y), P<float>(h->mlp_c), M, lambda))) return rc;
+    if ((rc = mlp_step(h, P<float>(h->mlp_x), nullptr, P<float>(h->mlp_y), P<float>(h->mlp_c), M, lambda, 0, false,
+                       0.f)))
+        return rc;
     if (loss) HIPCHK(h, hipMemcpyAsync(loss, h->mlp_loss.p, 4, hipMemcpyDeviceToHost, h->stream));
     if (grad) HIPCHK(h, hipMemcpyAsync(grad, h->mlp_g.p, 4ull * kNParams, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -511,65 +666,60 @@ int farm_mlp_train(farm_handle h, const float *X, const float *y, const float *c
     if (rc) return rc;
     if (n == 0 || batch <= 0 || epochs <= 0) return fail(h, FARM_EINVAL, "bad training arguments");
     HIPCHK(h, hipSetDevice(h->device));
-    DevBuf dX, dy, dc, dperm, bx;
+    // batches of an epoch: whole ones only (one short one when n < batch)
+    const int M = (int)std::min<uint64_t>((uint64_t)batch, n);
+    const uint64_t nb = n / M;
+    DevBuf dX, dy, dc, dperm;
     auto cleanup = [&]() {
+        (void)hipStreamSynchronize(h->stream);
         free_buf(dX);
         free_buf(dy);
         free_buf(dc);
         free_buf(dperm);
-        free_buf(bx);
     };
-    if ((rc = upload(h, dX, X, 4ull * n * kNFeat)) || (rc = upload(h, dy, y, 4ull * n)) ||
-        (rc = upload(h, dc, c, 4ull * n)) || (rc = ensure(h, dperm, 4ull * n)) ||
-        (rc = ensure(h, bx, 4ull * batch * kNFeat)) || (rc = mlp_buffers(h, batch))) {
-        cleanup();
-        return rc;
-    }
-    std::vector<uint32_t> perm(n);
+    // two orders in turn: one may still be in transfer while the next is made
+    std::vector<uint32_t> perms[2] = {std::vector<uint32_t>(n), std::vector<uint32_t>(n)};
     uint64_t s = seed * 6364136223846793005ull + 1442695040888963407ull;
-    for (int ep = 0; ep < epochs; ep++) {
+    auto shuffle = [&](std::vector<uint32_t> &perm) {
         for (uint64_t i = 0; i < n; i++) perm[i] = (uint32_t)i;
         for (uint64_t i = n - 1; i > 0; i--) {  // Fisher-Yates, PCG-style LCG
             s = s * 6364136223846793005ull + 1442695040888963407ull;
             const uint64_t j = (s >> 33) % (i + 1);
             std::swap(perm[i], perm[j]);
         }
-        if ((rc = upload(h, dperm, perm.data(), 4ull * n))) {
+    };
+    if ((rc = upload(h, dX, X, 4ull * n * kNFeat)) || (rc = upload(h, dy, y, 4ull * n)) ||
+        (rc = upload(h, dc, c, 4ull * n)) || (rc = ensure(h, dperm, 4ull * n)) || (rc = grad_buffers(h, M, nb))) {
+        cleanup();
+        return rc;
+    }
+    shuffle(perms[0]);
+    std::vector<float> losses(nb);
+    for (int ep = 0; ep < epochs; ep++) {
+        if ((rc = upload(h, dperm, perms[ep & 1].data(), 4ull * n))) {
             cleanup();
             return rc;
         }
-        double ep_loss = 0;
-        int nb = 0;
-        for (uint64_t b0 = 0; b0 + batch <= n || (b0 < n && nb == 0); b0 += batch) {
-            const int M = (int)std::min<uint64_t>(batch, n - b0);
-            const uint32_t *ix = P<uint32_t>(dperm) + b0;
-            hipLaunchKernelGGL(k_gather_rows, dim3(blocks_for((uint64_t)M * kNFeat)), dim3(256), 0, h->stream,
-                               (const float *)P<float>(dX), ix, M, kNFeat, P<float>(bx));
-            hipLaunchKernelGGL(k_gather_vec, dim3(blocks_for(M)), dim3(256), 0, h->stream, (const float *)P<float>(dy),
-                               ix, M, P<float>(h->mlp_y));
-            hipLaunchKernelGGL(k_gather_vec, dim3(blocks_for(M)), dim3(256), 0, h->stream, (const float *)P<float>(dc),
-                               ix, M, P<float>(h->mlp_c));
-            if ((rc = mlp_forward_dev(h, P<float>(bx), M)) ||
-                (rc = mlp_backward_dev(h, P<float>(bx), P<float>(h->mlp_y), P<float>(h->mlp_c), M, lambda))) {
+        // the epoch's steps are queued without a wait; the next shuffle runs
+        // on the host meanwhile
+        for (uint64_t b = 0; b < nb; b++) {
+            h->adam_t++;
+            if ((rc = mlp_step(h, P<float>(dX), P<uint32_t>(dperm) + b * M, P<float>(dy), P<float>(dc), M, lambda, b,
+                               true, lr))) {
                 cleanup();
                 return rc;
             }
-            h->adam_t++;
-            const float c1 = 1.f - powf(0.9f, (float)h->adam_t), c2 = 1.f - powf(0.999f, (float)h->adam_t);
-            hipLaunchKernelGGL(k_adam, dim3(blocks_for(kNParams)), dim3(256), 0, h->stream, P<float>(h->mlp_w),
-                               (const float *)P<float>(h->mlp_g), P<float>(h->mlp_m), P<float>(h->mlp_v), kNParams,
-                               lr, 0.9f, 0.999f, 1e-8f, c1, c2);
-            float L = 0;
-            hipError_t e = hipMemcpyAsync(&L, h->mlp_loss.p, 4, hipMemcpyDeviceToHost, h->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-            if (e != hipSuccess) {
-                cleanup();
-                return fail(h, FARM_EDEVICE, "training step failed: %s", hipGetErrorString(e));
-            }
-            ep_loss += L;
-            nb++;
         }
-        if (epoch_loss) epoch_loss[ep] = (float)(ep_loss / std::max(nb, 1));
+        if (ep + 1 < epochs) shuffle(perms[(ep + 1) & 1]);
+        hipError_t e = hipMemcpyAsync(losses.data(), h->mlp_loss.p, 4ull * nb, hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+        if (e != hipSuccess) {
+            cleanup();
+            return fail(h, FARM_EDEVICE, "training step failed: %s", hipGetErrorString(e));
+        }
+        double ep_loss = 0;
+        for (float L : losses) ep_loss += L;
+        if (epoch_loss) epoch_loss[ep] = (float)(ep_loss / nb);
     }
     cleanup();
     return FARM_OK;
@@ -609,12 +759,7 @@ int farm_mlp_predict_pairs(farm_handle h, uint64_t begin, uint64_t end, float *o
     const uint64_t n = end - begin;
     if ((rc = ensure(h, h->pred, 8ull * (n ? n : 1)))) return rc;
     if (!n) return FARM_OK;
-    // normalisation and the three layers in one pass (the logits of the
-    // three-launch path, bit for bit)
-    const unsigned grid = (unsigned)std::min<uint64_t>((n + kInferRows - 1) / kInferRows, 2ull * h->num_cus);
-    hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(256), 0, h->stream, (const float *)P<float>(h->feat),
-                       (const float *)P<float>(h->mlp_norm), (const float *)P<float>(h->mlp_w), n, P<float>(h->pred));
-    HIPCHK(h, hipGetLastError());
+    if ((rc = mlp_infer(h, P<float>(h->feat), P<float>(h->mlp_norm), n, P<float>(h->pred)))) return rc;
     if (out) HIPCHK(h, hipMemcpyAsync(out, h->pred.p, 8ull * n, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return FARM_OK;

@@ -49,6 +49,24 @@ def test_gradients_match_reference(device):
             o += n
 
 
+@pytest.mark.parametrize("m", [1, 31, 33, 8191, 8225])
+def test_gradients_at_tile_edges(device, m):
+    # one row, 32-row tiles with a part tile, and more tiles than workgroups;
+    # bf16 operands as in test_gradients_match_reference, hence its bounds
+    p, X, y, c = _rand_problem(70 + m, m)
+    device.mlp_set_params(p)
+    L, g = device.mlp_loss_grad(X, y, c, 0.05)
+    Lr, gr = mlp_ref.loss_grad(p.astype(np.float64), X, y.astype(np.float64), c.astype(np.float64), 0.05,
+                               rounding=True)
+    assert abs(L - Lr) <= 1e-4 * abs(Lr) + 1e-6
+    o = 0
+    for shp in learned.SHAPES:
+        n = int(np.prod(shp))
+        blk, ref = g[o:o + n], gr[o:o + n]
+        assert np.abs(blk - ref).max() < 3e-3 * (np.abs(ref).max() + 1e-12), (m, shp)
+        o += n
+
+
 def test_training_reduces_loss(device):
     rng = np.random.default_rng(3)
     X = rng.normal(0, 1, (20000, capi.NFEAT)).astype(np.float32)
