@@ -42,7 +42,7 @@ __global__ void k_plain(DevSet, const uint32_t *, const uint32_t *, uint32_t, ui
 __global__ void k_pixedges(DevSet, int64_t, uint32_t *);
 __global__ void k_vdiff(const float *, const float *, uint64_t, float4 *);
 __global__ void k_chunk_count(DevSet, int64_t, uint32_t, uint32_t *);
-__global__ void k_chunk_box(DevSet, int64_t, uint32_t, const uint32_t *, float4 *, uint2 *);
+__global__ void k_chunk_box(DevSet, int64_t, uint32_t, const uint32_t *, float4 *, uint4 *);
 __global__ void k_finalize(const uint32_t *, const IsxDesc *, unsigned long long *, unsigned long long *);
 }  // namespace farm
 
@@ -407,10 +407,10 @@ int build_chunk_boxes(farm_handle h, uint32_t C) {
     HIPCHK(h, hipMemcpyAsync(&nchunks, P<uint32_t>(h->choff) + nseqs, 4, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     if ((rc = ensure(h, h->chbox, 16ull * (nchunks + kRefScreen)))) return rc;
-    if ((rc = ensure(h, h->chseg, 8ull * (nchunks + kRefScreen)))) return rc;
+    if ((rc = ensure(h, h->chseg, 16ull * (nchunks + kRefScreen)))) return rc;
     if (h->npolys > 0) {
         hipLaunchKernelGGL(k_chunk_box, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys, C,
-                           (const uint32_t *)P<uint32_t>(h->choff), P<float4>(h->chbox), P<uint2>(h->chseg));
+                           (const uint32_t *)P<uint32_t>(h->choff), P<float4>(h->chbox), P<uint4>(h->chseg));
         HIPCHK(h, hipGetLastError());
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -440,7 +440,7 @@ int build_ix_boxes(farm_handle h) {
     if (h->npolys > 0) {
         hipLaunchKernelGGL(k_chunk_box, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys,
                            kIxChunk, (const uint32_t *)P<uint32_t>(h->ixoff), P<float4>(h->ixbox),
-                           (uint2 *)nullptr);
+                           (uint4 *)nullptr);
         HIPCHK(h, hipGetLastError());
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));

@@ -22,11 +22,11 @@ struct DevSet {
     // 16-byte load per target step)
     const float4 *xyd;
     // per edge sequence: index of its first C-step chunk box; the boxes
-    // (centre x, y, half extents x, y) and each chunk's first vertex and
-    // segment count, refinement only
+    // (centre x, y, half extents x, y) and each chunk's first vertex, segment
+    // count and direction mask (low, high word), refinement only
     const uint32_t *choff;
     const float4 *chbox;
-    const uint2 *chseg;
+    const uint4 *chseg;
     // the same for chunks of kIxChunk segments, for the intersection's chunk
     // skip (the refinement's arrays when C == kIxChunk; null: no skip)
     const uint32_t *ixoff;
@@ -52,6 +52,27 @@ constexpr uint32_t kRefChunkDefault = 16;
 // target segments per chunk of the intersection's collection screen
 constexpr uint32_t kIxChunk = 16;
 constexpr uint32_t kRefScreen = 4;
+
+constexpr uint32_t kChunkPoint = 0x10000u;  // in a chunk's segment count: one of them has length 0
+
+// Direction classes of lines: the direction (ux, uy), taken modulo pi with uy
+// >= 0, has the pseudo-angle s = 1 - ux / (|ux| + |uy|) in [0, 2), monotone in
+// the angle with slope in [1/2, 1]; kDirBins classes of equal width in s.  A
+// chunk's mask holds the classes within kDirTol of each of its segments'
+// pseudo-angles (cyclic), a source edge's mask its own class: an edge and a
+// segment whose lines meet at an angle of at most kDirTol share a bit.  Edges
+// too short for a reliable direction (or not finite) get every bit.
+constexpr int kDirBins = 64;
+constexpr float kDirTol = 0x1p-9f;
+
+__device__ __forceinline__ bool dir_angle(float ux, float uy, float &s) {
+    const float n = fabsf(ux) + fabsf(uy);
+    s = 1.f - (uy < 0.f ? -ux : ux) * __builtin_amdgcn_rcpf(n);
+    return n >= 0x1p-60f && n < 0x1p60f;  // false for NaN
+}
+__device__ __forceinline__ uint64_t dir_bit(float s) {
+    return 1ull << ((int)floorf(s * (kDirBins / 2)) & (kDirBins - 1));
+}
 
 // A BORDER x BORDER pixel pair of one candidate pair.
 struct PixPair {

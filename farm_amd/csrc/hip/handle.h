@@ -170,7 +170,7 @@ inline DevSet devset(farm_handle h) {
     S.cc = h->cc;
     S.choff = P<uint32_t>(h->choff);
     S.chbox = P<float4>(h->chbox);
-    S.chseg = P<uint2>(h->chseg);
+    S.chseg = P<uint4>(h->chseg);
     if (h->chunk == kIxChunk) {
         S.ixoff = S.choff;
         S.ixbox = S.chbox;

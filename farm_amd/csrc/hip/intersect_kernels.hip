@@ -409,10 +409,25 @@ __global__ __launch_bounds__(256) void k_tile_map(DevSet S, const uint32_t *__re
 // Per chunk every lane first tests its W edges against the chunk's box (an
 // exact prune: no edge whose line keeps the whole box at a safe distance can
 // meet a segment of the chunk under the reference predicate); the (lane,
-// chunk) pairs that survive are queued in LDS, and every 64 queued items are
-// evaluated one per lane: the lane's edges (read from LDS) against the
-// chunk's segments (its own loads), with the screen below and, for the rare
-// candidates, the exact reference predicate.
+// chunk) pairs that survive are queued in LDS and evaluated kDrain at a time:
+// the lane's edges (read from LDS) against the chunk's segments (loads of the
+// evaluating lane), with the screen below and, for the rare candidates, the
+// exact reference predicate.
+//
+// The line test alone keeps 6 % of the (lane, chunk) pairs on complex x lakes.
+// A second exact test drops four fifths of those: boxes apart on an axis leave
+// only crossings that rounding makes up, and those need lines that are nearly
+// parallel.  Let the lane's vertex box and the chunk's be apart by g >= 2^-8 q
+// on an axis (q the L1 reach).  The collinear branch needs box overlap, so a
+// true answer needs the computed signs of c, d against line ab and of a, b
+// against line cd to differ.  The f32 cross products err by less than 2^-22
+// times the L1 lengths of their two differences, i.e. by a distance below
+// delta = 2^-21.4 q to the line, so some point X of cd lies within delta of
+// line ab and some point Y of ab within delta of line cd.  X and Y are at
+// least g apart, so both lines make an angle below delta / g = 2^-13.4 with
+// XY, and less than 2^-12.4 with each other.  A chunk's direction mask holds
+// the classes within kDirTol = 2^-9 (>= 2^-10 in angle) of each of its
+// segments, so masks without a common bit rule the crossing out.
 // ------------------------------------------------------------------------
 
 // Boxes of the refinement's target chunks.  A sequence (first, len) is walked
@@ -420,11 +435,15 @@ __global__ __launch_bounds__(256) void k_tile_map(DevSet S, const uint32_t *__re
 // segments span vertices first + base - 1 .. first + base + n - 1.  The box is
 // stored as a centre and half extents rounded up, so [c - h, c + h] holds
 // every vertex of the chunk in exact arithmetic.  Infinite extents (the prune
-// never applies) go to a box that reaches past 2^40, holds a non-finite
-// vertex, or holds a segment of length 0: for c == d the reference's
-// c.cross(a, d) is 0 for every a, so segment_intersect takes its collinear
-// branch and answers with the bounding-box overlap alone, on either side of
-// line ab.
+// never applies) go to a box that reaches past 2^40 or holds a non-finite
+// vertex.  A chunk that holds a segment of length 0 is marked (kChunkPoint):
+// for c == d the reference's c.cross(a, d) is 0 for every a, so
+// segment_intersect takes its collinear branch and answers with the
+// bounding-box overlap alone, on either side of line ab.  Such a segment is
+// in play only for a lane whose box is not apart from the chunk's.  (Every
+// closed ring has one, its repeated first vertex; as a box that is never
+// pruned it put its chunk against all 512 edges of every tile, all of them
+// through the exact replay: half of the kernel's time.)
 __global__ __launch_bounds__(256) void k_chunk_count(DevSet S, int64_t npolys, uint32_t C,
                                                      uint32_t *__restrict__ cnt) {
     const int64_t p = blockIdx.x;
@@ -436,7 +455,7 @@ __global__ __launch_bounds__(256) void k_chunk_count(DevSet S, int64_t npolys, u
 
 __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uint32_t C,
                                                    const uint32_t *__restrict__ choff, float4 *__restrict__ box,
-                                                   uint2 *__restrict__ seg) {
+                                                   uint4 *__restrict__ seg) {
     const int64_t p = blockIdx.x;
     if (p >= npolys) return;
     const farm_raster_hdr H = S.hdr[p];
@@ -449,9 +468,14 @@ __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uin
             float x0 = x[sq.x + base - 1], x1 = x0, y0 = y[sq.x + base - 1], y1 = y0;
             bool open = isfinite(x0) && isfinite(y0);  // false: never prune this chunk
             float lx = x0, ly = y0;
+            uint64_t dirs = 0;
+            uint32_t mark = 0;
             for (uint32_t m = 0; m < n; m++) {
                 const float vx = x[sq.x + base + m], vy = y[sq.x + base + m];
-                open = open && isfinite(vx) && isfinite(vy) && !(vx == lx && vy == ly);
+                open = open && isfinite(vx) && isfinite(vy);
+                float s;
+                if (vx == lx && vy == ly) mark = kChunkPoint;
+                else dirs |= dir_angle(vx - lx, vy - ly, s) ? dir_bit(s - kDirTol) | dir_bit(s + kDirTol) : ~0ull;
                 lx = vx;
                 ly = vy;
                 x0 = fminf(x0, vx);
@@ -467,7 +491,7 @@ __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uin
             const float big = 0x1p40f;
             if (!(open && fabsf(cx) + hx < big && fabsf(cy) + hy < big)) hx = hy = INFINITY;
             box[o] = make_float4(cx, cy, hx, hy);
-            if (seg) seg[o] = make_uint2(sq.x + base - 1, n);
+            if (seg) seg[o] = make_uint4(sq.x + base - 1, n | mark, (uint32_t)dirs, (uint32_t)(dirs >> 32));
         }
     }
 }
@@ -477,6 +501,11 @@ __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uin
 typedef __attribute__((address_space(4))) const float cfloat;
 typedef __attribute__((address_space(4))) const uint32_t cuint;
 
+// Queued items are evaluated kDrain at a time, 2^kSplit lanes or more to an
+// item: measured on complex x lakes (496,000 pairs, 8 edges per lane, 16
+// segments per chunk) 9.87, 9.22 and 9.5 ms with 1, 2 and 4 lanes, as a wave
+// usually holds a few dozen items and fewer steps follow each other.
+constexpr uint32_t kSplit = 1, kDrain = 64u >> kSplit;
 constexpr uint32_t kRefQueue = 512;  // queued items per wave: a power of 2 above 63 + 64 kRefScreen
 
 template <int W, int C>
@@ -504,13 +533,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     float(*src)[2 * (W + 1)] = s_src[wv];
     uint32_t *sev = s_ev[wv];
     uint2 *ring = s_ring[wv];
-    // work counters: per tile in 32-bit lane registers, added at its end to
-    // the lane's own 64-bit totals in LDS (64-bit lane totals in registers
-    // push the kernel past its register budget; summing them over the wave
-    // per tile took 36 shuffles); the refine bytes are wave-uniform
-    __shared__ unsigned long long s_acc[4][2][64];  // tests, pruned tests
-    s_acc[wv][0][lane] = s_acc[wv][1][lane] = 0;
-    unsigned long long items = 0, rbytes = 0;
+    // and the directions of every lane's edges (dir_bit)
+    __shared__ uint2 s_dir[4][64];
+    uint2 *sdir = s_dir[wv];
+    // work counters: per tile in 32-bit lane registers, summed at its end
+    // into wave-uniform totals (64-bit lane totals push the kernel past its
+    // register budget)
+    unsigned long long items = 0, rbytes = 0, tests_w = 0, pruned_w = 0;
     // A wave takes `grab` consecutive tiles at a time, whose pairs' flags are
     // looked up together, one per lane (on jagged small polygons 70 % of the
     // tiles belong to pairs already decided; a descriptor and a flag load for
@@ -523,6 +552,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // position alone left waves idle (a call of 1.3e6 tiles of uneven cost
     // took 17.5 ms instead of 13.9).
     const uint32_t nwaves = gridDim.x * 4u, wid = blockIdx.x * 4u + (uint32_t)wv;
+    const uint32_t dir_all = prune ? 0u : ~0u;  // without the prune every direction matches
     const uint32_t grab = min(max(total / (nwaves * 16u), 1u), 16u);
     uint32_t home = wid & (kCtrShards - 1);
     uint32_t tbase = 0;
@@ -558,7 +588,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         }
         const uint32_t t = tbase + (uint32_t)__ffsll(live) - 1u;
         live &= live - 1;
-        uint32_t tests = 0, pruned = 0;
+        uint32_t tests = 0, queued = 0;
         // the tile's descriptor (one uniform load), then its pair's flag
         // again (an earlier tile of the grab may have decided it)
         const TileDesc td = tile_map[t];
@@ -654,13 +684,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 src[lane][E + 1 + v] = py[v];
             }
             sev[lane] = evb;
+            {
+                uint64_t dirs = 0;
+#pragma unroll
+                for (int e = 0; e < E; e++) {
+                    float s;
+                    const uint64_t b = dir_angle(px[e + 1] - px[e], py[e + 1] - py[e], s) ? dir_bit(s) : ~0ull;
+                    dirs |= ev[e] ? b : 0ull;
+                }
+                sdir[lane] = make_uint2((uint32_t)dirs, (uint32_t)(dirs >> 32));
+            }
             __builtin_amdgcn_wave_barrier();
             bool hit = false;
             bool stop = false;
             uint32_t qhead = 0, qn = 0, screened = 0;  // wave-uniform
             uint32_t scr_steps = 0, queued_steps = 0;  // target steps screened (uniform) / queued by this lane
 
-            // Evaluate the n <= 64 oldest queued items, one per lane: the source
+            // Evaluate the n <= kDrain oldest queued items: the source
             // lane's E edges against the chunk's nstep target segments.  Per
             // target vertex q and source edge (a, b):
             //   O(q) = a.cross(b, q)   -- o1/o2 of consecutive steps
@@ -670,13 +710,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             // superset filter (o1*o2 <= 0 or o3 == 0, and o3*o4 <= 0) sends
             // the rare candidates to the exact reference predicate.
             //
-            // Fewer than 64 items (a tile's last) are split over the lanes: k =
-            // 64 / n rounded down to a power of two (at most C) lanes per item,
-            // part j taking its steps j C / k .. (j + 1) C / k - 1.  A part is
-            // the item's segments from its own first vertex on, so the split
-            // evaluates the same tests in C / k steps instead of C.
+            // An item is split over k = 64 / n lanes, rounded down to a power
+            // of two (at most C), part j taking its steps j C / k .. (j + 1) C
+            // / k - 1.  A part is the item's segments from its own first vertex
+            // on, so the split evaluates the same tests in C / k steps instead
+            // of C.
             auto drain = [&](uint32_t n) {
-                uint32_t lk = 0;  // log2 k (uniform)
+                uint32_t lk = kSplit;  // log2 k (uniform)
                 while ((1u << lk) < (uint32_t)C && (n << (lk + 1)) <= 64u) lk++;
                 const uint32_t seg = (uint32_t)C >> lk;
                 const uint32_t item = (uint32_t)lane >> lk, m0 = ((uint32_t)lane & ((1u << lk) - 1u)) * seg;
@@ -772,8 +812,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 tests += (uint32_t)qnv * ns;
                 qhead = (qhead + n) & (kRefQueue - 1);
                 qn -= n;
-                if (__any(hit) || __hip_atomic_load(&result[pair], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                    stop = true;
+                if (__any(hit)) stop = true;
             };
 
             {
@@ -804,8 +843,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     // spread over the box and M in two more fmas the f32
                     // evaluation errs by at most about 13 2^-24 q |b - a|_1
                     // (every operand is within 2q of o), which M covers twice
-                    // over.  (A chunk with a segment of length 0 has an
-                    // infinite box and is never pruned.)
+                    // over.  (A segment of length 0 only answers with box
+                    // overlap: its chunk is kept for the lanes not apart.)
                     // this lane's slots again, from LDS (not kept in registers
                     // across the evaluation of queued items: the lane's index
                     // is made opaque, or the loads would move out of the loop)
@@ -838,6 +877,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                             scc[e] = ve ? fmaf(sbx[e], ayo, -(sby[e] * axo)) : INFINITY;
                         }
                     }
+                    const uint2 ldir = sdir[sln];
                     bool need[kRefScreen];
 #pragma unroll
                     for (int i = 0; i < (int)kRefScreen; i++) {
@@ -852,7 +892,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                         const float hx1 = bb.z * 1.000001f, hy1 = bb.w * 1.000001f;
                         // (ex1 > hx1 or -ex0 > hx1 or ey1 > hy1 or -ey0 > hy1, as two
                         // maxima and two compares)
-                        const bool apart = (fmaxf(ex1, -ex0) > hx1) | (fmaxf(ey1, -ey0) > hy1);
+                        const float sepx = fmaxf(ex1, -ex0), sepy = fmaxf(ey1, -ey0);
+                        const bool apart = (sepx > hx1) | (sepy > hy1);
+                        // Direction prune: apart by more than 2^-8 q on an axis
+                        // and no segment of the chunk within kDirTol of the
+                        // direction of any of the lane's edges.
+                        const bool far = fmaxf(sepx - hx1, sepy - hy1) > q * 0x1p-8f && q < 0x1p60f;
+                        const uint32_t cdl = cseg[4 * (g + i) + 2] | dir_all, cdh = cseg[4 * (g + i) + 3] | dir_all;
+                        const bool cand = !far || ((ldir.x & cdl) | (ldir.y & cdh)) != 0u;
+                        need[i] = false;
+                        if (!__ballot(cand)) continue;  // no lane's lines need a look
                         // (without the prune: the largest finite margin keeps every
                         // chunk for every slot with an edge)
                         const float k1 = !prune ? 0x1.fffffep127f : q * 0x1p-18f;
@@ -861,19 +910,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                         // |s_y| (hx + k1) + |s_x| (hy + k1) + k2
                         const float hxk = bb.z + k1, hyk = bb.w + k1;
                         const float cxo = bb.x - ox, cyo = bb.y - oy;
-                        need[i] = false;
+                        bool line = false;
 #pragma unroll
                         for (int e = 0; e < E; e++) {
                             const float oc = fmaf(sbx[e], cyo, -fmaf(sby[e], cxo, scc[e]));  // at the box centre
                             const float thr = fmaf(fabsf(sby[e]), hxk, fmaf(fabsf(sbx[e]), hyk, k2));
-                            need[i] = need[i] | !(fabsf(oc) > thr);  // bitwise: no branch per edge
+                            line = line | !(fabsf(oc) > thr);  // bitwise: no branch per edge
                         }
+                        need[i] = (line & cand) | (!apart && (cseg[4 * (g + i) + 1] & kChunkPoint));
                     }
 #pragma unroll
                     for (int i = 0; i < (int)kRefScreen; i++) {
                         const uint32_t c = g + i;
                         if (c >= nch) break;
-                        const uint32_t v0 = cseg[2 * c], nstep = cseg[2 * c + 1];
+                        const uint32_t v0 = cseg[4 * c], nstep = cseg[4 * c + 1] & ~kChunkPoint;
                         scr_steps += nstep;
                         const unsigned long long bm = __ballot(need[i]);
                         if (bm) {
@@ -888,9 +938,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                             qn += (uint32_t)__popcll(bm);
                         }
                     }
-                    while (qn >= 64 && !stop) {
+                    while (qn >= kDrain && !stop) {
                         __builtin_amdgcn_wave_barrier();
-                        drain(64);
+                        drain(kDrain);
                     }
                     if (!stop && (++screened & 7u) == 0 &&
                         __hip_atomic_load(&result[pair], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
@@ -911,31 +961,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 #pragma unroll
             for (int e = 0; e < E; e++) edges += (uint32_t)__popcll(__ballot((evb >> e) & 1u));
             rbytes += td_rbytes + edges * 8u;
-            // tests of this lane's edges the prune skipped: every screened step
-            // that was not queued
-            pruned += (uint32_t)nvalid * (scr_steps - queued_steps);
+            // tests the prune skipped: every edge's every screened step that was
+            // not queued
+            queued += (uint32_t)nvalid * queued_steps;
+            pruned_w += (unsigned long long)edges * scr_steps;
         };
         run(std::integral_constant<int, W>());
-        s_acc[wv][0][lane] += tests;
-        s_acc[wv][1][lane] += pruned;
-        if (pair_tests) {
-            // executed tests of this tile, for the cost labels
-            unsigned long long t64 = tests;
-            for (int o = 32; o > 0; o >>= 1) t64 += __shfl_xor(t64, o);
-            if (lane == 0) atomicAdd(&pair_tests[pair], (uint32_t)min(t64, 0xffffffffull));
-        }
-    }
-    unsigned long long t64 = s_acc[wv][0][lane], p64 = s_acc[wv][1][lane];
-    for (int o = 32; o > 0; o >>= 1) {
-        t64 += __shfl_xor(t64, o);
-        p64 += __shfl_xor(p64, o);
+        const unsigned long long t64 = wave_sum_u64(tests);
+        tests_w += t64;
+        pruned_w -= wave_sum_u64(queued);
+        // executed tests of this tile, for the cost labels
+        if (pair_tests && lane == 0) atomicAdd(&pair_tests[pair], (uint32_t)min(t64, 0xffffffffull));
     }
     if (lane == 0 && items) {
         unsigned long long *sh = ctr_shard(shards, wid);
-        atomicAdd(&sh[kCtrTests], t64);
+        atomicAdd(&sh[kCtrTests], tests_w);
         atomicAdd(&sh[kCtrItems], items);
         atomicAdd(&sh[kCtrRefineBytes], rbytes);
-        atomicAdd(&sh[kCtrPruned], p64);
+        atomicAdd(&sh[kCtrPruned], pruned_w);
     }
 }
 

@@ -52,6 +52,25 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 __device__ __forceinline__ bool wave_any(bool p) { return __ballot(p) != 0; }
 
+// Sum of v over the wave (64 lanes) modulo 2^32, by DPP adds (no LDS): row
+// shifts leave a row's sum in its lane 15, two row broadcasts add the rows up
+// in lane 63.
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, true);
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The same sum in 64 bits.
+__device__ __forceinline__ unsigned long long wave_sum_u64(uint32_t v) {
+    if (!__ballot((v >> 26) != 0)) return wave_sum_u32(v);  // no carry out of 32 bits
+    return ((unsigned long long)wave_sum_u32(v >> 16) << 16) + wave_sum_u32(v & 0xffffu);
+}
+
 // Exclusive prefix sum of v over the wave; *total gets the sum.
 __device__ __forceinline__ uint32_t wave_excl_scan(uint32_t v, int lane, uint32_t *total) {
     uint32_t s = v;
