@@ -437,10 +437,11 @@ int build_ix_boxes(farm_handle h) {
     HIPCHK(h, hipMemcpyAsync(&nchunks, P<uint32_t>(h->ixoff) + nseqs, 4, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     if ((rc = ensure(h, h->ixbox, 16ull * (nchunks + 1)))) return rc;
+    if ((rc = ensure(h, h->ixseg, 16ull * (nchunks + 1)))) return rc;
     if (h->npolys > 0) {
         hipLaunchKernelGGL(k_chunk_box, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys,
                            kIxChunk, (const uint32_t *)P<uint32_t>(h->ixoff), P<float4>(h->ixbox),
-                           (uint4 *)nullptr);
+                           P<uint4>(h->ixseg));
         HIPCHK(h, hipGetLastError());
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -703,7 +704,7 @@ int farm_close(farm_handle h) {
         if (h->stage[k]) (void)hipHostFree(h->stage[k]);
         if (h->stage_ev[k]) (void)hipEventDestroy(h->stage_ev[k]);
     }
-    DevBuf *bufs[] = {&h->hdr,    &h->status,  &h->pixoff, &h->seqs,   &h->x,      &h->y,        &h->xyd,      &h->fill,     &h->choff,  &h->chcnt,  &h->chbox,  &h->chseg,  &h->ixcnt, &h->ixoff, &h->ixbox, &h->voff,
+    DevBuf *bufs[] = {&h->hdr,    &h->status,  &h->pixoff, &h->seqs,   &h->x,      &h->y,        &h->xyd,      &h->fill,     &h->choff,  &h->chcnt,  &h->chbox,  &h->chseg,  &h->ixcnt, &h->ixoff, &h->ixbox, &h->ixseg, &h->voff,
                       &h->vnodes, &h->pixedges, &h->shape_ctr, &h->pa, &h->pb, &h->isx,
                       &h->scan_tmp, &h->pair_tests, &h->mlp_w, &h->mlp_m, &h->mlp_v, &h->mlp_g,
                       &h->mlp_norm, &h->mlp_wb, &h->mlp_x, &h->mlp_z3, &h->mlp_y, &h->mlp_c, &h->mlp_loss,

@@ -27,10 +27,11 @@ struct DevSet {
     const uint32_t *choff;
     const float4 *chbox;
     const uint4 *chseg;
-    // the same for chunks of kIxChunk segments, for the intersection's chunk
-    // skip (the refinement's arrays when C == kIxChunk; null: no skip)
+    // the same for chunks of kIxChunk segments, for the intersection's
+    // collection (the refinement's arrays when C == kIxChunk)
     const uint32_t *ixoff;
     const float4 *ixbox;
+    const uint4 *ixseg;
     const uint32_t *pixedges;  // per pixel: sum of sequence lengths (BORDER), else 0
     const uint32_t *voff;
     const double *vnodes;
@@ -49,7 +50,7 @@ struct DevSet {
 // screens kRefScreen chunk boxes per scalar load (the box and chunk arrays keep
 // kRefScreen spare entries past their end).
 constexpr uint32_t kRefChunkDefault = 16;
-// target segments per chunk of the intersection's collection screen
+// segments per chunk of the intersection's collection screens
 constexpr uint32_t kIxChunk = 16;
 constexpr uint32_t kRefScreen = 4;
 

@@ -44,9 +44,9 @@ struct farm_handle_s {
     farm::DevBuf fill;    // -w fill classes (when the set has them)
     int cc = FARM_CATEGORY_COUNT;
     farm::DevBuf hdr, status, pixoff, seqs, x, y, xyd, choff, chcnt, chbox, chseg, voff, vnodes, pixedges, shape_ctr;
-    // 16-segment chunk boxes for the intersection's chunk skip when the
+    // 16-segment chunks for the intersection's collection when the
     // refinement's boxes are of another size (built for set generation ix_gen)
-    farm::DevBuf ixcnt, ixoff, ixbox;
+    farm::DevBuf ixcnt, ixoff, ixbox, ixseg;
     uint64_t ix_gen = ~0ull;
     uint64_t nstatus = 0;
     // array lengths of the set (farm_polyset's counts)
@@ -174,12 +174,15 @@ inline DevSet devset(farm_handle h) {
     if (h->chunk == kIxChunk) {
         S.ixoff = S.choff;
         S.ixbox = S.chbox;
+        S.ixseg = S.chseg;
     } else if (h->ix_gen == h->set_gen) {
         S.ixoff = P<uint32_t>(h->ixoff);
         S.ixbox = P<float4>(h->ixbox);
+        S.ixseg = P<uint4>(h->ixseg);
     } else {
         S.ixoff = nullptr;
         S.ixbox = nullptr;
+        S.ixseg = nullptr;
     }
     S.pixedges = P<uint32_t>(h->pixedges);
     S.voff = P<uint32_t>(h->voff);

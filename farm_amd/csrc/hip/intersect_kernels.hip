@@ -491,7 +491,7 @@ __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uin
             const float big = 0x1p40f;
             if (!(open && fabsf(cx) + hx < big && fabsf(cy) + hy < big)) hx = hy = INFINITY;
             box[o] = make_float4(cx, cy, hx, hy);
-            if (seg) seg[o] = make_uint4(sq.x + base - 1, n | mark, (uint32_t)dirs, (uint32_t)(dirs >> 32));
+            seg[o] = make_uint4(sq.x + base - 1, n | mark, (uint32_t)dirs, (uint32_t)(dirs >> 32));
         }
     }
 }

@@ -17,13 +17,12 @@
 // One wavefront per pair:
 //  1. the source raster's window over the target MBB; all OUT / all IN
 //     windows end the pair (the reference's early return)
-//  2. every edge pair of every BORDER x BORDER pixel pair's sequence pairs:
-//     source edges on lanes, target vertices streamed; a line screen (the
-//     side of each target vertex against the source edge's line, with a
-//     margin above the f32 rounding) drops edge pairs that cannot cross;
-//     the rest are queued in LDS and take the reference's exact f32 / f64
-//     test a wave at a time; hits are appended to a per-wave record slab in
-//     global memory
+//  2. every edge pair of every BORDER x BORDER pixel pair: screens over the
+//     pixels' 16-segment chunks (boxes and directions, then the sides of a
+//     box and of each vertex against the source edge's line, with margins
+//     above the f32 rounding) drop edge pairs that cannot cross; the rest
+//     take the reference's exact f32 / f64 test a wave at a time; hits are
+//     appended to a per-wave record slab in global memory
 //  3. bitonic sorts of the slab (by point; by source edge and parameter;
 //     by target edge and parameter), de-duplication, pieces, their statuses
 //     (point-in-polygon tests, wave-cooperative when a chunk holds few
@@ -454,235 +453,189 @@ __device__ __forceinline__ void edge_test(float ax, float ay, float d1x, float d
     }
 }
 
-// Edge pairs that passed the line screen below, waiting for the exact test:
-// vertex indexes of the source and target edge's first vertex.
-constexpr uint32_t kQueue = 128;  // flushed once 64 are queued, so one push always fits
-struct EdgeQueue {
-    uint32_t ea[kQueue];
-    uint32_t eb[kQueue];
-};
-
-// The exact test (edge_test) of every queued edge pair, one per lane.
-__device__ __forceinline__ void flush_edges(const float *AX, const float *AY, const float *BX, const float *BY,
-                                            EdgeQueue &Q, uint32_t &qn, Rec *R, uint32_t cap, uint32_t *cnt,
-                                            int lane) {
-    wave_sync();
-    for (uint32_t k = lane; k < qn; k += 64) {
-        const uint32_t ea = Q.ea[k], eb = Q.eb[k];
-        const float ax = AX[ea], ay = AY[ea], bx = BX[eb], by = BY[eb];
-        edge_test(ax, ay, AX[ea + 1] - ax, AY[ea + 1] - ay, bx, by, BX[eb + 1] - bx, BY[eb + 1] - by, ea, eb, R,
-                  cap, cnt);
-    }
-    qn = 0;
-    wave_sync();
-}
-
-// Appends the lanes with cand set (ballot prefix); qn is wave-uniform.
-__device__ __forceinline__ void push_edge(bool cand, uint32_t ea, uint32_t eb, const float *AX, const float *AY,
-                                          const float *BX, const float *BY, EdgeQueue &Q, uint32_t &qn, Rec *R,
-                                          uint32_t cap, uint32_t *cnt, int lane) {
-    const uint64_t m = __ballot(cand);
-    if (m == 0) return;
-    if (cand) {
-        const uint32_t pos = qn + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        Q.ea[pos] = ea;
-        Q.eb[pos] = eb;
-    }
-    qn = uni(qn + (uint32_t)__popcll(m));
-    if (qn >= 64) flush_edges(AX, AY, BX, BY, Q, qn, R, cap, cnt, lane);
-}
-
-// Line screen.  For the source edge a + s*d1 of a lane, o_j = (b_j - a) x d1
-// is computed with edge_test's own c1 expression, once per target vertex, and
-// serves the two target edges that meet at b_j.  edge_test accepts edge j only
-// if u = o_j / dn lies in [-1e-9, 1 + 1e-9]; in exact arithmetic o_{j+1} =
-// o_j - dn, and the rounding of o_j, o_{j+1} and dn (each product and
-// difference rounded once, f32) moves o_{j+1} - (o_j - dn) by at most
-// 2^-21 * |d1|max * (R_j + R_{j+1}), R = |b - a|_1, while 1e-9 * |dn| stays
-// below 2^-29 of the same scale.  So an accepted edge has min(o_j, o_{j+1})
-// <= m and max(o_j, o_{j+1}) >= -m for m = 2^-19 * |d1|_1 * (R_j + R_{j+1})
-// (four times the bound, which absorbs the rounding of m itself); edges that
-// fail the screen cannot produce a record, and the rest go to the exact test.
-struct LineProbe {
-    float o, r;
-};
-__device__ __forceinline__ LineProbe line_probe(float ax, float ay, float d1x, float d1y, float bx, float by) {
-    const float rx = bx - ax, ry = by - ay;
-    return {rx * d1y - ry * d1x, fabsf(rx) + fabsf(ry)};
-}
-__device__ __forceinline__ bool line_pass(LineProbe p0, LineProbe p1, float k) {
-    const float m = k * (p0.r + p1.r);
-    return (p0.o <= m || p1.o <= m) && (p0.o >= -m || p1.o >= -m);
-}
-
-// Target vertices read through the constant address space: the vertex arrays
-// do not change during a launch, and uniform addresses then become scalar
-// loads.
-typedef __attribute__((address_space(4))) const float cfloat;
-constexpr int kScreenChunk = 16;  // target vertices per chunk (<= the vertex padding)
-static_assert(kScreenChunk == (int)kIxChunk, "the chunk skip reads kIxChunk-segment boxes");
-
-// Queues the lanes of mask (vertex indexes ea per lane, eb uniform).
-__device__ __forceinline__ void push_mask(uint64_t mask, uint32_t ea, uint32_t eb, const float *AX, const float *AY,
-                                          const float *BX, const float *BY, EdgeQueue &Q, uint32_t &qn, Rec *R,
-                                          uint32_t cap, uint32_t *cnt, int lane) {
-    if ((mask >> lane) & 1ull) {
-        const uint32_t pos = qn + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-        Q.ea[pos] = ea;
-        Q.eb[pos] = eb;
-    }
-    qn = uni(qn + (uint32_t)__popcll(mask));
-    if (qn >= 64) flush_edges(AX, AY, BX, BY, Q, qn, R, cap, cnt, lane);
-}
-
-// One lane's source edge for the chunked screen, and the side masks of a
-// target vertex: o = (q - a) x d1 (fused: the screen's own value, within the
-// same error bound as the reference's c1, which the margin M covers); bits of
-// gt / lt set where o > M / o < -M (fcmp predicates 2 and 4, ordered).
-struct ScreenLane {
-    float ax, ay, d1x, d1y, M;
-};
-__device__ __forceinline__ void screen_side(const ScreenLane &L, float qx, float qy, uint64_t &gt, uint64_t &lt) {
-    const float o = fmaf(qx - L.ax, L.d1y, -((qy - L.ay) * L.d1x));
-    gt = __builtin_amdgcn_fcmpf(o, L.M, 2);
-    lt = __builtin_amdgcn_fcmpf(o, -L.M, 4);
-}
-
-// Target edges j0 .. j0 + nstep - 1 (nstep == kScreenChunk unless TAIL): the
-// vertices of the chunk are uniform scalar loads, which may read up to
-// kScreenChunk - 1 vertices past the sequence, inside the zeroed padding that
-// follows the vertex arrays at worst.  An edge passes unless both its
-// vertices lie beyond the margin on one side.
-template <bool TAIL>
-__device__ __forceinline__ void screen_chunk(const ScreenLane &L, const cfloat *bxc, const cfloat *byc, uint32_t j0,
-                                             uint32_t nstep, uint64_t on_mask, uint64_t &gt, uint64_t &lt,
-                                             uint32_t ea, uint32_t lb, const float *AX, const float *AY,
-                                             const float *BX, const float *BY, EdgeQueue &Q, uint32_t &qn, Rec *R,
-                                             uint32_t cap, uint32_t *cnt, int lane) {
-    float qx[kScreenChunk], qy[kScreenChunk];
-#pragma unroll
-    for (int m = 0; m < kScreenChunk; m++) {
-        qx[m] = bxc[j0 + 1 + m];
-        qy[m] = byc[j0 + 1 + m];
-    }
-    // the failing lanes of each step; the active-lane mask is applied once,
-    // to the chunk's summary and to the steps that push
-    uint64_t fail[kScreenChunk];
-    uint64_t all_fail = ~0ull;
-#pragma unroll
-    for (int m = 0; m < kScreenChunk; m++) {
-        uint64_t gt1, lt1;
-        screen_side(L, qx[m], qy[m], gt1, lt1);
-        fail[m] = (gt & gt1) | (lt & lt1);
-        if (TAIL && (uint32_t)m >= nstep) fail[m] = ~0ull;
-        all_fail &= fail[m];
-        gt = gt1;
-        lt = lt1;
-    }
-    if (~all_fail & on_mask) {
-#pragma unroll
-        for (int m = 0; m < kScreenChunk; m++) {
-            const uint64_t pass = ~fail[m] & on_mask;
-            if (pass) push_mask(pass, ea, lb + j0 + m, AX, AY, BX, BY, Q, qn, R, cap, cnt, lane);
-        }
-    }
-}
-
-// All edge pairs of one sequence pair.  Source edges go to lanes and stay in
-// registers; when the source sequence fills the wave, the target vertices
-// stream in uniform chunks (scalar loads), else lanes split into phases, each
-// over a contiguous block of the target edges.  Pairs passing the line screen
-// are queued for the exact test.
+// ------------------------------------------------------------------------
+// Collection: the edge pairs of one BORDER x BORDER pixel pair that may cross,
+// narrowed down over the pixels' kIxChunk-segment chunks (a pixel's chunks are
+// one consecutive range, whatever sequences they belong to) through three
+// queues in LDS, each worked off 64 items or more at a time:
+//   1. every (source chunk, target chunk) pair, one per lane: kept unless
+//      their boxes are apart and their direction masks have no common bit;
+//   2. every (edge of the source chunk, target chunk), 16 lanes to a pair:
+//      kept unless the target box lies on one side of the edge's line;
+//   3. every segment of the target chunk against the edge, one (edge, chunk)
+//      per lane: kept unless both its ends lie on one side of the line;
+//   4. the exact test (edge_test).
+// On complex x lakes 1 keeps a fifth of the chunk pairs, 2 a tenth of their
+// edges.  Walking the sequence pairs one by one, a wave of source edges against
+// each target chunk, took 58 % of the kernel there (259 ms for 618,000 pairs,
+// 138 with this), and more on jagged rings (pixels of 8 sequences of 3 edges).
 //
-// Chunk skip (cbox: the target sequence's kIxChunk-segment chunk boxes,
-// centre and rounded-up half extents; null: none).  Every vertex q of a chunk
-// lies in its box, so the exact o(q) = (q - a) x d1 is within
-// S = |d1y| hx + |d1x| hy of o at the centre c.  The f32 o of the screen errs
-// by at most 2^-22 |d1|_1 R + 2^-24 |o| (R = |q - a|_1 <= Rmax, the box lies
-// in the sequence's box), i.e. by M / 16 and a relative ulp, and so does the
-// f32 o(c).  When the f32 o(c) exceeds T = S (1 + 2^-20) + 2 M + 2^-100 in
-// magnitude, every vertex's f32 o lies beyond M on the side of o(c): the
-// screen would fail every edge of the chunk, and the vertices' side masks are
-// those of the sign of o(c).  A chunk every active lane skips is passed over
-// whole (its vertices are not loaded).  An infinite box (a zero-length
-// segment, a non-finite vertex) makes T infinite or NaN and is never skipped.
-__device__ __forceinline__ void collect_seq_pair(const float *AX, const float *AY, const float *BX, const float *BY,
-                                                 uint2 e1, uint2 e2, const cfloat *cbox, EdgeQueue &Q, uint32_t &qn,
-                                                 Rec *R, uint32_t cap, uint32_t *cnt, int lane) {
-    const uint32_t la = e1.x, na = e1.y, lb = e2.x, nb = e2.y;  // first edge, edge count
-    if (na == 0 || nb == 0) return;
-    if (na >= 48) {
-        // the target sequence's box bounds every R_j of the screen: with
-        // R_j, R_j+1 <= Rmax = max|bx - ax| + max|by - ay| over the box, one
-        // margin M = 2^-19 * |d1|_1 * 2 * Rmax >= m serves the whole
-        // sequence, and each vertex's side of the line (o > M, o < -M) is a
-        // lane mask shared by its two edges
-        float bx0 = INFINITY, by0 = INFINITY, nbx1 = INFINITY, nby1 = INFINITY;
-        for (uint32_t v = lane; v <= nb; v += 64) {
-            const float x = BX[lb + v], y = BY[lb + v];
-            bx0 = fminf(bx0, x);
-            by0 = fminf(by0, y);
-            nbx1 = fminf(nbx1, -x);
-            nby1 = fminf(nby1, -y);
+// 1 is the refinement's direction prune.  A record needs t, u within 1e-9 of
+// [0, 1]; the f32 crosses err by less than 2^-22 times the L1 lengths of their
+// operands, so u puts a point of the target segment within (2^-22 3 q + 1e-9
+// 2 q) sqrt 2 < 2^-20 q of the source line and t one of the source edge that
+// near the target line (q the L1 reach).  With the boxes apart by g >= 2^-8 q
+// the two lines then meet at less than 2 2^-20 q / g = 2^-11, and chunks that
+// hold such segments share a direction bit (kDirTol = 2^-9).  Segments of
+// length 0 give no record (dn = 0).
+//
+// 2 and 3: for the source edge a + s*d1, o(q) = (q - a) x d1 is the side of
+// target vertex q.  edge_test accepts edge j only if u = o_j / dn lies in
+// [-1e-9, 1 + 1e-9]; in exact arithmetic o_{j+1} = o_j - dn, and the rounding
+// of o_j, o_{j+1} and dn (each product and difference rounded once, f32) moves
+// o_{j+1} - (o_j - dn) by at most 2^-21 |d1|max (R_j + R_{j+1}), R = |q - a|_1,
+// while 1e-9 |dn| stays below 2^-29 of the same scale.  So an accepted edge has
+// min(o_j, o_{j+1}) <= M and max(o_j, o_{j+1}) >= -M for M = 2^-18 |d1|_1 Rmax,
+// Rmax the reach of the chunk's box (four times the bound, which absorbs the
+// rounding of M and of the fused o of the screen).  Every vertex q of a chunk
+// lies in its box, so o(q) is within S = |d1y| hx + |d1x| hy of o at the centre
+// c; the f32 o errs by at most M / 16 and a relative ulp.  When the f32 |o(c)|
+// exceeds T = S (1 + 2^-20) + 2 M + 2^-100, every vertex lies beyond M on the
+// side of o(c).  An infinite box (a non-finite vertex) makes T infinite or NaN
+// and is never dropped.
+// ------------------------------------------------------------------------
+constexpr uint32_t kQueue = 128;  // flushed once 64 are queued, so one push always fits
+struct PairQueue {
+    uint32_t a[kQueue];
+    uint32_t b[kQueue];
+};
+struct Queues {
+    PairQueue chunks;  // source chunk, target chunk
+    PairQueue lines;   // source edge's first vertex, target chunk
+    PairQueue edges;   // first vertices of the source and target edge
+};
+
+// Wave-uniform state of one pair's collection.
+struct Collect {
+    const float4 *box;  // DevSet::ixbox / ixseg
+    const uint4 *seg;
+    const float *AX, *AY, *BX, *BY;
+    Queues *q;
+    uint32_t nc, nl, ne;  // queued items
+    Rec *R;
+    uint32_t cap;
+    uint32_t *cnt;
+    int lane;
+};
+
+__device__ __forceinline__ void push_pair(PairQueue &q, uint32_t &n, bool keep, uint32_t a, uint32_t b, int lane) {
+    const uint64_t m = __ballot(keep);
+    if (keep) {
+        const uint32_t pos = n + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        q.a[pos] = a;
+        q.b[pos] = b;
+    }
+    n = uni(n + (uint32_t)__popcll(m));
+}
+
+// 4: the exact test of every queued edge pair, one per lane.
+__device__ __forceinline__ void flush_edges(Collect &C) {
+    wave_sync();
+    for (uint32_t k = C.lane; k < C.ne; k += 64) {
+        const uint32_t ea = C.q->edges.a[k], eb = C.q->edges.b[k];
+        const float ax = C.AX[ea], ay = C.AY[ea], bx = C.BX[eb], by = C.BY[eb];
+        edge_test(ax, ay, C.AX[ea + 1] - ax, C.AY[ea + 1] - ay, bx, by, C.BX[eb + 1] - bx, C.BY[eb + 1] - by, ea, eb,
+                  C.R, C.cap, C.cnt);
+    }
+    C.ne = 0;
+    wave_sync();
+}
+
+// the margin M of edge a + s * d1 against a chunk's box
+__device__ __forceinline__ float line_margin(float ax, float ay, float d1x, float d1y, float4 bb) {
+    const float r = ((fabsf(bb.x - ax) + bb.z) + (fabsf(bb.y - ay) + bb.w)) * 1.000001f;
+    return 0x1p-18f * (fabsf(d1x) + fabsf(d1y)) * r;
+}
+
+// 3: the first n <= 64 queued (edge, chunk) items, one per lane.
+__device__ __forceinline__ void flush_lines(Collect &C, uint32_t n) {
+    wave_sync();
+    const bool on = (uint32_t)C.lane < n;
+    const uint32_t k = on ? (uint32_t)C.lane : 0u;
+    const uint32_t ea = C.q->lines.a[k], cb = C.q->lines.b[k];
+    const uint4 sg = C.seg[cb];
+    const float4 bb = C.box[cb];
+    const uint32_t v0 = sg.x, ns = on ? sg.y & (kChunkPoint - 1u) : 0u;
+    const float ax = C.AX[ea], ay = C.AY[ea];
+    const float d1x = C.AX[ea + 1] - ax, d1y = C.AY[ea + 1] - ay;
+    const float M = line_margin(ax, ay, d1x, d1y, bb);
+    // the items behind the first 64 move up (read before they are overwritten)
+    const bool more = (uint32_t)C.lane + n < C.nl;
+    const uint32_t ma = more ? C.q->lines.a[C.lane + n] : 0u, mb = more ? C.q->lines.b[C.lane + n] : 0u;
+    wave_sync();
+    if (more) {
+        C.q->lines.a[C.lane] = ma;
+        C.q->lines.b[C.lane] = mb;
+    }
+    C.nl -= n;
+    auto side = [&](uint32_t v) { return fmaf(C.BX[v] - ax, d1y, -((C.BY[v] - ay) * d1x)); };
+    float o = side(v0);
+    for (uint32_t m = 0; __ballot(m < ns); m++) {
+        const uint32_t v = v0 + min(m + 1, ns);
+        const float p = side(v);
+        const bool keep = m < ns && !((o > M && p > M) || (o < -M && p < -M));
+        if (__ballot(keep)) {
+            push_pair(C.q->edges, C.ne, keep, ea, v0 + m, C.lane);
+            if (C.ne >= 64) flush_edges(C);
         }
-        bx0 = wave_min(bx0);
-        by0 = wave_min(by0);
-        const float bx1 = -wave_min(nbx1), by1 = -wave_min(nby1);
-        const cfloat *bxc = (const cfloat *)(BX + lb), *byc = (const cfloat *)(BY + lb);
-        for (uint32_t i0 = 0; i0 < na; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            const bool on = i < na;
-            const uint32_t ea = la + (on ? i : 0);
-            const float ax = AX[ea], ay = AY[ea];
-            const float d1x = AX[ea + 1] - ax, d1y = AY[ea + 1] - ay;
-            const float rmax = fmaxf(fabsf(bx0 - ax), fabsf(bx1 - ax)) + fmaxf(fabsf(by0 - ay), fabsf(by1 - ay));
-            const float M = 0x1p-18f * (fabsf(d1x) + fabsf(d1y)) * rmax;
-            const uint64_t on_mask = __ballot(on);
-            ScreenLane L{ax, ay, d1x, d1y, M};
-            uint64_t gt, lt;
-            screen_side(L, bxc[0], byc[0], gt, lt);
-            const float ad1x = fabsf(d1x), ad1y = fabsf(d1y);
-            const float T0 = fmaf(M, 2.f, 0x1p-100f);
-            // true when every active lane skips chunk c (then gt / lt are the
-            // side masks of its last vertex)
-            auto skip_chunk = [&](uint32_t c) -> bool {
-                if (!cbox) return false;
-                const float cx = cbox[4 * c], cy = cbox[4 * c + 1], hx = cbox[4 * c + 2], hy = cbox[4 * c + 3];
-                const float oc = fmaf(cx - ax, d1y, -((cy - ay) * d1x));
-                const float T = fmaf(fmaf(ad1y, hx, ad1x * hy), 1.000001f, T0);
-                if (__ballot(on && !(fabsf(oc) > T))) return false;
-                gt = __ballot(oc > 0.f);
-                lt = __ballot(oc < 0.f);
-                return true;
-            };
-            const uint32_t nfull = nb / kScreenChunk * kScreenChunk;
-            for (uint32_t j0 = 0; j0 < nfull; j0 += kScreenChunk) {
-                if (skip_chunk(j0 / kScreenChunk)) continue;
-                screen_chunk<false>(L, bxc, byc, j0, kScreenChunk, on_mask, gt, lt, ea, lb, AX, AY, BX, BY, Q, qn, R,
-                                    cap, cnt, lane);
+        o = p;
+    }
+}
+
+// 2: every queued (source chunk, target chunk) pair, 4 per round: lane 16 i + e
+// takes edge e of pair i.
+__device__ __forceinline__ void flush_chunks(Collect &C) {
+    wave_sync();
+    const uint32_t e = (uint32_t)C.lane & 15u, sub = (uint32_t)C.lane >> 4;
+    for (uint32_t k0 = 0; k0 < C.nc; k0 += 4) {
+        const uint32_t k = k0 + sub;
+        bool keep = false;
+        uint32_t ea = 0, cb = 0;
+        if (k < C.nc) {
+            const uint4 sg = C.seg[C.q->chunks.a[k]];
+            cb = C.q->chunks.b[k];
+            if (e < (sg.y & (kChunkPoint - 1u))) {
+                const float4 bb = C.box[cb];
+                ea = sg.x + e;
+                const float ax = C.AX[ea], ay = C.AY[ea];
+                const float d1x = C.AX[ea + 1] - ax, d1y = C.AY[ea + 1] - ay;
+                const float M = line_margin(ax, ay, d1x, d1y, bb);
+                const float oc = fmaf(bb.x - ax, d1y, -((bb.y - ay) * d1x));
+                const float T = fmaf(fmaf(fabsf(d1y), bb.z, fabsf(d1x) * bb.w), 1.000001f, fmaf(M, 2.f, 0x1p-100f));
+                keep = !(fabsf(oc) > T);
             }
-            if (nfull < nb && !skip_chunk(nfull / kScreenChunk))
-                screen_chunk<true>(L, bxc, byc, nfull, nb - nfull, on_mask, gt, lt, ea, lb, AX, AY, BX, BY, Q, qn, R,
-                                   cap, cnt, lane);
         }
-    } else {
-        const uint32_t phases = 64 / na;  // >= 1
-        const uint32_t blk = (nb + phases - 1) / phases;
-        const uint32_t i = lane % na, ph = lane / na;
-        const bool on = ph < phases;
-        const uint32_t j0 = on ? min(ph * blk, nb) : nb, j1 = on ? min(j0 + blk, nb) : nb;
-        const uint32_t ea = la + i;
-        const float ax = AX[ea], ay = AY[ea];
-        const float d1x = AX[ea + 1] - ax, d1y = AY[ea + 1] - ay;
-        const float k = 0x1p-19f * (fabsf(d1x) + fabsf(d1y));
-        LineProbe p0 = line_probe(ax, ay, d1x, d1y, BX[lb + j0], BY[lb + j0]);
-        for (uint32_t t = 0; t < blk; t++) {
-            const uint32_t j = j0 + t;
-            const bool act = j < j1;
-            const uint32_t v = act ? j + 1 : j0;  // vertex lb + v is within the sequence
-            const LineProbe p1 = line_probe(ax, ay, d1x, d1y, BX[lb + v], BY[lb + v]);
-            push_edge(act && line_pass(p0, p1, k), ea, lb + j, AX, AY, BX, BY, Q, qn, R, cap, cnt, lane);
-            p0 = p1;
+        push_pair(C.q->lines, C.nl, keep, ea, cb, C.lane);
+        if (C.nl >= 64) flush_lines(C, 64);
+    }
+    C.nc = 0;
+    wave_sync();
+}
+
+// 1: all chunk pairs of source chunks [a0, a1) and target chunks [b0, b1).
+__device__ __forceinline__ void collect_chunks(Collect &C, uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1) {
+    const uint32_t na = a1 - a0, nb = b1 - b0;
+    if (na == 0 || nb == 0) return;
+    uint32_t i = (uint32_t)C.lane / nb, j = (uint32_t)C.lane - i * nb;
+    const uint32_t qi = 64u / nb, rj = 64u - qi * nb;
+    while (__ballot(i < na)) {
+        bool keep = false;
+        if (i < na) {
+            const float4 A = C.box[a0 + i], B = C.box[b0 + j];
+            const uint4 sa = C.seg[a0 + i], sb = C.seg[b0 + j];
+            const float sx = fabsf(A.x - B.x), sy = fabsf(A.y - B.y), hx = A.z + B.z, hy = A.w + B.w;
+            const float q = ((sx + hx) + (sy + hy)) * 1.000001f;
+            const float gap = fmaxf(sx - hx * 1.000001f, sy - hy * 1.000001f);
+            const bool far = gap > q * 0x1p-8f && q < 0x1p60f;
+            keep = !far || ((sa.z & sb.z) | (sa.w & sb.w)) != 0u;
+        }
+        push_pair(C.q->chunks, C.nc, keep, a0 + i, b0 + j, C.lane);
+        if (C.nc >= 64) flush_chunks(C);
+        i += qi;
+        j += rj;
+        if (j >= nb) {
+            j -= nb;
+            i++;
         }
     }
 }
@@ -690,7 +643,7 @@ __device__ __forceinline__ void collect_seq_pair(const float *AX, const float *A
 // Ideal::intersection for one pair plus the area; R / D: the wave's two
 // record slabs of cap records each (cap a power of two).
 __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const double *ring2a, uint32_t ia, uint32_t ib,
-                                                     Rec *R, Rec *D, uint32_t cap, uint32_t *cnt, EdgeQueue &Q,
+                                                     Rec *R, Rec *D, uint32_t cap, uint32_t *cnt, Queues &Q,
                                                      int lane, const PieceOut &po) {
     PairRes r;
     for (int k = 0; k < 5; k++) r.c[k] = 0;
@@ -729,7 +682,7 @@ __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const doub
     const float *BX = S.x + hB.vert_start, *BY = S.y + hB.vert_start;
     if (lane == 0) *cnt = 0u;
     wave_sync();
-    uint32_t qn = 0;
+    Collect C{S.ixbox, S.ixseg, AX, AY, BX, BY, &Q, 0u, 0u, 0u, R, cap, cnt, lane};
     for (int x = w.x0; x <= w.x1; x++) {
         for (int y = w.y0; y <= w.y1; y++) {
             const uint32_t pa = (uint32_t)(y * hA.dimx + x);
@@ -737,28 +690,24 @@ __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const doub
             double lx, ly, hx, hy;
             pixel_box(hA, x, y, lx, ly, hx, hy);
             const Window v = window_of(hB, lx, ly, hx, hy);
+            const uint32_t sa0 = S.pixoff[hA.pixoff_start + pa], sa1 = S.pixoff[hA.pixoff_start + pa + 1];
+            const uint32_t ca0 = uni(S.ixoff[hA.seq_start + sa0]), ca1 = uni(S.ixoff[hA.seq_start + sa1]);
+            const uint64_t na = S.pixedges[hA.pix_start + pa];
             for (int x2 = v.x0; x2 <= v.x1; x2++) {
                 for (int y2 = v.y0; y2 <= v.y1; y2++) {
                     const uint32_t pb = (uint32_t)(y2 * hB.dimx + x2);
                     if (show(S.status[hB.pix_start + pb]) != 1) continue;
                     r.bb++;
-                    const uint32_t sa0 = S.pixoff[hA.pixoff_start + pa], sa1 = S.pixoff[hA.pixoff_start + pa + 1];
                     const uint32_t sb0 = S.pixoff[hB.pixoff_start + pb], sb1 = S.pixoff[hB.pixoff_start + pb + 1];
-                    for (uint32_t sa = sa0; sa < sa1; sa++) {
-                        const uint2 e1 = S.seqs[hA.seq_start + sa];
-                        for (uint32_t sb = sb0; sb < sb1; sb++) {
-                            const uint2 e2 = S.seqs[hB.seq_start + sb];
-                            r.tests += (uint64_t)e1.y * e2.y;
-                            const cfloat *cb =
-                                S.ixbox ? (const cfloat *)(S.ixbox + S.ixoff[hB.seq_start + sb]) : nullptr;
-                            collect_seq_pair(AX, AY, BX, BY, e1, e2, cb, Q, qn, R, cap, cnt, lane);
-                        }
-                    }
+                    r.tests += na * S.pixedges[hB.pix_start + pb];
+                    collect_chunks(C, ca0, ca1, uni(S.ixoff[hB.seq_start + sb0]), uni(S.ixoff[hB.seq_start + sb1]));
                 }
             }
         }
     }
-    if (qn) flush_edges(AX, AY, BX, BY, Q, qn, R, cap, cnt, lane);
+    if (C.nc) flush_chunks(C);
+    while (C.nl) flush_lines(C, min(C.nl, 64u));
+    if (C.ne) flush_edges(C);
     wave_sync();
     const uint32_t nrec = uni(*cnt);
     r.raw = nrec;
@@ -862,9 +811,9 @@ __global__ __launch_bounds__(256) void k_intersection(DevSet S, const double *__
     Rec *R = slab + gw * 2ull * cap;
     Rec *D = R + cap;
     __shared__ uint32_t rec_cnt[kWaves];
-    __shared__ EdgeQueue queues[kWaves];
+    __shared__ Queues queues[kWaves];
     uint32_t *cnt = &rec_cnt[threadIdx.x >> 6];
-    EdgeQueue &Q = queues[threadIdx.x >> 6];
+    Queues &Q = queues[threadIdx.x >> 6];
     unsigned long long bb = 0, tests = 0, raw = 0, found = 0;
     for (;;) {
         uint32_t base = 0;
