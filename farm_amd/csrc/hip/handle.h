@@ -101,7 +101,7 @@ struct farm_handle_s {
     farm::DevBuf wctr, wovf, wslab, wslab_big, wout, wmd;
     // intersection
     bool ring_area_ready = false;
-    farm::DevBuf ring2a, icounts, iarea, ipieces;
+    farm::DevBuf ring2a, icounts, iarea, ipieces, ixlist, ixflag;
     // candidate generation
     farm::DevBuf cg_boxa, cg_boxq, cg_cellcnt, cg_celloff, cg_items, cg_uoff, cg_cnt, cg_off, cg_keys, cg_keys2;
     // pinned staging of the streamed vertex upload (two buffers, their DMA events)

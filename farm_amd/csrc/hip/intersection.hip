@@ -14,7 +14,8 @@
 // midpoint of its longest sub-segment is).  Without two distinct crossing
 // points the pair is contained (first vertex IN the other) or disjoint.
 //
-// One wavefront per pair:
+// One wavefront per pair, or the four of a workgroup for a pair with much work
+// (k_ix_heavy) and for calls of few pairs:
 //  1. the source raster's window over the target MBB; all OUT / all IN
 //     windows end the pair (the reference's early return)
 //  2. every edge pair of every BORDER x BORDER pixel pair: screens over the
@@ -25,8 +26,8 @@
 //     appended to a per-wave record slab in global memory
 //  3. bitonic sorts of the slab (by point; by source edge and parameter;
 //     by target edge and parameter), de-duplication, pieces, their statuses
-//     (point-in-polygon tests, wave-cooperative when a chunk holds few
-//     pieces) and the wave-cooperative path sums of the IN pieces
+//     (point-in-polygon tests, all of a wave's points together) and the
+//     wave-cooperative path sums of the IN pieces
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -51,7 +52,6 @@ struct Rec {
 constexpr int kWaves = 4;
 constexpr uint32_t kRecCap = 2048;     // records per wave slab (power of two)
 constexpr uint32_t kRecCapBig = 65536;  // second pass for pairs beyond kRecCap (a third sizes to the largest)
-constexpr uint32_t kChunk = 2;          // pairs per queue grab
 
 // Point::operator== (Point.h:32)
 __device__ __forceinline__ bool pt_eq(float ax, float ay, float bx, float by) {
@@ -93,331 +93,41 @@ __device__ __forceinline__ Rec pad_rec() {
     return r;
 }
 
+// The lanes that share one pair: one wave (NW = 1), or the NW waves of a
+// workgroup.
+template <int NW>
+struct Team {
+    int lane, wv;
+    __device__ __forceinline__ uint32_t tid() const { return (uint32_t)(NW == 1 ? lane : wv * 64 + lane); }
+    __device__ __forceinline__ bool first() const { return NW == 1 || wv == 0; }
+    __device__ __forceinline__ void sync() const {
+        if constexpr (NW == 1) wave_sync();
+        else __syncthreads();
+    }
+};
+
 // Bitonic sort of R[0, n) in place; R has room for next_pow2(n) records.
-template <int K>
-__device__ void bitonic(Rec *R, uint32_t n, int lane) {
+template <int K, int NW>
+__device__ void bitonic(Rec *R, uint32_t n, const Team<NW> &tm) {
     uint32_t m = 1;
     while (m < n) m <<= 1;
-    for (uint32_t i = n + lane; i < m; i += 64) R[i] = pad_rec();
-    wave_sync();
+    for (uint32_t i = n + tm.tid(); i < m; i += 64 * NW) R[i] = pad_rec();
+    tm.sync();
     for (uint32_t k = 2; k <= m; k <<= 1) {
         for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            for (uint32_t i = lane; i < m; i += 64) {
-                const uint32_t l = i ^ j;
-                if (l > i) {
-                    const Rec a = R[i], b = R[l];
-                    const bool up = (i & k) == 0;
-                    if (rec_less<K>(b, a) == up) {
-                        R[i] = b;
-                        R[l] = a;
-                    }
+            // pair p of this stage: i has bit j clear, l = i | j
+            for (uint32_t p = tm.tid(); p < m / 2; p += 64 * NW) {
+                const uint32_t i = 2 * p - (p & (j - 1)), l = i | j;
+                const Rec a = R[i], b = R[l];
+                const bool up = (i & k) == 0;
+                if (rec_less<K>(b, a) == up) {
+                    R[i] = b;
+                    R[l] = a;
                 }
             }
-            wave_sync();
+            tm.sync();
         }
     }
-}
-
-// Ideal::segment_contain with count_intersection_nodes (Ideal.cpp:988-1006):
-// 0 OUT, 1 BORDER (on the boundary), 2 IN
-__device__ int seg_contain(const DevSet &S, const farm_raster_hdr &h, float px, float py) {
-    const int x = off_axis((double)px, h.mbr[0], h.step[0], h.dimx);
-    const int y = off_axis((double)py, h.mbr[1], h.step[1], h.dimy);
-    const uint32_t id = (uint32_t)(y * h.dimx + x);
-    const uint8_t st = S.status[h.pix_start + id];
-    if (st == kCC - 1) return 2;
-    if (st == 0) return 0;
-    const double bx_high = h.mbr[0] + (x + 1) * h.step[0];
-    bool ret = false;
-    const uint32_t s0 = S.pixoff[h.pixoff_start + id], s1 = S.pixoff[h.pixoff_start + id + 1];
-    const float *X = S.x + h.vert_start, *Y = S.y + h.vert_start;
-    for (uint32_t e = s0; e < s1; e++) {
-        const uint2 sq = S.seqs[h.seq_start + e];
-        for (uint32_t k = 0; k < sq.y; k++) {
-            const float v1x = X[sq.x + k], v1y = Y[sq.x + k];
-            const float v2x = X[sq.x + k + 1], v2y = Y[sq.x + k + 1];
-            if (pt_eq(px, py, v1x, v1y) || pt_eq(px, py, v2x, v2y)) return 1;
-            if ((v1y >= py) != (v2y >= py)) {
-                const double dx = (double)(v2x - v1x);
-                const double dy = (double)(v2y - v1y);
-                const double pyd = (double)(py - v1y);
-                if (fabs(dy) > 1e-9) {
-                    const double ix = dx * pyd / dy + (double)v1x;
-                    if (fabs((double)px - ix) < 1e-9) return 1;
-                    if ((double)px < ix && ix <= bx_high) ret = !ret;
-                }
-            } else if (v1y == py && v2y == py && ((v1x >= px) != (v2x >= px))) {
-                return 1;
-            }
-        }
-    }
-    const uint32_t *vo = S.voff + h.vline_start;
-    uint32_t i = vo[x + 1];
-    const uint32_t j = vo[x + 2];
-    int cnt = 0;
-    while (i < j && S.vnodes[h.vnode_start + i] < (double)py) {
-        cnt++;
-        i++;
-    }
-    if (cnt & 1) ret = !ret;
-    return ret ? 2 : 0;
-}
-
-// seg_contain for one point (the same for every lane), the whole wave
-// testing the pixel's edges together.  The serial form returns 1 at the first
-// edge that puts the point on the boundary, else the parity of the crossings
-// to the right within the pixel and of the sorted grid-line nodes below it:
-// neither depends on the order the edges are visited in, so "on" is a wave
-// any, the parity a ballot count, and the node prefix a count of nodes < py.
-__device__ int seg_contain_wave(const DevSet &S, const farm_raster_hdr &h, float px, float py, int lane) {
-    const int x = off_axis((double)px, h.mbr[0], h.step[0], h.dimx);
-    const int y = off_axis((double)py, h.mbr[1], h.step[1], h.dimy);
-    const uint32_t id = (uint32_t)(y * h.dimx + x);
-    const uint8_t st = S.status[h.pix_start + id];
-    if (st == kCC - 1) return 2;
-    if (st == 0) return 0;
-    const double bx_high = h.mbr[0] + (x + 1) * h.step[0];
-    bool on = false, par = false;
-    const uint32_t s0 = S.pixoff[h.pixoff_start + id], s1 = S.pixoff[h.pixoff_start + id + 1];
-    const float *X = S.x + h.vert_start, *Y = S.y + h.vert_start;
-    for (uint32_t e = s0; e < s1; e++) {
-        const uint2 sq = S.seqs[h.seq_start + e];
-        for (uint32_t k = lane; k < sq.y; k += 64) {
-            const float v1x = X[sq.x + k], v1y = Y[sq.x + k];
-            const float v2x = X[sq.x + k + 1], v2y = Y[sq.x + k + 1];
-            if (pt_eq(px, py, v1x, v1y) || pt_eq(px, py, v2x, v2y)) on = true;
-            if ((v1y >= py) != (v2y >= py)) {
-                const double dx = (double)(v2x - v1x);
-                const double dy = (double)(v2y - v1y);
-                const double pyd = (double)(py - v1y);
-                if (fabs(dy) > 1e-9) {
-                    const double ix = dx * pyd / dy + (double)v1x;
-                    if (fabs((double)px - ix) < 1e-9) on = true;
-                    if ((double)px < ix && ix <= bx_high) par = !par;
-                }
-            } else if (v1y == py && v2y == py && ((v1x >= px) != (v2x >= px))) {
-                on = true;
-            }
-        }
-    }
-    if (wave_any(on)) return 1;
-    uint32_t cnt = (uint32_t)__popcll(__ballot(par));
-    const uint32_t *vo = S.voff + h.vline_start;
-    const uint32_t i = vo[x + 1], j = vo[x + 2];
-    for (uint32_t k0 = i; k0 < j; k0 += 64) {
-        const uint32_t k = k0 + lane;
-        cnt += (uint32_t)__popcll(__ballot(k < j && S.vnodes[h.vnode_start + k] < (double)py));
-    }
-    return (cnt & 1) ? 2 : 0;
-}
-
-// The IN pieces of a pair go to buf (when requested), one atomic per wave
-// and chunk; beyond cap they are only counted.
-struct PieceOut {
-    farm_piece *buf;
-    uint32_t *cnt;
-    uint32_t cap;
-    uint32_t pair;
-};
-
-__device__ __forceinline__ void put_pieces(const PieceOut &po, bool mine, const farm_piece &p, int lane) {
-    const uint64_t m = __ballot(mine);
-    if (!po.buf || !m) return;
-    uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(po.cnt, (uint32_t)__popcll(m));
-    base = uni(__shfl(base, 0, 64));
-    if (mine) {
-        const uint32_t k = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        if (k < po.cap) po.buf[k] = p;
-    }
-}
-
-struct PairRes {
-    int32_t c[5];  // [crossing points, pieces, IN, OUT, BORDER]
-    double area;
-    uint64_t bb, tests, raw;
-    bool over;
-};
-
-// Path point k of an area piece: 0 = a, 1..nvert = ring vertices from
-// `first` (cyclic over m), nvert + 1 = b.
-__device__ __forceinline__ void path_pt(const float *X, const float *Y, int m, int first, int nvert, float ax,
-                                        float ay, float bx, float by, int k, float &x, float &y) {
-    if (k == 0) {
-        x = ax;
-        y = ay;
-    } else if (k == nvert + 1) {
-        x = bx;
-        y = by;
-    } else {
-        int v = first + k - 1;
-        if (v >= m) v -= m;
-        x = X[v];
-        y = Y[v];
-    }
-}
-
-constexpr int kLanePath = 16;  // area-piece paths of at most this many segments are searched by one lane
-
-// One ring's pieces: D[0, n) sorted by this ring's (edge, parameter).
-// Counts the reference pieces by status into r and returns this lane's part
-// of the cross-product sum of the area pieces IN the other polygon.
-template <bool SRC>
-__device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const farm_raster_hdr &hq, const Rec *D,
-                              uint32_t n, double ox, double oy, int lane, PairRes &r, uint32_t &pieces,
-                              const PieceOut &po) {
-    const float *X = S.x + hp.vert_start, *Y = S.y + hp.vert_start;
-    const int m = (int)hp.nverts - 1;
-    const double eps = (double)1e-6f;  // util.h:44
-    double acc = 0.0;
-    for (uint32_t c0 = 0; c0 < n; c0 += 64) {
-        const uint32_t i = c0 + lane;
-        bool piece = false, in_area = false, long_path = false;
-        int st = 0, first = 0, nvert = 0;
-        float ax = 0, ay = 0, bx = 0, by = 0;
-        float rx = 0, ry = 0, mx = 0, my = 0;  // the two points tested against the other polygon
-        if (i < n) {
-            const Rec a = D[i], b = D[(i + 1) % n];
-            ax = a.px;
-            ay = a.py;
-            bx = b.px;
-            by = b.py;
-            if (!pt_eq(a.px, a.py, b.px, b.py)) {
-                piece = true;
-                // the reference's segment (Ideal.cpp:1559-1581, 1592-1614)
-                const int ea0 = SRC ? a.ei : a.ej, eb0 = SRC ? b.ei : b.ej;
-                const double ta0 = SRC ? a.t : a.u, tb0 = SRC ? b.t : b.u;
-                int ae = ea0, be = eb0;
-                double ap = ta0, bp = tb0;
-                if (fabs(ap - 1.0) < eps) {
-                    ae = (ae + 1) % m;
-                    ap = 0.0;
-                }
-                if (fabs(bp) < eps) {
-                    be--;
-                    bp = 1.0;
-                }
-                if (ae == be && ap < bp) {
-                    rx = (a.px + b.px) * 0.5f;
-                    ry = (a.py + b.py) * 0.5f;
-                } else {
-                    rx = X[ae + 1];
-                    ry = Y[ae + 1];
-                }
-                // the area piece: a -> ring vertices ea0 + 1 .. eb0 -> b
-                if (i + 1 < n) nvert = eb0 - ea0;
-                else nvert = (eb0 - ea0 + m) % m + ((eb0 == ea0 && tb0 <= ta0) ? m : 0);
-                if (nvert < 0) nvert = 0;
-                first = ea0 + 1;
-                // the area's test point: the midpoint of the path's longest
-                // sub-segment (the first on ties), well inside the piece; a
-                // path of more than kLanePath segments is searched by the
-                // whole wave below
-                if (nvert + 1 <= kLanePath) {
-                    float ux = ax, uy = ay, vx = ax, vy = ay, px = ax, py = ay;
-                    double best = -1.0;
-                    for (int k = 1; k <= nvert + 1; k++) {
-                        float qx, qy;
-                        path_pt(X, Y, m, first, nvert, ax, ay, bx, by, k, qx, qy);
-                        const double dx = (double)qx - px, dy = (double)qy - py;
-                        const double l = dx * dx + dy * dy;
-                        if (l > best) {
-                            best = l;
-                            ux = px;
-                            uy = py;
-                            vx = qx;
-                            vy = qy;
-                        }
-                        px = qx;
-                        py = qy;
-                    }
-                    mx = (ux + vx) * 0.5f;
-                    my = (uy + vy) * 0.5f;
-                } else {
-                    long_path = true;
-                }
-            }
-        }
-        // long paths, one at a time: segment k (points k - 1 -> k) on lane
-        // (k - 1) % 64; each lane keeps its first longest, then the wave takes
-        // the longest with the smallest k
-        uint64_t lp = __ballot(long_path);
-        while (lp) {
-            const int src = __ffsll((unsigned long long)lp) - 1;
-            lp &= lp - 1;
-            const int f = uni(__shfl(first, src, 64)), nv = uni(__shfl(nvert, src, 64));
-            const float pax = uni(__shfl(ax, src, 64)), pay = uni(__shfl(ay, src, 64));
-            const float pbx = uni(__shfl(bx, src, 64)), pby = uni(__shfl(by, src, 64));
-            double best = -1.0;
-            int bk = INT_MAX;
-            float ux = 0.f, uy = 0.f, vx = 0.f, vy = 0.f;
-            for (int k = 1 + lane; k <= nv + 1; k += 64) {
-                float x0, y0, x1, y1;
-                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k - 1, x0, y0);
-                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k, x1, y1);
-                const double dx = (double)x1 - x0, dy = (double)y1 - y0;
-                const double l = dx * dx + dy * dy;
-                if (l > best) {
-                    best = l;
-                    bk = k;
-                    ux = x0;
-                    uy = y0;
-                    vx = x1;
-                    vy = y1;
-                }
-            }
-            const double top = -wave_min(-best);
-            int kk = best == top ? bk : INT_MAX;
-            for (int o = 32; o > 0; o >>= 1) kk = min(kk, __shfl_xor(kk, o, 64));
-            const int wl = __ffsll((unsigned long long)__ballot(best == top && bk == kk)) - 1;
-            const float wmx = (__shfl(ux, wl, 64) + __shfl(vx, wl, 64)) * 0.5f;
-            const float wmy = (__shfl(uy, wl, 64) + __shfl(vy, wl, 64)) * 0.5f;
-            if (lane == src) {
-                mx = wmx;
-                my = wmy;
-            }
-        }
-        const uint64_t pm = __ballot(piece);
-        if (__popcll(pm) <= 32) {
-            // few pieces: the wave tests each point's pixel edges together
-            uint64_t q = pm;
-            while (q) {
-                const int src = __ffsll((unsigned long long)q) - 1;
-                q &= q - 1;
-                const int s1 = seg_contain_wave(S, hq, uni(__shfl(rx, src, 64)), uni(__shfl(ry, src, 64)), lane);
-                const int s2 = seg_contain_wave(S, hq, uni(__shfl(mx, src, 64)), uni(__shfl(my, src, 64)), lane);
-                if (lane == src) {
-                    st = s1;
-                    in_area = s2 == 2;
-                }
-            }
-        } else if (piece) {
-            st = seg_contain(S, hq, rx, ry);
-            in_area = seg_contain(S, hq, mx, my) == 2;
-        }
-        r.c[1] += __popcll(pm);
-        r.c[2] += __popcll(__ballot(piece && st == 2));
-        r.c[3] += __popcll(__ballot(piece && st == 0));
-        r.c[4] += __popcll(__ballot(piece && st == 1));
-        pieces += __popcll(pm);
-        put_pieces(po, in_area, farm_piece{po.pair, SRC ? 0 : 1, first, nvert, ax, ay, bx, by}, lane);
-        // wave-cooperative path sums of this chunk's IN pieces
-        uint64_t inm = __ballot(in_area);
-        while (inm) {
-            const int src = __ffsll((unsigned long long)inm) - 1;
-            inm &= inm - 1;
-            const int f = __shfl(first, src, 64), nv = __shfl(nvert, src, 64);
-            const float pax = __shfl(ax, src, 64), pay = __shfl(ay, src, 64);
-            const float pbx = __shfl(bx, src, 64), pby = __shfl(by, src, 64);
-            for (int k = lane; k <= nv; k += 64) {
-                float x0, y0, x1, y1;
-                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k, x0, y0);
-                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k + 1, x1, y1);
-                acc += ((double)x0 - ox) * ((double)y1 - oy) - ((double)x1 - ox) * ((double)y0 - oy);
-            }
-        }
-    }
-    return acc;
 }
 
 // The reference's crossing test of source edge ea and target edge eb
@@ -612,12 +322,16 @@ __device__ __forceinline__ void flush_chunks(Collect &C) {
     wave_sync();
 }
 
-// 1: all chunk pairs of source chunks [a0, a1) and target chunks [b0, b1).
-__device__ __forceinline__ void collect_chunks(Collect &C, uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1) {
+// 1: the chunk pairs of source chunks [a0, a1) and target chunks [b0, b1), 64
+// at a time: rounds start, start + NW, ..
+template <int NW>
+__device__ __forceinline__ void collect_chunks(Collect &C, uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1,
+                                               uint32_t start) {
     const uint32_t na = a1 - a0, nb = b1 - b0;
     if (na == 0 || nb == 0) return;
-    uint32_t i = (uint32_t)C.lane / nb, j = (uint32_t)C.lane - i * nb;
-    const uint32_t qi = 64u / nb, rj = 64u - qi * nb;
+    const uint32_t f = 64u * start + (uint32_t)C.lane;
+    uint32_t i = f / nb, j = f - i * nb;
+    const uint32_t qi = 64u * NW / nb, rj = 64u * NW - qi * nb;
     while (__ballot(i < na)) {
         bool keep = false;
         if (i < na) {
@@ -640,11 +354,348 @@ __device__ __forceinline__ void collect_chunks(Collect &C, uint32_t a0, uint32_t
     }
 }
 
-// Ideal::intersection for one pair plus the area; R / D: the wave's two
-// record slabs of cap records each (cap a power of two).
+// Ideal::segment_contain with count_intersection_nodes (Ideal.cpp:988-1006) for
+// one point per lane (active lanes): 0 OUT, 1 BORDER (on the boundary), 2 IN.
+// The serial form returns 1 at the first edge that puts the point on the
+// boundary, else the parity of the crossings to the right within the pixel and
+// of the sorted grid-line nodes below the point; neither depends on the order
+// the edges are visited in.  So all points share the wave: (point, chunk of its
+// pixel) items, one per lane, drop the chunks that cannot matter (entirely
+// above, below or to the left of the point: no vertex of such a chunk is the
+// point, no edge of it straddles the point's y or crosses to its right); the
+// rest are queued and their edges tested, 16 lanes to a chunk, the answers
+// gathered per point in LDS.  (One point after the other, the wave over its
+// pixel's edges, each took a chain of six dependent loads: two thirds of the
+// kernel on complex x lakes.)
+__device__ __forceinline__ int contain_points(const DevSet &S, const farm_raster_hdr &h, float px, float py, bool active, int lane,
+                              Queues &Q) {
+    uint32_t *flag = Q.edges.a, *gx = Q.edges.a + 64;     // 1: odd crossings, 2: on the boundary; the pixel's x
+    uint32_t *pre = Q.edges.b, *ch0 = Q.edges.b + 64;     // first item and first chunk of each point
+    float *fx = (float *)Q.lines.a, *fy = (float *)Q.lines.b;
+    int res = 0, x = 0;
+    uint32_t c0 = 0, nch = 0;
+    if (active) {
+        x = off_axis((double)px, h.mbr[0], h.step[0], h.dimx);
+        const int y = off_axis((double)py, h.mbr[1], h.step[1], h.dimy);
+        const uint32_t id = (uint32_t)(y * h.dimx + x);
+        const uint8_t st = S.status[h.pix_start + id];
+        if (st == kCC - 1) res = 2;
+        else if (st != 0) {
+            const uint32_t s0 = S.pixoff[h.pixoff_start + id], s1 = S.pixoff[h.pixoff_start + id + 1];
+            c0 = S.ixoff[h.seq_start + s0];
+            nch = S.ixoff[h.seq_start + s1] - c0;
+            res = -1;
+        }
+    }
+    const bool todo = res < 0;
+    if (!__ballot(todo)) return res;
+    uint32_t total;
+    const uint32_t first = wave_excl_scan(nch, lane, &total);
+    flag[lane] = 0u;
+    gx[lane] = (uint32_t)x;
+    pre[lane] = first;
+    ch0[lane] = c0;
+    fx[lane] = px;
+    fy[lane] = py;
+    wave_sync();
+    const float *X = S.x + h.vert_start, *Y = S.y + h.vert_start;
+    uint32_t nq = 0;
+    auto flush = [&]() {
+        wave_sync();
+        const uint32_t e = (uint32_t)lane & 15u, sub = (uint32_t)lane >> 4;
+#pragma unroll 2
+        for (uint32_t k0 = 0; k0 < nq; k0 += 4) {
+            const uint32_t k = k0 + sub;
+            if (k >= nq) continue;
+            const uint32_t p = Q.chunks.a[k];
+            const uint4 sg = S.ixseg[Q.chunks.b[k]];
+            if (e >= (sg.y & (kChunkPoint - 1u))) continue;
+            const uint32_t v = sg.x + e;
+            const float v1x = X[v], v1y = Y[v], v2x = X[v + 1], v2y = Y[v + 1];
+            const float qx = fx[p], qy = fy[p];
+            bool on = pt_eq(qx, qy, v1x, v1y) || pt_eq(qx, qy, v2x, v2y), cross = false;
+            if ((v1y >= qy) != (v2y >= qy)) {
+                const double dx = (double)(v2x - v1x);
+                const double dy = (double)(v2y - v1y);
+                const double pyd = (double)(qy - v1y);
+                if (fabs(dy) > 1e-9) {
+                    const double ix = dx * pyd / dy + (double)v1x;
+                    const double bx_high = h.mbr[0] + ((int)gx[p] + 1) * h.step[0];
+                    if (fabs((double)qx - ix) < 1e-9) on = true;
+                    cross = (double)qx < ix && ix <= bx_high;
+                }
+            } else if (v1y == qy && v2y == qy && ((v1x >= qx) != (v2x >= qx))) {
+                on = true;
+            }
+            if (on) atomicOr(&flag[p], 2u);
+            if (cross) atomicXor(&flag[p], 1u);
+        }
+        nq = 0;
+        wave_sync();
+    };
+    for (uint32_t u0 = 0; u0 < total; u0 += 64) {
+        const uint32_t u = u0 + (uint32_t)lane;
+        bool keep = false;
+        uint32_t p = 0, ch = 0;
+        if (u < total) {
+            // the last point whose first item is at or before u
+#pragma unroll
+            for (uint32_t step = 32; step > 0; step >>= 1)
+                if (pre[p + step] <= u) p += step;
+            ch = ch0[p] + (u - pre[p]);
+            const float4 bb = S.ixbox[ch];
+            const double qx = (double)fx[p], qy = (double)fy[p];
+            const double ylo = (double)bb.y - (double)bb.w, yhi = (double)bb.y + (double)bb.w;
+            const double xhi = (double)bb.x + (double)bb.z * 1.00001;  // (and a crossing's rounding beyond it)
+            keep = !(qy > yhi + 1e-8 || qy < ylo - 1e-8 || qx > xhi + 1e-8);
+        }
+        push_pair(Q.chunks, nq, keep, p, ch, lane);
+        if (nq >= 64) flush();
+    }
+    if (nq) flush();
+    if (todo) {
+        const uint32_t f = flag[lane];
+        if (f & 2u) {
+            res = 1;
+        } else {
+            // grid-line nodes below the point (sorted: a binary search)
+            const uint32_t *vo = S.voff + h.vline_start;
+            uint32_t lo = vo[x + 1], hi = vo[x + 2];
+            const uint32_t i = lo;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2;
+                if (S.vnodes[h.vnode_start + mid] < (double)py) lo = mid + 1;
+                else hi = mid;
+            }
+            res = ((f ^ (lo - i)) & 1u) ? 2 : 0;
+        }
+    }
+    wave_sync();
+    return res;
+}
+
+// The IN pieces of a pair go to buf (when requested), one atomic per wave
+// and chunk; beyond cap they are only counted.
+struct PieceOut {
+    farm_piece *buf;
+    uint32_t *cnt;
+    uint32_t cap;
+    uint32_t pair;
+};
+
+__device__ __forceinline__ void put_pieces(const PieceOut &po, bool mine, const farm_piece &p, int lane) {
+    const uint64_t m = __ballot(mine);
+    if (!po.buf || !m) return;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(po.cnt, (uint32_t)__popcll(m));
+    base = uni(__shfl(base, 0, 64));
+    if (mine) {
+        const uint32_t k = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+        if (k < po.cap) po.buf[k] = p;
+    }
+}
+
+struct PairRes {
+    int32_t c[5];  // [crossing points, pieces, IN, OUT, BORDER]
+    double area;
+    uint64_t bb, tests, raw;
+    bool over;
+};
+
+// Path point k of an area piece: 0 = a, 1..nvert = ring vertices from
+// `first` (cyclic over m), nvert + 1 = b.
+__device__ __forceinline__ void path_pt(const float *X, const float *Y, int m, int first, int nvert, float ax,
+                                        float ay, float bx, float by, int k, float &x, float &y) {
+    if (k == 0) {
+        x = ax;
+        y = ay;
+    } else if (k == nvert + 1) {
+        x = bx;
+        y = by;
+    } else {
+        int v = first + k - 1;
+        if (v >= m) v -= m;
+        x = X[v];
+        y = Y[v];
+    }
+}
+
+constexpr int kLanePath = 16;  // area-piece paths of at most this many segments are searched by one lane
+
+// One ring's pieces: D[0, n) sorted by this ring's (edge, parameter).
+// Counts the reference pieces by status into r and returns this lane's part
+// of the cross-product sum of the area pieces IN the other polygon.
+// The team's waves take 64 pieces each in turn; r gets this wave's counts.
+template <bool SRC, int NW>
+__device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const farm_raster_hdr &hq, const Rec *D,
+                              uint32_t n, double ox, double oy, const Team<NW> &tm, PairRes &r, const PieceOut &po,
+                              Queues &Q) {
+    const int lane = tm.lane;
+    const float *X = S.x + hp.vert_start, *Y = S.y + hp.vert_start;
+    const int m = (int)hp.nverts - 1;
+    const double eps = (double)1e-6f;  // util.h:44
+    double acc = 0.0;
+    for (uint32_t c0 = NW == 1 ? 0u : 64u * tm.wv; c0 < n; c0 += 64 * NW) {
+        const uint32_t i = c0 + lane;
+        bool piece = false, in_area = false, long_path = false;
+        int st = 0, first = 0, nvert = 0;
+        float ax = 0, ay = 0, bx = 0, by = 0;
+        float rx = 0, ry = 0, mx = 0, my = 0;  // the two points tested against the other polygon
+        if (i < n) {
+            const Rec a = D[i], b = D[(i + 1) % n];
+            ax = a.px;
+            ay = a.py;
+            bx = b.px;
+            by = b.py;
+            if (!pt_eq(a.px, a.py, b.px, b.py)) {
+                piece = true;
+                // the reference's segment (Ideal.cpp:1559-1581, 1592-1614)
+                const int ea0 = SRC ? a.ei : a.ej, eb0 = SRC ? b.ei : b.ej;
+                const double ta0 = SRC ? a.t : a.u, tb0 = SRC ? b.t : b.u;
+                int ae = ea0, be = eb0;
+                double ap = ta0, bp = tb0;
+                if (fabs(ap - 1.0) < eps) {
+                    ae = (ae + 1) % m;
+                    ap = 0.0;
+                }
+                if (fabs(bp) < eps) {
+                    be--;
+                    bp = 1.0;
+                }
+                if (ae == be && ap < bp) {
+                    rx = (a.px + b.px) * 0.5f;
+                    ry = (a.py + b.py) * 0.5f;
+                } else {
+                    rx = X[ae + 1];
+                    ry = Y[ae + 1];
+                }
+                // the area piece: a -> ring vertices ea0 + 1 .. eb0 -> b
+                if (i + 1 < n) nvert = eb0 - ea0;
+                else nvert = (eb0 - ea0 + m) % m + ((eb0 == ea0 && tb0 <= ta0) ? m : 0);
+                if (nvert < 0) nvert = 0;
+                first = ea0 + 1;
+                // the area's test point: the midpoint of the path's longest
+                // sub-segment (the first on ties), well inside the piece; a
+                // path of more than kLanePath segments is searched by the
+                // whole wave below
+                if (nvert + 1 <= kLanePath) {
+                    float ux = ax, uy = ay, vx = ax, vy = ay, px = ax, py = ay;
+                    double best = -1.0;
+                    for (int k = 1; k <= nvert + 1; k++) {
+                        float qx, qy;
+                        path_pt(X, Y, m, first, nvert, ax, ay, bx, by, k, qx, qy);
+                        const double dx = (double)qx - px, dy = (double)qy - py;
+                        const double l = dx * dx + dy * dy;
+                        if (l > best) {
+                            best = l;
+                            ux = px;
+                            uy = py;
+                            vx = qx;
+                            vy = qy;
+                        }
+                        px = qx;
+                        py = qy;
+                    }
+                    mx = (ux + vx) * 0.5f;
+                    my = (uy + vy) * 0.5f;
+                } else {
+                    long_path = true;
+                }
+            }
+        }
+        // long paths, one at a time: segment k (points k - 1 -> k) on lane
+        // (k - 1) % 64; each lane keeps its first longest, then the wave takes
+        // the longest with the smallest k
+        uint64_t lp = __ballot(long_path);
+        while (lp) {
+            const int src = __ffsll((unsigned long long)lp) - 1;
+            lp &= lp - 1;
+            const int f = uni(__shfl(first, src, 64)), nv = uni(__shfl(nvert, src, 64));
+            const float pax = uni(__shfl(ax, src, 64)), pay = uni(__shfl(ay, src, 64));
+            const float pbx = uni(__shfl(bx, src, 64)), pby = uni(__shfl(by, src, 64));
+            double best = -1.0;
+            int bk = INT_MAX;
+            float ux = 0.f, uy = 0.f, vx = 0.f, vy = 0.f;
+            for (int k = 1 + lane; k <= nv + 1; k += 64) {
+                float x0, y0, x1, y1;
+                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k - 1, x0, y0);
+                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k, x1, y1);
+                const double dx = (double)x1 - x0, dy = (double)y1 - y0;
+                const double l = dx * dx + dy * dy;
+                if (l > best) {
+                    best = l;
+                    bk = k;
+                    ux = x0;
+                    uy = y0;
+                    vx = x1;
+                    vy = y1;
+                }
+            }
+            const double top = -wave_min(-best);
+            int kk = best == top ? bk : INT_MAX;
+            for (int o = 32; o > 0; o >>= 1) kk = min(kk, __shfl_xor(kk, o, 64));
+            const int wl = __ffsll((unsigned long long)__ballot(best == top && bk == kk)) - 1;
+            const float wmx = (__shfl(ux, wl, 64) + __shfl(vx, wl, 64)) * 0.5f;
+            const float wmy = (__shfl(uy, wl, 64) + __shfl(vy, wl, 64)) * 0.5f;
+            if (lane == src) {
+                mx = wmx;
+                my = wmy;
+            }
+        }
+        const uint64_t pm = __ballot(piece);
+        if (min(n - c0, 64u) <= 32) {
+            // both points of every piece at once: lane 32 + k takes piece k's second
+            const float qx = __shfl(mx, lane & 31, 64), qy = __shfl(my, lane & 31, 64);
+            const bool up = lane >= 32, act = (pm >> (lane & 31)) & 1u;
+            const int s = contain_points(S, hq, up ? qx : rx, up ? qy : ry, act, lane, Q);
+            const int s2 = __shfl(s, (lane + 32) & 63, 64);
+            if (piece) {
+                st = s;
+                in_area = s2 == 2;
+            }
+        } else {
+            st = contain_points(S, hq, rx, ry, piece, lane, Q);
+            in_area = contain_points(S, hq, mx, my, piece, lane, Q) == 2 && piece;
+        }
+        r.c[1] += __popcll(pm);
+        r.c[2] += __popcll(__ballot(piece && st == 2));
+        r.c[3] += __popcll(__ballot(piece && st == 0));
+        r.c[4] += __popcll(__ballot(piece && st == 1));
+        put_pieces(po, in_area, farm_piece{po.pair, SRC ? 0 : 1, first, nvert, ax, ay, bx, by}, lane);
+        // wave-cooperative path sums of this chunk's IN pieces
+        uint64_t inm = __ballot(in_area);
+        while (inm) {
+            const int src = __ffsll((unsigned long long)inm) - 1;
+            inm &= inm - 1;
+            const int f = __shfl(first, src, 64), nv = __shfl(nvert, src, 64);
+            const float pax = __shfl(ax, src, 64), pay = __shfl(ay, src, 64);
+            const float pbx = __shfl(bx, src, 64), pby = __shfl(by, src, 64);
+            for (int k = lane; k <= nv; k += 64) {
+                float x0, y0, x1, y1;
+                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k, x0, y0);
+                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k + 1, x1, y1);
+                acc += ((double)x0 - ox) * ((double)y1 - oy) - ((double)x1 - ox) * ((double)y0 - oy);
+            }
+        }
+    }
+    return acc;
+}
+
+// What the waves of a team add up over a pair, in LDS.
+struct TeamSum {
+    uint32_t cnt, nk;
+    int32_t c[5];
+    double side[2][kWaves];
+};
+
+// Ideal::intersection for one pair plus the area; R / D: the team's two record
+// slabs of cap records each (cap a power of two).  Every wave of the team
+// returns the same result.
+template <int NW>
 __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const double *ring2a, uint32_t ia, uint32_t ib,
-                                                     Rec *R, Rec *D, uint32_t cap, uint32_t *cnt, Queues &Q,
-                                                     int lane, const PieceOut &po) {
+                                                     Rec *R, Rec *D, uint32_t cap, TeamSum &T, Queues &Q,
+                                                     const Team<NW> &tm, const PieceOut &po) {
+    const int lane = tm.lane;
     PairRes r;
     for (int k = 0; k < 5; k++) r.c[k] = 0;
     r.area = 0.0;
@@ -674,33 +725,74 @@ __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const doub
     if (itn == npx) {
         r.c[0] = -2;
         r.area = fabs(ring2a[ib]) / 2.0;
-        put_pieces(po, lane == 0, farm_piece{po.pair, 1, 0, -1, 0.f, 0.f, 0.f, 0.f}, lane);  // all of B
+        put_pieces(po, tm.tid() == 0, farm_piece{po.pair, 1, 0, -1, 0.f, 0.f, 0.f, 0.f}, lane);  // all of B
         return r;
     }
-    // 2. crossing points of the edges of BORDER x BORDER pixel pairs
+    // 2. crossing points of the edges of BORDER x BORDER pixel pairs.  Lanes
+    // take 64 source pixels, then the window of one of them, so that a pixel
+    // pair needs no loads of its own before its chunks.
     const float *AX = S.x + hA.vert_start, *AY = S.y + hA.vert_start;
     const float *BX = S.x + hB.vert_start, *BY = S.y + hB.vert_start;
-    if (lane == 0) *cnt = 0u;
-    wave_sync();
-    Collect C{S.ixbox, S.ixseg, AX, AY, BX, BY, &Q, 0u, 0u, 0u, R, cap, cnt, lane};
-    for (int x = w.x0; x <= w.x1; x++) {
-        for (int y = w.y0; y <= w.y1; y++) {
+    if (tm.tid() == 0) {
+        T.cnt = 0u;
+        T.nk = 0u;
+        for (int k = 0; k < 5; k++) T.c[k] = 0;
+    }
+    tm.sync();
+    Collect C{S.ixbox, S.ixseg, AX, AY, BX, BY, &Q, 0u, 0u, 0u, R, cap, &T.cnt, lane};
+    uint32_t turn = NW == 1 ? 0u : (uint32_t)tm.wv;  // the team's waves start at different rounds
+    for (uint32_t k0 = 0; k0 < npx; k0 += 64) {
+        const uint32_t k = k0 + lane;
+        bool live = false;
+        uint32_t ca0 = 0, ca1 = 0, na = 0;
+        Window v{0, -1, 0, -1};
+        if (k < npx) {
+            const int x = w.x0 + (int)(k / wy), y = w.y0 + (int)(k % wy);
             const uint32_t pa = (uint32_t)(y * hA.dimx + x);
-            if (show(S.status[hA.pix_start + pa]) != 1) continue;
-            double lx, ly, hx, hy;
-            pixel_box(hA, x, y, lx, ly, hx, hy);
-            const Window v = window_of(hB, lx, ly, hx, hy);
-            const uint32_t sa0 = S.pixoff[hA.pixoff_start + pa], sa1 = S.pixoff[hA.pixoff_start + pa + 1];
-            const uint32_t ca0 = uni(S.ixoff[hA.seq_start + sa0]), ca1 = uni(S.ixoff[hA.seq_start + sa1]);
-            const uint64_t na = S.pixedges[hA.pix_start + pa];
-            for (int x2 = v.x0; x2 <= v.x1; x2++) {
-                for (int y2 = v.y0; y2 <= v.y1; y2++) {
-                    const uint32_t pb = (uint32_t)(y2 * hB.dimx + x2);
-                    if (show(S.status[hB.pix_start + pb]) != 1) continue;
+            live = show(S.status[hA.pix_start + pa]) == 1;
+            if (live) {
+                double lx, ly, hx, hy;
+                pixel_box(hA, x, y, lx, ly, hx, hy);
+                v = window_of(hB, lx, ly, hx, hy);
+                const uint32_t s0 = S.pixoff[hA.pixoff_start + pa], s1 = S.pixoff[hA.pixoff_start + pa + 1];
+                ca0 = S.ixoff[hA.seq_start + s0];
+                ca1 = S.ixoff[hA.seq_start + s1];
+                na = S.pixedges[hA.pix_start + pa];
+            }
+        }
+        uint64_t lm = __ballot(live);
+        while (lm) {
+            const int src = __ffsll((unsigned long long)lm) - 1;
+            lm &= lm - 1;
+            const int vx0 = __builtin_amdgcn_readlane(v.x0, src), vx1 = __builtin_amdgcn_readlane(v.x1, src);
+            const int vy0 = __builtin_amdgcn_readlane(v.y0, src), vy1 = __builtin_amdgcn_readlane(v.y1, src);
+            const uint32_t a0 = __builtin_amdgcn_readlane(ca0, src), a1 = __builtin_amdgcn_readlane(ca1, src);
+            const uint64_t ea = (uint32_t)__builtin_amdgcn_readlane(na, src);
+            const uint32_t hgt = (uint32_t)(vy1 - vy0 + 1);
+            const uint32_t nt = vx1 >= vx0 && vy1 >= vy0 ? (uint32_t)(vx1 - vx0 + 1) * hgt : 0u;
+            for (uint32_t t0 = 0; t0 < nt; t0 += 64) {
+                const uint32_t t = t0 + lane;
+                bool tl = false;
+                uint32_t cb0 = 0, cb1 = 0, nb = 0;
+                if (t < nt) {
+                    const uint32_t pb = (uint32_t)((vy0 + (int)(t % hgt)) * hB.dimx + vx0 + (int)(t / hgt));
+                    tl = show(S.status[hB.pix_start + pb]) == 1;
+                    if (tl) {
+                        const uint32_t s0 = S.pixoff[hB.pixoff_start + pb], s1 = S.pixoff[hB.pixoff_start + pb + 1];
+                        cb0 = S.ixoff[hB.seq_start + s0];
+                        cb1 = S.ixoff[hB.seq_start + s1];
+                        nb = S.pixedges[hB.pix_start + pb];
+                    }
+                }
+                uint64_t bm = __ballot(tl);
+                while (bm) {
+                    const int s2 = __ffsll((unsigned long long)bm) - 1;
+                    bm &= bm - 1;
                     r.bb++;
-                    const uint32_t sb0 = S.pixoff[hB.pixoff_start + pb], sb1 = S.pixoff[hB.pixoff_start + pb + 1];
-                    r.tests += na * S.pixedges[hB.pix_start + pb];
-                    collect_chunks(C, ca0, ca1, uni(S.ixoff[hB.seq_start + sb0]), uni(S.ixoff[hB.seq_start + sb1]));
+                    r.tests += ea * (uint32_t)__builtin_amdgcn_readlane(nb, s2);
+                    collect_chunks<NW>(C, a0, a1, (uint32_t)__builtin_amdgcn_readlane(cb0, s2),
+                                       (uint32_t)__builtin_amdgcn_readlane(cb1, s2), turn);
+                    if (NW > 1) turn = turn + 1 == NW ? 0 : turn + 1;
                 }
             }
         }
@@ -708,72 +800,91 @@ __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const doub
     if (C.nc) flush_chunks(C);
     while (C.nl) flush_lines(C, min(C.nl, 64u));
     if (C.ne) flush_edges(C);
-    wave_sync();
-    const uint32_t nrec = uni(*cnt);
+    tm.sync();
+    const uint32_t nrec = uni(T.cnt);
     r.raw = nrec;
     if (nrec > cap) {
         r.over = true;
         return r;
     }
-    wave_sync();
     const double ox = fmax(hA.mbr[0], hB.mbr[0]), oy = fmax(hA.mbr[1], hB.mbr[1]);
     uint32_t nk = 0;
     if (nrec > 0) {
         // 3. sort by point, keep the first of each run of equal points
-        bitonic<0>(R, nrec, lane);
+        bitonic<0>(R, nrec, tm);
         bool small = false;
-        for (uint32_t k = lane; k < nrec; k += 64) {
-            const Rec e = R[k];
-            small |= fabsf(e.px) < 0.015625f || fabsf(e.py) < 0.015625f;
-        }
-        if (!wave_any(small)) {
-            // above 2^-6 the 1e-9 tolerance is float equality: a record is
-            // kept when it differs from its predecessor
-            for (uint32_t c0 = 0; c0 < nrec; c0 += 64) {
-                const uint32_t k = c0 + lane;
-                bool keep = false;
-                Rec e;
-                if (k < nrec) {
-                    e = R[k];
-                    keep = k == 0 || !pt_eq(R[k - 1].px, R[k - 1].py, e.px, e.py);
-                }
-                const uint64_t km = __ballot(keep);
-                if (keep) D[nk + (uint32_t)__popcll(km & ((1ull << lane) - 1ull))] = e;
-                nk += (uint32_t)__popcll(km);
-            }
-        } else if (lane == 0) {
-            // std::unique: compare with the last kept record
-            for (uint32_t k = 0; k < nrec; k++) {
+        if (tm.first()) {
+            for (uint32_t k = lane; k < nrec; k += 64) {
                 const Rec e = R[k];
-                if (nk == 0 || !pt_eq(D[nk - 1].px, D[nk - 1].py, e.px, e.py)) D[nk++] = e;
+                small |= fabsf(e.px) < 0.015625f || fabsf(e.py) < 0.015625f;
             }
+            if (!wave_any(small)) {
+                // above 2^-6 the 1e-9 tolerance is float equality: a record is
+                // kept when it differs from its predecessor
+                for (uint32_t c0 = 0; c0 < nrec; c0 += 64) {
+                    const uint32_t k = c0 + lane;
+                    bool keep = false;
+                    Rec e;
+                    if (k < nrec) {
+                        e = R[k];
+                        keep = k == 0 || !pt_eq(R[k - 1].px, R[k - 1].py, e.px, e.py);
+                    }
+                    const uint64_t km = __ballot(keep);
+                    if (keep) D[nk + (uint32_t)__popcll(km & ((1ull << lane) - 1ull))] = e;
+                    nk += (uint32_t)__popcll(km);
+                }
+            } else if (lane == 0) {
+                // std::unique: compare with the last kept record
+                for (uint32_t k = 0; k < nrec; k++) {
+                    const Rec e = R[k];
+                    if (nk == 0 || !pt_eq(D[nk - 1].px, D[nk - 1].py, e.px, e.py)) D[nk++] = e;
+                }
+            }
+            if (lane == 0) T.nk = nk;
         }
-        nk = uni(__shfl(nk, 0, 64));
-        wave_sync();
+        tm.sync();
+        nk = uni(T.nk);
     }
     r.c[0] = (int32_t)nk;
-    uint32_t pieces = 0;
     double acc_a = 0.0, acc_b = 0.0;
     if (nk > 0) {
-        bitonic<1>(D, nk, lane);
-        acc_a = ring_pieces<true>(S, hA, hB, D, nk, ox, oy, lane, r, pieces, po);
-        wave_sync();
-        bitonic<2>(D, nk, lane);
-        acc_b = ring_pieces<false>(S, hB, hA, D, nk, ox, oy, lane, r, pieces, po);
+        bitonic<1>(D, nk, tm);
+        acc_a = ring_pieces<true>(S, hA, hB, D, nk, ox, oy, tm, r, po, Q);
+        tm.sync();
+        bitonic<2>(D, nk, tm);
+        acc_b = ring_pieces<false>(S, hB, hA, D, nk, ox, oy, tm, r, po, Q);
     }
-    if (pieces == 0) {
-        // containment or disjoint
-        if (seg_contain_wave(S, hB, AX[0], AY[0], lane) == 2) {
+    double side_a = wave_sum(acc_a), side_b = wave_sum(acc_b);
+    if constexpr (NW > 1) {
+        if (lane == 0) {
+            for (int k = 1; k < 5; k++)
+                if (r.c[k]) atomicAdd(&T.c[k], r.c[k]);
+            T.side[0][tm.wv] = side_a;
+            T.side[1][tm.wv] = side_b;
+        }
+        tm.sync();
+        for (int k = 1; k < 5; k++) r.c[k] = T.c[k];
+        side_a = side_b = 0.0;
+        for (int k = 0; k < NW; k++) {
+            side_a += T.side[0][k];
+            side_b += T.side[1][k];
+        }
+    }
+    if (r.c[1] == 0) {
+        // containment or disjoint: the first vertex of A in B, of B in A
+        const int in_b = uni(__shfl(contain_points(S, hB, AX[0], AY[0], lane == 0, lane, Q), 0, 64));
+        const int in_a = in_b == 2 ? 0 : uni(__shfl(contain_points(S, hA, BX[0], BY[0], lane == 0, lane, Q), 0, 64));
+        const bool mine = tm.tid() == 0;
+        if (in_b == 2) {
             r.area = fabs(ring2a[ia]) / 2.0;
-            put_pieces(po, lane == 0, farm_piece{po.pair, 0, 0, -1, 0.f, 0.f, 0.f, 0.f}, lane);  // all of A
-        } else if (seg_contain_wave(S, hA, BX[0], BY[0], lane) == 2) {
+            put_pieces(po, mine, farm_piece{po.pair, 0, 0, -1, 0.f, 0.f, 0.f, 0.f}, lane);  // all of A
+        } else if (in_a == 2) {
             r.area = fabs(ring2a[ib]) / 2.0;
-            put_pieces(po, lane == 0, farm_piece{po.pair, 1, 0, -1, 0.f, 0.f, 0.f, 0.f}, lane);  // all of B
+            put_pieces(po, mine, farm_piece{po.pair, 1, 0, -1, 0.f, 0.f, 0.f, 0.f}, lane);  // all of B
         }
         return r;
     }
     const double sa = ring2a[ia] < 0 ? -1.0 : 1.0, sb = ring2a[ib] < 0 ? -1.0 : 1.0;
-    const double side_a = wave_sum(acc_a), side_b = wave_sum(acc_b);
     r.area = fabs(sa * side_a + sb * side_b) / 2.0;
     return r;
 }
@@ -796,62 +907,119 @@ __global__ __launch_bounds__(256) void k_ring_area(DevSet S, int64_t npolys, dou
     if (lane == 0) out[p] = acc;
 }
 
-// Persistent waves over pairs; BIG: the pairs in `list` with larger slabs.
+// Pairs for a whole workgroup: their indices to list (count at ctr[kIxHeavy]),
+// and flags[k] = 1.  A pair's collection runs over up to (chunks of A in the
+// overlap of the boxes) x (chunks of B in it) chunk pairs, estimated from the
+// overlap's share of each box; beyond kHeavyChunks one wave would be at it for
+// milliseconds (a 200,000-vertex ring against one over all of it took 57 ms of a
+// 138 ms call).  all: every pair (a call too small to fill the chip with one
+// wave per pair).
+enum : int { kIxHead = 0, kIxOver = 1, kIxPieces = 2, kIxHeavy = 3, kIxHeavyHead = 4 };
+constexpr float kHeavyChunks = 8192.f;
+
+__global__ __launch_bounds__(256) void k_ix_heavy(DevSet S, const uint32_t *__restrict__ pa,
+                                                  const uint32_t *__restrict__ pb, uint32_t n, int all,
+                                                  uint8_t *__restrict__ flags, uint32_t *__restrict__ list,
+                                                  uint32_t *__restrict__ ctr) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    bool heavy = false;
+    if (k < n) {
+        const farm_raster_hdr &A = S.hdr[pa[k]], &B = S.hdr[pb[k]];
+        auto part = [&](int lo, int hi, float &fa, float &fb) {
+            const float w = (float)(fmin(A.mbr[hi], B.mbr[hi]) - fmax(A.mbr[lo], B.mbr[lo]));
+            fa *= fminf(fmaxf(w, 0.f) / fmaxf((float)(A.mbr[hi] - A.mbr[lo]), 1e-30f), 1.f);
+            fb *= fminf(fmaxf(w, 0.f) / fmaxf((float)(B.mbr[hi] - B.mbr[lo]), 1e-30f), 1.f);
+        };
+        float fa = 1.f, fb = 1.f;
+        part(0, 2, fa, fb);
+        part(1, 3, fa, fb);
+        heavy = all || (A.nverts * fa / kIxChunk) * (B.nverts * fb / kIxChunk) > kHeavyChunks;
+        flags[k] = heavy ? 1 : 0;
+    }
+    const uint64_t m = __ballot(heavy);
+    uint32_t base = 0;
+    if (lane == 0 && m) base = atomicAdd(&ctr[kIxHeavy], (uint32_t)__popcll(m));
+    base = uni(__shfl(base, 0, 64));
+    if (heavy) list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = k;
+}
+
+// Persistent workgroups: first the pairs of list[0 .. *nlist), all four waves
+// on one pair (records in slabs of kWaves * cap), then, wave by wave, the other
+// pairs of the window (flags; slabs of cap).  BIG: pairs that overflowed the
+// first launch's slabs, all on the list (n = 0).
+// Four waves per SIMD (128 registers, 13 of them spilled): 61.8 ms for 618,000
+// complex x lakes pairs against 66.7 ms at three.
 template <bool BIG>
-__global__ __launch_bounds__(256) void k_intersection(DevSet S, const double *__restrict__ ring2a,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_intersection(DevSet S, const double *__restrict__ ring2a,
                                                       const uint32_t *__restrict__ pa, const uint32_t *__restrict__ pb,
-                                                      uint32_t n, const uint32_t *__restrict__ list,
+                                                      uint32_t n, const uint8_t *__restrict__ flags,
+                                                      const uint32_t *__restrict__ list,
+                                                      const uint32_t *__restrict__ nlist,
                                                       int32_t *__restrict__ counts, double *__restrict__ area,
                                                       Rec *__restrict__ slab, uint32_t cap,
                                                       uint32_t *__restrict__ ctr, uint32_t *__restrict__ ovf,
                                                       unsigned long long *__restrict__ stats,
                                                       farm_piece *__restrict__ pcs, uint32_t pcap) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t gw = (uint64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
-    Rec *R = slab + gw * 2ull * cap;
-    Rec *D = R + cap;
-    __shared__ uint32_t rec_cnt[kWaves];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    Rec *block_slab = slab + (uint64_t)blockIdx.x * kWaves * 2ull * cap;
+    __shared__ TeamSum sums[kWaves];
     __shared__ Queues queues[kWaves];
-    uint32_t *cnt = &rec_cnt[threadIdx.x >> 6];
-    Queues &Q = queues[threadIdx.x >> 6];
+    __shared__ uint32_t s_next;
     unsigned long long bb = 0, tests = 0, raw = 0, found = 0;
-    for (;;) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(&ctr[0], kChunk);
-        base = uni(__shfl(base, 0, 64));
-        if (base >= n) break;
-        const uint32_t end = min(base + kChunk, n);
-        for (uint32_t k = base; k < end; k++) {
-            const uint32_t idx = BIG ? list[k] : k;
-            const uint32_t ia = pa[idx], ib = pb[idx];
-            if ((S.hdr[ia].flags | S.hdr[ib].flags) & FARM_HDR_REJECTED) {
-                if (lane < 5) counts[5ull * idx + lane] = lane == 0 ? -3 : 0;
-                if (lane == 0) area[idx] = 0.0;
-                continue;
-            }
-            const PieceOut po{pcs, ctr + 2, pcap, idx};
-            const PairRes r = intersection_pair(S, ring2a, ia, ib, R, D, cap, cnt, Q, lane, po);
-            if (r.over) {
-                if (lane == 0) {
-                    if (BIG) {  // still too many: the host reruns it with larger slabs
-                        counts[5ull * idx] = -4;
-                        counts[5ull * idx + 1] = (int32_t)min(r.raw, (uint32_t)INT_MAX);
-                    } else {
-                        const uint32_t slot = atomicAdd(&ctr[1], 1u);
-                        ovf[slot] = idx;
-                    }
+    // one pair by a team; `writer` stores its results
+    auto run = [&](auto tm, uint32_t idx, Rec *R, Rec *D, uint32_t rcap, TeamSum &T, bool writer) {
+        const uint32_t ia = pa[idx], ib = pb[idx];
+        if ((S.hdr[ia].flags | S.hdr[ib].flags) & FARM_HDR_REJECTED) {
+            if (writer && lane < 5) counts[5ull * idx + lane] = lane == 0 ? -3 : 0;
+            if (writer && lane == 0) area[idx] = 0.0;
+            return;
+        }
+        const PieceOut po{pcs, ctr + kIxPieces, pcap, idx};
+        const PairRes r = intersection_pair(S, ring2a, ia, ib, R, D, rcap, T, queues[wv], tm, po);
+        if (!writer) return;
+        if (r.over) {
+            if (lane == 0) {
+                if (BIG) {  // still too many: the host reruns it with larger slabs
+                    counts[5ull * idx] = -4;
+                    counts[5ull * idx + 1] = (int32_t)min(r.raw, (uint64_t)INT_MAX);
+                } else {
+                    ovf[atomicAdd(&ctr[kIxOver], 1u)] = idx;
                 }
-                continue;
             }
-            bb += r.bb;
-            tests += r.tests;
-            raw += r.raw;
-            found += r.area > 0.0;
-            if (lane < 5) counts[5ull * idx + lane] = r.c[lane];
-            if (lane == 0) area[idx] = r.area;
+            return;
+        }
+        bb += r.bb;
+        tests += r.tests;
+        raw += r.raw;
+        found += r.area > 0.0;
+        if (lane < 5) counts[5ull * idx + lane] = r.c[lane];
+        if (lane == 0) area[idx] = r.area;
+    };
+    const uint32_t nl = *nlist;
+    for (;;) {
+        __syncthreads();  // the team's last pair is done with the shared state
+        if (threadIdx.x == 0) s_next = atomicAdd(&ctr[kIxHeavyHead], 1u);
+        __syncthreads();
+        const uint32_t k = uni(s_next);
+        if (k >= nl) break;
+        run(Team<kWaves>{lane, wv}, list[k], block_slab, block_slab + (uint64_t)kWaves * cap, kWaves * cap, sums[0],
+            wv == 0);
+    }
+    if constexpr (!BIG) {
+        Rec *R = block_slab + wv * 2ull * cap;
+        const uint32_t grab = min(max(n / (gridDim.x * kWaves * 16u), 1u), 8u);
+        for (;;) {
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(&ctr[kIxHead], grab);
+            base = uni(__shfl(base, 0, 64));
+            if (base >= n) break;
+            const uint32_t end = min(base + grab, n);
+            for (uint32_t k = base; k < end; k++)
+                if (!flags[k]) run(Team<1>{lane, wv}, k, R, R + cap, cap, sums[wv], true);
         }
     }
-    if (lane == 0) {
+    if (lane == 0 && (bb || tests || raw || found)) {
         atomicAdd(&stats[0], bb);
         atomicAdd(&stats[1], tests);
         atomicAdd(&stats[2], raw);
@@ -860,11 +1028,13 @@ __global__ __launch_bounds__(256) void k_intersection(DevSet S, const double *__
 }
 
 template __global__ void k_intersection<false>(DevSet, const double *, const uint32_t *, const uint32_t *, uint32_t,
-                                               const uint32_t *, int32_t *, double *, Rec *, uint32_t, uint32_t *,
-                                               uint32_t *, unsigned long long *, farm_piece *, uint32_t);
+                                               const uint8_t *, const uint32_t *, const uint32_t *, int32_t *,
+                                               double *, Rec *, uint32_t, uint32_t *, uint32_t *,
+                                               unsigned long long *, farm_piece *, uint32_t);
 template __global__ void k_intersection<true>(DevSet, const double *, const uint32_t *, const uint32_t *, uint32_t,
-                                              const uint32_t *, int32_t *, double *, Rec *, uint32_t, uint32_t *,
-                                              uint32_t *, unsigned long long *, farm_piece *, uint32_t);
+                                              const uint8_t *, const uint32_t *, const uint32_t *, int32_t *,
+                                              double *, Rec *, uint32_t, uint32_t *, uint32_t *,
+                                              unsigned long long *, farm_piece *, uint32_t);
 
 }  // namespace farm
 
@@ -905,6 +1075,8 @@ int run_intersection(farm_handle h, uint64_t begin, uint64_t end, int32_t *count
     const uint32_t *pb = P<uint32_t>(h->pb) + begin;
     if ((rc = ensure(h, h->wctr, 64))) return rc;
     if ((rc = ensure(h, h->wovf, 4ull * n))) return rc;
+    if ((rc = ensure(h, h->ixlist, 4ull * n))) return rc;
+    if ((rc = ensure(h, h->ixflag, n))) return rc;
     uint32_t *ctr = P<uint32_t>(h->wctr);
     unsigned long long *ist = reinterpret_cast<unsigned long long *>(ctr + 8);
     if ((rc = fill_u32(h, ctr, 16, 0))) return rc;
@@ -912,22 +1084,27 @@ int run_intersection(farm_handle h, uint64_t begin, uint64_t end, int32_t *count
     const uint64_t nwaves = (uint64_t)nblocks * kWaves;
     if ((rc = ensure(h, h->wslab, nwaves * 2ull * kRecCap * sizeof(Rec)))) return rc;
     HIPCHK(h, hipEventRecord(h->ev[0], h->stream));
+    // fewer than 8 pairs to a workgroup: all of them by whole workgroups
+    hipLaunchKernelGGL(k_ix_heavy, dim3(blocks_for(n)), dim3(256), 0, h->stream, S, pa, pb, n, n < 8 * nblocks ? 1 : 0,
+                       P<uint8_t>(h->ixflag), P<uint32_t>(h->ixlist), ctr);
+    HIPCHK(h, hipGetLastError());
     hipLaunchKernelGGL(k_intersection<false>, dim3(nblocks), dim3(64 * kWaves), 0, h->stream, S,
-                       (const double *)P<double>(h->ring2a), pa, pb, n, (const uint32_t *)nullptr, counts_dev, area_dev,
-                       P<Rec>(h->wslab), kRecCap, ctr, P<uint32_t>(h->wovf), ist, pcs_dev, pcap);
+                       (const double *)P<double>(h->ring2a), pa, pb, n, (const uint8_t *)P<uint8_t>(h->ixflag),
+                       (const uint32_t *)P<uint32_t>(h->ixlist), (const uint32_t *)(ctr + kIxHeavy), counts_dev,
+                       area_dev, P<Rec>(h->wslab), kRecCap, ctr, P<uint32_t>(h->wovf), ist, pcs_dev, pcap);
     HIPCHK(h, hipGetLastError());
     uint32_t novf = 0;
-    HIPCHK(h, hipMemcpyAsync(&novf, ctr + 1, 4, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipMemcpyAsync(&novf, ctr + kIxOver, 4, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     if (novf) {
         // pairs with more raw crossing records than the first slabs hold
         const unsigned bblocks = 16;
         if ((rc = ensure(h, h->wslab_big, (uint64_t)bblocks * kWaves * 2ull * kRecCapBig * sizeof(Rec)))) return rc;
-        if ((rc = fill_u32(h, ctr, 1, 0))) return rc;
+        if ((rc = fill_u32(h, ctr + kIxHeavyHead, 1, 0))) return rc;
         hipLaunchKernelGGL(k_intersection<true>, dim3(bblocks), dim3(64 * kWaves), 0, h->stream, S,
-                           (const double *)P<double>(h->ring2a), pa, pb, novf, (const uint32_t *)P<uint32_t>(h->wovf),
-                           counts_dev, area_dev, P<Rec>(h->wslab_big), kRecCapBig, ctr, P<uint32_t>(h->wovf), ist,
-                           pcs_dev, pcap);
+                           (const double *)P<double>(h->ring2a), pa, pb, 0u, (const uint8_t *)nullptr,
+                           (const uint32_t *)P<uint32_t>(h->wovf), (const uint32_t *)(ctr + kIxOver), counts_dev,
+                           area_dev, P<Rec>(h->wslab_big), kRecCapBig, ctr, P<uint32_t>(h->wovf), ist, pcs_dev, pcap);
         HIPCHK(h, hipGetLastError());
     }
     HIPCHK(h, hipEventRecord(h->ev[1], h->stream));
@@ -949,21 +1126,23 @@ int run_intersection(farm_handle h, uint64_t begin, uint64_t end, int32_t *count
             }
         }
         if (!big.empty()) {
-            uint64_t cap = 2ull * kRecCapBig;
-            while (cap < most) cap <<= 1;
-            if (cap > (1ull << 26))
+            if (most > (1u << 26))
                 return fail(h, FARM_ECAPACITY, "a pair has %u crossing records (limit 2^26)", most);
+            uint64_t cap = 2ull * kRecCapBig;  // a workgroup's slabs hold kWaves * cap records each
+            while (kWaves * cap < most) cap <<= 1;
             const uint64_t per_wave = 2ull * cap * sizeof(Rec);
             const uint64_t waves = std::max<uint64_t>(kWaves, std::min<uint64_t>(64, (8ull << 30) / per_wave));
             const unsigned blocks = (unsigned)(waves / kWaves);
             if ((rc = ensure(h, h->wslab_big, (uint64_t)blocks * kWaves * per_wave))) return rc;
             HIPCHK(h, hipMemcpyAsync(P<uint32_t>(h->wovf), big.data(), 4ull * big.size(), hipMemcpyHostToDevice,
                                      h->stream));
-            if ((rc = fill_u32(h, ctr, 1, 0))) return rc;
+            const uint32_t nbig = (uint32_t)big.size();
+            HIPCHK(h, hipMemcpyAsync(ctr + kIxOver, &nbig, 4, hipMemcpyHostToDevice, h->stream));
+            if ((rc = fill_u32(h, ctr + kIxHeavyHead, 1, 0))) return rc;
             hipLaunchKernelGGL(k_intersection<true>, dim3(blocks), dim3(64 * kWaves), 0, h->stream, S,
-                               (const double *)P<double>(h->ring2a), pa, pb, (uint32_t)big.size(),
-                               (const uint32_t *)P<uint32_t>(h->wovf), counts_dev, area_dev, P<Rec>(h->wslab_big),
-                               (uint32_t)cap, ctr, P<uint32_t>(h->wovf), ist, pcs_dev, pcap);
+                               (const double *)P<double>(h->ring2a), pa, pb, 0u, (const uint8_t *)nullptr,
+                               (const uint32_t *)P<uint32_t>(h->wovf), (const uint32_t *)(ctr + kIxOver), counts_dev,
+                               area_dev, P<Rec>(h->wslab_big), (uint32_t)cap, ctr, P<uint32_t>(h->wovf), ist, pcs_dev, pcap);
             HIPCHK(h, hipGetLastError());
             HIPCHK(h, hipEventRecord(h->ev[1], h->stream));
             HIPCHK(h, hipMemcpyAsync(hst, ist, sizeof hst, hipMemcpyDeviceToHost, h->stream));
@@ -973,13 +1152,13 @@ int run_intersection(farm_handle h, uint64_t begin, uint64_t end, int32_t *count
                 HIPCHK(h, hipMemcpy(&c0, counts_dev + 5ull * idx, 4, hipMemcpyDeviceToHost));
                 if (c0 == -4)
                     return fail(h, FARM_ECAPACITY, "pair %llu: more than %llu crossing records",
-                                (unsigned long long)(begin + idx), (unsigned long long)cap);
+                                (unsigned long long)(begin + idx), (unsigned long long)(kWaves * cap));
             }
         }
     }
     if (npcs) {
         uint32_t np = 0;
-        HIPCHK(h, hipMemcpy(&np, ctr + 2, 4, hipMemcpyDeviceToHost));
+        HIPCHK(h, hipMemcpy(&np, ctr + kIxPieces, 4, hipMemcpyDeviceToHost));
         *npcs = np;
     }
     if (st) {

@@ -205,3 +205,29 @@ def test_intersection_polygons_areas_match(device, seed):
     check_wkt_areas({k: capi.wkt_multipolygon_area(t) for k, t in lines.items()},
                     {int(k): float(area[k]) for k in nz})
     assert set(lines) <= set(nz.tolist()) | set(np.nonzero(counts[:, 2] > 0)[0].tolist())
+
+
+@pytest.mark.parametrize("npairs", [60, 9001])
+def test_pairs_by_workgroups_and_by_waves(device, npairs):
+    # fewer pairs than 8 per workgroup: each by a whole workgroup; more: one
+    # wave each, but for the pairs of two long rings (some with more pieces
+    # than lanes, some contained)
+    a = rings_from_list([_wavy(6000, 0.0, 0.0, 1.0), _wavy(40, 0.3, 0.2, 0.5), _wavy(900, 5.0, 5.0, 0.4)])
+    b = rings_from_list([_wavy(5000, 0.2, 0.1, 0.9), _wavy(700, 0.1, 0.0, 0.7), _wavy(15, 0.0, 0.1, 0.05),
+                         _wavy(300, 5.1, 5.0, 0.35)])
+    base = Workload(a, b, vpr=30)
+    rep = -(-npairs // len(base.pa))
+    w = Workload(a, b, vpr=30, pairs=(np.tile(base.pa, rep)[:npairs], np.tile(base.pb, rep)[:npairs]))
+    want_c, want_a = oracle.intersection(base.OA, base.OB, base.pa, base.pb)
+    assert (want_c[:, 1] > 64).any() and ((want_c[:, 1] == 0) & (want_a > 0)).any()
+    w.upload(device)
+    c, area, _ = device.intersection_area()
+    assert np.array_equal(c, np.tile(want_c, (rep, 1))[:npairs])
+    want = np.tile(want_a, rep)[:npairs]
+    assert (np.abs(area - want) <= AREA_RTOL * np.abs(want) + AREA_ATOL).all()
+
+
+def _wavy(n, cx, cy, r):
+    t = np.linspace(0, 2 * np.pi, n, endpoint=False)
+    q = r * (1.0 + 0.1 * np.sin(7 * t) + 0.15 * np.sin(61 * t + 9 * cx))
+    return np.stack([3.0 + cx + q * np.cos(t), 3.0 + cy + q * np.sin(t)], 1)
