@@ -43,6 +43,9 @@ struct DevSet {
     const farm_layer *layers;
     const uint8_t *lstatus;
     const double *areas;
+    // per pixel: the box of its sequences, their edges and count (within only)
+    const float4 *pixbox;
+    const uint2 *pixlen;
 };
 
 // The refinement walks a target edge sequence in chunks of C steps (8, 16 or

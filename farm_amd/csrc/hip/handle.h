@@ -98,6 +98,8 @@ struct farm_handle_s {
     uint64_t max_border_pix = 0;  // most BORDER pixels of a finest layer
     farm::DevBuf layers, lstatus, areas;
     bool areas_ready = false;  // areas hold the set's per-pixel clipped areas
+    farm::DevBuf pixbox, pixlen;  // built for set generation pixrec_gen
+    uint64_t pixrec_gen = ~0ull;
     farm::DevBuf wctr, wovf, wslab, wslab_big, wout, wmd;
     // intersection
     bool ring_area_ready = false;
@@ -190,6 +192,8 @@ inline DevSet devset(farm_handle h) {
     S.layers = h->has_layers ? P<farm_layer>(h->layers) : nullptr;
     S.lstatus = h->has_layers ? P<uint8_t>(h->lstatus) : nullptr;
     S.areas = h->has_layers ? P<double>(h->areas) : nullptr;
+    S.pixbox = P<float4>(h->pixbox);
+    S.pixlen = P<uint2>(h->pixlen);
     return S;
 }
 

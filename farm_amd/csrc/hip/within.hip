@@ -65,7 +65,7 @@ constexpr double kFar = 100000.0;           // the reference's "no distance yet"
 constexpr int kWaves = 4;                   // wavefronts per workgroup
 constexpr int kPixMax = 512;                // pixels of a layer handled in LDS
 constexpr int kBitWords = kPixMax / 32;
-constexpr uint32_t kChunk = 8;              // pairs per queue grab
+constexpr uint32_t kChunk = 8;              // most pairs per queue grab
 
 struct Cand {
     double apx, lo, hi;
@@ -99,6 +99,13 @@ __device__ __forceinline__ LGrid lgrid(const DevSet &S, const farm_raster_hdr &h
     return g;
 }
 
+// The two polygons' layers, read by the whole wave once per pair (a layer
+// looked up in global memory is two dependent loads, about eight times a level).
+constexpr int kLayC = 16;
+struct LayC {
+    LGrid g[2][kLayC];
+};
+
 __device__ __forceinline__ bool border(uint8_t s) { return s != 0 && s != kCC - 1; }
 
 // degree_per_kilometer_longitude(lat) (util.h:88-96); the index is clamped
@@ -116,6 +123,7 @@ __device__ __forceinline__ int km_idx(double lat) {
 constexpr int kKmC = 16;
 struct KmC {
     double v[kKmC], inv[kKmC];
+    double inv_max;  // 1 / the largest entry the pair can need
     int lo, n;
 };
 
@@ -273,19 +281,26 @@ __device__ __forceinline__ int unpack_y(T v) {
     return (int)((uint32_t)v >> SH);
 }
 
-// Pixel set -> compact list (ascending ids): rounds of 64 ids, one per lane,
-// each member placed by the ballot count of the members below it.  (x, y)
-// of a lane's id is advanced by 64 ids per round instead of divided out.
+// Pixel sets of both polygons -> compact lists (ascending ids): rounds of 64
+// ids, one per lane, each member placed by the ballot count of the members
+// below it.  (x, y) of a lane's id is advanced by 64 ids per round instead of
+// divided out.  Both sides go through one loop, so that their LDS latencies
+// overlap.
 template <int SH, class T>
-__device__ __forceinline__ uint32_t compact(const uint32_t *bits, int npix, int dimx, T *list, int lane) {
-    const uint64_t below = (1ull << lane) - 1ull;
-    const uint32_t ux = (uint32_t)dimx;
-    uint32_t y = (uint32_t)lane / ux, x = (uint32_t)lane - y * ux;
-    const uint32_t sy = 64u / ux, sx = 64u - sy * ux;  // sx < dimx
-    uint32_t total = 0;
-    for (int id0 = 0; id0 < npix; id0 += 64) {
-        const int id = id0 + lane;
-        const bool in = id < npix && ((bits[id >> 5] >> (id & 31)) & 1u);
+struct Compact {
+    const uint32_t *bits;
+    T *list;
+    int npix;
+    uint32_t ux, x, y, sx, sy, total;
+    __device__ __forceinline__ Compact(const uint32_t *bits_, int npix_, int dimx, T *list_, int lane)
+        : bits(bits_), list(list_), npix(npix_), ux((uint32_t)dimx), total(0) {
+        y = (uint32_t)lane / ux;
+        x = (uint32_t)lane - y * ux;
+        sy = 64u / ux;
+        sx = 64u - sy * ux;  // < dimx
+    }
+    __device__ __forceinline__ bool member(int id) const { return id < npix && ((bits[id >> 5] >> (id & 31)) & 1u); }
+    __device__ __forceinline__ void place(bool in, uint64_t below) {
         const uint64_t m = __ballot(in);
         if (in) list[total + (uint32_t)__popcll(m & below)] = pack_xy<SH, T>(x, y);
         total += (uint32_t)__popcll(m);
@@ -296,13 +311,30 @@ __device__ __forceinline__ uint32_t compact(const uint32_t *bits, int npix, int 
             y++;
         }
     }
+};
+
+template <int SH, class T>
+__device__ __forceinline__ void compact_both(const uint32_t *sb, int npix_s, int dimx_s, T *sl, uint32_t &ns,
+                                             const uint32_t *tb, int npix_t, int dimx_t, T *tl, uint32_t &nt,
+                                             int lane) {
+    const uint64_t below = (1ull << lane) - 1ull;
+    Compact<SH, T> s(sb, npix_s, dimx_s, sl, lane), t(tb, npix_t, dimx_t, tl, lane);
+    for (int id0 = 0; id0 < max(npix_s, npix_t); id0 += 64) {
+        const bool is = s.member(id0 + lane), it = t.member(id0 + lane);
+        s.place(is, below);
+        t.place(it, below);
+    }
     wave_sync();
-    return uni(total);
+    ns = uni(s.total);
+    nt = uni(t.total);
 }
 
-__device__ __forceinline__ void clear_bits(uint32_t *bits, int npix, int lane) {
-    const int nw = (npix + 31) >> 5;
-    for (int w = lane; w < nw; w += 64) bits[w] = 0u;
+__device__ __forceinline__ void clear_bits(uint32_t *sb, int npix_s, uint32_t *tb, int npix_t, int lane) {
+    const int ws = (npix_s + 31) >> 5, wt = (npix_t + 31) >> 5;
+    for (int w = lane; w < max(ws, wt); w += 64) {
+        if (w < ws) sb[w] = 0u;
+        if (w < wt) tb[w] = 0u;
+    }
     wave_sync();
 }
 
@@ -316,51 +348,82 @@ struct PairOut {
     uint64_t boxes;   // box-pair distances evaluated in the descent
 };
 
-// Descend one side: children (at layer g) of every parent in list (at layer
-// pg), or (same layer) the members themselves; BORDER ones go to bits.
+// Descend: children (at layer g) of every parent in list (at layer pg), or (same
+// layer) the members themselves; BORDER ones go to bits.  A parent's children
+// are 2 x 2 to 3 x 3 pixels as a rule: their classes are loaded together, and
+// those of both sides before either is used (one after the other, nine load
+// latencies a side and level, this was a third of the kernel).
 template <int SH, class T>
-__device__ __forceinline__ void expand_side(const T *list, uint32_t n, bool next, const LGrid &pg,
-                                            const LGrid &g, const uint8_t *st, uint32_t *bits, int lane) {
+struct Expand {
+    const LGrid &pg, &g;
+    uint32_t *bits;
+    bool next;
+    double ystep;
+    int sx, sy, ex, ey;
+    uint8_t c[9];
+    __device__ __forceinline__ Expand(bool next_, const LGrid &pg_, const LGrid &g_, uint32_t *bits_)
+        : pg(pg_), g(g_), bits(bits_), next(next_), ystep(next_ ? 1.0 / g_.step : 0.0) {}
     // get_offset_x/_y's (v - low) / step through the step's reciprocal
     // (div_rcp: the same rounded quotient)
-    const double ystep = next ? 1.0 / g.step : 0.0;
-    auto off = [&](double v, double lo, int dim) {
+    __device__ __forceinline__ int off(double v, double lo, int dim) const {
         return min(max(d2i(div_rcp(v - lo, g.step, ystep)), 0), dim - 1);
-    };
-    for (uint32_t k = lane; k < n; k += 64) {
-        const T v = list[k];
-        const int px = unpack_x<SH>(v), py = unpack_y<SH>(v);
-        if (!next) {
-            const uint32_t id = (uint32_t)(py * g.dimx + px);
-            if (border(st[id])) set_bit(bits, id);
-            continue;
+    }
+    // parent v's window and the classes of its first 3 x 3 pixels
+    __device__ __forceinline__ void load(bool on, T v) {
+        sx = ex = unpack_x<SH>(v);
+        sy = ey = unpack_y<SH>(v);
+        if (next) {
+            // the parent box shrunk by 1e-6, then retrieve_pixels'
+            // own 1e-6 (MyRaster.cpp:332-346), in that order
+            double b[4];
+            pbox(pg, sx, sy, b);
+            b[0] += 1e-6;
+            b[1] += 1e-6;
+            b[2] -= 1e-6;
+            b[3] -= 1e-6;
+            sx = off(b[0] + 1e-6, g.lx, g.dimx);
+            sy = off(b[1] + 1e-6, g.ly, g.dimy);
+            ex = off(b[2] - 1e-6, g.lx, g.dimx);
+            ey = off(b[3] - 1e-6, g.ly, g.dimy);
         }
-        // the parent box shrunk by 1e-6, then retrieve_pixels'
-        // own 1e-6 (MyRaster.cpp:332-346), in that order
-        double b[4];
-        pbox(pg, px, py, b);
-        b[0] += 1e-6;
-        b[1] += 1e-6;
-        b[2] -= 1e-6;
-        b[3] -= 1e-6;
-        const int sx = off(b[0] + 1e-6, g.lx, g.dimx);
-        const int sy = off(b[1] + 1e-6, g.ly, g.dimy);
-        const int ex = off(b[2] - 1e-6, g.lx, g.dimx);
-        const int ey = off(b[3] - 1e-6, g.ly, g.dimy);
+        if (!on) ex = sx - 1;  // no pixel
+#pragma unroll
+        for (int q = 0; q < 9; q++) {
+            const int x = sx + q % 3, y = sy + q / 3;
+            c[q] = x <= ex && y <= ey ? g.st[y * g.dimx + x] : (uint8_t)0;
+        }
+    }
+    __device__ __forceinline__ void mark() {
+#pragma unroll
+        for (int q = 0; q < 9; q++)
+            if (border(c[q])) set_bit(bits, (uint32_t)((sy + q / 3) * g.dimx + sx + q % 3));
+        if (ex - sx < 3 && ey - sy < 3) return;
         for (int x = sx; x <= ex; x++)
             for (int y = sy; y <= ey; y++) {
                 const uint32_t id = (uint32_t)(y * g.dimx + x);
-                if (border(st[id])) set_bit(bits, id);
+                if (border(g.st[id])) set_bit(bits, id);
             }
+    }
+};
+
+template <int SH, class T>
+__device__ __forceinline__ void expand_both(Expand<SH, T> s, const T *sl, uint32_t ns, Expand<SH, T> t, const T *tl,
+                                            uint32_t nt, int lane) {
+    for (uint32_t k = lane; k < max(ns, nt); k += 64) {
+        s.load(k < ns, k < ns ? sl[k] : (T)0);
+        t.load(k < nt, k < nt ? tl[k] : (T)0);
+        s.mark();
+        t.mark();
     }
     wave_sync();
 }
 
 // Edge-sequence pairs of one candidate pixel pair, 64 at a time.
 struct SeqTab {
-    uint32_t fa[64], la[64], fb[64], lb[64], w1[64], pre[65];
+    uint32_t fa[64], la[64], fb[64], lb[64], pre[65];
     unsigned long long mins[64];  // squared distance bits (non-negative doubles order as integers)
     KmC km;                       // the km table entries of the current pair
+    LayC lay;                     // its layers
     Cand stage[64];               // last-level candidates waiting to be merged into the best 64
 };
 
@@ -375,15 +438,38 @@ struct CandBatch {
     double ref[kBatch];
 };
 
-// floor(n / m) for n < 2^22 and 1 <= m: the binary32 quotient is within one
-// of it (relative error below 2^-22), and one step against the remainder
-// corrects it.
-__device__ __forceinline__ uint32_t udiv_small(uint32_t n, uint32_t m) {
-    uint32_t q = (uint32_t)((float)n * __builtin_amdgcn_rcpf((float)m));
-    const int r = (int)n - (int)(q * m);
-    if (r < 0) q--;
-    else if (r >= (int)m) q++;
-    return q;
+// Box of an edge sequence: the union of its chunks' boxes (DevSet::ixbox);
+// false when it has more chunks than are worth looking at, or an open box.
+__device__ __forceinline__ bool seq_box(const DevSet &S, uint32_t seq, double b[4]) {
+    const uint32_t c0 = S.ixoff[seq], c1 = S.ixoff[seq + 1];
+    if (c1 - c0 > 4) return false;
+    b[0] = b[1] = INFINITY;
+    b[2] = b[3] = -INFINITY;
+    for (uint32_t c = c0; c < c1; c++) {
+        const float4 q = S.ixbox[c];
+        if (!(fabsf(q.x) + q.z + fabsf(q.y) + q.w < INFINITY)) return false;
+        b[0] = fmin(b[0], (double)q.x - (double)q.z);
+        b[1] = fmin(b[1], (double)q.y - (double)q.w);
+        b[2] = fmax(b[2], (double)q.x + (double)q.z);
+        b[3] = fmax(b[3], (double)q.y + (double)q.w);
+    }
+    return true;
+}
+
+// Lower bound of the squared distance in km between anything in boxes p and q
+// (low x, low y, high x, high y), as the evaluations compute distances: with
+// the largest km table entry of the pair's latitudes, less 1e-6 of the boxes'
+// extents, which covers the binary32 rounding of the evaluations' differences
+// (2^-24 of a segment).  NaN or 0 for an infinite box.
+__device__ __forceinline__ double box_low_d2(const double p[4], const double q[4], double inv_max) {
+    const double gx = fmax(q[0] - p[2], p[0] - q[2]) - 1e-6 * ((p[2] - p[0]) + (q[2] - q[0]));
+    const double gy = fmax(q[1] - p[3], p[1] - q[3]) - 1e-6 * ((p[3] - p[1]) + (q[3] - q[1]));
+    const double dx = fmax(gx, 0.0) * inv_max, dy = fmax(gy, 0.0) * kKmLatInv;
+    return dx * dx + dy * dy;
+}
+// that bound beyond distance v, with a margin for the double arithmetic
+__device__ __forceinline__ bool beyond(double low_d2, double v) {
+    return low_d2 * (1.0 - 1e-9) > v * v * (1.0 + 1e-9);
 }
 
 // Refines a batch of candidate pixel pairs: the truncated distances of all
@@ -394,18 +480,27 @@ __device__ __forceinline__ uint32_t udiv_small(uint32_t n, uint32_t m) {
 // after every valid sequence pair (running minimum < d: within; < the row's
 // candidate's reference_dist: not within) become a running-minimum scan and
 // the first lane that passes one.  Returns 1 / 0 when decided, 2 to go on.
+//
+// A row is not evaluated when the two sequences' boxes are further apart than
+// the running minimum before the batch, d and the candidate's reference_dist:
+// its distance then neither lowers the running minimum nor passes a check by
+// itself, so every check and minimum after it is unchanged.  (The first valid
+// row of a candidate always is: its check may pass on the earlier minimum.)
+// In pairs with hundreds of candidates (nine tenths of the evaluations) few
+// rows are left after the first ones.
+// Evaluations are counted as if every row were evaluated.
 __device__ __forceinline__ int refine_batch(const DevSet &S, const farm_raster_hdr &hs, const farm_raster_hdr &ht,
                                             const CandBatch &cb, double d, double &min_dist, PairOut &r,
                                             SeqTab &tab, int lane) {
     const uint32_t nrows = cb.nrows;
-    const float *sxv = S.x + hs.vert_start, *syv = S.y + hs.vert_start;
-    const float *txv = S.x + ht.vert_start, *tyv = S.y + ht.vert_start;
+    const float4 *sv = S.xyd + hs.vert_start, *tv = S.xyd + ht.vert_start;  // (x, y of a vertex in one load)
     for (uint32_t c0 = 0; c0 < nrows; c0 += 64) {
         const uint32_t k = c0 + lane;
-        uint32_t la = 0, lb = 0, fa = 0, fb = 0;
+        uint32_t la = 0, lb = 0, fa = 0, fb = 0, rr = 0;
         double ref = kFar;
+        bool apart = false;
         if (k < nrows) {
-            uint32_t s0 = 0, t0 = 0, n2 = 1, rr = 0;
+            uint32_t s0 = 0, t0 = 0, n2 = 1;
 #pragma unroll
             for (int q = 0; q < kBatch; q++) {
                 if (q < cb.n && k >= cb.row0[q]) {
@@ -423,53 +518,101 @@ __device__ __forceinline__ int refine_batch(const DevSet &S, const farm_raster_h
             la = e1.y;
             fb = e2.x;
             lb = e2.y;
+            double p[4], q[4];
+            const double thr = fmax(fmax(min_dist, d), ref);
+            if (thr < kFar && seq_box(S, hs.seq_start + s0 + a, p) && seq_box(S, ht.seq_start + t0 + b, q)) {
+                apart = beyond(box_low_d2(p, q, tab.km.inv_max), thr);
+            }
         }
         // sequences of fewer than 2 edges are skipped (Ideal.cpp:2630)
         const bool ok = k < nrows && la >= 2 && lb >= 2;
+        // the candidate's first valid row among these 64
+        const uint64_t okm = __ballot(ok);
+        const uint32_t start = rr > c0 ? rr - c0 : 0u;  // its first lane
+        const bool lead = ok && ((okm & ((1ull << lane) - 1ull)) >> start) == 0ull;
         const uint32_t w1 = ok ? lb * (la - 1) : 0u;
-        const uint32_t w = ok ? w1 + la * (lb - 1) : 0u;
-        uint32_t W;
+        const uint32_t wall = ok ? w1 + la * (lb - 1) : 0u;
+        const uint32_t w = lead || !apart ? wall : 0u;
+        uint32_t W, Wall;
         const uint32_t pre = wave_excl_scan(w, lane, &W);
+        const uint32_t pall = wave_excl_scan(wall, lane, &Wall) + wall;
         tab.fa[lane] = fa;
         tab.la[lane] = la;
         tab.fb[lane] = fb;
         tab.lb[lane] = lb;
-        tab.w1[lane] = w1;
         tab.pre[lane] = pre;
         if (lane == 63) tab.pre[64] = W;
         tab.mins[lane] = ~0ull;
         wave_sync();
-        // e < w1: point i of the target sequence, segment j of the source
-        // one; else point i of the source sequence, segment j of the target
-        // one.  One distance per lane either way: the operands are selected,
-        // so lanes on both sides of w1 share one evaluation.
-        auto sweep = [&](auto small_tag) {
-            constexpr bool SM = decltype(small_tag)::value;
-            int kk = 0, cur = -1;
+        // Each lane takes ceil(W / 64) consecutive evaluations.  Within a row,
+        // e < w1: point i of the target sequence, segment j of the source one;
+        // else point i of the source sequence, segment j of the target one.
+        // One distance per lane and step either way: the operands are
+        // selected, so lanes on both sides of w1 share one evaluation, and a
+        // step along the segments loads one vertex.
+        {
+            const uint32_t per = (W + 63) / 64;
+            uint32_t u = (uint32_t)lane * per;
+            const uint32_t uend = min(u + per, W);
+            uint32_t kk = 0;
+            // the row that holds u
+#pragma unroll
+            for (uint32_t step = 32; step > 0; step >>= 1)
+                if (tab.pre[kk + step] <= u) kk += step;
+            uint32_t rowend = 0, turn = 0;  // ends of the row and of its first half
+            uint32_t j = 0, m = 0;
+            const float4 *pt = sv, *sg = sv;
+            float2 p = make_float2(0.f, 0.f), a = p;
+            auto xy = [](const float4 *v) { return *reinterpret_cast<const float2 *>(v); };
             double acc = INFINITY;
-            for (uint32_t u = lane; u < W; u += 64) {
-                while (tab.pre[kk + 1] <= u) kk++;
-                if (kk != cur) {
-                    if (cur >= 0) atomicMin(&tab.mins[cur], (unsigned long long)__double_as_longlong(acc));
-                    cur = kk;
-                    acc = INFINITY;
+            // the operands of evaluation e of row kk
+            auto seek = [&]() {
+                const uint32_t base = tab.pre[kk], e = u - base;
+                const uint32_t la_ = tab.la[kk], lb_ = tab.lb[kk], half = lb_ * (la_ - 1);
+                rowend = min(tab.pre[kk + 1], uend);
+                turn = base + half;
+                const bool tgt_pt = e < half;
+                const uint32_t e2 = tgt_pt ? e : e - half;
+                m = (tgt_pt ? la_ : lb_) - 1;
+                const uint32_t i = e2 / m;
+                j = e2 - i * m;
+                const uint32_t fa_ = tab.fa[kk], fb_ = tab.fb[kk];
+                pt = (tgt_pt ? tv + fb_ : sv + fa_) + i;
+                sg = tgt_pt ? sv + fa_ : tv + fb_;
+                p = xy(pt);
+                a = xy(sg + j);
+            };
+            if (u < uend) seek();
+            for (uint32_t s = 0; s < per; s++) {
+                if (u < uend) {
+                    j++;
+                    const float2 b = xy(sg + j);
+                    acc = fmin(acc, pt_seg_d2(p.x, p.y, a.x, a.y, b.x, b.y, tab.km));
+                    u++;
+                    a = b;
+                    if (u == rowend) {
+                        atomicMin(&tab.mins[kk], (unsigned long long)__double_as_longlong(acc));
+                        acc = INFINITY;
+                        if (u < uend) {
+                            do kk++;
+                            while (tab.pre[kk + 1] <= u);  // (rows without evaluations)
+                            seek();
+                        }
+                    } else if (u == turn) {
+                        seek();
+                    } else if (j == m) {
+                        pt++;
+                        p = xy(pt);
+                        j = 0;
+                        a = xy(sg);
+                    }
                 }
-                const uint32_t e = u - tab.pre[kk];
-                const uint32_t fa_ = tab.fa[kk], fb_ = tab.fb[kk], w1_ = tab.w1[kk];
-                const bool tgt_pt = e < w1_;
-                const uint32_t e2 = tgt_pt ? e : e - w1_, m = (tgt_pt ? tab.la[kk] : tab.lb[kk]) - 1;
-                const uint32_t i = SM ? udiv_small(e2, m) : e2 / m, j = e2 - i * m;
-                const float *ptx = tgt_pt ? txv + fb_ : sxv + fa_, *pty = tgt_pt ? tyv + fb_ : syv + fa_;
-                const float *sgx = tgt_pt ? sxv + fa_ : txv + fb_, *sgy = tgt_pt ? syv + fa_ : tyv + fb_;
-                acc = fmin(acc, pt_seg_d2(ptx[i], pty[i], sgx[j], sgy[j], sgx[j + 1], sgy[j + 1], tab.km));
             }
-            if (cur >= 0) atomicMin(&tab.mins[cur], (unsigned long long)__double_as_longlong(acc));
-        };
-        if (W < (1u << 22)) sweep(std::true_type());  // every e2 below 2^22
-        else sweep(std::false_type());
+        }
         wave_sync();
-        // min of the square roots = square root of the min (sqrt is monotone)
-        const double dist = ok ? sqrt(__longlong_as_double((long long)tab.mins[lane])) : INFINITY;
+        // min of the square roots = square root of the min (sqrt is monotone);
+        // a row that was not evaluated has no distance
+        const double dist = ok && w ? sqrt(__longlong_as_double((long long)tab.mins[lane])) : INFINITY;
         double run = dist;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
@@ -481,13 +624,13 @@ __device__ __forceinline__ int refine_batch(const DevSet &S, const farm_raster_h
         if (hit) {
             const int ks = uni(__ffsll(hit) - 1);
             const double md = uni(__shfl(run, ks, 64));
-            r.evals += tab.pre[ks + 1];
+            r.evals += uni(__shfl(pall, ks, 64));
             min_dist = md;
             r.min_dist = md;
             return md < d ? 1 : 0;
         }
-        r.evals += W;
-        if (__ballot(ok)) {
+        r.evals += Wall;
+        if (okm) {
             min_dist = uni(__shfl(run, 63, 64));
             r.min_dist = min_dist;
         }
@@ -643,29 +786,45 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
         if (lane == 0) {
             tab.km.lo = i0;
             tab.km.n = n;
+            tab.km.inv_max = c_km_lon_inv[min(i1 + 1, 899)];  // (the table grows with the latitude)
         }
         wave_sync();
     }
     // every layer must fit the pixel buffers (the finest is the largest,
-    // but check all: a coarse layer may be one pixel wider)
-    for (int k = 0; k <= s_level; k++) {
-        const LGrid g = lgrid(S, hs, k);
-        if ((uint64_t)g.dimx * g.dimy > pixcap || g.dimx > (1 << SH) || g.dimy > (1 << SH)) {
-            r.bit = 3;
-            return r;
-        }
+    // but check all: a coarse layer may be one pixel wider); lane k < 32 looks
+    // at layer k of the source, lane 32 + k at the target's
+    bool big = false;
+    for (int k = lane & 31; k <= max(s_level, t_level); k += 32) {
+        const bool src = lane < 32;
+        if (k > (src ? s_level : t_level)) continue;
+        const LGrid g = lgrid(S, src ? hs : ht, k);
+        big = big || (uint64_t)g.dimx * g.dimy > pixcap || g.dimx > (1 << SH) || g.dimy > (1 << SH);
+        if (k < kLayC) tab.lay.g[src ? 0 : 1][k] = g;
     }
-    for (int k = 0; k <= t_level; k++) {
-        const LGrid g = lgrid(S, ht, k);
-        if ((uint64_t)g.dimx * g.dimy > pixcap || g.dimx > (1 << SH) || g.dimy > (1 << SH)) {
-            r.bit = 3;
-            return r;
-        }
+    if (wave_any(big)) {
+        r.bit = 3;
+        return r;
     }
+    wave_sync();
+    auto lay = [&](int side, int k) {
+        if (k >= kLayC) return lgrid(S, side ? ht : hs, k);
+        const LGrid &c = tab.lay.g[side][k];  // (uniform: into scalar registers)
+        LGrid g;
+        g.lx = uni(c.lx);
+        g.ly = uni(c.ly);
+        g.step = uni(c.step);
+        g.dimx = uni(c.dimx);
+        g.dimy = uni(c.dimy);
+        const uint64_t st = (uint64_t)c.st;
+        g.st = (const uint8_t *)(((uint64_t)uni((uint32_t)(st >> 32)) << 32) | uni((uint32_t)st));
+        return g;
+    };
+    auto slay = [&](int k) { return lay(0, k); };
+    auto tlay = [&](int k) { return lay(1, k); };
     // level 0: every pixel of both top layers
     uint32_t ns, nt;
     {
-        const LGrid gs = lgrid(S, hs, 0), gt = lgrid(S, ht, 0);
+        const LGrid gs = slay(0), gt = tlay(0);
         ns = (uint32_t)(gs.dimx * gs.dimy);
         nt = (uint32_t)(gt.dimx * gt.dimy);
         for (uint32_t k = lane; k < ns; k += 64) sl[k] = pack_xy<SH, T>(k % gs.dimx, k / gs.dimx);
@@ -677,11 +836,11 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
     // the LDS path keeps the last level's grids, lists and bound for its own
     // candidate generation (below); the global path writes its candidates to
     // the slab
-    LGrid fgs = lgrid(S, hs, 0), fgt = lgrid(S, ht, 0);
+    LGrid fgs = slay(0), fgt = tlay(0);
     uint32_t fns = 0, fnt = 0;
     double fkeep2 = -1.0;
     for (;;) {
-        const double s_step = lgrid(S, hs, i).step, t_step = lgrid(S, ht, j).step;
+        const double s_step = slay(i).step, t_step = tlay(j).step;
         bool s_next = false, t_next = false;
         if (i < s_level && (s_step >= t_step || j >= t_level)) {
             i++;
@@ -693,15 +852,15 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
         }
         if (ns == 0 || nt == 0) break;  // the queue of pixel pairs is empty
         final_level = !s_next && !t_next;
-        const LGrid gs = lgrid(S, hs, i), gt = lgrid(S, ht, j);
+        const LGrid gs = slay(i), gt = tlay(j);
         const int npix_s = gs.dimx * gs.dimy, npix_t = gt.dimx * gt.dimy;
-        clear_bits(sb, npix_s, lane);
-        clear_bits(tb, npix_t, lane);
-        const uint8_t *sts = gs.st, *stt = gt.st;
-        expand_side<SH>(sl, ns, s_next, s_next ? lgrid(S, hs, i - 1) : gs, gs, sts, sb, lane);
-        expand_side<SH>(tl, nt, t_next, t_next ? lgrid(S, ht, j - 1) : gt, gt, stt, tb, lane);
-        ns = compact<SH>(sb, npix_s, gs.dimx, sl, lane);
-        nt = compact<SH>(tb, npix_t, gt.dimx, tl, lane);
+        clear_bits(sb, npix_s, tb, npix_t, lane);
+        {
+            const LGrid ps = s_next ? slay(i - 1) : gs, pt = t_next ? tlay(j - 1) : gt;
+            expand_both<SH, T>(Expand<SH, T>(s_next, ps, gs, sb), sl, ns, Expand<SH, T>(t_next, pt, gt, tb), tl, nt,
+                               lane);
+        }
+        compact_both<SH, T>(sb, npix_s, gs.dimx, sl, ns, tb, npix_t, gt.dimx, tl, nt, lane);
         if (ns == 0 || nt == 0) break;  // no BORDER pixel on a side: nothing to refine
         // pass 1: any BORDER box pair within d by its farthest corners
         // decides; else the smallest such maximum bounds the useful pairs
@@ -751,8 +910,7 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
         // pass 2: keep pairs with min distance <= d and below maxd; their
         // projections are the next level's sets, or (last level) they are
         // the candidates
-        clear_bits(sb, npix_s, lane);
-        clear_bits(tb, npix_t, lane);
+        clear_bits(sb, npix_s, tb, npix_t, lane);
         uint32_t nc = 0;
         bool over = false;
         const double sa = gs.step * gs.step, ta = gt.step * gt.step;
@@ -819,8 +977,7 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
             r.ncand = nc;
             break;
         }
-        ns = compact<SH>(sb, npix_s, gs.dimx, sl, lane);
-        nt = compact<SH>(tb, npix_t, gt.dimx, tl, lane);
+        compact_both<SH, T>(sb, npix_s, gs.dimx, sl, ns, tb, npix_t, gt.dimx, tl, nt, lane);
     }
     if (!final_level) return r;
     if constexpr (SH == 8) {
@@ -947,13 +1104,40 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
             const double later = __shfl_down(sfx, 1, 64);
             const double rref = fmin(kFar, fmin(lane < 63 ? later : INFINITY, rest));
             const uint32_t rids = (best.id1 & 0xffffu) | (best.id2 << 16);
+            // What lane k's candidate comes to without a look at its sequences:
+            // the evaluations of its rows and a bound of their distances.
+            unsigned long long cev = 0;
+            double clow = 0.0;
+            if ((uint32_t)lane < nb) {
+                const uint64_t p1 = hs.pix_start + best.id1, p2 = ht.pix_start + best.id2;
+                const float4 b1 = S.pixbox[p1], b2 = S.pixbox[p2];
+                const uint2 l1 = S.pixlen[p1], l2 = S.pixlen[p2];
+                // sum over the sequence pairs of lb (la - 1) + la (lb - 1)
+                cev = 2ull * l1.x * l2.x - (unsigned long long)l1.x * l2.y - (unsigned long long)l2.x * l1.y;
+                const double p[4] = {b1.x, b1.y, b1.z, b1.w}, q[4] = {b2.x, b2.y, b2.z, b2.w};
+                clow = box_low_d2(p, q, tab.km.inv_max);
+            }
             uint32_t k = 0;
             while (k < nb) {
+                // Candidates that neither lower the running minimum nor pass a
+                // check: out of its reach, and the minimum (>= d so far) is not
+                // below their reference_dist either.  A run of them is counted
+                // and passed over.
+                const uint64_t im = __ballot((uint32_t)lane < nb && min_dist >= rref && beyond(clow, min_dist)) >> k;
+                if (im & 1ull) {
+                    const uint32_t run = ~im ? (uint32_t)__ffsll((unsigned long long)~im) - 1u : 64u;
+                    unsigned long long v = (uint32_t)lane >= k && (uint32_t)lane < k + run ? cev : 0ull;
+                    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+                    r.evals += uni((uint32_t)v) | ((uint64_t)uni((uint32_t)(v >> 32)) << 32);
+                    k += run;
+                    continue;
+                }
+                const uint32_t k0 = k;
                 CandBatch cb;
                 bool open = true;
 #pragma unroll
                 for (int qq = 0; qq < kBatch; qq++) {
-                    if (open && k < nb) {
+                    if (open && k < nb && !((im >> (k - k0)) & 1ull)) {
                         const int kk = (int)k;
                         const uint32_t ids = (uint32_t)__builtin_amdgcn_readlane((int)rids, kk);
                         const uint32_t id1 = ids & 0xffffu, id2 = ids >> 16;
@@ -978,6 +1162,8 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
                             k++;
                             if (cb.nrows >= 64) open = false;
                         }
+                    } else {
+                        open = false;
                     }
                 }
                 const int res = refine_batch(S, hs, ht, cb, d, min_dist, r, tab, lane);
@@ -1045,6 +1231,46 @@ __device__ __forceinline__ PairOut within_pair(const DevSet &S, uint32_t ia, uin
 
 }  // namespace
 
+// Per pixel: the box of its edge sequences (low x, low y, high x, high y) and,
+// of the sequences of 2 edges or more, the edges and the count.
+__global__ __launch_bounds__(256) void k_pixrec(DevSet S, int64_t npolys, float4 *__restrict__ box,
+                                                uint2 *__restrict__ len) {
+    const int64_t p = blockIdx.x;
+    if (p >= npolys) return;
+    const farm_raster_hdr H = S.hdr[p];
+    const uint32_t npix = (uint32_t)H.dimx * (uint32_t)H.dimy;
+    for (uint32_t i = threadIdx.x; i < npix; i += blockDim.x) {
+        const uint32_t s0 = S.pixoff[H.pixoff_start + i], s1 = S.pixoff[H.pixoff_start + i + 1];
+        float4 b = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+        uint2 l = make_uint2(0u, 0u);
+        for (uint32_t s = s0; s < s1; s++) {
+            const uint32_t n = S.seqs[H.seq_start + s].y;
+            if (n >= 2) {
+                l.x += n;
+                l.y++;
+            }
+        }
+        if (s1 > s0) {
+            const uint32_t c1 = S.ixoff[H.seq_start + s1];
+            for (uint32_t c = S.ixoff[H.seq_start + s0]; c < c1; c++) {
+                const float4 q = S.ixbox[c];
+                if (!(fabsf(q.x) + q.z + fabsf(q.y) + q.w < INFINITY)) {  // an open box
+                    b = make_float4(-INFINITY, -INFINITY, INFINITY, INFINITY);
+                    break;
+                }
+                // (rounded outwards: a sum of two floats is within 2^-24 of its value)
+                const float ex = (fabsf(q.x) + q.z) * 0x1p-23f, ey = (fabsf(q.y) + q.w) * 0x1p-23f;
+                b.x = fminf(b.x, (q.x - q.z) - ex);
+                b.y = fminf(b.y, (q.y - q.w) - ey);
+                b.z = fmaxf(b.z, (q.x + q.z) + ex);
+                b.w = fmaxf(b.w, (q.y + q.w) + ey);
+            }
+        }
+        box[H.pix_start + i] = b;
+        len[H.pix_start + i] = l;
+    }
+}
+
 // Persistent waves take pairs in chunks from a global counter.  BIG: the
 // pair indices come from `list` (pairs the LDS path could not hold) and the
 // lists / bits live in a per-wave global slab.
@@ -1082,12 +1308,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         cand = reinterpret_cast<Cand *>(base + (((2ull * pixcap + 2 * wbits) * 4 + 255) & ~255ull));
     }
     unsigned long long ncand = 0, evals = 0, found = 0, boxes = 0;
+    // (consecutive pairs share their target: a few at a time, but not so many
+    // that a large target's pairs all fall to one wave of a small call)
+    const uint32_t grab = min(max(n / (gridDim.x * kWaves * 16u), 1u), kChunk);
     for (;;) {
         uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(&ctr[0], kChunk);
+        if (lane == 0) base = atomicAdd(&ctr[0], grab);
         base = uni(__shfl(base, 0, 64));
         if (base >= n) break;
-        const uint32_t end = min(base + kChunk, n);
+        const uint32_t end = min(base + grab, n);
         for (uint32_t k = base; k < end; k++) {
             const uint32_t idx = BIG ? list[k] : k;
             const uint32_t ia = pa[idx], ib = pb[idx];
@@ -1141,6 +1370,10 @@ template __global__ void k_within<true>(DevSet, const uint32_t *, const uint32_t
 
 using namespace farm;
 
+namespace farm {
+int build_ix_boxes(farm_handle h);
+}  // namespace farm
+
 namespace {
 
 int within_consts(farm_handle h) {
@@ -1153,6 +1386,20 @@ int within_consts(farm_handle h) {
     HIPCHK(h, hipMemcpyToSymbol(HIP_SYMBOL(c_km_lon_inv), inv, sizeof inv));
     HIPCHK(h, hipMemcpyToSymbol(HIP_SYMBOL(c_mean), mean, sizeof mean));
     h->within_consts_ready = true;
+    return FARM_OK;
+}
+
+// The pixels' records (k_pixrec), once per set.
+int build_pixrec(farm_handle h) {
+    int rc;
+    if ((rc = build_ix_boxes(h))) return rc;
+    if (h->pixrec_gen == h->set_gen) return FARM_OK;
+    if ((rc = ensure(h, h->pixbox, 16 * h->nstatus))) return rc;
+    if ((rc = ensure(h, h->pixlen, 8 * h->nstatus))) return rc;
+    hipLaunchKernelGGL(k_pixrec, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys,
+                       P<float4>(h->pixbox), P<uint2>(h->pixlen));
+    HIPCHK(h, hipGetLastError());
+    h->pixrec_gen = h->set_gen;
     return FARM_OK;
 }
 
@@ -1171,6 +1418,7 @@ int run_within(farm_handle h, uint64_t begin, uint64_t end, double d_km, uint8_t
     HIPCHK(h, hipSetDevice(h->device));
     int rc;
     if ((rc = within_consts(h))) return rc;
+    if (n && (rc = build_pixrec(h))) return rc;
     if (st) memset(st, 0, sizeof *st);
     if (st) st->pairs = n;
     if (n == 0) return FARM_OK;

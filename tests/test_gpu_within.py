@@ -119,3 +119,24 @@ def test_empty_window(device):
     device.upload_pairs(np.zeros(1, np.uint32), np.ones(1, np.uint32))
     bits, md, st = device.within(10.0, 0, 0)
     assert len(bits) == 0 and st["found"] == 0
+
+
+@pytest.mark.parametrize("chunk", [16, 32])
+@pytest.mark.parametrize("vpr", [10, 150])
+def test_candidates_and_rows_out_of_reach(vpr, chunk):
+    # large lakes near small and large ones: hundreds of candidates a pair, most
+    # of them passed over by their pixels' boxes or row by row; at vpr 150
+    # sequences of many chunks (and of more than the box of a row looks at);
+    # with 32-segment refinement chunks the boxes are a set of their own
+    rng = np.random.default_rng(61)
+    nv = np.concatenate([rng.integers(300, 1500, 30), rng.integers(20, 200, 60)])
+    ro, xy = datagen.star_polygons(rng, 90, 0.0, 1.5, nv, np.log(0.12), 0.9)
+    dev = capi.Device(0)
+    try:
+        dev.set_tuning(4, chunk, 8)
+        for d_km in (4.0, 15.0):
+            want, md, st = _run(dev, ro, xy, d_km=d_km, vpr=vpr)
+            assert (want == 0).sum() > 50 and (want == 1).sum() > 50
+        assert st["bb_pixel_pairs"] > 64 * 10
+    finally:
+        dev.close()
