@@ -460,38 +460,54 @@ __global__ __launch_bounds__(256) void k_chunk_box(DevSet S, int64_t npolys, uin
     if (p >= npolys) return;
     const farm_raster_hdr H = S.hdr[p];
     const float *x = S.x + H.vert_start, *y = S.y + H.vert_start;
-    for (uint32_t s = threadIdx.x; s < H.nseqs; s += blockDim.x) {
-        const uint2 sq = S.seqs[H.seq_start + s];
-        uint32_t o = choff[H.seq_start + s];
-        for (uint32_t base = 1; base <= sq.y; base += C, o++) {
-            const uint32_t n = min(C, sq.y - base + 1);
-            float x0 = x[sq.x + base - 1], x1 = x0, y0 = y[sq.x + base - 1], y1 = y0;
-            bool open = isfinite(x0) && isfinite(y0);  // false: never prune this chunk
-            float lx = x0, ly = y0;
-            uint64_t dirs = 0;
-            uint32_t mark = 0;
-            for (uint32_t m = 0; m < n; m++) {
-                const float vx = x[sq.x + base + m], vy = y[sq.x + base + m];
-                open = open && isfinite(vx) && isfinite(vy);
-                float s;
-                if (vx == lx && vy == ly) mark = kChunkPoint;
-                else dirs |= dir_angle(vx - lx, vy - ly, s) ? dir_bit(s - kDirTol) | dir_bit(s + kDirTol) : ~0ull;
-                lx = vx;
-                ly = vy;
-                x0 = fminf(x0, vx);
-                x1 = fmaxf(x1, vx);
-                y0 = fminf(y0, vy);
-                y1 = fmaxf(y1, vy);
-            }
-            const float cx = 0.5f * x0 + 0.5f * x1, cy = 0.5f * y0 + 0.5f * y1;
-            // a rounded difference is within 2^-24 of the exact one; the
-            // factor and the smallest normal cover it and the product's rounding
-            float hx = fmaxf(x1 - cx, cx - x0) * 1.0000003f + 1.1754944e-38f;
-            float hy = fmaxf(y1 - cy, cy - y0) * 1.0000003f + 1.1754944e-38f;
-            const float big = 0x1p40f;
-            if (!(open && fabsf(cx) + hx < big && fabsf(cy) + hy < big)) hx = hy = INFINITY;
-            box[o] = make_float4(cx, cy, hx, hy);
-            seg[o] = make_uint4(sq.x + base - 1, n | mark, (uint32_t)dirs, (uint32_t)(dirs >> 32));
+    // chunk o of sequence sq, whose segments start at step base
+    auto put = [&](uint2 sq, uint32_t base, uint32_t o) {
+        const uint32_t n = min(C, sq.y - base + 1);
+        float x0 = x[sq.x + base - 1], x1 = x0, y0 = y[sq.x + base - 1], y1 = y0;
+        bool open = isfinite(x0) && isfinite(y0);  // false: never prune this chunk
+        float lx = x0, ly = y0;
+        uint64_t dirs = 0;
+        uint32_t mark = 0;
+        for (uint32_t m = 0; m < n; m++) {
+            const float vx = x[sq.x + base + m], vy = y[sq.x + base + m];
+            open = open && isfinite(vx) && isfinite(vy);
+            float s;
+            if (vx == lx && vy == ly) mark = kChunkPoint;
+            else dirs |= dir_angle(vx - lx, vy - ly, s) ? dir_bit(s - kDirTol) | dir_bit(s + kDirTol) : ~0ull;
+            lx = vx;
+            ly = vy;
+            x0 = fminf(x0, vx);
+            x1 = fmaxf(x1, vx);
+            y0 = fminf(y0, vy);
+            y1 = fmaxf(y1, vy);
+        }
+        const float cx = 0.5f * x0 + 0.5f * x1, cy = 0.5f * y0 + 0.5f * y1;
+        // a rounded difference is within 2^-24 of the exact one; the
+        // factor and the smallest normal cover it and the product's rounding
+        float hx = fmaxf(x1 - cx, cx - x0) * 1.0000003f + 1.1754944e-38f;
+        float hy = fmaxf(y1 - cy, cy - y0) * 1.0000003f + 1.1754944e-38f;
+        const float big = 0x1p40f;
+        if (!(open && fabsf(cx) + hx < big && fabsf(cy) + hy < big)) hx = hy = INFINITY;
+        box[o] = make_float4(cx, cy, hx, hy);
+        seg[o] = make_uint4(sq.x + base - 1, n | mark, (uint32_t)dirs, (uint32_t)(dirs >> 32));
+    };
+    // a lane takes a short sequence whole; the chunks of a longer one are
+    // shared by the wave (1.18 -> 0.58 ms for 400 rings of 1.6 M vertices in
+    // all and 10,000 lakes, where one lane had sequences of 10,000 segments)
+    const int lane = threadIdx.x & 63;
+    for (uint32_t s0 = threadIdx.x & ~63u; s0 < H.nseqs; s0 += blockDim.x) {
+        const uint32_t s = s0 + lane;
+        const uint2 sq = s < H.nseqs ? S.seqs[H.seq_start + s] : make_uint2(0u, 0u);
+        const uint32_t o = s < H.nseqs ? choff[H.seq_start + s] : 0u;
+        const bool wide = sq.y > 4 * C;
+        if (!wide)
+            for (uint32_t k = 0; k * C < sq.y; k++) put(sq, 1 + k * C, o + k);
+        for (uint64_t m = __ballot(wide); m; m &= m - 1) {
+            const int src = __ffsll((unsigned long long)m) - 1;
+            const uint2 w = make_uint2((uint32_t)__builtin_amdgcn_readlane((int)sq.x, src),
+                                       (uint32_t)__builtin_amdgcn_readlane((int)sq.y, src));
+            const uint32_t wo = (uint32_t)__builtin_amdgcn_readlane((int)o, src);
+            for (uint32_t k = lane; k * C < w.y; k += 64) put(w, 1 + k * C, wo + k);
         }
     }
 }

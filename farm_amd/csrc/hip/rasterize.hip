@@ -542,15 +542,16 @@ __global__ __launch_bounds__(kRB) void k_rscan(const RPoly *__restrict__ P, cons
 // ---------------------------------------------------- fill classes ----
 
 // Column and row bounds as the reference accumulates them (Xi += step_x),
-// and the number of columns / rows its loops visit.
+// the number of columns / rows its loops visit, and each column's polygon.
 __global__ __launch_bounds__(kRB) void k_rbounds(const RPoly *__restrict__ P, int64_t np,
                                                  uint32_t *__restrict__ rflag, double *__restrict__ colx,
                                                  double *__restrict__ rowy, int *__restrict__ ncols,
-                                                 int *__restrict__ nrows) {
+                                                 int *__restrict__ nrows, uint32_t *__restrict__ colpoly) {
     const int64_t i = (int64_t)blockIdx.x * kRB + threadIdx.x;
     if (i >= np) return;
     const RPoly g = P[i];
     ncols[i] = nrows[i] = 0;
+    for (int c = 0; c < g.dimx + 2; c++) colpoly[g.vl + c] = (uint32_t)i;
     if (rflag[i]) return;
     bool over = false;
     {
@@ -674,20 +675,27 @@ __device__ __forceinline__ uint32_t hash_put(unsigned long long *keys, uint32_t 
 
 // Candidate counts of every column strip (PASS 0, before dedup) or the
 // strips themselves (PASS 1): kept points in order, the first repeated at
-// the end, their count and largest |y|.
+// the end, their count and largest |y|.  One workgroup per column: a ring of
+// 200,000 vertices has 28 of them, and one workgroup went through them in turn
+// (both passes 13.2 ms for 400 rings of 1,000 to 130,000 vertices and 10,000
+// lakes; 2.1 ms so, the longest strip's serial batches).
 template <int PASS>
 __global__ __launch_bounds__(kRB) void k_rstrip(const RPoly *__restrict__ P, const float *__restrict__ X,
                                                 const float *__restrict__ Y, const float *__restrict__ absx,
                                                 uint32_t *__restrict__ rflag, const int *__restrict__ ncols,
                                                 const int *__restrict__ nrows, const double *__restrict__ colx,
+                                                const uint32_t *__restrict__ colpoly, uint64_t slot0,
                                                 uint32_t *__restrict__ stripc, const uint64_t *__restrict__ stripo,
                                                 const uint64_t *__restrict__ hasho, float2 *__restrict__ pool,
+                                                float2 *__restrict__ nearpool,
                                                 unsigned long long *__restrict__ hkeys, uint32_t *__restrict__ hidx,
                                                 uint32_t *__restrict__ stripn, float *__restrict__ stripmy) {
-    const int64_t i = blockIdx.x;
+    const uint64_t cs = slot0 + blockIdx.x;
+    const uint32_t i = colpoly[cs];
     if (rflag[i]) return;
     const RPoly g = P[i];
-    const int ncol = ncols[i], nrow = nrows[i];
+    const int ncol = ncols[i], nrow = nrows[i], c = (int)(cs - g.vl);
+    if (c >= ncol) return;
     const Bucket bk(g.x0, g.sx, g.dimx + 2, (double)absx[i]);
     const float *Xp = X + g.v, *Yp = Y + g.v;
     const int ne = (int)g.nv - 1;
@@ -696,131 +704,257 @@ __global__ __launch_bounds__(kRB) void k_rstrip(const RPoly *__restrict__ P, con
     __shared__ uint32_t s_idx[PASS ? kLdsSlots : 1];
     __shared__ float2 s_cand[PASS ? kChunkCands : 1];
     __shared__ uint8_t s_keep[PASS ? kChunkCands : 1], s_near[PASS ? kChunkCands : 1];
+    __shared__ uint16_t s_list[PASS ? kChunkCands : 1];
+    __shared__ uint32_t s_nkept;
     __shared__ float s_my[kRB / 64];
     bool fail = false;
-    for (int c = 0; c < ncol; c++) {
-        const double Xi = colx[g.vl + c], Xi1 = colx[g.vl + c + 1];
-        if (PASS == 0) {
-            uint32_t cnt = 0;
-            for (int e = threadIdx.x; e < ne; e += kRB) {
-                const float ax = Xp[e], bx = Xp[e + 1];
-                if (!bk.reaches(ax, bx, c)) continue;
-                float2 pts[4];
-                cnt += strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, pts);
-            }
-            uint32_t tot;
-            block_scan(cnt, sh, &tot);
-            if (threadIdx.x == 0) stripc[g.vl + c] = tot;
-            continue;
+    const double Xi = colx[g.vl + c], Xi1 = colx[g.vl + c + 1];
+    if (PASS == 0) {
+        uint32_t cnt = 0;
+        for (int e = threadIdx.x; e < ne; e += kRB) {
+            const float ax = Xp[e], bx = Xp[e + 1];
+            if (!bk.reaches(ax, bx, c)) continue;
+            float2 pts[4];
+            cnt += strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, pts);
         }
-        const uint32_t cnt = stripc[g.vl + c];
-        if (cnt == 0) {
-            if (threadIdx.x == 0) stripn[g.vl + c] = 0;
-            continue;
+        uint32_t tot;
+        block_scan(cnt, sh, &tot);
+        if (threadIdx.x == 0) stripc[g.vl + c] = tot;
+        return;
+    }
+    const uint32_t cnt = stripc[g.vl + c];
+    if (cnt == 0) {
+        if (threadIdx.x == 0) stripn[g.vl + c] = 0;
+        return;
+    }
+    float2 *pts = pool + stripo[g.vl + c], *nearp = nearpool + stripo[g.vl + c];
+    if (threadIdx.x == 0) s_nkept = 0;
+    const bool lds = cnt <= kLdsCands;
+    uint32_t slots = kLdsSlots;
+    if (!lds) {
+        slots = 1;
+        while (slots < 2 * cnt) slots <<= 1;
+    }
+    unsigned long long *gkeys = hkeys + (lds ? 0 : hasho[g.vl + c]);
+    uint32_t *gix = hidx + (lds ? 0 : hasho[g.vl + c]);
+    const uint32_t mask = slots - 1;
+    if (lds) {
+        for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
+            s_keys[s] = 0;
+            s_idx[s] = 0xffffffffu;
         }
-        float2 *pts = pool + stripo[g.vl + c];
-        const bool lds = cnt <= kLdsCands;
-        uint32_t slots = kLdsSlots;
-        if (!lds) {
-            slots = 1;
-            while (slots < 2 * cnt) slots <<= 1;
+    } else {
+        for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
+            gkeys[s] = 0;
+            gix[s] = 0xffffffffu;
         }
-        unsigned long long *gkeys = hkeys + (lds ? 0 : hasho[g.vl + c]);
-        uint32_t *gix = hidx + (lds ? 0 : hasho[g.vl + c]);
-        const uint32_t mask = slots - 1;
-        if (lds) {
-            for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
-                s_keys[s] = 0;
-                s_idx[s] = 0xffffffffu;
+    }
+    __syncthreads();
+    uint32_t base = 0, kept = 0;
+    float my = 0.f;
+    for (int c0 = 0; c0 < ne; c0 += kRB) {
+        // most batches of a long ring miss the column: four at a time are
+        // passed over with one barrier
+        if ((c0 & (4 * kRB - 1)) == 0) {
+            bool any = false;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int e = c0 + q * kRB + (int)threadIdx.x;
+                any = any || (e < ne && bk.reaches(Xp[e], Xp[e + 1], c));
             }
-        } else {
-            for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
-                gkeys[s] = 0;
-                gix[s] = 0xffffffffu;
+            if (!__syncthreads_or(any)) {
+                c0 += 3 * kRB;
+                continue;
             }
+        }
+        const int e = c0 + threadIdx.x;
+        float2 loc[4];
+        uint32_t n = 0;
+        if (e < ne) {
+            const float ax = Xp[e], bx = Xp[e + 1];
+            if (bk.reaches(ax, bx, c)) n = strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, loc);
+        }
+        if (!__syncthreads_or(n != 0)) continue;
+        uint32_t tot;
+        const uint32_t off = block_scan(n, sh, &tot);
+        uint32_t slot[4];
+        uint32_t nnear = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) {
+            if (j >= n) break;
+            s_cand[off + j] = loc[j];
+            const bool nr = near_axis(loc[j]);
+            s_near[off + j] = nr;
+            nnear += nr;
+            if (!nr)
+                slot[j] = lds ? hash_put(s_keys, s_idx, mask, pt_key(loc[j]), base + off + j)
+                              : hash_put(gkeys, gix, mask, pt_key(loc[j]), base + off + j);
         }
         __syncthreads();
-        uint32_t base = 0, kept = 0;
-        float my = 0.f;
-        for (int c0 = 0; c0 < ne; c0 += kRB) {
-            const int e = c0 + threadIdx.x;
-            float2 loc[4];
-            uint32_t n = 0;
-            if (e < ne) {
-                const float ax = Xp[e], bx = Xp[e + 1];
-                if (bk.reaches(ax, bx, c)) n = strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, loc);
-            }
-            uint32_t tot;
-            const uint32_t off = block_scan(n, sh, &tot);
-            if (tot == 0) continue;
-            uint32_t slot[4];
-            bool anynear = false;
 #pragma unroll
-            for (uint32_t j = 0; j < 4; j++) {
-                if (j >= n) break;
-                s_cand[off + j] = loc[j];
-                const bool nr = near_axis(loc[j]);
-                s_near[off + j] = nr;
-                anynear |= nr;
-                if (!nr)
-                    slot[j] = lds ? hash_put(s_keys, s_idx, mask, pt_key(loc[j]), base + off + j)
-                                  : hash_put(gkeys, gix, mask, pt_key(loc[j]), base + off + j);
+        for (uint32_t j = 0; j < 4; j++) {
+            if (j >= n) break;
+            s_keep[off + j] =
+                s_near[off + j] || ((lds ? s_idx[slot[j]] : gix[slot[j]]) == base + off + j);
+        }
+        if (__syncthreads_or(nnear != 0)) {
+            // Points near an axis, in order, against every point kept before
+            // them.  Only another point near an axis can equal one: a
+            // coordinate of kNearAxis or more equals its own bits alone.  All
+            // the batch's are compared with the kept ones of earlier batches
+            // and with each other at once; only those that equal an earlier
+            // one of their own batch go in turn, as that one may be dropped.
+            // (Every point in turn against all kept ones held a 75,000-point
+            // ring at the axis for 5.8 ms of the pass; 1.9 ms so.)
+            uint32_t nn;
+            uint32_t no = block_scan(nnear, sh, &nn);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                if (j < n && s_near[off + j]) s_list[no++] = (uint16_t)(off + j);
+            __syncthreads();
+            const uint32_t prior = s_nkept;
+            for (uint32_t q = 0; q < nn; q++) {
+                const uint32_t j = s_list[q];
+                const float2 p = s_cand[j];
+                bool found = false, twin = false;
+                for (uint32_t k = threadIdx.x; k < prior; k += kRB) found |= same_pt(nearp[k], p);
+                for (uint32_t k = threadIdx.x; k < q; k += kRB) twin |= same_pt(s_cand[s_list[k]], p);
+                if (found) s_keep[j] = 0;
+                if (twin) s_near[j] = 2;
             }
             __syncthreads();
-#pragma unroll
-            for (uint32_t j = 0; j < 4; j++) {
-                if (j >= n) break;
-                s_keep[off + j] =
-                    s_near[off + j] ? 0 : ((lds ? s_idx[slot[j]] : gix[slot[j]]) == base + off + j);
+            for (uint32_t q = 0; q < nn; q++) {
+                const uint32_t j = s_list[q];
+                if (s_near[j] != 2 || !s_keep[j]) continue;
+                const float2 p = s_cand[j];
+                bool found = false;
+                for (uint32_t k = threadIdx.x; k < q; k += kRB)
+                    found |= s_keep[s_list[k]] && same_pt(s_cand[s_list[k]], p);
+                found = __syncthreads_or(found);
+                if (threadIdx.x == 0) s_keep[j] = !found;
+                __syncthreads();
             }
-            if (__syncthreads_or(anynear)) {
-                // points near an axis, in order, against every point kept before them
-                for (uint32_t j = 0; j < tot; j++) {
-                    if (!s_near[j]) continue;
-                    const float2 p = s_cand[j];
-                    bool found = false;
-                    for (uint32_t k = threadIdx.x; k < kept; k += kRB) found |= same_pt(pts[k], p);
-                    for (uint32_t k = threadIdx.x; k < j; k += kRB) found |= s_keep[k] && same_pt(s_cand[k], p);
-                    found = __syncthreads_or(found);
-                    if (threadIdx.x == 0) s_keep[j] = !found;
-                    __syncthreads();
-                }
+            for (uint32_t q = threadIdx.x; q < nn; q += kRB)
+                if (s_keep[s_list[q]]) nearp[atomicAdd(&s_nkept, 1u)] = s_cand[s_list[q]];
+        }
+        uint32_t nk = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+            if (j < n) nk += s_keep[off + j];
+        uint32_t ktot;
+        uint32_t ko = block_scan(nk, sh, &ktot);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+            if (j < n && s_keep[off + j]) {
+                pts[kept + ko++] = loc[j];
+                my = smax(my, fabsf(loc[j].y));
             }
-            uint32_t nk = 0;
-#pragma unroll
-            for (uint32_t j = 0; j < 4; j++)
-                if (j < n) nk += s_keep[off + j];
-            uint32_t ktot;
-            uint32_t ko = block_scan(nk, sh, &ktot);
-#pragma unroll
-            for (uint32_t j = 0; j < 4; j++)
-                if (j < n && s_keep[off + j]) {
-                    pts[kept + ko++] = loc[j];
-                    my = smax(my, fabsf(loc[j].y));
-                }
-            base += tot;
-            kept += ktot;
-        }
-        // the largest |y| of the strip (the row buckets' margin scale)
-        const float wm = wave_max(my);
-        if ((threadIdx.x & 63) == 0) s_my[threadIdx.x >> 6] = wm;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            float m = s_my[0];
-            for (int w = 1; w < kRB / 64; w++) m = smax(m, s_my[w]);
-            if (kept > 0) pts[kept] = pts[0];
-            stripn[g.vl + c] = kept ? kept + 1 : 0;
-            stripmy[g.vl + c] = m;
-            // a non-empty strip outside the grid: the reference asserts
-            if (kept > 0 && (c >= g.dimx || nrow > g.dimy)) fail = true;
-        }
-        __syncthreads();
+        base += tot;
+        kept += ktot;
     }
+    // the largest |y| of the strip (the row buckets' margin scale)
+    const float wm = wave_max(my);
+    if ((threadIdx.x & 63) == 0) s_my[threadIdx.x >> 6] = wm;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float m = s_my[0];
+        for (int w = 1; w < kRB / 64; w++) m = smax(m, s_my[w]);
+        if (kept > 0) pts[kept] = pts[0];
+        stripn[g.vl + c] = kept ? kept + 1 : 0;
+        stripmy[g.vl + c] = m;
+        // a non-empty strip outside the grid: the reference asserts
+        if (kept > 0 && (c >= g.dimx || nrow > g.dimy)) fail = true;
+    }
+    __syncthreads();
     if (PASS == 1 && threadIdx.x == 0 && fail) atomicOr(&rflag[i], kRejFill);
 }
 
-// Ideal::calculate_fullness, y pass and encodePixelArea (Ideal.cpp:64-88),
-// one lane per pixel of a visited cell.
+// Points strip edge (A, B) adds to row [Yi, Yi1] (Ideal::calculate_fullness,
+// its y pass), in order; their count.
+__device__ __forceinline__ uint32_t cell_points(float2 A, float2 B, double Yi, double Yi1, float2 *out) {
+    bool skip = false, ok0 = true, ok1 = true;
+    double xi = 0, xi1 = 0;
+    if (A.x == B.x) {
+        xi = A.x;
+        xi1 = A.x;
+    } else {
+        const float den = B.x - A.x;
+        const double slope = ((double)B.y - A.y) / den;
+        if (A.y == B.y) {
+            if (A.y == Yi) {
+                xi = A.x;
+                ok1 = false;
+            } else if (A.y == Yi1) {
+                ok0 = false;
+                xi1 = A.x;
+            } else {
+                skip = true;
+            }
+        } else {
+            xi = ((Yi - B.y) / slope) + B.x;
+            xi1 = ((Yi1 - B.y) / slope) + B.x;
+        }
+    }
+    // constant indexes only, so that out[] stays in registers
+    uint32_t n = 0;
+    auto app = [&](float2 p) {
+#pragma unroll
+        for (uint32_t j = 0; j < 3; j++)
+            if (n == j) out[j] = p;
+        n++;
+    };
+    if (within(Yi, Yi1, A.y)) app(A);
+    if (!skip) {
+        const float2 q0 = make_float2((float)xi, (float)Yi), q1 = make_float2((float)xi1, (float)Yi1);
+        const float mny = smin(A.y, B.y), mxy = smax(A.y, B.y);
+        const float mnx = smin(A.x, B.x), mxx = smax(A.x, B.x);
+        const bool in0 = ok0 && within(mnx, mxx, q0.x) && within(mny, mxy, q0.y);
+        const bool in1 = ok1 && within(mnx, mxx, q1.x) && within(mny, mxy, q1.y);
+        if (A.y < B.y) {
+            if (in0) app(q0);
+            if (in1) app(q1);
+        } else {
+            if (in1) app(q1);
+            if (in0) app(q0);
+        }
+    }
+    return n;
+}
+
+// A cell's points so far and the shoelace over them, in the host's order.
+struct CellSum {
+    double area;
+    uint32_t cnt;
+    float2 first, prv;
+};
+__device__ __forceinline__ double shoelace(float2 p, float2 q) { return (double)p.x * q.y - (double)q.x * p.y; }
+
+// encodePixelArea (Ideal.cpp:64-88) of a BORDER pixel from its points.
+__device__ __forceinline__ void put_cell(CellSum c, double pix_area, uint8_t *status, double *area_out) {
+    if (c.cnt > 0 && !same_pt(c.first, c.prv)) {
+        c.area += shoelace(c.prv, c.first);
+        c.cnt++;
+    }
+    const double area = c.cnt >= 3 ? fabs(c.area) / 2.0 : 0.0;
+    int cls;
+    const double ratio = area / pix_area;
+    if (fabs(ratio - 1.0) < 1e-9) cls = kCC - 1;
+    else if (fabs(ratio) < 1e-9) cls = 0;
+    else {
+        cls = cvt_x86(ceil(ratio * (kCC - 2)));
+        if (cls >= kCC) cls = kCC - 1;
+        cls = (uint8_t)cls;
+    }
+    *status = (uint8_t)max(1, min(cls, kCC - 2));
+    *area_out = area;
+}
+
+// Ideal::calculate_fullness, y pass and encodePixelArea, one lane per pixel of
+// a visited cell; the BORDER pixels of a strip of more than kWaveStrip points
+// are left to k_rcells_wide (a lane alone with a strip of 10,000 points held
+// the kernel for 7.1 ms on those sets; 0.15 and 0.62 ms in the two).
+constexpr uint32_t kWaveStrip = 128;
+
 __global__ __launch_bounds__(kRB) void k_rcells(const RPoly *__restrict__ P, const uint32_t *__restrict__ pixpoly,
                                                 uint64_t npix, const uint32_t *__restrict__ rflag,
                                                 const int *__restrict__ ncols, const int *__restrict__ nrows,
@@ -839,87 +973,107 @@ __global__ __launch_bounds__(kRB) void k_rcells(const RPoly *__restrict__ P, con
         if (n == 0) continue;
         const uint8_t st = status[p];
         const double pix_area = g.sx * g.sy;
-        if (st == kRawIn) {
-            status[p] = kCC - 1;
-            areas[p] = pix_area;
-            continue;
-        }
-        if (st != kRawBorder) {
-            status[p] = 0;
-            areas[p] = 0.0;
+        if (st == kRawBorder) {
+            if (n > kWaveStrip) continue;
+        } else {
+            status[p] = st == kRawIn ? kCC - 1 : 0;
+            areas[p] = st == kRawIn ? pix_area : 0.0;
             continue;
         }
         const double Yi = rowy[g.hl + row], Yi1 = rowy[g.hl + row + 1];
         const Bucket bk(g.y0, g.sy, g.dimy + 2, (double)stripmy[g.vl + col]);
         const float2 *V = pool + stripo[g.vl + col];
         // the cell's points, summed into the shoelace as they come
-        double area = 0.0;
-        uint32_t cnt = 0;
-        float2 first = make_float2(0.f, 0.f), prv = first;
-        auto push = [&](float2 q) {
-            if (cnt == 0) first = q;
-            else area += ((double)prv.x * q.y - (double)q.x * prv.y);
-            prv = q;
-            cnt++;
-        };
+        CellSum c{0.0, 0u, make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
         float2 A = V[0];
         for (uint32_t k = 0; k + 1 < n; k++) {
             const float2 B = V[k + 1];
             if (bk.reaches(A.y, B.y, row)) {
-                bool skip = false, ok0 = true, ok1 = true;
-                double xi = 0, xi1 = 0;
-                if (A.x == B.x) {
-                    xi = A.x;
-                    xi1 = A.x;
-                } else {
-                    const float den = B.x - A.x;
-                    const double slope = ((double)B.y - A.y) / den;
-                    if (A.y == B.y) {
-                        if (A.y == Yi) {
-                            xi = A.x;
-                            ok1 = false;
-                        } else if (A.y == Yi1) {
-                            ok0 = false;
-                            xi1 = A.x;
-                        } else {
-                            skip = true;
-                        }
-                    } else {
-                        xi = ((Yi - B.y) / slope) + B.x;
-                        xi1 = ((Yi1 - B.y) / slope) + B.x;
+                float2 pts[3];
+                const uint32_t m = cell_points(A, B, Yi, Yi1, pts);
+#pragma unroll
+                for (uint32_t j = 0; j < 3; j++)
+                    if (j < m) {
+                        if (c.cnt == 0) c.first = pts[j];
+                        else c.area += shoelace(c.prv, pts[j]);
+                        c.prv = pts[j];
+                        c.cnt++;
                     }
-                }
-                if (within(Yi, Yi1, A.y)) push(A);
-                if (!skip) {
-                    const float2 q0 = make_float2((float)xi, (float)Yi), q1 = make_float2((float)xi1, (float)Yi1);
-                    const float mny = smin(A.y, B.y), mxy = smax(A.y, B.y);
-                    const float mnx = smin(A.x, B.x), mxx = smax(A.x, B.x);
-                    const bool in0 = ok0 && within(mnx, mxx, q0.x) && within(mny, mxy, q0.y);
-                    const bool in1 = ok1 && within(mnx, mxx, q1.x) && within(mny, mxy, q1.y);
-                    if (A.y < B.y) {
-                        if (in0) push(q0);
-                        if (in1) push(q1);
-                    } else {
-                        if (in1) push(q1);
-                        if (in0) push(q0);
-                    }
-                }
             }
             A = B;
         }
-        if (cnt > 0 && !same_pt(first, prv)) push(first);
-        area = cnt >= 3 ? fabs(area) / 2.0 : 0.0;
-        int cls;
-        const double ratio = area / pix_area;
-        if (fabs(ratio - 1.0) < 1e-9) cls = kCC - 1;
-        else if (fabs(ratio) < 1e-9) cls = 0;
-        else {
-            cls = cvt_x86(ceil(ratio * (kCC - 2)));
-            if (cls >= kCC) cls = kCC - 1;
-            cls = (uint8_t)cls;
+        put_cell(c, pix_area, status + p, areas + p);
+    }
+}
+
+// The BORDER pixels of the long strips: one workgroup per column, a wave per
+// pixel, 64 strip edges at a time.  Every lane tests and clips its edge and
+// takes its points' shoelace terms; the terms are added one after the other in
+// the strip's order, as the host adds them.
+__global__ __launch_bounds__(kRB) void k_rcells_wide(const RPoly *__restrict__ P, const uint32_t *__restrict__ colpoly,
+                                                     uint64_t slot0, const uint32_t *__restrict__ rflag,
+                                                     const int *__restrict__ ncols, const int *__restrict__ nrows,
+                                                     const double *__restrict__ rowy,
+                                                     const uint64_t *__restrict__ stripo,
+                                                     const uint32_t *__restrict__ stripn,
+                                                     const float *__restrict__ stripmy,
+                                                     const float2 *__restrict__ pool, uint8_t *__restrict__ status,
+                                                     double *__restrict__ areas) {
+    const uint64_t cs = slot0 + blockIdx.x;
+    const uint32_t n = stripn[cs];
+    if (n <= kWaveStrip) return;
+    const uint32_t i = colpoly[cs];
+    if (rflag[i]) return;
+    const RPoly g = P[i];
+    const int col = (int)(cs - g.vl), lane = threadIdx.x & 63;
+    if (col >= ncols[i] || col >= g.dimx) return;
+    const Bucket bk(g.y0, g.sy, g.dimy + 2, (double)stripmy[cs]);
+    const float2 *V = pool + stripo[cs];
+    for (int row = threadIdx.x >> 6; row < min(nrows[i], g.dimy); row += kRB / 64) {
+        const uint64_t p = g.pix + (uint64_t)row * g.dimx + col;
+        if (status[p] != kRawBorder) continue;
+        const double Yi = rowy[g.hl + row], Yi1 = rowy[g.hl + row + 1];
+        CellSum c{0.0, 0u, make_float2(0.f, 0.f), make_float2(0.f, 0.f)};
+        for (uint32_t k0 = 0; k0 + 1 < n; k0 += 64) {
+            const uint32_t k = k0 + lane;
+            uint32_t m = 0;
+            const float2 none = make_float2(0.f, 0.f);
+            float2 pts[3] = {none, none, none}, last = none;
+            if (k + 1 < n) {
+                const float2 A = V[k], B = V[k + 1];
+                if (bk.reaches(A.y, B.y, row)) m = cell_points(A, B, Yi, Yi1, pts);
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 3; j++)
+                if (j < m) last = pts[j];
+            const uint64_t have = __ballot(m != 0);
+            if (!have) continue;
+            // the point before this lane's first: the last one of the nearest
+            // lower lane that has any, else the cell's last so far
+            const uint64_t below = have & ((1ull << lane) - 1ull);
+            const int pl = below ? 63 - __clzll((long long)below) : lane;
+            const float bx = __shfl(last.x, pl, 64), by = __shfl(last.y, pl, 64);
+            const float2 prv = below ? make_float2(bx, by) : c.prv;
+            const double t[3] = {shoelace(prv, pts[0]), shoelace(pts[0], pts[1]), shoelace(pts[1], pts[2])};
+            const int f = __ffsll((unsigned long long)have) - 1;
+            if (c.cnt == 0) c.first = make_float2(uni(__shfl(pts[0].x, f, 64)), uni(__shfl(pts[0].y, f, 64)));
+            for (uint64_t todo = have; todo; todo &= todo - 1) {
+                const int s = __ffsll((unsigned long long)todo) - 1;
+                const uint32_t ms = (uint32_t)__builtin_amdgcn_readlane((int)m, s);
+#pragma unroll
+                for (uint32_t j = 0; j < 3; j++)
+                    if (j < ms) {
+                        const long long tb = __double_as_longlong(t[j]);
+                        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)tb, s);
+                        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(tb >> 32), s);
+                        if (c.cnt != 0) c.area += __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+                        c.cnt++;
+                    }
+            }
+            const int l = 63 - __clzll((long long)have);
+            c.prv = make_float2(uni(__shfl(last.x, l, 64)), uni(__shfl(last.y, l, 64)));
         }
-        status[p] = (uint8_t)max(1, min(cls, kCC - 2));
-        areas[p] = area;
+        if (lane == 0) put_cell(c, g.sx * g.sy, status + p, areas + p);
     }
 }
 
@@ -1355,11 +1509,12 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
 
     // ---- fill classes ----
     double *colx, *rowy;
+    uint32_t *colpoly;
     int *ncols, *nrows;
     uint32_t *stripc, *stripn;
     uint64_t *psz, *stripo, *hsz, *hasho;
     float *stripmy;
-    if ((rc = T.get(h, &colx, nvl)) || (rc = T.get(h, &rowy, nhl)) || (rc = T.get(h, &ncols, np)) ||
+    if ((rc = T.get(h, &colx, nvl)) || (rc = T.get(h, &colpoly, nvl)) || (rc = T.get(h, &rowy, nhl)) || (rc = T.get(h, &ncols, np)) ||
         (rc = T.get(h, &nrows, np)) || (rc = T.get(h, &stripc, nvl)) || (rc = T.get(h, &stripn, nvl)) ||
         (rc = T.get(h, &stripmy, nvl)) || (rc = T.get(h, &psz, nvl + 1)) || (rc = T.get(h, &stripo, nvl + 1)) ||
         (rc = T.get(h, &hsz, nvl + 1)) || (rc = T.get(h, &hasho, nvl + 1)))
@@ -1368,15 +1523,23 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
     HIPCHK(h, hipMemsetAsync(stripn, 0, 4 * nvl, h->stream));
     if (np) {
         hipLaunchKernelGGL(k_rbounds, dim3(blocks_for(np)), dim3(kRB), 0, h->stream, (const RPoly *)d_rp, np, d_flag,
-                           colx, rowy, ncols, nrows);
-        HIPCHK(h, hipGetLastError());
-        hipLaunchKernelGGL(k_rstrip<0>, dim3((unsigned)np), dim3(kRB), 0, h->stream, (const RPoly *)d_rp,
-                           P<float>(h->x), P<float>(h->y), (const float *)d_absx, d_flag, (const int *)ncols,
-                           (const int *)nrows, (const double *)colx, stripc, (const uint64_t *)nullptr,
-                           (const uint64_t *)nullptr, (float2 *)nullptr, (unsigned long long *)nullptr,
-                           (uint32_t *)nullptr, stripn, stripmy);
+                           colx, rowy, ncols, nrows, colpoly);
         HIPCHK(h, hipGetLastError());
     }
+    // one workgroup per column slot (several launches beyond 2^30 of them)
+    auto strips = [&](auto kernel, const uint64_t *so, const uint64_t *hof, float2 *pool, float2 *nearpool,
+                      unsigned long long *hkeys, uint32_t *hidx) -> int {
+        for (uint64_t s0 = 0; s0 < nvl; s0 += 1ull << 30) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<uint64_t>(nvl - s0, 1ull << 30)), dim3(kRB), 0,
+                               h->stream, (const RPoly *)d_rp, P<float>(h->x), P<float>(h->y), (const float *)d_absx,
+                               d_flag, (const int *)ncols, (const int *)nrows, (const double *)colx,
+                               (const uint32_t *)colpoly, s0, stripc, so, hof, pool, nearpool, hkeys, hidx,
+                               stripn, stripmy);
+            HIPCHK(h, hipGetLastError());
+        }
+        return FARM_OK;
+    };
+    if ((rc = strips(k_rstrip<0>, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr))) return rc;
     // pool sizes: every candidate plus the closing point; hashes in HBM for
     // strips beyond the LDS table
     {
@@ -1399,17 +1562,11 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
         ho[nvl] = th;
         HIPCHK(h, hipMemcpyAsync(stripo, po.data(), 8 * (nvl + 1), hipMemcpyHostToDevice, h->stream));
         HIPCHK(h, hipMemcpyAsync(hasho, ho.data(), 8 * (nvl + 1), hipMemcpyHostToDevice, h->stream));
-        float2 *pool;
+        float2 *pool, *nearpool;
         unsigned long long *hkeys;
         uint32_t *hidx;
-        if ((rc = T.get(h, &pool, tp)) || (rc = T.get(h, &hkeys, th)) || (rc = T.get(h, &hidx, th))) return rc;
-        if (np) {
-            hipLaunchKernelGGL(k_rstrip<1>, dim3((unsigned)np), dim3(kRB), 0, h->stream, (const RPoly *)d_rp,
-                               P<float>(h->x), P<float>(h->y), (const float *)d_absx, d_flag, (const int *)ncols,
-                               (const int *)nrows, (const double *)colx, stripc, (const uint64_t *)stripo,
-                               (const uint64_t *)hasho, pool, hkeys, hidx, stripn, stripmy);
-            HIPCHK(h, hipGetLastError());
-        }
+        if ((rc = T.get(h, &pool, tp)) || (rc = T.get(h, &nearpool, tp)) || (rc = T.get(h, &hkeys, th)) || (rc = T.get(h, &hidx, th))) return rc;
+        if ((rc = strips(k_rstrip<1>, stripo, hasho, pool, nearpool, hkeys, hidx))) return rc;
         if (npix) {
             hipLaunchKernelGGL(k_rcells, dim3(grid_for(npix)), dim3(kRB), 0, h->stream, (const RPoly *)d_rp,
                                (const uint32_t *)d_pixpoly, npix, (const uint32_t *)d_flag, (const int *)ncols,
@@ -1417,6 +1574,15 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
                                (const uint32_t *)stripn, (const float *)stripmy, (const float2 *)pool,
                                P<uint8_t>(h->status), P<double>(h->areas));
             HIPCHK(h, hipGetLastError());
+            for (uint64_t s0 = 0; s0 < nvl; s0 += 1ull << 30) {
+                hipLaunchKernelGGL(k_rcells_wide, dim3((unsigned)std::min<uint64_t>(nvl - s0, 1ull << 30)), dim3(kRB),
+                                   0, h->stream, (const RPoly *)d_rp, (const uint32_t *)colpoly, s0,
+                                   (const uint32_t *)d_flag, (const int *)ncols, (const int *)nrows,
+                                   (const double *)rowy, (const uint64_t *)stripo, (const uint32_t *)stripn,
+                                   (const float *)stripmy, (const float2 *)pool, P<uint8_t>(h->status),
+                                   P<double>(h->areas));
+                HIPCHK(h, hipGetLastError());
+            }
         }
         HIPCHK(h, hipStreamSynchronize(h->stream));
     }

@@ -98,6 +98,31 @@ def _square(x0, y0, x1, y1):
     return np.array([[x0, y0], [x1, y0], [x1, y1], [x0, y1]], dtype=np.float32)
 
 
+@pytest.mark.parametrize("n", [120, 126, 130, 300, 1100, 5000])
+def test_long_strips_and_points_near_axes(device, n):
+    """Column strips around the sizes at which a pixel's points are taken by a
+    wave and a strip's points leave the shared-memory table; rings across and
+    along the axes, where points less than 1e-9 apart are the same point: every
+    third vertex is followed by one or two such twins.  Byte equality with the
+    host builder."""
+    t = np.linspace(0.0, 2.0 * np.pi, n, endpoint=False)
+    wave = 1.0 + 0.3 * np.sin(11.0 * t)
+    rings = []
+    for r, cx, cy in [(0.004, 0.0, 0.0), (1.0, 0.0, 0.0), (0.5, 0.5, 7.0), (0.01, 3.0, 0.002)]:
+        ring = np.stack([cx + r * wave * np.cos(t), cy + r * wave * np.sin(t)], axis=1).astype(np.float32)
+        twins = []
+        for i, v in enumerate(ring):
+            twins.append(v)
+            if i % 3 == 0:
+                twins.append((v.astype(np.float64) + (6e-10, -6e-10)).astype(np.float32))
+            if i % 6 == 0:
+                twins.append((v.astype(np.float64) + (1.2e-9, -6e-10)).astype(np.float32))
+        rings += [ring, np.array(twins, dtype=np.float32)]
+    H = capi.HostSet.from_rings(*rings_from_list(rings))
+    for vpr in (n, max(1, n // 16)):
+        _check(device, H, vpr)
+
+
 def test_degenerate_rings(device):
     # axis-aligned edges on grid lines, one-pixel rings, repeated vertices,
     # a ring revisiting a vertex, collinear runs and rings the reference
