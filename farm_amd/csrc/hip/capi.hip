@@ -42,6 +42,8 @@ __global__ void k_plain(DevSet, const uint32_t *, const uint32_t *, uint32_t, ui
 __global__ void k_pixedges(DevSet, int64_t, uint32_t *);
 __global__ void k_vdiff(const float *, const float *, uint64_t, float4 *);
 __global__ void k_chunk_count(DevSet, int64_t, uint32_t, uint32_t *);
+__global__ void k_most_chunks(DevSet, int64_t, const uint32_t *, uint32_t *);
+__global__ void k_chunk_group(const float4 *, const uint4 *, uint32_t, float4 *, uint4 *);
 __global__ void k_chunk_box(DevSet, int64_t, uint32_t, const uint32_t *, float4 *, uint4 *);
 __global__ void k_finalize(const uint32_t *, const IsxDesc *, unsigned long long *, unsigned long long *);
 }  // namespace farm
@@ -413,6 +415,26 @@ int build_chunk_boxes(farm_handle h, uint32_t C) {
                            (const uint32_t *)P<uint32_t>(h->choff), P<float4>(h->chbox), P<uint4>(h->chseg));
         HIPCHK(h, hipGetLastError());
     }
+    h->wide_tiles = true;
+    if (nchunks >= kItemChunks) {
+        uint32_t most = 0, *d_most = P<uint32_t>(h->chcnt);
+        if ((rc = fill_u32(h, d_most, 1, 0))) return rc;
+        hipLaunchKernelGGL(k_most_chunks, dim3(256), dim3(256), 0, h->stream, devset(h), h->npolys,
+                           (const uint32_t *)P<uint32_t>(h->choff), d_most);
+        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, hipMemcpyAsync(&most, d_most, 4, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        h->wide_tiles = most < kItemChunks;
+    }
+    const uint32_t ngroups = (nchunks + kGroup - 1) / kGroup;
+    if ((rc = ensure(h, h->cgbox, 16ull * (ngroups + kRefScreen)))) return rc;
+    if ((rc = ensure(h, h->cgseg, 16ull * (ngroups + kRefScreen)))) return rc;
+    if (ngroups) {
+        hipLaunchKernelGGL(k_chunk_group, dim3((ngroups + 255) / 256), dim3(256), 0, h->stream,
+                           (const float4 *)P<float4>(h->chbox), (const uint4 *)P<uint4>(h->chseg), nchunks,
+                           P<float4>(h->cgbox), P<uint4>(h->cgseg));
+        HIPCHK(h, hipGetLastError());
+    }
     HIPCHK(h, hipStreamSynchronize(h->stream));
     h->chunk = C;
     return FARM_OK;
@@ -704,7 +726,7 @@ int farm_close(farm_handle h) {
         if (h->stage[k]) (void)hipHostFree(h->stage[k]);
         if (h->stage_ev[k]) (void)hipEventDestroy(h->stage_ev[k]);
     }
-    DevBuf *bufs[] = {&h->hdr,    &h->status,  &h->pixoff, &h->seqs,   &h->x,      &h->y,        &h->xyd,      &h->fill,     &h->choff,  &h->chcnt,  &h->chbox,  &h->chseg,  &h->ixcnt, &h->ixoff, &h->ixbox, &h->ixseg, &h->voff,
+    DevBuf *bufs[] = {&h->hdr,    &h->status,  &h->pixoff, &h->seqs,   &h->x,      &h->y,        &h->xyd,      &h->fill,     &h->choff,  &h->chcnt,  &h->chbox,  &h->chseg, &h->cgbox, &h->cgseg,  &h->ixcnt, &h->ixoff, &h->ixbox, &h->ixseg, &h->voff,
                       &h->vnodes, &h->pixedges, &h->shape_ctr, &h->pa, &h->pb, &h->isx,
                       &h->scan_tmp, &h->pair_tests, &h->mlp_w, &h->mlp_m, &h->mlp_v, &h->mlp_g,
                       &h->mlp_norm, &h->mlp_wb, &h->mlp_x, &h->mlp_z3, &h->mlp_y, &h->mlp_c, &h->mlp_loss,
@@ -845,6 +867,7 @@ static int run_intersect(farm_handle h, uint64_t begin, uint64_t end, const farm
     const int mode = opts ? opts->mode : FARM_MODE_EXACT_BATCHED;
     int E = opts && opts->tile_a ? opts->tile_a : h->tuned_tile;
     if (E != 1 && E != 2 && E != 4 && E != 8) return fail(h, FARM_EINVAL, "tile_a must be 1, 2, 4 or 8");
+    if (!h->wide_tiles && E > 2) E = 2;
     // chunk size: the call's, else the tuned one (the built one for the
     // fixed-scratch entry, which never rebuilds the boxes on its own)
     const int C = opts && opts->tile_b ? opts->tile_b : (fixed ? (int)h->chunk : h->tuned_chunk);

@@ -27,6 +27,8 @@ struct DevSet {
     const uint32_t *choff;
     const float4 *chbox;
     const uint4 *chseg;
+    const float4 *cgbox;  // the same for groups of kGroup chunks
+    const uint4 *cgseg;
     // the same for chunks of kIxChunk segments, for the intersection's
     // collection (the refinement's arrays when C == kIxChunk)
     const uint32_t *ixoff;
@@ -52,10 +54,12 @@ struct DevSet {
 // 32; kRefChunkDefault until the autotuner or the caller picks another) and
 // screens kRefScreen chunk boxes per scalar load (the box and chunk arrays keep
 // kRefScreen spare entries past their end).
+// Wide tiles screen aligned groups of kGroup chunks first.
 constexpr uint32_t kRefChunkDefault = 16;
 // segments per chunk of the intersection's collection screens
 constexpr uint32_t kIxChunk = 16;
-constexpr uint32_t kRefScreen = 4;
+constexpr uint32_t kRefScreen = 4, kGroup = 4;
+constexpr uint32_t kItemChunks = (1u << 26) - 2 * kGroup;  // a queued item's chunk has 26 bits
 
 constexpr uint32_t kChunkPoint = 0x10000u;  // in a chunk's segment count: one of them has length 0
 

@@ -43,7 +43,7 @@ struct farm_handle_s {
     int64_t npolys = 0;
     farm::DevBuf fill;    // -w fill classes (when the set has them)
     int cc = FARM_CATEGORY_COUNT;
-    farm::DevBuf hdr, status, pixoff, seqs, x, y, xyd, choff, chcnt, chbox, chseg, voff, vnodes, pixedges, shape_ctr;
+    farm::DevBuf hdr, status, pixoff, seqs, x, y, xyd, choff, chcnt, chbox, chseg, cgbox, cgseg, voff, vnodes, pixedges, shape_ctr;
     // 16-segment chunks for the intersection's collection when the
     // refinement's boxes are of another size (built for set generation ix_gen)
     farm::DevBuf ixcnt, ixoff, ixbox, ixseg;
@@ -80,6 +80,7 @@ struct farm_handle_s {
     int tuned_chunk = 16;
     int tuned_bpc = 8;
     uint32_t chunk = 16;
+    bool wide_tiles = true;  // no polygon of the set has kItemChunks chunks (4 and 8 edges per lane allowed)
     int shape_bucket = 0;
     std::map<int, farm_tuning> tunings;
     // learned part
@@ -173,6 +174,8 @@ inline DevSet devset(farm_handle h) {
     S.choff = P<uint32_t>(h->choff);
     S.chbox = P<float4>(h->chbox);
     S.chseg = P<uint4>(h->chseg);
+    S.cgbox = P<float4>(h->cgbox);
+    S.cgseg = P<uint4>(h->cgseg);
     if (h->chunk == kIxChunk) {
         S.ixoff = S.choff;
         S.ixbox = S.chbox;

@@ -90,6 +90,31 @@ def test_chunk_sizes(device, chunk):
             assert diff.size == 0, f"tile {tile} chunk {chunk}: {diff.size} pairs differ, first {diff[:10]}"
 
 
+@pytest.mark.parametrize("vpr", [40, 300])
+@pytest.mark.parametrize("chunk", [8, 16, 32])
+def test_groups_of_chunks(device, chunk, vpr):
+    # pixels of a few to hundreds of chunks, which begin and end anywhere in an
+    # aligned group of them: the answers, and on pairs that all answer false
+    # (so that nothing ends early) every test accounted for as run or pruned
+    from farm_amd import datagen
+
+    a, b = datagen.complex_set(41, 12, lo=0.0, hi=3.0), datagen.lake_set(42, 150, lo=0.0, hi=3.0)
+    w = Workload(a, b, vpr=vpr)
+    want, _ = w.oracle(0)
+    w.upload(device)
+    for tile in (1, 4, 8):
+        r = device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=tile, chunk=chunk)
+        assert np.array_equal(r.bits, (want == 1).astype(np.uint8)), tile
+    apart = want == 0
+    device.upload_pairs(w.pa[apart], w.pb[apart] + len(w.A))
+    full = device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=1, chunk=chunk, flags=capi.FLAG_NO_PRUNE).stats
+    assert full["pruned_tests"] == 0 and full["segment_tests"] > 0
+    for tile in (1, 4, 8):
+        st = device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=tile, chunk=chunk).stats
+        print(f"  -v {vpr} tile={tile} chunk={chunk}: {st['segment_tests']} run", flush=True)
+        assert st["segment_tests"] + st["pruned_tests"] == full["segment_tests"]
+
+
 def test_tuning_rejects_bad_values(device):
     w = star_pairs(8, n=200)
     w.upload(device)
