@@ -730,7 +730,7 @@ int farm_close(farm_handle h) {
                       &h->vnodes, &h->pixedges, &h->shape_ctr, &h->pa, &h->pb, &h->isx,
                       &h->scan_tmp, &h->pair_tests, &h->mlp_w, &h->mlp_m, &h->mlp_v, &h->mlp_g,
                       &h->mlp_norm, &h->mlp_wb, &h->mlp_x, &h->mlp_z3, &h->mlp_y, &h->mlp_c, &h->mlp_loss,
-                      &h->mlp_part, &h->mlp_lpart, &h->feat, &h->decided, &h->pred,
+                      &h->mlp_act, &h->mlp_part, &h->mlp_lpart, &h->feat, &h->decided, &h->pred,
                       &h->skipbuf, &h->pixbox, &h->pixlen, &h->layers, &h->lstatus, &h->areas, &h->wctr, &h->wovf, &h->wslab,
                       &h->wslab_big, &h->wout, &h->wmd, &h->ring2a, &h->icounts, &h->iarea, &h->ipieces, &h->ixlist, &h->ixflag, &h->cg_boxa,
                       &h->cg_boxq, &h->cg_cellcnt, &h->cg_celloff, &h->cg_items, &h->cg_cnt, &h->cg_off,

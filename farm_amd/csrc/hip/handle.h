@@ -88,7 +88,7 @@ struct farm_handle_s {
     farm::DevBuf mlp_w, mlp_m, mlp_v, mlp_g;  // f32 master params, Adam moments, grads
     farm::DevBuf mlp_norm;                    // per feature: mean, 1/std (2 * kNFeat)
     farm::DevBuf mlp_wb;                      // bf16 copies of the weights
-    farm::DevBuf mlp_x, mlp_z3, mlp_y, mlp_c, mlp_loss, mlp_part, mlp_lpart;
+    farm::DevBuf mlp_x, mlp_z3, mlp_y, mlp_c, mlp_loss, mlp_act, mlp_part, mlp_lpart;
     farm::DevBuf feat, decided, pred;  // per-pair features / decided flags / predictions
     farm::DevBuf skipbuf;              // pairs decided before the exact filter
     uint64_t adam_t = 0;

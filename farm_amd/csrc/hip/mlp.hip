@@ -3,10 +3,9 @@
 //
 // The products run on MFMA (v_mfma_f32_16x16x16_bf16): operands are rounded
 // to bf16 when staged (round to nearest even), products accumulate in fp32.
-// Inference is one kernel (k_mlp_infer); a training step is two: k_mlp_grad
-// (forward, loss and every gradient of 32 rows at a time, the activations
-// never leaving LDS) and k_mlp_step (the sum of the workgroups' gradients and
-// Adam).  The reference has no learned component; the features come from the
+// Inference is one kernel (k_mlp_infer); a training step is three: k_mlp_rows
+// (forward and backward of 32 rows at a time), k_mlp_wgrad (the sums over the
+// rows: weight and bias gradients, the loss) and k_mlp_step (Adam).  The reference has no learned component; the features come from the
 // same raster windows as the filter (Ideal::intersect, Ideal.cpp:1329-1357).
 #include <hip/hip_runtime.h>
 
@@ -216,23 +215,43 @@ __global__ __launch_bounds__(256) void k_mlp_infer(const float *__restrict__ fea
 // ------------------------------------------------------------------------
 // Training.  loss = mean(BCE-with-logits(z0, y)) + lambda * mean((z1 - c)^2).
 //
-// k_mlp_grad: one workgroup takes kGradRows rows at a time through the
-// forward pass, the loss and the backward pass, and keeps its part of every
-// weight gradient in MFMA accumulators until its last tile.  Each activation
-// and each dL/dactivation is staged in LDS as bf16 twice: row-major (the A
-// operand of the next product) and transposed (an operand of a weight
-// gradient, whose inner dimension is the rows), padded so that the 8-byte
-// fragment reads of a wave fall two to a bank.  The weights come as bf16 from
-// L2, in the layout each product reads with one 8-byte load per fragment
-// (MlpPacked).  A step of 2,048 rows is bound by latency (64 workgroups, one
-// chain of seven dependent products); with a launch per product, bias and
-// ReLU (20 launches, two 64-row blocks of work per product, a host wait per
-// step) it took 560 us, 165 us of it in each of the two large weight
-// gradients; the two kernels of a step together take 27 us.
+// Three kernels a step.  k_mlp_rows takes 32 rows a workgroup through the
+// forward pass and back: the operands of the next product row-major in LDS as
+// bf16, padded so that a wave's 8-byte fragment reads fall two to a bank; the
+// weights as bf16 from L2, in the layout each product reads with one 8-byte
+// load per fragment (MlpPacked).  Every activation and dL/dactivation leaves
+// it transposed, ready to be an operand of a weight gradient, whose inner
+// dimension is the rows (MlpAct).  k_mlp_wgrad sums over the rows: a wave per
+// 16 x 16 tile of a weight gradient and chunk of about 1,024 rows, one MFMA
+// chain in row order; a workgroup per bias; the loss.  k_mlp_step adds the
+// chunks up and applies Adam.
+//
+// The orders of these sums are part of the result: a last bit of dL/dh turns a
+// bf16 rounding, Adam's division amplifies it, and a run's weights then differ
+// by 1e-3 in norm.  So a step's sums do not depend on how its rows are spread
+// over the chip: chunks of the rows as grad_chunk() cuts them, and within one
+// 16 rows an MFMA in ascending order.  (Gradients kept per workgroup gave
+// other weights and were no faster.)
+//
+// A step of 2,048 rows is bound by latency: a chain of five dependent products
+// for 64 workgroups (16.3 us), then one of 64 MFMAs a wave (8.0 us; 10.2 with
+// 8 blocks' loads in flight instead of 32), then Adam (5 us).  65,536 rows in
+// batches of 2,048, two epochs: 2.85 ms, as with gradients per workgroup.
 // ------------------------------------------------------------------------
 constexpr int kGradRows = 32;
-constexpr int kTPad = kGradRows + 4;
-constexpr int kGradBlocks = 256;  // most workgroups of one step
+constexpr int kGradParts = 256;  // most chunks whose sums are kept apart
+
+// What k_mlp_rows leaves for k_mlp_wgrad, M rows padded to Mp (a multiple of
+// kGradRows).  xt .. dzt: bf16, in blocks of 16 rows, [block][column][row], so
+// that a fragment (4 rows of a column) is one 8-byte load and a wave's 64
+// fragments are 512 consecutive bytes; rows past M are 0.  f2, f1, fz:
+// dL/d(layer output) before its rounding to bf16, z: the logits, [column][row].
+struct MlpAct {
+    short *xt, *h1t, *h2t, *d2t, *d1t, *dzt;
+    float *f2, *f1, *fz, *z;
+    size_t Mp;
+};
+constexpr uint64_t kActBytesPerRow = 2ull * (kNFeat + 4 * kHidden + kOut) + 4ull * (2 * kHidden + 2 * kOut);
 
 // bf16 copies of the weights: W1^T, W2^T, W2, W3^T (16 rows, 2 used), W3
 struct MlpPacked {
@@ -295,38 +314,41 @@ __device__ __forceinline__ void tile_product(const short *A, const short *__rest
         }
 }
 
-// rows: the rows' indices into X, y and c (null: rows 0 .. M - 1).  part:
-// kNParams gradients per workgroup; loss_part: one loss per workgroup.
-__global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ X, const uint32_t *__restrict__ rows,
+// rows: the rows' indices into X, y and c (null: rows 0 .. M - 1).
+__global__ __launch_bounds__(256) void k_mlp_rows(const float *__restrict__ X, const uint32_t *__restrict__ rows,
                                                    const float *__restrict__ y, const float *__restrict__ cst, int M,
                                                    float lambda, const float *__restrict__ W,
-                                                   const MlpPacked *__restrict__ P, float *__restrict__ part,
-                                                   float *__restrict__ loss_part) {
+                                                   const MlpPacked *__restrict__ P, MlpAct act) {
     constexpr int SX = kNFeat + 8, SH = kHidden + 8;
-    __shared__ __align__(16) short sX[kGradRows * SX], sXT[kNFeat * kTPad];
-    __shared__ __align__(16) short sH1[kGradRows * SH], sH1T[kHidden * kTPad];
-    __shared__ __align__(16) short sH2[kGradRows * SH], sH2T[kHidden * kTPad];
-    __shared__ __align__(16) short sD2[kGradRows * SH], sD2T[kHidden * kTPad];
-    __shared__ __align__(16) short sD1T[kHidden * kTPad];
-    __shared__ __align__(16) short sDz[kGradRows * 4], sDzT[16 * kTPad];
+    __shared__ __align__(16) short sX[kGradRows * SX], sH1[kGradRows * SH], sH2[kGradRows * SH], sD2[kGradRows * SH];
+    __shared__ __align__(16) short sDz[kGradRows * 4];
     __shared__ uint32_t sRow[kGradRows];
-    __shared__ float sLoss[2], sB3[2][kOut];
     const int t = threadIdx.x, w = t >> 6, l = t & 63, c = l & 15, q = 4 * (l >> 4);
-    for (int i = t; i < 16 * kTPad; i += 256) sDzT[i] = 0;
-    f32x4 g1[5][2], g2[2][8], g3[2];
-    float gb1[2] = {0.f, 0.f}, gb2[2] = {0.f, 0.f}, gb3 = 0.f, loss = 0.f;
-#pragma unroll
-    for (int i = 0; i < 5; i++)
-#pragma unroll
-        for (int n = 0; n < 2; n++) g1[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-#pragma unroll
-        for (int n = 0; n < 8; n++) g2[i][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-        g3[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    const int r0 = blockIdx.x * kGradRows;
     const bf16x4 zero = {0, 0, 0, 0};
-    // this wave's tile of a layer's output: + bias, ReLU, staged both ways
+    if (t < kGradRows) sRow[t] = r0 + t < M ? (rows ? rows[r0 + t] : (uint32_t)(r0 + t)) : 0xffffffffu;
+    __syncthreads();
+    for (int i = t; i < kGradRows * (kNFeat / 4); i += 256) {
+        const int r = i / (kNFeat / 4), k = 4 * (i % (kNFeat / 4));
+        const uint32_t src = sRow[r];
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (src != 0xffffffffu) v = *reinterpret_cast<const float4 *>(X + (size_t)src * kNFeat + k);
+        *reinterpret_cast<bf16x4 *>(sX + r * SX + k) = bf16x4{f2bf(v.x), f2bf(v.y), f2bf(v.z), f2bf(v.w)};
+    }
+    __syncthreads();
+    // fragment f of ncol columns: rows 16 m + q .. + 3 of this lane's column
+    auto at = [&](short *T, int ncol, int m, int col, int rq) {
+        return reinterpret_cast<bf16x4 *>(T + (((size_t)2 * blockIdx.x + m) * ncol + col) * 16 + rq);
+    };
+    for (int i = t; i < 2 * kNFeat * 4; i += 256) {
+        const int rq = 4 * (i & 3), col = (i >> 2) % kNFeat, m = (i >> 2) / kNFeat;
+        bf16x4 b;
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[j] = sX[(16 * m + rq + j) * SX + col];
+        *at(act.xt, kNFeat, m, col, rq) = b;
+    }
+    // this wave's tile of a layer's output, staged for the next product (R) and
+    // for the weight gradients (T; rows past M as 0)
     auto put = [&](const f32x4 v, int m, int n, short *R, short *T) {
         const int col = 16 * (2 * w + n) + c;
         bf16x4 b;
@@ -334,196 +356,204 @@ __global__ __launch_bounds__(256) void k_mlp_grad(const float *__restrict__ X, c
         for (int j = 0; j < 4; j++) {
             b[j] = f2bf(v[j]);
             if (R) R[(16 * m + q + j) * SH + col] = b[j];
+            if (r0 + 16 * m + q + j >= M) b[j] = 0;
         }
-        *reinterpret_cast<bf16x4 *>(T + col * kTPad + 16 * m + q) = b;
+        *at(T, kHidden, m, col, q) = b;
     };
-    const int tiles = (M + kGradRows - 1) / kGradRows;
-    for (int tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const int r0 = tile * kGradRows;
-        __syncthreads();  // the previous tile's reads are done
-        if (t < kGradRows) sRow[t] = r0 + t < M ? (rows ? rows[r0 + t] : (uint32_t)(r0 + t)) : 0xffffffffu;
-        __syncthreads();
-        for (int i = t; i < kGradRows * (kNFeat / 4); i += 256) {
-            const int r = i / (kNFeat / 4), k = 4 * (i % (kNFeat / 4));
-            const uint32_t src = sRow[r];
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (src != 0xffffffffu) v = *reinterpret_cast<const float4 *>(X + (size_t)src * kNFeat + k);
-            const bf16x4 b = {f2bf(v.x), f2bf(v.y), f2bf(v.z), f2bf(v.w)};
-            *reinterpret_cast<bf16x4 *>(sX + r * SX + k) = b;
-#pragma unroll
-            for (int j = 0; j < 4; j++) sXT[(k + j) * kTPad + r] = b[j];
-        }
-        __syncthreads();
-        f32x4 h1[2][2], h2[2][2], d[2][2];
-        auto relu_layer = [&](f32x4(&h)[2][2], const float *bias, short *R, short *T) {
-#pragma unroll
-            for (int m = 0; m < 2; m++)
-#pragma unroll
-                for (int n = 0; n < 2; n++) {
-                    const float b = bias[16 * (2 * w + n) + c];
-#pragma unroll
-                    for (int j = 0; j < 4; j++) h[m][n][j] = fmaxf(h[m][n][j] + b, 0.f);
-                    put(h[m][n], m, n, R, T);
-                }
-        };
-        tile_product<kNFeat, SX>(sX, P->w1t, w, l, h1);
-        relu_layer(h1, W + kOffB1, sH1, sH1T);
-        __syncthreads();
-        tile_product<kHidden, SH>(sH1, P->w2t, w, l, h2);
-        relu_layer(h2, W + kOffB2, sH2, sH2T);
-        __syncthreads();
-        if (w < 2) {
-            // logits of rows 16w ..: lane column 0 the logit, 1 the cost
-            f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k = 0; k < kHidden / 16; k++)
-                z = mfma(frag(sH2 + (16 * w + c) * SH + 16 * k + q), frag(P->w3t + c * kHidden + 16 * k + q), z);
-            bf16x4 dz = zero;
-            if (c < kOut) {
-                const float b = W[kOffB3 + c];
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const uint32_t src = sRow[16 * w + q + j];
-                    if (src == 0xffffffffu) continue;
-                    const float zj = z[j] + b;
-                    float g;
-                    if (c == 0) {
-                        const float yj = y[src];
-                        const float s = 1.f / (1.f + expf(-zj));
-                        g = (s - yj) / M;
-                        loss += (fmaxf(zj, 0.f) - zj * yj + log1pf(expf(-fabsf(zj)))) / M;
-                    } else {
-                        const float e = zj - cst[src];
-                        g = 2.f * lambda * e / M;
-                        loss += lambda * e * e / M;
-                    }
-                    gb3 += g;
-                    dz[j] = f2bf(g);
-                }
-                *reinterpret_cast<bf16x4 *>(sDzT + c * kTPad + 16 * w + q) = dz;
-            }
-            if (c < 4)
-#pragma unroll
-                for (int j = 0; j < 4; j++) sDz[(16 * w + q + j) * 4 + c] = dz[j];
-        }
-        __syncthreads();
-        // dL/dh2 = dz W3^T (two inner terms, the rest of the 16 zero), masked
-#pragma unroll
-        for (int n = 0; n < 2; n++) {
-            bf16x4 b = zero;
-            if (q == 0) {
-                const short *p = P->w3 + (16 * (2 * w + n) + c) * kOut;
-                b[0] = p[0];
-                b[1] = p[1];
-            }
-#pragma unroll
-            for (int m = 0; m < 2; m++) {
-                const bf16x4 a = q == 0 ? frag(sDz + (16 * m + c) * 4) : zero;
-                f32x4 v = mfma(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    v[j] = h2[m][n][j] > 0.f ? v[j] : 0.f;
-                    gb2[n] += v[j];
-                }
-                put(v, m, n, sD2, sD2T);
-            }
-        }
-        __syncthreads();
-        tile_product<kHidden, SH>(sD2, P->w2, w, l, d);
+    f32x4 h1[2][2], h2[2][2], d[2][2];
+    auto relu_layer = [&](f32x4(&h)[2][2], const float *bias, short *R, short *T) {
 #pragma unroll
         for (int m = 0; m < 2; m++)
 #pragma unroll
             for (int n = 0; n < 2; n++) {
+                const float b = bias[16 * (2 * w + n) + c];
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    d[m][n][j] = h1[m][n][j] > 0.f ? d[m][n][j] : 0.f;
-                    gb1[n] += d[m][n][j];
+                for (int j = 0; j < 4; j++) h[m][n][j] = fmaxf(h[m][n][j] + b, 0.f);
+                put(h[m][n], m, n, R, T);
+            }
+    };
+    tile_product<kNFeat, SX>(sX, P->w1t, w, l, h1);
+    relu_layer(h1, W + kOffB1, sH1, act.h1t);
+    __syncthreads();
+    tile_product<kHidden, SH>(sH1, P->w2t, w, l, h2);
+    relu_layer(h2, W + kOffB2, sH2, act.h2t);
+    __syncthreads();
+    if (w < 2) {
+        // logits of rows 16w ..: lane column 0 the logit, 1 the cost
+        f32x4 z = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < kHidden / 16; k++)
+            z = mfma(frag(sH2 + (16 * w + c) * SH + 16 * k + q), frag(P->w3t + c * kHidden + 16 * k + q), z);
+        bf16x4 dz = zero;
+        if (c < kOut) {
+            f32x4 g = f32x4{0.f, 0.f, 0.f, 0.f};
+            const float b = W[kOffB3 + c];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                z[j] += b;
+                const uint32_t src = sRow[16 * w + q + j];
+                if (src == 0xffffffffu) continue;
+                if (c == 0) {
+                    const float s = 1.f / (1.f + expf(-z[j]));
+                    g[j] = (s - y[src]) / M;
+                } else {
+                    g[j] = 2.f * lambda * (z[j] - cst[src]) / M;
                 }
-                put(d[m][n], m, n, nullptr, sD1T);
+                dz[j] = f2bf(g[j]);
             }
-        // weight gradients of layers 3 and 2 (rows are the inner dimension)
-#pragma unroll
-        for (int k = 0; k < kGradRows / 16; k++) {
-#pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const int m = 2 * w + i;
-                g3[i] = mfma(frag(sH2T + (16 * m + c) * kTPad + 16 * k + q), frag(sDzT + c * kTPad + 16 * k + q),
-                             g3[i]);
-                const bf16x4 a = frag(sH1T + (16 * m + c) * kTPad + 16 * k + q);
-#pragma unroll
-                for (int n = 0; n < 8; n++)
-                    g2[i][n] = mfma(a, frag(sD2T + (16 * n + c) * kTPad + 16 * k + q), g2[i][n]);
-            }
+            const size_t o = (size_t)c * act.Mp + r0 + 16 * w + q;
+            *reinterpret_cast<f32x4 *>(act.z + o) = z;
+            *reinterpret_cast<f32x4 *>(act.fz + o) = g;
+            *at(act.dzt, kOut, w, c, q) = dz;
         }
-        __syncthreads();
+        if (c < 4)
 #pragma unroll
-        for (int k = 0; k < kGradRows / 16; k++)
-#pragma unroll
-            for (int n = 0; n < 2; n++) {
-                const bf16x4 b = frag(sD1T + (16 * (2 * w + n) + c) * kTPad + 16 * k + q);
-#pragma unroll
-                for (int i = 0; i < 5; i++)
-                    g1[i][n] = mfma(frag(sXT + (16 * i + c) * kTPad + 16 * k + q), b, g1[i][n]);
-            }
+            for (int j = 0; j < 4; j++) sDz[(16 * w + q + j) * 4 + c] = dz[j];
     }
-    float *G = part + (size_t)blockIdx.x * kNParams;
+    __syncthreads();
+    // dL/dh2 = dz W3^T (two inner terms, the rest of the 16 zero), masked
 #pragma unroll
     for (int n = 0; n < 2; n++) {
         const int col = 16 * (2 * w + n) + c;
-#pragma unroll
-        for (int i = 0; i < 5; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) G[kOffW1 + (16 * i + q + j) * kHidden + col] = g1[i][n][j];
-        float s1 = gb1[n], s2 = gb2[n];
-        s1 += __shfl_xor(s1, 16);
-        s1 += __shfl_xor(s1, 32);
-        s2 += __shfl_xor(s2, 16);
-        s2 += __shfl_xor(s2, 32);
+        bf16x4 b = zero;
         if (q == 0) {
-            G[kOffB1 + col] = s1;
-            G[kOffB2 + col] = s2;
+            const short *p = P->w3 + col * kOut;
+            b[0] = p[0];
+            b[1] = p[1];
+        }
+#pragma unroll
+        for (int m = 0; m < 2; m++) {
+            const bf16x4 a = q == 0 ? frag(sDz + (16 * m + c) * 4) : zero;
+            f32x4 v = mfma(a, b, f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = h2[m][n][j] > 0.f ? v[j] : 0.f;
+            *reinterpret_cast<f32x4 *>(act.f2 + (size_t)col * act.Mp + r0 + 16 * m + q) = v;
+            put(v, m, n, sD2, act.d2t);
         }
     }
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int row = 16 * (2 * w + i) + q + j;
-#pragma unroll
-            for (int n = 0; n < 8; n++) G[kOffW2 + row * kHidden + 16 * n + c] = g2[i][n][j];
-            if (c < kOut) G[kOffW3 + row * kOut + c] = g3[i][j];
-        }
-    // waves 0 and 1 hold the losses and the output bias gradients
-    if (w < 2) {
-        for (int o = 32; o > 0; o >>= 1) loss += __shfl_xor(loss, o);
-        if (l == 0) sLoss[w] = loss;
-    }
-    gb3 += __shfl_xor(gb3, 16);
-    gb3 += __shfl_xor(gb3, 32);
-    if (w < 2 && l < kOut) sB3[w][l] = gb3;
     __syncthreads();
-    if (t < kOut) G[kOffB3 + t] = sB3[0][t] + sB3[1][t];
-    if (t == 0) loss_part[blockIdx.x] = sLoss[0] + sLoss[1];
+    tile_product<kHidden, SH>(sD2, P->w2, w, l, d);
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            const int col = 16 * (2 * w + n) + c;
+#pragma unroll
+            for (int j = 0; j < 4; j++) d[m][n][j] = h1[m][n][j] > 0.f ? d[m][n][j] : 0.f;
+            *reinterpret_cast<f32x4 *>(act.f1 + (size_t)col * act.Mp + r0 + 16 * m + q) = d[m][n];
+            put(d[m][n], m, n, nullptr, act.d1t);
+        }
 }
 
-// The step's gradients (the workgroups' parts, summed in order) into g when
-// given, and Adam on w and its bf16 copies when adam != 0; the loss to *loss.
+// Weight gradient tiles of 16 x 16: 5 x 8 of W1, 8 x 8 of W2, 8 x 1 of W3.
+constexpr int kTilesW1 = (kNFeat / 16) * (kHidden / 16), kTilesW2 = (kHidden / 16) * (kHidden / 16),
+              kGradTiles = kTilesW1 + kTilesW2 + kHidden / 16;
+constexpr int kBiases = 2 * kHidden + kOut;
+
+// Workgroups [0, gw): the weight gradients, a wave per tile and part p of np,
+// which takes the row chunks p, p + np, ..; [gw, gw + kBiases): a bias each;
+// the rest: 256 rows' losses, one sum per wave.
+__global__ __launch_bounds__(256) void k_mlp_wgrad(MlpAct act, const uint32_t *__restrict__ rows,
+                                                    const float *__restrict__ y, const float *__restrict__ cst, int M,
+                                                    float lambda, int chunk, int np, int gw, float *__restrict__ part,
+                                                    float *__restrict__ loss_part) {
+    const int t = threadIdx.x, w = t >> 6, l = t & 63, c = l & 15, q = 4 * (l >> 4);
+    const int b = blockIdx.x;
+    if (b < gw) {
+        const int task = 4 * b + w, tile = task % kGradTiles, p = task / kGradTiles;
+        if (p >= np) return;
+        // operands and output of this tile
+        const short *A, *B;
+        int na, nb, mt, nt, off, ld;
+        if (tile < kTilesW1) {
+            A = act.xt, B = act.d1t, na = kNFeat, nb = kHidden, off = kOffW1, ld = kHidden;
+            mt = tile / (kHidden / 16), nt = tile % (kHidden / 16);
+        } else if (tile < kTilesW1 + kTilesW2) {
+            A = act.h1t, B = act.d2t, na = nb = kHidden, off = kOffW2, ld = kHidden;
+            mt = (tile - kTilesW1) / (kHidden / 16), nt = (tile - kTilesW1) % (kHidden / 16);
+        } else {
+            A = act.h2t, B = act.dzt, na = kHidden, nb = kOut, off = kOffW3, ld = kOut;
+            mt = tile - kTilesW1 - kTilesW2, nt = 0;
+        }
+        const bool col = 16 * nt + c < nb;  // W3 has 2 of the 16 columns
+        const bf16x4 zero = {0, 0, 0, 0};
+        A += (size_t)(16 * mt + c) * 16 + q;
+        B += col ? (size_t)(16 * nt + c) * 16 + q : 0;
+        f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int k0 = p * chunk; k0 < M; k0 += np * chunk) {
+            const int rb1 = (min(M, k0 + chunk) + 15) / 16;
+            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+            // (32 blocks' loads together, then their products in turn)
+            for (int rb = k0 / 16; rb < rb1; rb += 32) {
+                bf16x4 fa[32], fb[32];
+#pragma unroll
+                for (int u = 0; u < 32; u++) {
+                    const size_t r = min(rb + u, rb1 - 1);
+                    fa[u] = frag(A + r * na * 16);
+                    fb[u] = frag(B + r * nb * 16);
+                }
+#pragma unroll
+                for (int u = 0; u < 32; u++)
+                    if (rb + u < rb1) acc = mfma(fa[u], col ? fb[u] : zero, acc);
+            }
+            sum += acc;
+        }
+        if (!col) return;
+        float *G = part + (size_t)p * kNParams + off;
+#pragma unroll
+        for (int j = 0; j < 4; j++) G[(16 * mt + q + j) * ld + 16 * nt + c] = sum[j];
+        return;
+    }
+    if (b < gw + kBiases) {
+        // the column's sum in f32: rows t, t + 256, .. a lane
+        __shared__ float sum[4];
+        const int k = b - gw;
+        const float *f;
+        int i;
+        if (k < kHidden) f = act.f1 + (size_t)k * act.Mp, i = kOffB1 + k;
+        else if (k < 2 * kHidden) f = act.f2 + (size_t)(k - kHidden) * act.Mp, i = kOffB2 + k - kHidden;
+        else f = act.fz + (size_t)(k - 2 * kHidden) * act.Mp, i = kOffB3 + k - 2 * kHidden;
+        float s = 0.f;
+#pragma unroll 8
+        for (int64_t r = t; r < M; r += 256) s += f[r];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (l == 0) sum[w] = s;
+        __syncthreads();
+        if (t == 0) part[i] = sum[0] + sum[1] + sum[2] + sum[3];
+        return;
+    }
+    const int g = b - gw - kBiases, r = 256 * g + t;
+    float L = 0.f;
+    if (r < M) {
+        const uint32_t src = rows ? rows[r] : (uint32_t)r;
+        const float z0 = act.z[r], e = act.z[act.Mp + r] - cst[src];
+        L = (fmaxf(z0, 0.f) - z0 * y[src] + log1pf(expf(-fabsf(z0)))) / M + lambda * e * e / M;
+    }
+    for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
+    if (l == 0) loss_part[4 * g + w] = L;
+}
+
+// The step's gradients (the chunks' parts, summed in order) into g when given,
+// and Adam on w and its bf16 copies when adam != 0; the loss, the sum of nloss
+// parts, to *loss.
 __global__ __launch_bounds__(256) void k_mlp_step(const float *__restrict__ part, const float *__restrict__ loss_part,
-                                                   int nblocks, float *__restrict__ g, float *__restrict__ loss,
+                                                   int np, int nloss, float *__restrict__ g, float *__restrict__ loss,
                                                    int adam, float *__restrict__ w, MlpPacked *__restrict__ P,
                                                    float *__restrict__ m, float *__restrict__ v, float lr, float b1,
                                                    float b2, float eps, float c1, float c2) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x == 0 && threadIdx.x < 64) {
         float L = 0.f;
-        for (int k = threadIdx.x; k < nblocks; k += 64) L += loss_part[k];
+        for (int k = threadIdx.x; k < nloss; k += 64) L += loss_part[k];
         for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o);
         if (threadIdx.x == 0) *loss = L;
     }
     if (i >= kNParams) return;
+    // (a bias is one sum over all rows, in the first part)
+    const bool bias = (i >= kOffB1 && i < kOffW2) || (i >= kOffB2 && i < kOffW3) || i >= kOffB3;
     float gi = 0.f;
-#pragma unroll 16
-    for (int k = 0; k < nblocks; k++) gi += part[(size_t)k * kNParams + i];
+#pragma unroll 8
+    for (int k = 0; k < (bias ? 1 : np); k++) gi += part[(size_t)k * kNParams + i];
     if (g) g[i] = gi;
     if (!adam) return;
     const float mi = b1 * m[i] + (1.f - b1) * gi;
@@ -541,28 +571,71 @@ using namespace farm;
 
 namespace {
 
-// Workgroups of a step of M rows, and the buffers of their gradients.
-int grad_blocks(int M) { return std::min((M + kGradRows - 1) / kGradRows, kGradBlocks); }
+// Rows of a chunk of the weight gradients: M / (M / 1024) of them, to a whole
+// number of 16.
+int grad_chunk(int M) {
+    const int n = std::max(1, M / 1024);
+    return ((M + n - 1) / n + 15) / 16 * 16;
+}
+int grad_parts(int M) {
+    const int chunk = grad_chunk(M);
+    return std::min((M + chunk - 1) / chunk, kGradParts);
+}
+uint64_t grad_rows(int M) { return ((uint64_t)M + kGradRows - 1) / kGradRows * kGradRows; }
+int loss_blocks(int M) { return (M + 255) / 256; }
 
 int grad_buffers(farm_handle h, int M, uint64_t losses) {
     int rc;
-    if ((rc = ensure(h, h->mlp_part, 4ull * kNParams * grad_blocks(M)))) return rc;
-    if ((rc = ensure(h, h->mlp_lpart, 4ull * kGradBlocks))) return rc;
+    if ((rc = ensure(h, h->mlp_act, kActBytesPerRow * grad_rows(M)))) return rc;
+    if ((rc = ensure(h, h->mlp_part, 4ull * kNParams * grad_parts(M)))) return rc;
+    if ((rc = ensure(h, h->mlp_lpart, 16ull * loss_blocks(M)))) return rc;
     return ensure(h, h->mlp_loss, 4ull * losses);
+}
+
+// the arrays of M rows in mlp_act (Mp is a multiple of 32: each is aligned to 64 bytes)
+MlpAct carve_act(farm_handle h, int M) {
+    MlpAct a;
+    const size_t Mp = a.Mp = grad_rows(M);
+    float *f = P<float>(h->mlp_act);
+    auto floats = [&](int ncol) {
+        float *p = f;
+        f += Mp * ncol;
+        return p;
+    };
+    a.f2 = floats(kHidden);
+    a.f1 = floats(kHidden);
+    a.fz = floats(kOut);
+    a.z = floats(kOut);
+    short *s = reinterpret_cast<short *>(f);
+    auto shorts = [&](int ncol) {
+        short *p = s;
+        s += Mp * ncol;
+        return p;
+    };
+    a.xt = shorts(kNFeat);
+    a.h1t = shorts(kHidden);
+    a.h2t = shorts(kHidden);
+    a.d2t = shorts(kHidden);
+    a.d1t = shorts(kHidden);
+    a.dzt = shorts(kOut);
+    return a;
 }
 
 // loss (to mlp_loss[slot]) and gradients of M rows of X, y, c (device; rows:
 // their indices, or null), then Adam (step adam_t) or the gradients to mlp_g
 int mlp_step(farm_handle h, const float *X, const uint32_t *rows, const float *y, const float *c, int M, float lambda,
              uint64_t slot, bool adam, float lr) {
-    const int nb = grad_blocks(M);
-    hipLaunchKernelGGL(k_mlp_grad, dim3(nb), dim3(256), 0, h->stream, X, rows, y, c, M, lambda,
-                       (const float *)P<float>(h->mlp_w), (const MlpPacked *)P<MlpPacked>(h->mlp_wb),
-                       P<float>(h->mlp_part), P<float>(h->mlp_lpart));
+    const MlpAct act = carve_act(h, M);
+    const int np = grad_parts(M), gw = (np * kGradTiles + 3) / 4, gl = loss_blocks(M);
+    hipLaunchKernelGGL(k_mlp_rows, dim3((unsigned)(act.Mp / kGradRows)), dim3(256), 0, h->stream, X, rows, y, c, M,
+                       lambda, (const float *)P<float>(h->mlp_w), (const MlpPacked *)P<MlpPacked>(h->mlp_wb), act);
+    HIPCHK(h, hipGetLastError());
+    hipLaunchKernelGGL(k_mlp_wgrad, dim3(gw + kBiases + gl), dim3(256), 0, h->stream, act, rows, y, c, M, lambda,
+                       grad_chunk(M), np, gw, P<float>(h->mlp_part), P<float>(h->mlp_lpart));
     HIPCHK(h, hipGetLastError());
     const float c1 = 1.f - powf(0.9f, (float)h->adam_t), c2 = 1.f - powf(0.999f, (float)h->adam_t);
     hipLaunchKernelGGL(k_mlp_step, dim3(blocks_for(kNParams)), dim3(256), 0, h->stream,
-                       (const float *)P<float>(h->mlp_part), (const float *)P<float>(h->mlp_lpart), nb,
+                       (const float *)P<float>(h->mlp_part), (const float *)P<float>(h->mlp_lpart), np, 4 * gl,
                        adam ? (float *)nullptr : P<float>(h->mlp_g), P<float>(h->mlp_loss) + slot, adam ? 1 : 0,
                        P<float>(h->mlp_w), P<MlpPacked>(h->mlp_wb), P<float>(h->mlp_m), P<float>(h->mlp_v), lr, 0.9f,
                        0.999f, 1e-8f, c1, c2);

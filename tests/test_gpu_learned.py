@@ -2,6 +2,8 @@
 reference MLP (oracle/mlp_ref.py); training; the learned -a mode against the
 exact labels and against the reference heuristic; learned queue order keeps
 exact mode bit-exact."""
+import zlib
+
 import numpy as np
 import pytest
 
@@ -64,6 +66,52 @@ def test_gradients_at_tile_edges(device, m):
         n = int(np.prod(shp))
         blk, ref = g[o:o + n], gr[o:o + n]
         assert np.abs(blk - ref).max() < 3e-3 * (np.abs(ref).max() + 1e-12), (m, shp)
+        o += n
+
+
+# CRC-32 of the gradients (+ 0.0, so that -0 is 0) of _rand_problem(300 + m, m)
+# and of the weights after training on _rand_problem(900 + rows + batch, rows):
+# the sums over a batch's rows have one order (chunks of about 1,024 rows, 16
+# rows an MFMA; a bias's rows 256 lanes apart), so these bytes do not change
+# with the kernels' split of the work.  (Batches of one or two chunks: two
+# parts have one sum.)
+GRADIENT_CRC = {1: 861706529, 31: 4110951442, 33: 1722800055, 500: 3327316183, 1000: 4024023936, 2048: 3128967534,
+                2900: 166222546, 3000: 855922505, 3071: 1708108478}
+WEIGHTS_CRC = {(700, 1000, 2): 2570756007, (5000, 512, 2): 317308398, (9000, 1000, 1): 3392893631,
+               (9000, 2048, 2): 883283139, (65536, 2048, 2): 1539214011}
+
+
+@pytest.mark.parametrize("m", list(GRADIENT_CRC))
+def test_gradient_bytes(device, m):
+    p, X, y, c = _rand_problem(300 + m, m)
+    device.mlp_set_params(p)
+    _, g = device.mlp_loss_grad(X, y, c, 0.05)
+    assert zlib.crc32(np.ascontiguousarray(g + np.float32(0)).tobytes()) == GRADIENT_CRC[m]
+
+
+@pytest.mark.parametrize("rows,batch,epochs", list(WEIGHTS_CRC))
+def test_trained_weight_bytes(device, rows, batch, epochs):
+    p, X, y, c = _rand_problem(900 + rows + batch, rows)
+    device.mlp_set_params(p)
+    device.mlp_train(X, y, c, epochs, batch, 2e-3, 0.05, 1)
+    w = device.mlp_get_params()
+    assert zlib.crc32(np.ascontiguousarray(w).tobytes()) == WEIGHTS_CRC[rows, batch, epochs]
+
+
+def test_gradients_of_more_chunks_than_parts(device):
+    # 268 chunks of the rows: a wave sums two of them; bf16 operands as in
+    # test_gradients_match_reference, hence its bounds
+    m = 275_000
+    p, X, y, c = _rand_problem(71, m)
+    device.mlp_set_params(p)
+    L, g = device.mlp_loss_grad(X, y, c, 0.05)
+    Lr, gr = mlp_ref.loss_grad(p.astype(np.float64), X, y.astype(np.float64), c.astype(np.float64), 0.05,
+                               rounding=True)
+    assert abs(L - Lr) <= 1e-4 * abs(Lr) + 1e-6
+    o = 0
+    for shp in learned.SHAPES:
+        n = int(np.prod(shp))
+        assert np.abs(g[o:o + n] - gr[o:o + n]).max() < 3e-3 * (np.abs(gr[o:o + n]).max() + 1e-12), shp
         o += n
 
 
