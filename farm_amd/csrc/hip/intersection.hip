@@ -525,16 +525,38 @@ constexpr int kLanePath = 16;  // area-piece paths of at most this many segments
 // One ring's pieces: D[0, n) sorted by this ring's (edge, parameter).
 // Counts the reference pieces by status into r and returns this lane's part
 // of the cross-product sum of the area pieces IN the other polygon.
-// The team's waves take 64 pieces each in turn; r gets this wave's counts.
+// The team's waves take 64 pieces each in turn; r gets this wave's counts.  The
+// sum has one order whatever the team, as its last bits are part of the area
+// and which pairs go to a team depends on the call's size: lane k adds segments
+// k, k + 64, .. of one piece after the other.  A team's lanes work out the
+// segments of a piece each, up to kRow of them, into a row of memory (0 past
+// the piece's last and for other pieces, which adds nothing), and its first
+// wave adds the rows in order, the longer pieces by itself; the other waves
+// return 0.
+constexpr int kRow = 4;
+constexpr int kRowLong = 0x7ff8b17e;  // high word of a longer piece's row: a NaN no sum makes
 template <bool SRC, int NW>
 __device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const farm_raster_hdr &hq, const Rec *D,
-                              uint32_t n, double ox, double oy, const Team<NW> &tm, PairRes &r, const PieceOut &po,
-                              Queues &Q) {
+                              uint32_t n, double *rows, double ox, double oy, const Team<NW> &tm, PairRes &r,
+                              const PieceOut &po, Queues &Q) {
     const int lane = tm.lane;
     const float *X = S.x + hp.vert_start, *Y = S.y + hp.vert_start;
     const int m = (int)hp.nverts - 1;
     const double eps = (double)1e-6f;  // util.h:44
     double acc = 0.0;
+    // ring vertices on the way from record i (a) to the next (b)
+    auto path_len = [&](uint32_t i, const Rec &a, const Rec &b) {
+        const int e0 = SRC ? a.ei : a.ej, e1 = SRC ? b.ei : b.ej;
+        const double t0 = SRC ? a.t : a.u, t1 = SRC ? b.t : b.u;
+        return i + 1 < n ? max(e1 - e0, 0) : (e1 - e0 + m) % m + ((e1 == e0 && t1 <= t0) ? m : 0);
+    };
+    // segment k of the path from a to b
+    auto term = [&](int f, int nv, float pax, float pay, float pbx, float pby, int k) {
+        float x0, y0, x1, y1;
+        path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k, x0, y0);
+        path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k + 1, x1, y1);
+        return ((double)x0 - ox) * ((double)y1 - oy) - ((double)x1 - ox) * ((double)y0 - oy);
+    };
     for (uint32_t c0 = NW == 1 ? 0u : 64u * tm.wv; c0 < n; c0 += 64 * NW) {
         const uint32_t i = c0 + lane;
         bool piece = false, in_area = false, long_path = false;
@@ -570,9 +592,7 @@ __device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const 
                     ry = Y[ae + 1];
                 }
                 // the area piece: a -> ring vertices ea0 + 1 .. eb0 -> b
-                if (i + 1 < n) nvert = eb0 - ea0;
-                else nvert = (eb0 - ea0 + m) % m + ((eb0 == ea0 && tb0 <= ta0) ? m : 0);
-                if (nvert < 0) nvert = 0;
+                nvert = path_len(i, a, b);
                 first = ea0 + 1;
                 // the area's test point: the midpoint of the path's longest
                 // sub-segment (the first on ties), well inside the piece; a
@@ -662,21 +682,57 @@ __device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const 
         r.c[3] += __popcll(__ballot(piece && st == 0));
         r.c[4] += __popcll(__ballot(piece && st == 1));
         put_pieces(po, in_area, farm_piece{po.pair, SRC ? 0 : 1, first, nvert, ax, ay, bx, by}, lane);
-        // wave-cooperative path sums of this chunk's IN pieces
-        uint64_t inm = __ballot(in_area);
-        while (inm) {
-            const int src = __ffsll((unsigned long long)inm) - 1;
-            inm &= inm - 1;
-            const int f = __shfl(first, src, 64), nv = __shfl(nvert, src, 64);
-            const float pax = __shfl(ax, src, 64), pay = __shfl(ay, src, 64);
-            const float pbx = __shfl(bx, src, 64), pby = __shfl(by, src, 64);
-            for (int k = lane; k <= nv; k += 64) {
-                float x0, y0, x1, y1;
-                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k, x0, y0);
-                path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k + 1, x1, y1);
-                acc += ((double)x0 - ox) * ((double)y1 - oy) - ((double)x1 - ox) * ((double)y0 - oy);
+        if constexpr (NW > 1) {
+            if (i < n) {
+                double t[kRow] = {0.0, 0.0, 0.0, 0.0};
+                if (in_area && nvert < kRow) {
+#pragma unroll
+                    for (int k = 0; k < kRow; k++)
+                        if (k <= nvert) t[k] = term(first, nvert, ax, ay, bx, by, k);
+                } else if (in_area) {
+                    t[0] = __hiloint2double(kRowLong, 0);
+                }
+#pragma unroll
+                for (int k = 0; k < kRow; k += 2)
+                    *reinterpret_cast<double2 *>(rows + (uint64_t)kRow * i + k) = make_double2(t[k], t[k + 1]);
+            }
+        } else {
+            // the wave over one IN piece after the other
+            uint64_t inm = __ballot(in_area);
+            while (inm) {
+                const int src = __ffsll((unsigned long long)inm) - 1;
+                inm &= inm - 1;
+                const int f = __shfl(first, src, 64), nv = __shfl(nvert, src, 64);
+                const float pax = __shfl(ax, src, 64), pay = __shfl(ay, src, 64);
+                const float pbx = __shfl(bx, src, 64), pby = __shfl(by, src, 64);
+                for (int k = lane; k <= nv; k += 64) acc += term(f, nv, pax, pay, pbx, pby, k);
             }
         }
+    }
+    if constexpr (NW > 1) {
+        tm.sync();
+        if (tm.first())
+            for (uint32_t p0 = 0; p0 < n; p0 += 64) {
+                const uint32_t np = min(n - p0, 64u);
+                const double *row = rows + (uint64_t)kRow * p0;
+                const bool wide = (uint32_t)lane < np && __double2hiint(row[kRow * lane]) == kRowLong;
+                uint64_t wm = __ballot(wide);
+                for (uint32_t p = 0; p < np;) {
+                    // the rows up to the next longer piece
+                    const uint32_t end = wm ? (uint32_t)__ffsll((unsigned long long)wm) - 1u : np;
+                    if (lane < kRow) {
+#pragma unroll 8
+                        for (; p < end; p++) acc += row[kRow * p + lane];
+                    }
+                    p = end;
+                    if (!wm) break;
+                    wm &= wm - 1;
+                    const Rec a = D[p0 + p], b = D[(p0 + p + 1) % n];
+                    const int nv = path_len(p0 + p, a, b), f = (SRC ? a.ei : a.ej) + 1;
+                    for (int k = lane; k <= nv; k += 64) acc += term(f, nv, a.px, a.py, b.px, b.py, k);
+                    p++;
+                }
+            }
     }
     return acc;
 }
@@ -847,12 +903,14 @@ __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const doub
     }
     r.c[0] = (int32_t)nk;
     double acc_a = 0.0, acc_b = 0.0;
+    static_assert(kRow * sizeof(double) == sizeof(Rec), "a row per record");
+    double *rows = reinterpret_cast<double *>(R);  // (the raw records are done with)
     if (nk > 0) {
         bitonic<1>(D, nk, tm);
-        acc_a = ring_pieces<true>(S, hA, hB, D, nk, ox, oy, tm, r, po, Q);
+        acc_a = ring_pieces<true>(S, hA, hB, D, nk, rows, ox, oy, tm, r, po, Q);
         tm.sync();
         bitonic<2>(D, nk, tm);
-        acc_b = ring_pieces<false>(S, hB, hA, D, nk, ox, oy, tm, r, po, Q);
+        acc_b = ring_pieces<false>(S, hB, hA, D, nk, rows, ox, oy, tm, r, po, Q);
     }
     double side_a = wave_sum(acc_a), side_b = wave_sum(acc_b);
     if constexpr (NW > 1) {

@@ -227,6 +227,25 @@ def test_pairs_by_workgroups_and_by_waves(device, npairs):
     assert (np.abs(area - want) <= AREA_RTOL * np.abs(want) + AREA_ATOL).all()
 
 
+def test_areas_do_not_depend_on_the_calls_size(device):
+    # pairs of some hundred short pieces (jagged rings) and of few long ones,
+    # all in one call (a wave each) and 500 at a time (a workgroup each): the
+    # path sums have one order, so the areas are the same bytes
+    (sa, sxy), (ta, txy) = datagen.star_pair_set(13, 4400, 4400, 0.0, 148.0)
+    a = [sxy[sa[i]:sa[i + 1] - 1] for i in range(len(sa) - 1)] + [_wavy(900, 0.0, 0.0, 1.0), _wavy(61, 0.3, 0.2, 0.5)]
+    b = [txy[ta[i]:ta[i + 1] - 1] for i in range(len(ta) - 1)] + [_wavy(300, 0.1, 0.0, 0.9), _wavy(700, 0.2, 0.3, 0.8)]
+    w = Workload(rings_from_list(a), rings_from_list(b), vpr=10)
+    n = len(w.pa)
+    assert n > 8192 + 500
+    w.upload(device)
+    c, area, _ = device.intersection_area()
+    assert (c[:, 1] > 128).any() and (c[:, 1] > 0).sum() > 2000
+    parts = [device.intersection_area(k, min(k + 500, n)) for k in range(0, n, 500)]
+    assert np.array_equal(np.concatenate([p[0] for p in parts]), c)
+    diff = np.concatenate([p[1] for p in parts]).view(np.uint64) != area.view(np.uint64)
+    assert not diff.any(), f"{diff.sum()} of {n} areas differ"
+
+
 def _wavy(n, cx, cy, r):
     t = np.linspace(0, 2 * np.pi, n, endpoint=False)
     q = r * (1.0 + 0.1 * np.sin(7 * t) + 0.15 * np.sin(61 * t + 9 * cx))
