@@ -307,6 +307,7 @@ EXPORTS = {
     "farm_hostset_rasterize_device": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int,
                                                 C.POINTER(RasterInfo)]),
     "farm_set_staging": (C.c_int, [C.c_void_p, C.c_uint64]),
+    "farm_set_raster_groups": (C.c_int, [C.c_void_p, C.c_uint64]),
     "farm_hostset_rasterize": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
     "farm_hostset_rasterize_h": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int]),
     "farm_hostset_layer": (C.c_int, [C.c_void_p, C.c_int64, C.c_int, C.POINTER(Layer), C.POINTER(C.c_void_p)]),
@@ -650,6 +651,10 @@ class Device:
 
     def set_staging(self, vertices: int) -> None:
         self._check(lib.farm_set_staging(self._h, int(vertices)), "set_staging")
+
+    def set_raster_groups(self, groups: int) -> None:
+        """Workgroups per launch of the raster builder's column kernels (0: the default)."""
+        self._check(lib.farm_set_raster_groups(self._h, int(groups)), "set_raster_groups")
 
     def download_polyset(self) -> dict:
         """The device set's arrays (after rasterize), as HostSet.layout names them."""

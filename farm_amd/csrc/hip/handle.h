@@ -31,6 +31,10 @@ constexpr int kW1 = kNFeat * kHidden, kB1 = kHidden, kW2 = kHidden * kHidden, kB
 constexpr int kOffW1 = 0, kOffB1 = kOffW1 + kW1, kOffW2 = kOffB1 + kB1, kOffB2 = kOffW2 + kW2, kOffW3 = kOffB2 + kB2,
               kOffB3 = kOffW3 + kW3, kNParams = kOffB3 + kB3;
 
+
+// HIP takes fewer than 2^32 work items a launch: the most workgroups of 256
+constexpr uint64_t kMaxLaunchGroups = (1ull << 24) - 1;
+
 }  // namespace farm
 
 struct farm_handle_s {
@@ -111,6 +115,7 @@ struct farm_handle_s {
     void *stage[2] = {nullptr, nullptr};
     hipEvent_t stage_ev[2] = {};
     uint64_t stage_verts = 1ull << 22;  // vertices per staging buffer (8 B each)
+    uint64_t raster_groups = farm::kMaxLaunchGroups;  // workgroups per launch of the raster builder's column kernels
 };
 
 namespace farm {

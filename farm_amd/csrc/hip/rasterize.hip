@@ -1526,11 +1526,12 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
                            colx, rowy, ncols, nrows, colpoly);
         HIPCHK(h, hipGetLastError());
     }
-    // one workgroup per column slot (several launches beyond 2^30 of them)
+    // one workgroup per column slot, h->raster_groups of them a launch
+    const uint64_t slice = h->raster_groups;
     auto strips = [&](auto kernel, const uint64_t *so, const uint64_t *hof, float2 *pool, float2 *nearpool,
                       unsigned long long *hkeys, uint32_t *hidx) -> int {
-        for (uint64_t s0 = 0; s0 < nvl; s0 += 1ull << 30) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min<uint64_t>(nvl - s0, 1ull << 30)), dim3(kRB), 0,
+        for (uint64_t s0 = 0; s0 < nvl; s0 += slice) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(nvl - s0, slice)), dim3(kRB), 0,
                                h->stream, (const RPoly *)d_rp, P<float>(h->x), P<float>(h->y), (const float *)d_absx,
                                d_flag, (const int *)ncols, (const int *)nrows, (const double *)colx,
                                (const uint32_t *)colpoly, s0, stripc, so, hof, pool, nearpool, hkeys, hidx,
@@ -1574,9 +1575,8 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
                                (const uint32_t *)stripn, (const float *)stripmy, (const float2 *)pool,
                                P<uint8_t>(h->status), P<double>(h->areas));
             HIPCHK(h, hipGetLastError());
-            for (uint64_t s0 = 0; s0 < nvl; s0 += 1ull << 30) {
-                hipLaunchKernelGGL(k_rcells_wide, dim3((unsigned)std::min<uint64_t>(nvl - s0, 1ull << 30)), dim3(kRB),
-                                   0, h->stream, (const RPoly *)d_rp, (const uint32_t *)colpoly, s0,
+            for (uint64_t s0 = 0; s0 < nvl; s0 += slice) {
+                hipLaunchKernelGGL(k_rcells_wide, dim3((unsigned)std::min(nvl - s0, slice)), dim3(kRB), 0, h->stream, (const RPoly *)d_rp, (const uint32_t *)colpoly, s0,
                                    (const uint32_t *)d_flag, (const int *)ncols, (const int *)nrows,
                                    (const double *)rowy, (const uint64_t *)stripo, (const uint32_t *)stripn,
                                    (const float *)stripmy, (const float2 *)pool, P<uint8_t>(h->status),
@@ -1794,6 +1794,16 @@ extern "C" int farm_hostset_rasterize_device(farm_handle h, const farm_hostset *
     rc = rasterize_uploaded(h, np, voff, nvt, vpr, nlow, info);
     if (!rc && info) info->upload_ms = up_ms;
     return rc;
+}
+
+// a launch of 2^32 work items or more is refused
+static_assert((uint64_t)kMaxLaunchGroups * kRB < (1ull << 32), "launch size");
+
+extern "C" int farm_set_raster_groups(farm_handle h, uint64_t groups) {
+    if (!h || groups > kMaxLaunchGroups) return fail(h, FARM_EINVAL, "%llu workgroups a launch",
+                                                     (unsigned long long)groups);
+    h->raster_groups = groups ? groups : kMaxLaunchGroups;
+    return FARM_OK;
 }
 
 extern "C" int farm_set_staging(farm_handle h, uint64_t vertices) {

@@ -57,6 +57,11 @@ int farm_hostset_rasterize_device(farm_handle h, const farm_hostset *s, int vpr,
  * longer than that goes through a pinned buffer of its own.  No counterpart
  * in the reference (its upload is one pageable copy). */
 int farm_set_staging(farm_handle h, uint64_t vertices);
+/* Workgroups per launch of the device raster builder's column kernels
+ * (default and maximum 2^24 - 1, the most of 256 work items that HIP takes;
+ * 0 restores it).  A set with more raster columns takes several launches; the
+ * result does not depend on it.  No counterpart in the reference. */
+int farm_set_raster_groups(farm_handle h, uint64_t groups);
 /* The rings as the raster builder reads them (each stored ring plus its
  * first vertex once more), for farm_rasterize: vert_off gets npolys + 1
  * offsets; x / y (may be NULL: offsets only) vert_off[npolys] floats each. */

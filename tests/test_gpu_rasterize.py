@@ -223,6 +223,38 @@ def test_fill_categories_on_the_device(device, bits):
     device.set_categories(4)
 
 
+def _thin_triangles(seed, n):
+    # rings of three vertices, 10,000 times wider than high: 200 columns of one pixel at -v 1
+    rng = np.random.default_rng(seed)
+    x, y = rng.uniform(1, 50, n), rng.uniform(1, 50, n)
+    t = np.stack([np.stack([x, y], 1), np.stack([x + 1.0, y + 2e-5 * rng.uniform(1, 5, n)], 1),
+                  np.stack([x + rng.uniform(0.2, 0.8, n), y + 1e-4], 1)], 1)
+    t = np.concatenate([t, t[:, :1]], 1).astype(np.float32)
+    return capi.HostSet.from_rings(np.arange(n + 1, dtype=np.uint64) * 4, t.reshape(-1, 2))
+
+
+@pytest.mark.parametrize("groups", [1, 7, 64])
+def test_column_kernels_in_several_launches(device, groups):
+    # long strips (the wide cell kernel) and short ones, sliced anywhere
+    c = datagen.complex_set(41, 2, 0.0, 3.0, nv_cap=6000)
+    s = datagen.star_pair_set(42, 6, 6, 0.0, 4.0)[0]
+    H = capi.HostSet.concat(capi.HostSet.from_rings(*c), capi.HostSet.from_rings(*s))
+    try:
+        device.set_raster_groups(groups)
+        _check(device, H, 64)
+    finally:
+        device.set_raster_groups(0)
+    with pytest.raises(capi.FarmError):
+        device.set_raster_groups(1 << 24)
+
+
+def test_more_columns_than_one_launch_takes(device):
+    # 2^24 workgroups of 256 are 2^32 work items, which HIP refuses
+    H = _thin_triangles(1, 80_000)
+    _, D = _check(device, H, 1)
+    assert int((D["hdr"]["dimx"].astype(np.int64) + 2).sum()) > 1 << 24
+
+
 def test_streamed_upload_through_pinned_staging(device):
     # farm_hostset_rasterize_device: the same set as farm_rasterize, with the
     # rings streamed through two pinned buffers -- many chunks, and one ring
