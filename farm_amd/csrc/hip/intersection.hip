@@ -979,27 +979,29 @@ __global__ __launch_bounds__(256) void k_ix_heavy(DevSet S, const uint32_t *__re
                                                   const uint32_t *__restrict__ pb, uint32_t n, int all,
                                                   uint8_t *__restrict__ flags, uint32_t *__restrict__ list,
                                                   uint32_t *__restrict__ ctr) {
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    bool heavy = false;
-    if (k < n) {
-        const farm_raster_hdr &A = S.hdr[pa[k]], &B = S.hdr[pb[k]];
-        auto part = [&](int lo, int hi, float &fa, float &fb) {
-            const float w = (float)(fmin(A.mbr[hi], B.mbr[hi]) - fmax(A.mbr[lo], B.mbr[lo]));
-            fa *= fminf(fmaxf(w, 0.f) / fmaxf((float)(A.mbr[hi] - A.mbr[lo]), 1e-30f), 1.f);
-            fb *= fminf(fmaxf(w, 0.f) / fmaxf((float)(B.mbr[hi] - B.mbr[lo]), 1e-30f), 1.f);
-        };
-        float fa = 1.f, fb = 1.f;
-        part(0, 2, fa, fb);
-        part(1, 3, fa, fb);
-        heavy = all || (A.nverts * fa / kIxChunk) * (B.nverts * fb / kIxChunk) > kHeavyChunks;
-        flags[k] = heavy ? 1 : 0;
+    for (uint64_t k0 = (uint64_t)blockIdx.x * blockDim.x; k0 < n; k0 += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t k = k0 + threadIdx.x;
+        bool heavy = false;
+        if (k < n) {
+            const farm_raster_hdr &A = S.hdr[pa[k]], &B = S.hdr[pb[k]];
+            auto part = [&](int lo, int hi, float &fa, float &fb) {
+                const float w = (float)(fmin(A.mbr[hi], B.mbr[hi]) - fmax(A.mbr[lo], B.mbr[lo]));
+                fa *= fminf(fmaxf(w, 0.f) / fmaxf((float)(A.mbr[hi] - A.mbr[lo]), 1e-30f), 1.f);
+                fb *= fminf(fmaxf(w, 0.f) / fmaxf((float)(B.mbr[hi] - B.mbr[lo]), 1e-30f), 1.f);
+            };
+            float fa = 1.f, fb = 1.f;
+            part(0, 2, fa, fb);
+            part(1, 3, fa, fb);
+            heavy = all || (A.nverts * fa / kIxChunk) * (B.nverts * fb / kIxChunk) > kHeavyChunks;
+            flags[k] = heavy ? 1 : 0;
+        }
+        const uint64_t m = __ballot(heavy);
+        uint32_t base = 0;
+        if (lane == 0 && m) base = atomicAdd(&ctr[kIxHeavy], (uint32_t)__popcll(m));
+        base = uni(__shfl(base, 0, 64));
+        if (heavy) list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint32_t)k;
     }
-    const uint64_t m = __ballot(heavy);
-    uint32_t base = 0;
-    if (lane == 0 && m) base = atomicAdd(&ctr[kIxHeavy], (uint32_t)__popcll(m));
-    base = uni(__shfl(base, 0, 64));
-    if (heavy) list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = k;
 }
 
 // Persistent workgroups: first the pairs of list[0 .. *nlist), all four waves
@@ -1143,7 +1145,7 @@ int run_intersection(farm_handle h, uint64_t begin, uint64_t end, int32_t *count
     if ((rc = ensure(h, h->wslab, nwaves * 2ull * kRecCap * sizeof(Rec)))) return rc;
     HIPCHK(h, hipEventRecord(h->ev[0], h->stream));
     // fewer than 8 pairs to a workgroup: all of them by whole workgroups
-    hipLaunchKernelGGL(k_ix_heavy, dim3(blocks_for(n)), dim3(256), 0, h->stream, S, pa, pb, n, n < 8 * nblocks ? 1 : 0,
+    hipLaunchKernelGGL(k_ix_heavy, dim3((unsigned)std::min<uint64_t>(blocks_for(n), kMaxLaunchGroups)), dim3(256), 0, h->stream, S, pa, pb, n, n < 8 * nblocks ? 1 : 0,
                        P<uint8_t>(h->ixflag), P<uint32_t>(h->ixlist), ctr);
     HIPCHK(h, hipGetLastError());
     hipLaunchKernelGGL(k_intersection<false>, dim3(nblocks), dim3(64 * kWaves), 0, h->stream, S,
