@@ -375,6 +375,7 @@ int finish_set(farm_handle h) {
     h->shape_bucket = hs[1] ? (int)std::floor(2.0 * std::log2(std::max(1.0, (double)hs[0] / (double)hs[1]))) : 0;
     // the bucket's tuned configuration, if the table holds one
     auto it = h->tunings.find(h->shape_bucket);
+    h->tile_auto = false;
     if (it != h->tunings.end()) {
         h->tuned_tile = it->second.tile_a;
         h->tuned_chunk = it->second.chunk;
@@ -385,6 +386,7 @@ int finish_set(farm_handle h) {
         // lie below 64, 128 and 256)
         const double e = hs[1] ? (double)hs[0] / (double)hs[1] : 0.0;
         h->tuned_tile = e < kTileEdges ? 1 : e < 2 * kTileEdges ? 2 : e < 4 * kTileEdges ? 4 : 8;
+        h->tile_auto = true;
     }
     return build_chunk_boxes(h, (uint32_t)h->tuned_chunk);
 }
@@ -516,6 +518,7 @@ static bool valid_tuning(const farm_tuning &t) {
 static int apply_tuning(farm_handle h, const farm_tuning &t) {
     h->tuned_tile = t.tile_a;
     h->tile_chosen = true;
+    h->tile_auto = false;
     h->tuned_chunk = t.chunk;
     h->tuned_bpc = t.blocks_per_cu;
     farm_tuning e = t;
@@ -593,6 +596,7 @@ int farm_set_tile(farm_handle h, int tile) {
     if (tile != 1 && tile != 2 && tile != 4 && tile != 8) return fail(h, FARM_EINVAL, "tile must be 1, 2, 4 or 8");
     h->tuned_tile = tile;
     h->tile_chosen = true;
+    h->tile_auto = false;
     return FARM_OK;
 }
 
@@ -896,10 +900,25 @@ static int run_intersect(farm_handle h, uint64_t begin, uint64_t end, const farm
     const DevSet S = devset(h);
     unsigned long long c[kCtrSlots];
     IsxWork W;
+    // A width that nobody chose gives way where its tiles have no room: the
+    // window is repeated at 4 edges per lane, the fewest tiles that a call
+    // which names no width may need (a quarter of those at 1).
+    bool narrow = E < 4 && h->wide_tiles && h->tile_auto && !(opts && opts->tile_a);
+    auto widen = [&]() {
+        const bool could = narrow;
+        if (narrow) E = 4;
+        narrow = false;
+        return could;
+    };
     for (int attempt = 0;; attempt++) {
         int rc;
-        if (fixed) W = isx_carve(h->scratch, kNaPairs, kNaPixPairs, kNaTiles);
-        else if ((rc = isx_reserve(h, n, &W))) return rc;
+        if (fixed) {
+            W = isx_carve(h->scratch, kNaPairs, kNaPixPairs, kNaTiles);
+        } else if ((rc = isx_reserve(h, n, &W))) {
+            if (rc != FARM_ENOMEM || attempt == 0 || !widen()) return rc;
+            h->isx_want_tiles = h->isx_want_pp;
+            if ((rc = isx_reserve(h, n, &W))) return rc;
+        }
         uint8_t *outp = out_kind == OUT_DEV ? out : (out_kind == OUT_HOST ? W.bits : nullptr);
         hipLaunchKernelGGL(k_set_desc, dim3(blocks_for(kIsxClear)), dim3(256), 0, h->stream, W.desc,
                            (unsigned long long)begin, (unsigned long long)n, outp, pair_tests, (uint32_t *)W.ctr);
@@ -980,6 +999,7 @@ static int run_intersect(farm_handle h, uint64_t begin, uint64_t end, const farm
             h->isx_want_tiles = std::max(h->isx_want_tiles, h->isx_want_pp);
             continue;
         }
+        if ((ntiles > 0xffffffffull || (fixed && ntiles > W.cap_tiles)) && widen()) continue;
         if (ntiles > 0xffffffffull)
             return fail(h, FARM_ECAPACITY, "%llu refinement tiles exceed 32-bit offsets; use smaller batches", ntiles);
         if (ntiles > W.cap_tiles) {
