@@ -289,6 +289,7 @@ EXPORTS = {
     "farm_autotune": (C.c_int, [C.c_void_p, C.c_uint64, C.c_uint64, C.POINTER(C.c_int)]),
     "farm_autotune_config": (C.c_int, [C.c_void_p, C.c_uint64, C.c_uint64, C.POINTER(Tuning)]),
     "farm_set_tile": (C.c_int, [C.c_void_p, C.c_int]),
+    "farm_set_wide_tile_limit": (C.c_int, [C.c_void_p, C.c_uint32]),
     "farm_get_tuning": (C.c_int, [C.c_void_p, C.POINTER(Tuning)]),
     "farm_set_tuning": (C.c_int, [C.c_void_p, C.POINTER(Tuning)]),
     "farm_tuning_save": (C.c_int, [C.c_void_p, C.c_char_p]),
@@ -881,6 +882,10 @@ class Device:
         if cache:
             self._check(lib.farm_tuning_save(self._h, cache.encode()), "tuning_save")
         return best.as_dict()
+
+    def set_wide_tile_limit(self, chunks: int) -> None:
+        """Chunks of one polygon from which tiles of 4 and 8 run at 2 (0: the default)."""
+        self._check(lib.farm_set_wide_tile_limit(self._h, chunks), "set_wide_tile_limit")
 
     def tuning(self) -> dict:
         """The configuration calls with tile_a / tile_b == 0 use."""

@@ -418,7 +418,7 @@ int build_chunk_boxes(farm_handle h, uint32_t C) {
         HIPCHK(h, hipGetLastError());
     }
     h->wide_tiles = true;
-    if (nchunks >= kItemChunks) {
+    if (nchunks >= h->item_chunks) {
         uint32_t most = 0, *d_most = P<uint32_t>(h->chcnt);
         if ((rc = fill_u32(h, d_most, 1, 0))) return rc;
         hipLaunchKernelGGL(k_most_chunks, dim3(256), dim3(256), 0, h->stream, devset(h), h->npolys,
@@ -426,7 +426,7 @@ int build_chunk_boxes(farm_handle h, uint32_t C) {
         HIPCHK(h, hipGetLastError());
         HIPCHK(h, hipMemcpyAsync(&most, d_most, 4, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
-        h->wide_tiles = most < kItemChunks;
+        h->wide_tiles = most < h->item_chunks;
     }
     const uint32_t ngroups = (nchunks + kGroup - 1) / kGroup;
     if ((rc = ensure(h, h->cgbox, 16ull * (ngroups + kRefScreen)))) return rc;
@@ -598,6 +598,13 @@ int farm_set_tile(farm_handle h, int tile) {
     h->tile_chosen = true;
     h->tile_auto = false;
     return FARM_OK;
+}
+
+int farm_set_wide_tile_limit(farm_handle h, uint32_t chunks) {
+    if (!h || chunks > kItemChunks) return fail(h, FARM_EINVAL, "%u chunks: at most %u", chunks, kItemChunks);
+    HIPCHK(h, hipSetDevice(h->device));
+    h->item_chunks = chunks ? chunks : kItemChunks;
+    return h->npolys > 0 ? build_chunk_boxes(h, h->chunk) : FARM_OK;
 }
 
 int farm_get_tuning(farm_handle h, farm_tuning *out) {
@@ -871,7 +878,6 @@ static int run_intersect(farm_handle h, uint64_t begin, uint64_t end, const farm
     const int mode = opts ? opts->mode : FARM_MODE_EXACT_BATCHED;
     int E = opts && opts->tile_a ? opts->tile_a : h->tuned_tile;
     if (E != 1 && E != 2 && E != 4 && E != 8) return fail(h, FARM_EINVAL, "tile_a must be 1, 2, 4 or 8");
-    if (!h->wide_tiles && E > 2) E = 2;
     // chunk size: the call's, else the tuned one (the built one for the
     // fixed-scratch entry, which never rebuilds the boxes on its own)
     const int C = opts && opts->tile_b ? opts->tile_b : (fixed ? (int)h->chunk : h->tuned_chunk);
@@ -897,6 +903,7 @@ static int run_intersect(farm_handle h, uint64_t begin, uint64_t end, const farm
         int rc = build_chunk_boxes(h, (uint32_t)C);
         if (rc) return rc;
     }
+    if (!h->wide_tiles && E > 2) E = 2;  // (of the boxes the call runs with)
     const DevSet S = devset(h);
     unsigned long long c[kCtrSlots];
     IsxWork W;

@@ -85,7 +85,8 @@ struct farm_handle_s {
     int tuned_chunk = 16;
     int tuned_bpc = 8;
     uint32_t chunk = 16;
-    bool wide_tiles = true;  // no polygon of the set has kItemChunks chunks (4 and 8 edges per lane allowed)
+    uint32_t item_chunks = farm::kItemChunks;  // a polygon of this many chunks runs at 2 edges per lane or fewer
+    bool wide_tiles = true;  // no polygon of the set has them, in chunks of the built size
     int shape_bucket = 0;
     std::map<int, farm_tuning> tunings;
     // learned part

@@ -416,6 +416,11 @@ int farm_autotune_config(farm_handle h, uint64_t begin, uint64_t end, farm_tunin
 int farm_autotune(farm_handle h, uint64_t begin, uint64_t end, int *best_tile);
 /* Set the tile width used when opts->tile_a is 0 (e.g. a persisted choice). */
 int farm_set_tile(farm_handle h, int tile);
+/* 4 and 8 edges per lane queue a polygon's chunks by 26-bit numbers: sets with
+ * a polygon of `chunks` chunks or more (default and maximum 2^26 - 8; 0
+ * restores it) run at 2 edges per lane where 4 or 8 are asked for, with the
+ * same answers. */
+int farm_set_wide_tile_limit(farm_handle h, uint32_t chunks);
 /* The configuration calls with opts->tile_a / tile_b == 0 use, and the set's
  * shape bucket. */
 int farm_get_tuning(farm_handle h, farm_tuning *out);

@@ -115,6 +115,41 @@ def test_groups_of_chunks(device, chunk, vpr):
         assert st["segment_tests"] + st["pruned_tests"] == full["segment_tests"]
 
 
+def test_wide_tile_limit_holds_for_the_chunks_of_the_call(device):
+    # a polygon beyond the limit in chunks of 8 segments and below it in chunks
+    # of 32: which widths run is decided by the chunks that the call runs with,
+    # whatever they were before it (the limit itself, 2^26 chunks, takes a ring
+    # of 5e8 vertices)
+    from farm_amd import datagen
+
+    a, b = datagen.complex_set(41, 12, lo=0.0, hi=3.0), datagen.lake_set(42, 150, lo=0.0, hi=3.0)
+    w = Workload(a, b, vpr=300)
+    want, _ = w.oracle(0)
+    w.upload(device)
+    apart = want == 0
+    device.upload_pairs(w.pa[apart], w.pb[apart] + len(w.A))
+    nv = max(np.diff(np.asarray(r[0]).astype(np.int64)).max() for r in (a, b))
+
+    def tiles(tile, chunk):
+        r = device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=tile, chunk=chunk)
+        assert not r.bits.any()
+        return r.stats["refine_items"]  # every tile runs: no pair answers true
+
+    full = {t: tiles(t, 16) for t in (2, 4, 8)}
+    assert full[2] > full[4] > full[8]
+    try:
+        device.set_wide_tile_limit(int(nv) // 16)
+        for chunk, wide in ((32, True), (8, False), (32, True), (8, False)):
+            for t in (8, 4, 2):
+                got = tiles(t, chunk)
+                print(f"  chunks of {chunk}, tile {t}: {got} tiles", flush=True)
+                assert got == full[t if wide else 2]
+    finally:
+        device.set_wide_tile_limit(0)
+    assert tiles(8, 8) == full[8]
+    device.intersect(mode=capi.MODE_EXACT_BATCHED, chunk=16)
+
+
 def test_tuning_rejects_bad_values(device):
     w = star_pairs(8, n=200)
     w.upload(device)
