@@ -38,6 +38,7 @@
 #include <chrono>
 #include <hipcub/hipcub.hpp>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "../../../include/farm_host.h"
@@ -675,198 +676,239 @@ __device__ __forceinline__ uint32_t hash_put(unsigned long long *keys, uint32_t 
 
 // Candidate counts of every column strip (PASS 0, before dedup) or the
 // strips themselves (PASS 1): kept points in order, the first repeated at
-// the end, their count and largest |y|.  One workgroup per column: a ring of
-// 200,000 vertices has 28 of them, and one workgroup went through them in turn
-// (both passes 13.2 ms for 400 rings of 1,000 to 130,000 vertices and 10,000
-// lakes; 2.1 ms so, the longest strip's serial batches).
+// the end, their count and largest |y|.  A workgroup's item is one column, or
+// with kItemWhole all columns of a ring in turn.  A ring of 200,000 vertices
+// has 28 columns, and one workgroup for all of them took 13.2 ms (both passes,
+// 400 rings of 1,000 to 130,000 vertices and 10,000 lakes; 3.8 ms by columns,
+// the longest strip's serial batches).  Short rings in large numbers fill the
+// chip either way, and a workgroup a column costs them its start and its
+// clearing of the table (300,000 lakes of up to 2,000 vertices: 60.5 ms by
+// columns, 50.8 whole).
+// LOOK: most batches of kRB edges of a long ring miss a column, and four at a
+// time are passed over with one barrier; rings of kShortRing batches or fewer
+// take the code without it (pass 1 on those 300,000 lakes 43.4 ms, and 49.9
+// with a look that is never taken).
+constexpr uint32_t kItemWhole = 0x80000000u;
+constexpr uint64_t kShortRing = 8;  // 4,000 complex rings: 15.8 ms at 8, 16.0 at 16, 16.4 at 32
+// A ring of nb batches is done whole where there are kWholeRings nb short rings
+// per CU or more: its workgroup, the longest of them, then ends with the rest.
+// 10,000 lakes (39 per CU), whole up to 0 / 2 / 4 / 8 batches: 2.20, 2.16, 2.24,
+// 3.73 ms; 30,000 (117 per CU), 0 / 3 / 7 / 8: 6.27, 6.06, 6.27, 5.99; 20,000
+// jagged rings of up to 500 vertices (78 per CU), 0 / 2: 1.12, 0.85.
+constexpr uint64_t kWholeRings = 16;
+
+template <int PASS>
+struct StripLds {
+    uint32_t sh[4];
+    unsigned long long keys[PASS ? kLdsSlots : 1];
+    uint32_t idx[PASS ? kLdsSlots : 1];
+    float2 cand[PASS ? kChunkCands : 1];
+    uint8_t keep[PASS ? kChunkCands : 1], near[PASS ? kChunkCands : 1];
+    uint16_t list[PASS ? kChunkCands : 1];
+    uint32_t nkept;
+    float my[kRB / 64];
+};
+
+// columns [c_begin, c_end) of ring g; false: the reference asserts
+template <int PASS, bool LOOK>
+__device__ __forceinline__ bool strip_columns(const RPoly &g, const float *X, const float *Y, double absx, int nrow,
+                                              int c_begin, int c_end, const double *__restrict__ colx,
+                                              uint32_t *__restrict__ stripc, const uint64_t *__restrict__ stripo,
+                                              const uint64_t *__restrict__ hasho, float2 *__restrict__ pool,
+                                              float2 *__restrict__ nearpool, unsigned long long *__restrict__ hkeys,
+                                              uint32_t *__restrict__ hidx, uint32_t *__restrict__ stripn,
+                                              float *__restrict__ stripmy, StripLds<PASS> &L) {
+    const Bucket bk(g.x0, g.sx, g.dimx + 2, absx);
+    const float *Xp = X + g.v, *Yp = Y + g.v;
+    const int ne = (int)g.nv - 1;
+    bool fail = false;
+    for (int c = c_begin; c < c_end; c++) {
+        const double Xi = colx[g.vl + c], Xi1 = colx[g.vl + c + 1];
+        if (PASS == 0) {
+            uint32_t cnt = 0;
+            for (int e = threadIdx.x; e < ne; e += kRB) {
+                const float ax = Xp[e], bx = Xp[e + 1];
+                if (!bk.reaches(ax, bx, c)) continue;
+                float2 pts[4];
+                cnt += strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, pts);
+            }
+            uint32_t tot;
+            block_scan(cnt, L.sh, &tot);
+            if (threadIdx.x == 0) stripc[g.vl + c] = tot;
+            continue;
+        }
+        const uint32_t cnt = stripc[g.vl + c];
+        if (cnt == 0) {
+            if (threadIdx.x == 0) stripn[g.vl + c] = 0;
+            continue;
+        }
+        float2 *pts = pool + stripo[g.vl + c], *nearp = nearpool + stripo[g.vl + c];
+        if (threadIdx.x == 0) L.nkept = 0;
+        const bool lds = cnt <= kLdsCands;
+        uint32_t slots = kLdsSlots;
+        if (!lds) {
+            slots = 1;
+            while (slots < 2 * cnt) slots <<= 1;
+        }
+        unsigned long long *gkeys = hkeys + (lds ? 0 : hasho[g.vl + c]);
+        uint32_t *gix = hidx + (lds ? 0 : hasho[g.vl + c]);
+        const uint32_t mask = slots - 1;
+        if (lds) {
+            for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
+                L.keys[s] = 0;
+                L.idx[s] = 0xffffffffu;
+            }
+        } else {
+            for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
+                gkeys[s] = 0;
+                gix[s] = 0xffffffffu;
+            }
+        }
+        __syncthreads();
+        uint32_t base = 0, kept = 0;
+        float my = 0.f;
+        for (int c0 = 0; c0 < ne; c0 += kRB) {
+            if (LOOK && (c0 & (4 * kRB - 1)) == 0) {
+                bool any = false;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int e = c0 + q * kRB + (int)threadIdx.x;
+                    any = any || (e < ne && bk.reaches(Xp[e], Xp[e + 1], c));
+                }
+                if (!__syncthreads_or(any)) {
+                    c0 += 3 * kRB;
+                    continue;
+                }
+            }
+            const int e = c0 + threadIdx.x;
+            float2 loc[4];
+            uint32_t n = 0;
+            if (e < ne) {
+                const float ax = Xp[e], bx = Xp[e + 1];
+                if (bk.reaches(ax, bx, c)) n = strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, loc);
+            }
+            if (LOOK && !__syncthreads_or(n != 0)) continue;
+            uint32_t tot;
+            const uint32_t off = block_scan(n, L.sh, &tot);
+            if (tot == 0) continue;
+            uint32_t slot[4];
+            uint32_t nnear = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                if (j >= n) break;
+                L.cand[off + j] = loc[j];
+                const bool nr = near_axis(loc[j]);
+                L.near[off + j] = nr;
+                nnear += nr;
+                if (!nr)
+                    slot[j] = lds ? hash_put(L.keys, L.idx, mask, pt_key(loc[j]), base + off + j)
+                                  : hash_put(gkeys, gix, mask, pt_key(loc[j]), base + off + j);
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++) {
+                if (j >= n) break;
+                L.keep[off + j] =
+                    L.near[off + j] || ((lds ? L.idx[slot[j]] : gix[slot[j]]) == base + off + j);
+            }
+            if (__syncthreads_or(nnear != 0)) {
+                // Points near an axis, in order, against every point kept before
+                // them.  Only another point near an axis can equal one: a
+                // coordinate of kNearAxis or more equals its own bits alone.  All
+                // the batch's are compared with the kept ones of earlier batches
+                // and with each other at once; only those that equal an earlier
+                // one of their own batch go in turn, as that one may be dropped.
+                // (Every point in turn against all kept ones held a 75,000-point
+                // ring at the axis for 5.8 ms of the pass; 1.9 ms so.)
+                uint32_t nn;
+                uint32_t no = block_scan(nnear, L.sh, &nn);
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++)
+                    if (j < n && L.near[off + j]) L.list[no++] = (uint16_t)(off + j);
+                __syncthreads();
+                const uint32_t prior = L.nkept;
+                for (uint32_t q = 0; q < nn; q++) {
+                    const uint32_t j = L.list[q];
+                    const float2 p = L.cand[j];
+                    bool found = false, twin = false;
+                    for (uint32_t k = threadIdx.x; k < prior; k += kRB) found |= same_pt(nearp[k], p);
+                    for (uint32_t k = threadIdx.x; k < q; k += kRB) twin |= same_pt(L.cand[L.list[k]], p);
+                    if (found) L.keep[j] = 0;
+                    if (twin) L.near[j] = 2;
+                }
+                __syncthreads();
+                for (uint32_t q = 0; q < nn; q++) {
+                    const uint32_t j = L.list[q];
+                    if (L.near[j] != 2 || !L.keep[j]) continue;
+                    const float2 p = L.cand[j];
+                    bool found = false;
+                    for (uint32_t k = threadIdx.x; k < q; k += kRB)
+                        found |= L.keep[L.list[k]] && same_pt(L.cand[L.list[k]], p);
+                    found = __syncthreads_or(found);
+                    if (threadIdx.x == 0) L.keep[j] = !found;
+                    __syncthreads();
+                }
+                for (uint32_t q = threadIdx.x; q < nn; q += kRB)
+                    if (L.keep[L.list[q]]) nearp[atomicAdd(&L.nkept, 1u)] = L.cand[L.list[q]];
+            }
+            uint32_t nk = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                if (j < n) nk += L.keep[off + j];
+            uint32_t ktot;
+            uint32_t ko = block_scan(nk, L.sh, &ktot);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; j++)
+                if (j < n && L.keep[off + j]) {
+                    pts[kept + ko++] = loc[j];
+                    my = smax(my, fabsf(loc[j].y));
+                }
+            base += tot;
+            kept += ktot;
+        }
+        // the largest |y| of the strip (the row buckets' margin scale)
+        const float wm = wave_max(my);
+        if ((threadIdx.x & 63) == 0) L.my[threadIdx.x >> 6] = wm;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            float m = L.my[0];
+            for (int w = 1; w < kRB / 64; w++) m = smax(m, L.my[w]);
+            if (kept > 0) pts[kept] = pts[0];
+            stripn[g.vl + c] = kept ? kept + 1 : 0;
+            stripmy[g.vl + c] = m;
+            // a non-empty strip outside the grid: the reference asserts
+            if (kept > 0 && (c >= g.dimx || nrow > g.dimy)) fail = true;
+        }
+        __syncthreads();
+    }
+    return !fail;
+}
+
 template <int PASS>
 __global__ __launch_bounds__(kRB) void k_rstrip(const RPoly *__restrict__ P, const float *__restrict__ X,
                                                 const float *__restrict__ Y, const float *__restrict__ absx,
                                                 uint32_t *__restrict__ rflag, const int *__restrict__ ncols,
                                                 const int *__restrict__ nrows, const double *__restrict__ colx,
-                                                const uint32_t *__restrict__ colpoly, uint64_t slot0,
+                                                const uint32_t *__restrict__ colpoly, const uint32_t *__restrict__ items,
                                                 uint32_t *__restrict__ stripc, const uint64_t *__restrict__ stripo,
                                                 const uint64_t *__restrict__ hasho, float2 *__restrict__ pool,
                                                 float2 *__restrict__ nearpool,
                                                 unsigned long long *__restrict__ hkeys, uint32_t *__restrict__ hidx,
                                                 uint32_t *__restrict__ stripn, float *__restrict__ stripmy) {
-    const uint64_t cs = slot0 + blockIdx.x;
+    const uint32_t item = items[blockIdx.x], cs = item & ~kItemWhole;
     const uint32_t i = colpoly[cs];
     if (rflag[i]) return;
     const RPoly g = P[i];
-    const int ncol = ncols[i], nrow = nrows[i], c = (int)(cs - g.vl);
-    if (c >= ncol) return;
-    const Bucket bk(g.x0, g.sx, g.dimx + 2, (double)absx[i]);
-    const float *Xp = X + g.v, *Yp = Y + g.v;
-    const int ne = (int)g.nv - 1;
-    __shared__ uint32_t sh[4];
-    __shared__ unsigned long long s_keys[PASS ? kLdsSlots : 1];
-    __shared__ uint32_t s_idx[PASS ? kLdsSlots : 1];
-    __shared__ float2 s_cand[PASS ? kChunkCands : 1];
-    __shared__ uint8_t s_keep[PASS ? kChunkCands : 1], s_near[PASS ? kChunkCands : 1];
-    __shared__ uint16_t s_list[PASS ? kChunkCands : 1];
-    __shared__ uint32_t s_nkept;
-    __shared__ float s_my[kRB / 64];
-    bool fail = false;
-    const double Xi = colx[g.vl + c], Xi1 = colx[g.vl + c + 1];
-    if (PASS == 0) {
-        uint32_t cnt = 0;
-        for (int e = threadIdx.x; e < ne; e += kRB) {
-            const float ax = Xp[e], bx = Xp[e + 1];
-            if (!bk.reaches(ax, bx, c)) continue;
-            float2 pts[4];
-            cnt += strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, pts);
-        }
-        uint32_t tot;
-        block_scan(cnt, sh, &tot);
-        if (threadIdx.x == 0) stripc[g.vl + c] = tot;
-        return;
-    }
-    const uint32_t cnt = stripc[g.vl + c];
-    if (cnt == 0) {
-        if (threadIdx.x == 0) stripn[g.vl + c] = 0;
-        return;
-    }
-    float2 *pts = pool + stripo[g.vl + c], *nearp = nearpool + stripo[g.vl + c];
-    if (threadIdx.x == 0) s_nkept = 0;
-    const bool lds = cnt <= kLdsCands;
-    uint32_t slots = kLdsSlots;
-    if (!lds) {
-        slots = 1;
-        while (slots < 2 * cnt) slots <<= 1;
-    }
-    unsigned long long *gkeys = hkeys + (lds ? 0 : hasho[g.vl + c]);
-    uint32_t *gix = hidx + (lds ? 0 : hasho[g.vl + c]);
-    const uint32_t mask = slots - 1;
-    if (lds) {
-        for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
-            s_keys[s] = 0;
-            s_idx[s] = 0xffffffffu;
-        }
-    } else {
-        for (uint32_t s = threadIdx.x; s < slots; s += kRB) {
-            gkeys[s] = 0;
-            gix[s] = 0xffffffffu;
-        }
-    }
-    __syncthreads();
-    uint32_t base = 0, kept = 0;
-    float my = 0.f;
-    for (int c0 = 0; c0 < ne; c0 += kRB) {
-        // most batches of a long ring miss the column: four at a time are
-        // passed over with one barrier
-        if ((c0 & (4 * kRB - 1)) == 0) {
-            bool any = false;
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int e = c0 + q * kRB + (int)threadIdx.x;
-                any = any || (e < ne && bk.reaches(Xp[e], Xp[e + 1], c));
-            }
-            if (!__syncthreads_or(any)) {
-                c0 += 3 * kRB;
-                continue;
-            }
-        }
-        const int e = c0 + threadIdx.x;
-        float2 loc[4];
-        uint32_t n = 0;
-        if (e < ne) {
-            const float ax = Xp[e], bx = Xp[e + 1];
-            if (bk.reaches(ax, bx, c)) n = strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, loc);
-        }
-        if (!__syncthreads_or(n != 0)) continue;
-        uint32_t tot;
-        const uint32_t off = block_scan(n, sh, &tot);
-        uint32_t slot[4];
-        uint32_t nnear = 0;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) {
-            if (j >= n) break;
-            s_cand[off + j] = loc[j];
-            const bool nr = near_axis(loc[j]);
-            s_near[off + j] = nr;
-            nnear += nr;
-            if (!nr)
-                slot[j] = lds ? hash_put(s_keys, s_idx, mask, pt_key(loc[j]), base + off + j)
-                              : hash_put(gkeys, gix, mask, pt_key(loc[j]), base + off + j);
-        }
-        __syncthreads();
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) {
-            if (j >= n) break;
-            s_keep[off + j] =
-                s_near[off + j] || ((lds ? s_idx[slot[j]] : gix[slot[j]]) == base + off + j);
-        }
-        if (__syncthreads_or(nnear != 0)) {
-            // Points near an axis, in order, against every point kept before
-            // them.  Only another point near an axis can equal one: a
-            // coordinate of kNearAxis or more equals its own bits alone.  All
-            // the batch's are compared with the kept ones of earlier batches
-            // and with each other at once; only those that equal an earlier
-            // one of their own batch go in turn, as that one may be dropped.
-            // (Every point in turn against all kept ones held a 75,000-point
-            // ring at the axis for 5.8 ms of the pass; 1.9 ms so.)
-            uint32_t nn;
-            uint32_t no = block_scan(nnear, sh, &nn);
-#pragma unroll
-            for (uint32_t j = 0; j < 4; j++)
-                if (j < n && s_near[off + j]) s_list[no++] = (uint16_t)(off + j);
-            __syncthreads();
-            const uint32_t prior = s_nkept;
-            for (uint32_t q = 0; q < nn; q++) {
-                const uint32_t j = s_list[q];
-                const float2 p = s_cand[j];
-                bool found = false, twin = false;
-                for (uint32_t k = threadIdx.x; k < prior; k += kRB) found |= same_pt(nearp[k], p);
-                for (uint32_t k = threadIdx.x; k < q; k += kRB) twin |= same_pt(s_cand[s_list[k]], p);
-                if (found) s_keep[j] = 0;
-                if (twin) s_near[j] = 2;
-            }
-            __syncthreads();
-            for (uint32_t q = 0; q < nn; q++) {
-                const uint32_t j = s_list[q];
-                if (s_near[j] != 2 || !s_keep[j]) continue;
-                const float2 p = s_cand[j];
-                bool found = false;
-                for (uint32_t k = threadIdx.x; k < q; k += kRB)
-                    found |= s_keep[s_list[k]] && same_pt(s_cand[s_list[k]], p);
-                found = __syncthreads_or(found);
-                if (threadIdx.x == 0) s_keep[j] = !found;
-                __syncthreads();
-            }
-            for (uint32_t q = threadIdx.x; q < nn; q += kRB)
-                if (s_keep[s_list[q]]) nearp[atomicAdd(&s_nkept, 1u)] = s_cand[s_list[q]];
-        }
-        uint32_t nk = 0;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++)
-            if (j < n) nk += s_keep[off + j];
-        uint32_t ktot;
-        uint32_t ko = block_scan(nk, sh, &ktot);
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++)
-            if (j < n && s_keep[off + j]) {
-                pts[kept + ko++] = loc[j];
-                my = smax(my, fabsf(loc[j].y));
-            }
-        base += tot;
-        kept += ktot;
-    }
-    // the largest |y| of the strip (the row buckets' margin scale)
-    const float wm = wave_max(my);
-    if ((threadIdx.x & 63) == 0) s_my[threadIdx.x >> 6] = wm;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float m = s_my[0];
-        for (int w = 1; w < kRB / 64; w++) m = smax(m, s_my[w]);
-        if (kept > 0) pts[kept] = pts[0];
-        stripn[g.vl + c] = kept ? kept + 1 : 0;
-        stripmy[g.vl + c] = m;
-        // a non-empty strip outside the grid: the reference asserts
-        if (kept > 0 && (c >= g.dimx || nrow > g.dimy)) fail = true;
-    }
-    __syncthreads();
-    if (PASS == 1 && threadIdx.x == 0 && fail) atomicOr(&rflag[i], kRejFill);
+    const int nrow = nrows[i], c_begin = (int)(cs - g.vl);
+    const int c_end = item & kItemWhole ? ncols[i] : min(c_begin + 1, ncols[i]);
+    __shared__ StripLds<PASS> L;
+    auto columns = [&](auto look) {
+        return strip_columns<PASS, decltype(look)::value>(g, X, Y, (double)absx[i], nrow, c_begin, c_end, colx, stripc,
+                                                          stripo, hasho, pool, nearpool, hkeys, hidx, stripn, stripmy,
+                                                          L);
+    };
+    const bool ok = PASS == 1 && g.nv > kShortRing * kRB + 1 ? columns(std::true_type()) : columns(std::false_type());
+    if (PASS == 1 && threadIdx.x == 0 && !ok) atomicOr(&rflag[i], kRejFill);
 }
 
 // Points strip edge (A, B) adds to row [Yi, Yi1] (Ideal::calculate_fullness,
@@ -1512,12 +1554,12 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
     uint32_t *colpoly;
     int *ncols, *nrows;
     uint32_t *stripc, *stripn;
-    uint64_t *psz, *stripo, *hsz, *hasho;
+    uint64_t *stripo, *hasho;
     float *stripmy;
     if ((rc = T.get(h, &colx, nvl)) || (rc = T.get(h, &colpoly, nvl)) || (rc = T.get(h, &rowy, nhl)) || (rc = T.get(h, &ncols, np)) ||
         (rc = T.get(h, &nrows, np)) || (rc = T.get(h, &stripc, nvl)) || (rc = T.get(h, &stripn, nvl)) ||
-        (rc = T.get(h, &stripmy, nvl)) || (rc = T.get(h, &psz, nvl + 1)) || (rc = T.get(h, &stripo, nvl + 1)) ||
-        (rc = T.get(h, &hsz, nvl + 1)) || (rc = T.get(h, &hasho, nvl + 1)))
+        (rc = T.get(h, &stripmy, nvl)) || (rc = T.get(h, &stripo, nvl + 1)) ||
+        (rc = T.get(h, &hasho, nvl + 1)))
         return rc;
     HIPCHK(h, hipMemsetAsync(stripc, 0, 4 * nvl, h->stream));
     HIPCHK(h, hipMemsetAsync(stripn, 0, 4 * nvl, h->stream));
@@ -1526,19 +1568,42 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
                            colx, rowy, ncols, nrows, colpoly);
         HIPCHK(h, hipGetLastError());
     }
-    // one workgroup per column slot, h->raster_groups of them a launch
-    const uint64_t slice = h->raster_groups;
-    auto strips = [&](auto kernel, const uint64_t *so, const uint64_t *hof, float2 *pool, float2 *nearpool,
-                      unsigned long long *hkeys, uint32_t *hidx) -> int {
-        for (uint64_t s0 = 0; s0 < nvl; s0 += slice) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(nvl - s0, slice)), dim3(kRB), 0,
-                               h->stream, (const RPoly *)d_rp, P<float>(h->x), P<float>(h->y), (const float *)d_absx,
-                               d_flag, (const int *)ncols, (const int *)nrows, (const double *)colx,
-                               (const uint32_t *)colpoly, s0, stripc, so, hof, pool, nearpool, hkeys, hidx,
-                               stripn, stripmy);
+    // work items of the strips, the columns of long rings first
+    std::vector<uint32_t> items, rest;
+    {
+        auto batches = [&](int64_t i) { return (voff[i + 1] - voff[i] + kRB - 2) / kRB; };
+        uint64_t nshort = 0;
+        for (int64_t i = 0; i < np; i++) nshort += batches(i) <= kShortRing;
+        for (int64_t i = 0; i < np; i++) {
+            const uint64_t nb = batches(i);
+            if (nb <= kShortRing && nb * kWholeRings * (uint64_t)h->num_cus <= nshort) {
+                rest.push_back((uint32_t)rp[i].vl | kItemWhole);
+                continue;
+            }
+            std::vector<uint32_t> &to = nb <= kShortRing ? rest : items;
+            for (int c = 0; c < rp[i].dimx + 2; c++) to.push_back((uint32_t)rp[i].vl + c);
+        }
+        items.insert(items.end(), rest.begin(), rest.end());
+    }
+    uint32_t *d_items;
+    if ((rc = T.get(h, &d_items, items.size()))) return rc;
+    HIPCHK(h, hipMemcpyAsync(d_items, items.data(), 4 * items.size(), hipMemcpyHostToDevice, h->stream));
+    // launch(first, workgroups) over n workgroups, h->raster_groups at a time
+    auto sliced = [&](uint64_t n, auto launch) -> int {
+        for (uint64_t s0 = 0; s0 < n; s0 += h->raster_groups) {
+            launch(s0, dim3((unsigned)std::min<uint64_t>(n - s0, h->raster_groups)));
             HIPCHK(h, hipGetLastError());
         }
         return FARM_OK;
+    };
+    auto strips = [&](auto kernel, const uint64_t *so, const uint64_t *hof, float2 *pool, float2 *nearpool,
+                      unsigned long long *hkeys, uint32_t *hidx) {
+        return sliced(items.size(), [&](uint64_t s0, dim3 groups) {
+            hipLaunchKernelGGL(kernel, groups, dim3(kRB), 0, h->stream, (const RPoly *)d_rp, P<float>(h->x),
+                               P<float>(h->y), (const float *)d_absx, d_flag, (const int *)ncols, (const int *)nrows,
+                               (const double *)colx, (const uint32_t *)colpoly, (const uint32_t *)d_items + s0, stripc,
+                               so, hof, pool, nearpool, hkeys, hidx, stripn, stripmy);
+        });
     };
     if ((rc = strips(k_rstrip<0>, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr))) return rc;
     // pool sizes: every candidate plus the closing point; hashes in HBM for
@@ -1575,19 +1640,18 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
                                (const uint32_t *)stripn, (const float *)stripmy, (const float2 *)pool,
                                P<uint8_t>(h->status), P<double>(h->areas));
             HIPCHK(h, hipGetLastError());
-            for (uint64_t s0 = 0; s0 < nvl; s0 += slice) {
-                hipLaunchKernelGGL(k_rcells_wide, dim3((unsigned)std::min(nvl - s0, slice)), dim3(kRB), 0, h->stream, (const RPoly *)d_rp, (const uint32_t *)colpoly, s0,
-                                   (const uint32_t *)d_flag, (const int *)ncols, (const int *)nrows,
-                                   (const double *)rowy, (const uint64_t *)stripo, (const uint32_t *)stripn,
-                                   (const float *)stripmy, (const float2 *)pool, P<uint8_t>(h->status),
-                                   P<double>(h->areas));
-                HIPCHK(h, hipGetLastError());
-            }
+            // one workgroup per column slot
+            rc = sliced(nvl, [&](uint64_t s0, dim3 groups) {
+                hipLaunchKernelGGL(k_rcells_wide, groups, dim3(kRB), 0, h->stream, (const RPoly *)d_rp,
+                                   (const uint32_t *)colpoly, s0, (const uint32_t *)d_flag, (const int *)ncols,
+                                   (const int *)nrows, (const double *)rowy, (const uint64_t *)stripo,
+                                   (const uint32_t *)stripn, (const float *)stripmy, (const float2 *)pool,
+                                   P<uint8_t>(h->status), P<double>(h->areas));
+            });
+            if (rc) return rc;
         }
         HIPCHK(h, hipStreamSynchronize(h->stream));
     }
-    (void)psz;
-    (void)hsz;
 
     // ---- final arrays ----
     uint64_t *nseq, *nvnf, *seqf, *vnf;

@@ -248,6 +248,21 @@ def test_column_kernels_in_several_launches(device, groups):
         device.set_raster_groups(1 << 24)
 
 
+@pytest.mark.parametrize("n", [4000, 4200, 8400])
+def test_short_rings_whole_and_by_columns(device, n):
+    # from 16 short rings per CU on (4,096 on 256 CUs) those of one batch of 256
+    # edges are one workgroup's, from 32 on those of two; longer ones go by
+    # columns, beyond 8 batches with the look ahead
+    rng = np.random.default_rng(43)
+    sizes = [255, 256, 257, 511, 512, 513, 2047, 2048, 2049, 2500] + [12] * n
+    rings = []
+    for nv in sizes:
+        t = np.sort(rng.uniform(0, 2 * np.pi, nv))
+        r = rng.uniform(0.1, 0.3) * (1 + 0.4 * rng.uniform(-1, 1, nv))
+        rings.append(rng.uniform(-3, 20, 2) + np.stack([r * np.cos(t), r * np.sin(t)], 1))
+    _check(device, capi.HostSet.from_rings(*rings_from_list(rings)), 10)
+
+
 def test_more_columns_than_one_launch_takes(device):
     # 2^24 workgroups of 256 are 2^32 work items, which HIP refuses
     H = _thin_triangles(1, 80_000)
