@@ -32,9 +32,9 @@ __global__ void k_bucket_scatter(const uint8_t *, const unsigned long long *, ui
 template <int E>
 __global__ void k_tiles(const PixPair *, const uint32_t *, const unsigned long long *, unsigned long long *, uint64_t,
                         uint32_t *);
-template <int E, int C>
+template <int E, int C, bool PRUNE>
 __global__ void k_refine(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *, const TileDesc *, uint64_t,
-                         uint64_t, uint32_t *, uint32_t *, const unsigned long long *, unsigned long long *, int);
+                         uint64_t, uint32_t *, uint32_t *, const unsigned long long *, unsigned long long *);
 __global__ void k_tile_map(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *, const PixPair *,
                            const uint32_t *, const uint32_t *, const unsigned long long *, uint64_t, uint64_t,
                            TileDesc *);
@@ -191,10 +191,13 @@ int isx_front(farm_handle h, const DevSet &S, const IsxWork &W, const IsxCfg &c)
 // The persistent refinement with the tile width and chunk size of the call.
 template <int E, int C>
 void launch_refine(farm_handle h, const DevSet &S, const IsxWork &W, const IsxCfg &c) {
-    const dim3 grid((unsigned)(h->num_cus * c.bpc)), blk(256);
-    hipLaunchKernelGGL((k_refine<E, C>), grid, blk, 0, h->stream, S, c.pa, c.pb, (const IsxDesc *)W.desc,
-                       (const TileDesc *)W.tile_map, W.cap_pp, W.cap_tiles, W.tcur, W.result,
-                       (const unsigned long long *)W.ctr, W.shards, c.prune);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(h->num_cus * c.bpc)), dim3(256), 0, h->stream, S, c.pa, c.pb,
+                           (const IsxDesc *)W.desc, (const TileDesc *)W.tile_map, W.cap_pp, W.cap_tiles, W.tcur,
+                           W.result, (const unsigned long long *)W.ctr, W.shards);
+    };
+    if (c.prune) launch(k_refine<E, C, true>);
+    else launch(k_refine<E, C, false>);
 }
 
 template <int E>

@@ -572,7 +572,7 @@ typedef __attribute__((address_space(4))) const uint32_t cuint;
 constexpr uint32_t kSplit = 1, kDrain = 64u >> kSplit;
 constexpr uint32_t kRefQueue = 512;  // queued items per wave: a power of 2 above 63 + 64 kRefScreen (or kGroup)
 
-template <int W, int C>
+template <int W, int C, bool PRUNE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_refine(DevSet S, const uint32_t *__restrict__ pa_all,
                                                  const uint32_t *__restrict__ pb_all,
                                                  const IsxDesc *__restrict__ desc,
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                                                  uint64_t cap_tiles, uint32_t *__restrict__ cursor,
                                                  uint32_t *__restrict__ result,
                                                  const unsigned long long *__restrict__ ctr,
-                                                 unsigned long long *__restrict__ shards, int prune) {
+                                                 unsigned long long *__restrict__ shards) {
     // the tile total, unless a buffer of an earlier phase overflowed (the
     // host then grows the workspace and repeats the call, or fails it)
     if (ctr[kCtrPixPairs] > cap_pp || ctr[kCtrTiles] > cap_tiles) return;
@@ -594,7 +594,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // (with groups: chunk of the pixel and source lane in one word each, and
     // in the other half a ring of groups and source lanes; sets with a
     // polygon of 2^26 chunks or more run at 2 edges per lane)
-    constexpr bool groups = W >= 4;
+    constexpr bool groups = PRUNE && W >= 4;
     __shared__ uint2 s_ring[4][kRefQueue];
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
@@ -621,7 +621,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     // position alone left waves idle (a call of 1.3e6 tiles of uneven cost
     // took 17.5 ms instead of 13.9).
     const uint32_t nwaves = gridDim.x * 4u, wid = blockIdx.x * 4u + (uint32_t)wv;
-    const uint32_t dir_all = prune ? 0u : ~0u;  // without the prune every direction matches
     const uint32_t grab = min(max(total / (nwaves * 16u), 1u), 16u);
     uint32_t home = wid & (kCtrShards - 1);
     uint32_t tbase = 0;
@@ -773,39 +772,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
             const uint4 *vseg = S.chseg + g0;
             uint32_t scr_steps = 0, queued_steps = 0;  // target steps screened (uniform) / queued by this lane
 
-            // Evaluate the n <= kDrain oldest queued items: the source
-            // lane's E edges against the chunk's nstep target segments.  Per
-            // target vertex q and source edge (a, b):
+            // Evaluate source lane sl's E edges against the ns <= C segments from
+            // target vertex vs on.  Per target vertex q and source edge (a, b):
             //   O(q) = a.cross(b, q)   -- o1/o2 of consecutive steps
             //   o(p) = c.cross(p, d)   -- per source vertex p, for the segment (c, d)
             // carried from step to step: tx/ty = p - c serves O(c) and, by the
             // antisymmetry of rounded subtraction, o(p) of the next step.  A
             // superset filter (o1*o2 <= 0 or o3 == 0, and o3*o4 <= 0) sends
             // the rare candidates to the exact reference predicate.
-            //
-            // An item is split over k = 64 / n lanes, rounded down to a power
-            // of two (at most C), part j taking its steps j C / k .. (j + 1) C
-            // / k - 1.  A part is the item's segments from its own first vertex
-            // on, so the split evaluates the same tests in C / k steps instead
-            // of C.
-            auto drain = [&](uint32_t n) {
-                uint32_t lk = kSplit;  // log2 k (uniform)
-                while ((1u << lk) < (uint32_t)C && (n << (lk + 1)) <= 64u) lk++;
-                const uint32_t seg = (uint32_t)C >> lk;
-                const uint32_t item = (uint32_t)lane >> lk, m0 = ((uint32_t)lane & ((1u << lk) - 1u)) * seg;
-                uint2 it;
-                if constexpr (groups) {
-                    const uint32_t w = ring4[(qhead + min(item, n - 1)) & (kRefQueue - 1)];
-                    const uint4 sg = vseg[w >> 6];
-                    it = make_uint2(sg.x, (w & 63u) | ((sg.y & ~kChunkPoint) << 8));
-                } else {
-                    it = ring[(qhead + item) & (kRefQueue - 1)];
-                }
-                const uint32_t nsf = item < n ? (it.y >> 8) : 0u;
-                const uint32_t ns = nsf > m0 ? min(seg, nsf - m0) : 0u;
-                const bool has = ns > 0u;
-                const uint32_t sl = has ? (it.y & 63u) : (uint32_t)lane;
-                const uint32_t vs = has ? it.x + m0 : 0u;  // the part's first vertex c
+            auto eval = [&](uint32_t sl, uint32_t vs, uint32_t ns) {
                 float qpx[E + 1], qpy[E + 1];
 #pragma unroll
                 for (int v = 0; v <= E; v++) {
@@ -890,6 +865,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                     }
                 }
                 tests += (uint32_t)qnv * ns;
+            };
+
+            // Evaluate the n <= kDrain (without the prune 64) oldest queued items: the source
+            // lane's E edges against the chunk's nstep target segments.
+            //
+            // An item is split over k = 64 / n lanes, rounded down to a power
+            // of two (at most C), part j taking its steps j C / k .. (j + 1) C
+            // / k - 1.  A part is the item's segments from its own first vertex
+            // on, so the split evaluates the same tests in C / k steps instead
+            // of C.
+            auto drain = [&](uint32_t n) {
+                uint32_t lk = PRUNE ? kSplit : 0u;  // log2 k (uniform)
+                while ((1u << lk) < (uint32_t)C && (n << (lk + 1)) <= 64u) lk++;
+                const uint32_t seg = (uint32_t)C >> lk;
+                const uint32_t item = (uint32_t)lane >> lk, m0 = ((uint32_t)lane & ((1u << lk) - 1u)) * seg;
+                uint2 it;
+                if constexpr (groups) {
+                    const uint32_t w = ring4[(qhead + min(item, n - 1)) & (kRefQueue - 1)];
+                    const uint4 sg = vseg[w >> 6];
+                    it = make_uint2(sg.x, (w & 63u) | ((sg.y & ~kChunkPoint) << 8));
+                } else {
+                    it = ring[(qhead + item) & (kRefQueue - 1)];
+                }
+                const uint32_t nsf = item < n ? (it.y >> 8) : 0u;
+                const uint32_t ns = nsf > m0 ? min(seg, nsf - m0) : 0u;
+                const bool has = ns > 0u;
+                const uint32_t sl = has ? (it.y & 63u) : (uint32_t)lane;
+                const uint32_t vs = has ? it.x + m0 : 0u;  // the part's first vertex c
+                eval(sl, vs, ns);
                 qhead = (qhead + n) & (kRefQueue - 1);
                 qn -= n;
                 if (__any(hit)) stop = true;
@@ -968,12 +972,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 // and no segment of the chunk within kDirTol of the
                 // direction of any of the lane's edges.
                 const bool far = fmaxf(sepx - hx1, sepy - hy1) > q * 0x1p-8f && q < 0x1p60f;
-                const bool cand = !far || ((L.dir.x & (cdl | dir_all)) | (L.dir.y & (cdh | dir_all))) != 0u;
+                const bool cand = !far || ((L.dir.x & cdl) | (L.dir.y & cdh)) != 0u;
                 if (!__ballot(cand)) return false;  // no lane's lines need a look
-                // (without the prune: the largest finite margin keeps every
-                // chunk for every slot with an edge)
-                const float k1 = !prune ? 0x1.fffffep127f : q * 0x1p-18f;
-                const float k2 = !prune ? 0x1.fffffep127f : (apart ? 0x1p-80f : fmaf(q, q * 0x1p-17f, 0x1p-80f));
+                const float k1 = q * 0x1p-18f;
+                const float k2 = apart ? 0x1p-80f : fmaf(q, q * 0x1p-17f, 0x1p-80f);
                 // |s_y| hx + |s_x| hy + (|s_x| + |s_y|) k1 + k2 as
                 // |s_y| (hx + k1) + |s_x| (hy + k1) + k2
                 const float hxk = bb.z + k1, hyk = bb.w + k1;
@@ -1018,7 +1020,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 gn -= n;
             };
 
-            {
+            if constexpr (!PRUNE) {
+                // every chunk for every lane that has an edge, 64 items at a
+                // time (straight from the chunks, each lane its own edges, a
+                // tile's empty lanes idle: 91 ms instead of 75 at 8 edges per
+                // lane on complex x lakes)
+                const cuint *cseg = (const cuint *)S.chseg;
+                const unsigned long long bm = __ballot(evb != 0);
+                for (uint32_t c = b_c0; c < b_c1 && !stop; c++) {
+                    const uint32_t v0 = cseg[4 * c], nstep = cseg[4 * c + 1] & ~kChunkPoint;
+                    scr_steps += nstep;
+                    if (evb) {
+                        ring[(qhead + qn + below(bm)) & (kRefQueue - 1)] = make_uint2(v0, (uint32_t)lane | (nstep << 8));
+                        queued_steps += nstep;
+                    }
+                    qn += (uint32_t)__popcll(bm);
+                    while (!stop && (qn >= 64 || (c + 1 == b_c1 && qn))) {
+                        __builtin_amdgcn_wave_barrier();
+                        drain(min(qn, 64u));
+                    }
+                    if ((++screened & 31u) == 0 &&
+                        __hip_atomic_load(&result[pair], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                        break;
+                }
+            } else {
                 // kRefScreen boxes at a time against every lane's edges (scalar
                 // loads; entries past the pixel's last are read, the arrays keep
                 // spare ones, but not used): of chunks at narrow tiles, whose
@@ -1348,26 +1373,26 @@ __global__ __launch_bounds__(256) void k_finalize(const uint32_t *__restrict__ r
 #define FARM_TILES_INST(EE)                                                                                    \
     template __global__ void k_tiles<EE>(const PixPair *, const uint32_t *, const unsigned long long *,          \
                                          unsigned long long *, uint64_t, uint32_t *);
-#define FARM_REFINE_INST(EE, CC)                                                                               \
-    template __global__ void k_refine<EE, CC>(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *,      \
-                                              const TileDesc *, uint64_t, uint64_t, uint32_t *, uint32_t *,     \
-                                              const unsigned long long *, unsigned long long *, int);
+#define FARM_REFINE_INST(EE, CC, PP)                                                                           \
+    template __global__ void k_refine<EE, CC, PP>(DevSet, const uint32_t *, const uint32_t *, const IsxDesc *,  \
+                                                  const TileDesc *, uint64_t, uint64_t, uint32_t *, uint32_t *, \
+                                                  const unsigned long long *, unsigned long long *);
+#define FARM_REFINE_INSTS(EE)     \
+    FARM_REFINE_INST(EE, 8, true)  \
+    FARM_REFINE_INST(EE, 16, true) \
+    FARM_REFINE_INST(EE, 32, true) \
+    FARM_REFINE_INST(EE, 8, false) \
+    FARM_REFINE_INST(EE, 16, false) \
+    FARM_REFINE_INST(EE, 32, false)
 FARM_TILES_INST(1)
 FARM_TILES_INST(2)
 FARM_TILES_INST(4)
 FARM_TILES_INST(8)
-FARM_REFINE_INST(1, 8)
-FARM_REFINE_INST(2, 8)
-FARM_REFINE_INST(4, 8)
-FARM_REFINE_INST(8, 8)
-FARM_REFINE_INST(1, 16)
-FARM_REFINE_INST(2, 16)
-FARM_REFINE_INST(4, 16)
-FARM_REFINE_INST(8, 16)
-FARM_REFINE_INST(1, 32)
-FARM_REFINE_INST(2, 32)
-FARM_REFINE_INST(4, 32)
-FARM_REFINE_INST(8, 32)
+FARM_REFINE_INSTS(1)
+FARM_REFINE_INSTS(2)
+FARM_REFINE_INSTS(4)
+FARM_REFINE_INSTS(8)
+#undef FARM_REFINE_INSTS
 #undef FARM_TILES_INST
 #undef FARM_REFINE_INST
 

@@ -115,6 +115,28 @@ def test_groups_of_chunks(device, chunk, vpr):
         assert st["segment_tests"] + st["pruned_tests"] == full["segment_tests"]
 
 
+@pytest.mark.parametrize("chunk", [8, 16, 32])
+def test_without_the_prune(device, chunk):
+    # another kernel of its own: every chunk for every lane with an edge, in
+    # rounds of 64 items and a part of one, at every tile width; on pairs that
+    # all answer false, the same tests at each
+    from farm_amd import datagen
+
+    a, b = datagen.complex_set(41, 12, lo=0.0, hi=3.0), datagen.lake_set(42, 150, lo=0.0, hi=3.0)
+    w = Workload(a, b, vpr=40)
+    want, _ = w.oracle(0)
+    w.upload(device)
+    for tile in (1, 2, 4, 8):
+        r = device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=tile, chunk=chunk, flags=capi.FLAG_NO_PRUNE)
+        assert np.array_equal(r.bits, (want == 1).astype(np.uint8)), tile
+    apart = want == 0
+    device.upload_pairs(w.pa[apart], w.pb[apart] + len(w.A))
+    run = [device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=t, chunk=chunk, flags=capi.FLAG_NO_PRUNE).stats
+           for t in (1, 2, 4, 8)]
+    assert run[0]["segment_tests"] > 0
+    assert all(s["pruned_tests"] == 0 and s["segment_tests"] == run[0]["segment_tests"] for s in run)
+
+
 def test_wide_tile_limit_holds_for_the_chunks_of_the_call(device):
     # a polygon beyond the limit in chunks of 8 segments and below it in chunks
     # of 32: which widths run is decided by the chunks that the call runs with,
