@@ -311,12 +311,28 @@ namespace farm {
 
 int build_chunk_boxes(farm_handle h, uint32_t C);
 
-// Mean edges per BORDER pixel below which the default tile is 1 edge per lane
-// (2 below twice that, 4 below four times).  Measured, k_refine at 1 / 4 / 8
-// edges per lane: 23 edges per pixel (jagged rings, -v 10, 8 sequences a
-// pixel) 2.5 / 3.2 / 4.6 ms; 560 to 740 (complex x lakes, -v 256) 22.4 / 14.6
-// / 13.9 ms.
-constexpr double kTileEdges = 48.0;
+// Edges per lane where nothing is tuned or set, from the set's mean edges and
+// chunks per BORDER pixel.  Narrow tiles end early at a pair's first crossing
+// and leave fewer lanes empty; 4 edges per lane read half the boxes of 2 and
+// screen them in groups, which pays from about 24 chunks a pixel on.  Measured,
+// k_refine in ms at 1 / 2 / 4 / 8 edges per lane (edges, chunks per pixel):
+//   jagged small rings  (23, 8)  .354 .364 .519 .601   (49, 10) .450 .474 .668 .841
+//                       (68, 9)  .535 .498 .744 .934   (149, 10) .570 .641 .777 .964
+//                       (230, 15) .633 .682 .755 .797  (274, 18) .770 .709 .774 .737
+//   complex x lakes     (22, 14) .395 .389 .439 .498   (47, 22) .516 .482 .498 .574
+//                       (62, 25) .841 .650 .621 .746   (138, 36) 4.89 3.42 1.85 2.31
+//                       (273, 34) 6.67 4.40 2.37 2.46  (574, 37) 7.97 5.01 2.71 2.68
+//   smooth rings, 300   (19, 2)  .253 .260 .379 .450   (60, 4) .541 .517 .826 1.08
+//   vertices            (153, 10) 1.14 .977 1.44 1.87  (344, 22) 1.60 1.30 1.75 2.15
+//   smooth rings, 3,000 (43, 3)  .086 .079 .102 .114   (97, 7) .202 .149 .160 .190
+//                       (154, 10) .355 .254 .228 .276  (259, 17) .601 .500 .429 .408
+//   complex x complex   (57, 4)  .062 .062 .070 .075   (130, 9) .104 .086 .106 .110
+//                       (354, 23) .535 .468 .401 .381  (657, 42) 1.61 1.15 .755 .832
+// 8 is the autotuner's to choose: it wins 5 % at most, and loses up to 22 %.
+int default_tile(double edges, double chunks) {
+    if (edges >= 128.0 || chunks >= 24.0) return 4;
+    return edges < 48.0 && chunks < 12.0 ? 1 : 2;
+}
 
 // Sum and count of the nonzero per-pixel edge counts (BORDER pixels).
 __global__ __launch_bounds__(256) void k_shape_stats(const uint32_t *__restrict__ pixedges, uint64_t n,
@@ -383,15 +399,13 @@ int finish_set(farm_handle h) {
         h->tuned_tile = it->second.tile_a;
         h->tuned_chunk = it->second.chunk;
         h->tuned_bpc = it->second.blocks_per_cu;
-    } else if (!h->tile_chosen) {
-        // nothing tuned or set: the narrowest tile whose 64 lanes hold a mean
-        // pixel's edges (short edge sequences add a slot each, so the lines
-        // lie below 64, 128 and 256)
-        const double e = hs[1] ? (double)hs[0] / (double)hs[1] : 0.0;
-        h->tuned_tile = e < kTileEdges ? 1 : e < 2 * kTileEdges ? 2 : e < 4 * kTileEdges ? 4 : 8;
-        h->tile_auto = true;
+    } else {
+        h->tile_auto = !h->tile_chosen;
     }
-    return build_chunk_boxes(h, (uint32_t)h->tuned_chunk);
+    if ((rc = build_chunk_boxes(h, (uint32_t)h->tuned_chunk))) return rc;
+    if (h->tile_auto)
+        h->tuned_tile = hs[1] ? default_tile((double)hs[0] / (double)hs[1], (double)h->nchunks / (double)hs[1]) : 4;
+    return FARM_OK;
 }
 
 // Boxes of the refinement's C-step target chunks, per edge sequence.
@@ -420,6 +434,7 @@ int build_chunk_boxes(farm_handle h, uint32_t C) {
                            (const uint32_t *)P<uint32_t>(h->choff), P<float4>(h->chbox), P<uint4>(h->chseg));
         HIPCHK(h, hipGetLastError());
     }
+    h->nchunks = nchunks;
     h->wide_tiles = true;
     if (nchunks >= h->item_chunks) {
         uint32_t most = 0, *d_most = P<uint32_t>(h->chcnt);

@@ -81,7 +81,8 @@ struct farm_handle_s {
     // per shape bucket (farm_tuning_save / farm_tuning_load persist it)
     int tuned_tile = 4;
     bool tile_chosen = false;  // the caller (or the autotuner) named the tile width
-    bool tile_auto = false;    // tuned_tile comes from the set's edges per pixel alone
+    bool tile_auto = false;    // tuned_tile comes from the set's shape alone (default_tile)
+    uint32_t nchunks = 0;      // the set's chunks, of the built size
     int tuned_chunk = 16;
     int tuned_bpc = 8;
     uint32_t chunk = 16;

@@ -115,6 +115,30 @@ def test_groups_of_chunks(device, chunk, vpr):
         assert st["segment_tests"] + st["pruned_tests"] == full["segment_tests"]
 
 
+@pytest.mark.parametrize("shape,vpr,tile", [("star", 10, 1), ("star", 48, 2), ("lakes", 10, 2), ("lakes", 32, 4),
+                                            ("star", 300, 4)])
+def test_default_tile_by_shape(shape, vpr, tile):
+    # nothing tuned or set: few edges and chunks a pixel 1, up to 128 edges and
+    # 24 chunks 2, beyond either 4; a chosen width stays for later sets
+    from farm_amd import datagen
+
+    if shape == "star":
+        w = Workload(*datagen.star_pair_set(31, 300, 300, 0.0, 39.0), vpr=vpr)
+    else:
+        w = Workload(datagen.complex_set(41, 12, lo=0.0, hi=3.0), datagen.lake_set(42, 600, lo=0.0, hi=3.0), vpr=vpr)
+    want, _ = w.oracle(0)
+    dev = capi.Device(0)
+    try:
+        w.upload(dev)
+        assert dev.tuning()["tile_a"] == tile
+        assert np.array_equal(dev.intersect(mode=capi.MODE_EXACT_BATCHED).bits, (want == 1).astype(np.uint8))
+        dev.set_tuning(8, 16)
+        w.upload(dev)
+        assert dev.tuning()["tile_a"] == 8
+    finally:
+        dev.close()
+
+
 @pytest.mark.parametrize("chunk", [8, 16, 32])
 def test_without_the_prune(device, chunk):
     # another kernel of its own: every chunk for every lane with an edge, in
