@@ -209,7 +209,7 @@ struct PairQueue {
     uint32_t a[kQueue];
     uint32_t b[kQueue];
 };
-struct Queues {
+struct alignas(16) Queues {
     PairQueue chunks;  // source chunk, target chunk
     PairQueue lines;   // source edge's first vertex, target chunk
     PairQueue edges;   // first vertices of the source and target edge
@@ -522,40 +522,98 @@ __device__ __forceinline__ void path_pt(const float *X, const float *Y, int m, i
 
 constexpr int kLanePath = 16;  // area-piece paths of at most this many segments are searched by one lane
 
-// One ring's pieces: D[0, n) sorted by this ring's (edge, parameter).
-// Counts the reference pieces by status into r and returns this lane's part
-// of the cross-product sum of the area pieces IN the other polygon.
-// The team's waves take 64 pieces each in turn; r gets this wave's counts.  The
-// sum has one order whatever the team, as its last bits are part of the area
-// and which pairs go to a team depends on the call's size: lane k adds segments
-// k, k + 64, .. of one piece after the other.  A team's lanes work out the
-// segments of a piece each, up to kRow of them, into a row of memory (0 past
-// the piece's last and for other pieces, which adds nothing), and its first
-// wave adds the rows in order, the longer pieces by itself; the other waves
-// return 0.
-constexpr int kRow = 4;
+// A ring of m distinct vertices; cross products are taken relative to (ox, oy).
+struct Ring {
+    const float *X, *Y;
+    int m;
+    double ox, oy;
+    // segment k of the path from a through nv vertices to b
+    __device__ __forceinline__ double term(int f, int nv, float ax, float ay, float bx, float by, int k) const {
+        float x0, y0, x1, y1;
+        path_pt(X, Y, m, f, nv, ax, ay, bx, by, k, x0, y0);
+        path_pt(X, Y, m, f, nv, ax, ay, bx, by, k + 1, x1, y1);
+        return ((double)x0 - ox) * ((double)y1 - oy) - ((double)x1 - ox) * ((double)y0 - oy);
+    }
+};
+
+// A path sum has one order, whatever the team: lane k adds segments k, k + 64,
+// .. of one IN piece after the other.  (Its last bits are part of the area, and
+// which pairs go to a team depends on the call's size.)  A team's lanes work
+// out the segments of a piece each, up to `width` of them, into a row of memory
+// (0 past the piece's last and for other pieces, which adds nothing; a longer
+// piece's row has its vertices and ends), and one wave adds up the rows.
+constexpr int kRow = 8;
 constexpr int kRowLong = 0x7ff8b17e;  // high word of a longer piece's row: a NaN no sum makes
+
+// This lane's part of a ring's path sum, from the n rows.  (A call of its own:
+// inlined it spills the kernel's registers.  Both rings' sums by two waves, after
+// their pieces: 4,000 pairs of jagged rings, some hundred pieces each, 2.66 ms a
+// call; one after the other 2.84; every wave its own pieces, in no one order, 2.74.)
+__device__ __noinline__ double sum_rows(const Ring ring, const double *rows, uint32_t n, int width, int lane, Queues &Q) {
+    static_assert(sizeof(Queues) >= 32 * kRow * sizeof(double), "32 rows in a wave's queues");
+    double *lds = reinterpret_cast<double *>(&Q);
+    double acc = 0.0;
+    uint4 next[2];  // the next 32 rows, on their way
+    const uint64_t nval = (uint64_t)width * n;
+    const uint4 *rows4 = reinterpret_cast<const uint4 *>(rows);
+    uint4 *lds4 = reinterpret_cast<uint4 *>(lds);
+    auto load = [&](uint32_t p0) {
+#pragma unroll
+        for (uint32_t k = 0; k < 2; k++) {
+            const uint64_t o = (uint64_t)width / 2 * p0 + 64 * k + lane;
+            next[k] = rows4[o < nval / 2 ? o : 0];
+        }
+    };
+    load(0);
+    for (uint32_t p0 = 0; p0 < n; p0 += 32) {
+        const uint32_t np = min(n - p0, 32u);
+        wave_sync();
+#pragma unroll
+        for (uint32_t k = 0; k < 2; k++)
+            if ((int)(64 * k) < 16 * width) lds4[64 * k + lane] = next[k];
+        load(p0 + 32);
+        wave_sync();
+        uint32_t wm = (uint32_t)__ballot((uint32_t)lane < np && reinterpret_cast<const int *>(lds)[2 * width * (lane & 31) + 1] == kRowLong);
+        for (uint32_t p = 0; p < np; p++) {
+            // the rows up to the next longer piece
+            const uint32_t end = wm ? (uint32_t)__ffs((int)wm) - 1u : np;
+            if (lane < width) {
+#pragma unroll 8
+                for (; p < end; p++) acc += lds[width * p + lane];
+            }
+            p = end;
+            if (!wm) break;
+            wm &= wm - 1;
+            const int *w = reinterpret_cast<const int *>(lds + width * p);
+            const int f = uni(w[2]), nv = uni(w[3]);
+            const float ax = __int_as_float(w[4]), ay = __int_as_float(w[5]);
+            const float bx = __int_as_float(w[6]), by = __int_as_float(w[7]);
+            for (int k = lane; k <= nv; k += 64) acc += ring.term(f, nv, ax, ay, bx, by, k);
+        }
+    }
+    return acc;
+}
+
+// One ring's pieces: D[0, n) sorted by this ring's (edge, parameter).
+// Counts the reference pieces by status into r (this wave's, of a team whose
+// waves take 64 pieces each in turn) and returns this lane's part of the
+// cross-product sum of the area pieces IN the other polygon, or leaves it to
+// sum_rows (a team's).
 template <bool SRC, int NW>
 __device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const farm_raster_hdr &hq, const Rec *D,
-                              uint32_t n, double *rows, double ox, double oy, const Team<NW> &tm, PairRes &r,
+                              uint32_t n, double *rows, int width, double ox, double oy, const Team<NW> &tm, PairRes &r,
                               const PieceOut &po, Queues &Q) {
     const int lane = tm.lane;
     const float *X = S.x + hp.vert_start, *Y = S.y + hp.vert_start;
     const int m = (int)hp.nverts - 1;
     const double eps = (double)1e-6f;  // util.h:44
     double acc = 0.0;
+    const Ring ring{X, Y, m, ox, oy};
     // ring vertices on the way from record i (a) to the next (b)
     auto path_len = [&](uint32_t i, const Rec &a, const Rec &b) {
         const int e0 = SRC ? a.ei : a.ej, e1 = SRC ? b.ei : b.ej;
         const double t0 = SRC ? a.t : a.u, t1 = SRC ? b.t : b.u;
         return i + 1 < n ? max(e1 - e0, 0) : (e1 - e0 + m) % m + ((e1 == e0 && t1 <= t0) ? m : 0);
-    };
-    // segment k of the path from a to b
-    auto term = [&](int f, int nv, float pax, float pay, float pbx, float pby, int k) {
-        float x0, y0, x1, y1;
-        path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k, x0, y0);
-        path_pt(X, Y, m, f, nv, pax, pay, pbx, pby, k + 1, x1, y1);
-        return ((double)x0 - ox) * ((double)y1 - oy) - ((double)x1 - ox) * ((double)y0 - oy);
     };
     for (uint32_t c0 = NW == 1 ? 0u : 64u * tm.wv; c0 < n; c0 += 64 * NW) {
         const uint32_t i = c0 + lane;
@@ -684,17 +742,20 @@ __device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const 
         put_pieces(po, in_area, farm_piece{po.pair, SRC ? 0 : 1, first, nvert, ax, ay, bx, by}, lane);
         if constexpr (NW > 1) {
             if (i < n) {
-                double t[kRow] = {0.0, 0.0, 0.0, 0.0};
-                if (in_area && nvert < kRow) {
+                double t[kRow] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+                if (in_area && nvert < width) {
 #pragma unroll
                     for (int k = 0; k < kRow; k++)
-                        if (k <= nvert) t[k] = term(first, nvert, ax, ay, bx, by, k);
+                        if (k <= nvert) t[k] = ring.term(first, nvert, ax, ay, bx, by, k);
                 } else if (in_area) {
                     t[0] = __hiloint2double(kRowLong, 0);
+                    t[1] = __hiloint2double(nvert, first);
+                    t[2] = __hiloint2double(__float_as_int(ay), __float_as_int(ax));
+                    t[3] = __hiloint2double(__float_as_int(by), __float_as_int(bx));
                 }
 #pragma unroll
-                for (int k = 0; k < kRow; k += 2)
-                    *reinterpret_cast<double2 *>(rows + (uint64_t)kRow * i + k) = make_double2(t[k], t[k + 1]);
+                for (int k = 0; k < kRow; k++)
+                    if (k < width) rows[(uint64_t)width * i + k] = t[k];
             }
         } else {
             // the wave over one IN piece after the other
@@ -705,34 +766,9 @@ __device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const 
                 const int f = __shfl(first, src, 64), nv = __shfl(nvert, src, 64);
                 const float pax = __shfl(ax, src, 64), pay = __shfl(ay, src, 64);
                 const float pbx = __shfl(bx, src, 64), pby = __shfl(by, src, 64);
-                for (int k = lane; k <= nv; k += 64) acc += term(f, nv, pax, pay, pbx, pby, k);
+                for (int k = lane; k <= nv; k += 64) acc += ring.term(f, nv, pax, pay, pbx, pby, k);
             }
         }
-    }
-    if constexpr (NW > 1) {
-        tm.sync();
-        if (tm.first())
-            for (uint32_t p0 = 0; p0 < n; p0 += 64) {
-                const uint32_t np = min(n - p0, 64u);
-                const double *row = rows + (uint64_t)kRow * p0;
-                const bool wide = (uint32_t)lane < np && __double2hiint(row[kRow * lane]) == kRowLong;
-                uint64_t wm = __ballot(wide);
-                for (uint32_t p = 0; p < np;) {
-                    // the rows up to the next longer piece
-                    const uint32_t end = wm ? (uint32_t)__ffsll((unsigned long long)wm) - 1u : np;
-                    if (lane < kRow) {
-#pragma unroll 8
-                        for (; p < end; p++) acc += row[kRow * p + lane];
-                    }
-                    p = end;
-                    if (!wm) break;
-                    wm &= wm - 1;
-                    const Rec a = D[p0 + p], b = D[(p0 + p + 1) % n];
-                    const int nv = path_len(p0 + p, a, b), f = (SRC ? a.ei : a.ej) + 1;
-                    for (int k = lane; k <= nv; k += 64) acc += term(f, nv, a.px, a.py, b.px, b.py, k);
-                    p++;
-                }
-            }
     }
     return acc;
 }
@@ -903,14 +939,29 @@ __device__ __forceinline__ PairRes intersection_pair(const DevSet &S, const doub
     }
     r.c[0] = (int32_t)nk;
     double acc_a = 0.0, acc_b = 0.0;
-    static_assert(kRow * sizeof(double) == sizeof(Rec), "a row per record");
-    double *rows = reinterpret_cast<double *>(R);  // (the raw records are done with)
     if (nk > 0) {
+        // a team's rows take the place of the raw records, which are done with:
+        // both rings', and one wave adds up either; or one ring's at a time
+        static_assert(kRow * sizeof(double) == 2 * sizeof(Rec), "two records to a row");
+        double *rows = reinterpret_cast<double *>(R);
+        const int width = 4 * (uint64_t)nk <= cap ? kRow : kRow / 2;
+        const bool both = 2 * (uint64_t)nk <= cap;
+        const Ring ra{AX, AY, (int)hA.nverts - 1, ox, oy}, rb{BX, BY, (int)hB.nverts - 1, ox, oy};
         bitonic<1>(D, nk, tm);
-        acc_a = ring_pieces<true>(S, hA, hB, D, nk, rows, ox, oy, tm, r, po, Q);
+        acc_a = ring_pieces<true>(S, hA, hB, D, nk, rows, width, ox, oy, tm, r, po, Q);
         tm.sync();
+        if (NW > 1 && !both) {
+            if (tm.wv == 0) acc_a = sum_rows(ra, rows, nk, width, lane, Q);
+            tm.sync();
+        }
         bitonic<2>(D, nk, tm);
-        acc_b = ring_pieces<false>(S, hB, hA, D, nk, rows, ox, oy, tm, r, po, Q);
+        double *rows_b = both ? rows + (uint64_t)width * nk : rows;
+        acc_b = ring_pieces<false>(S, hB, hA, D, nk, rows_b, width, ox, oy, tm, r, po, Q);
+        if constexpr (NW > 1) {
+            tm.sync();
+            if (both && tm.wv == 0) acc_a = sum_rows(ra, rows, nk, width, lane, Q);
+            if (tm.wv == 1) acc_b = sum_rows(rb, rows_b, nk, width, lane, Q);
+        }
     }
     double side_a = wave_sum(acc_a), side_b = wave_sum(acc_b);
     if constexpr (NW > 1) {
@@ -968,12 +1019,22 @@ __global__ __launch_bounds__(256) void k_ring_area(DevSet S, int64_t npolys, dou
 // Pairs for a whole workgroup: their indices to list (count at ctr[kIxHeavy]),
 // and flags[k] = 1.  A pair's collection runs over up to (chunks of A in the
 // overlap of the boxes) x (chunks of B in it) chunk pairs, estimated from the
-// overlap's share of each box; beyond kHeavyChunks one wave would be at it for
-// milliseconds (a 200,000-vertex ring against one over all of it took 57 ms of a
-// 138 ms call).  all: every pair (a call too small to fill the chip with one
-// wave per pair).
+// overlap's share of each box.  Beyond kHeavyChunks one wave is at it too long,
+// or its crossing records outgrow the wave's slab and the pair is done again.
+// Measured, ms at 256 / 1,024 / 4,096 / 16,384 chunk pairs: complex x lakes
+// (479,000 pairs) -v 256 47.1 45.3 47.3 48.1, -v 64 51.2 47.1 45.4 45.7; jagged
+// rings -v 10 (237,000 pairs) 70.0 67.6 67.3 174; -v 33 (63,000) 14.0 14.5 18.3
+// 18.2.  (Chunks as they are: a jagged ring at 10 vertices per pixel has a third
+// of its vertices, not a sixteenth.)
+// all: every pair, in a call of fewer than kTeamPairs pairs to a workgroup, which
+// would not fill the chip evenly with one wave per pair.  Measured, ms with all
+// by workgroups and without, 1,024 workgroups: jagged rings -v 100 8,000 pairs
+// 2.93 / 5.02, 16,000 4.95 / 7.45, 32,000 9.09 / 9.22, 48,000 13.2 / 12.3;
+// complex x lakes -v 256 2,000 pairs 1.76 / 4.22, 8,000 6.58 / 6.39, 16,000 7.09 /
+// 6.58, 32,000 18.5 / 17.6.
 enum : int { kIxHead = 0, kIxOver = 1, kIxPieces = 2, kIxHeavy = 3, kIxHeavyHead = 4 };
-constexpr float kHeavyChunks = 8192.f;
+constexpr float kHeavyChunks = 1024.f;
+constexpr uint32_t kTeamPairs = 16;
 
 __global__ __launch_bounds__(256) void k_ix_heavy(DevSet S, const uint32_t *__restrict__ pa,
                                                   const uint32_t *__restrict__ pb, uint32_t n, int all,
@@ -993,7 +1054,9 @@ __global__ __launch_bounds__(256) void k_ix_heavy(DevSet S, const uint32_t *__re
             float fa = 1.f, fb = 1.f;
             part(0, 2, fa, fb);
             part(1, 3, fa, fb);
-            heavy = all || (A.nverts * fa / kIxChunk) * (B.nverts * fb / kIxChunk) > kHeavyChunks;
+            const float ca = (float)(S.ixoff[A.seq_start + A.nseqs] - S.ixoff[A.seq_start]);
+            const float cb = (float)(S.ixoff[B.seq_start + B.nseqs] - S.ixoff[B.seq_start]);
+            heavy = all || (ca * fa) * (cb * fb) > kHeavyChunks;
             flags[k] = heavy ? 1 : 0;
         }
         const uint64_t m = __ballot(heavy);
@@ -1144,8 +1207,8 @@ int run_intersection(farm_handle h, uint64_t begin, uint64_t end, int32_t *count
     const uint64_t nwaves = (uint64_t)nblocks * kWaves;
     if ((rc = ensure(h, h->wslab, nwaves * 2ull * kRecCap * sizeof(Rec)))) return rc;
     HIPCHK(h, hipEventRecord(h->ev[0], h->stream));
-    // fewer than 8 pairs to a workgroup: all of them by whole workgroups
-    hipLaunchKernelGGL(k_ix_heavy, dim3((unsigned)std::min<uint64_t>(blocks_for(n), kMaxLaunchGroups)), dim3(256), 0, h->stream, S, pa, pb, n, n < 8 * nblocks ? 1 : 0,
+    hipLaunchKernelGGL(k_ix_heavy, dim3((unsigned)std::min<uint64_t>(blocks_for(n), kMaxLaunchGroups)), dim3(256), 0, h->stream, S, pa, pb, n,
+                       n < kTeamPairs * nblocks ? 1 : 0,
                        P<uint8_t>(h->ixflag), P<uint32_t>(h->ixlist), ctr);
     HIPCHK(h, hipGetLastError());
     hipLaunchKernelGGL(k_intersection<false>, dim3(nblocks), dim3(64 * kWaves), 0, h->stream, S,

@@ -207,11 +207,11 @@ def test_intersection_polygons_areas_match(device, seed):
     assert set(lines) <= set(nz.tolist()) | set(np.nonzero(counts[:, 2] > 0)[0].tolist())
 
 
-@pytest.mark.parametrize("npairs", [60, 9001])
+@pytest.mark.parametrize("npairs", [60, 9001, 16385])
 def test_pairs_by_workgroups_and_by_waves(device, npairs):
-    # fewer pairs than 8 per workgroup: each by a whole workgroup; more: one
-    # wave each, but for the pairs of two long rings (some with more pieces
-    # than lanes, some contained)
+    # fewer pairs than 16 per workgroup (4 of them a CU): each by a whole
+    # workgroup; more: one wave each, but for the pairs of two long rings (some
+    # with more pieces than lanes, some contained)
     a = rings_from_list([_wavy(6000, 0.0, 0.0, 1.0), _wavy(40, 0.3, 0.2, 0.5), _wavy(900, 5.0, 5.0, 0.4)])
     b = rings_from_list([_wavy(5000, 0.2, 0.1, 0.9), _wavy(700, 0.1, 0.0, 0.7), _wavy(15, 0.0, 0.1, 0.05),
                          _wavy(300, 5.1, 5.0, 0.35)])
@@ -227,16 +227,32 @@ def test_pairs_by_workgroups_and_by_waves(device, npairs):
     assert (np.abs(area - want) <= AREA_RTOL * np.abs(want) + AREA_ATOL).all()
 
 
+@pytest.mark.parametrize("waves", [500, 1100, 1500, 2300])
+def test_many_pieces_by_a_workgroup(device, waves):
+    # two crossings a wave of one ring with the other: a workgroup's slab (8,192
+    # records) has room for both rings' rows of eight values, of four, for one
+    # ring's at a time; pieces of 0 to 9 vertices
+    t = np.linspace(0, 2 * np.pi, 8 * waves + 3, endpoint=False)
+    r = 1.0 + 0.1 * np.sin(waves * t + 0.3)
+    u = np.linspace(0.001, 2 * np.pi + 0.001, 3001, endpoint=False)
+    a = rings_from_list([np.stack([3.0 + r * np.cos(t), 3.0 + r * np.sin(t)], 1)])
+    b = rings_from_list([np.stack([3.0 + np.cos(u), 3.0 + np.sin(u)], 1)])
+    w = Workload(a, b, vpr=100)
+    c, area, st = _check(device, w)
+    assert c[0, 0] > 1.9 * waves and area[0] > 1.0
+    assert st["refine_items"] <= 8192  # (no rerun with larger slabs)
+
+
 def test_areas_do_not_depend_on_the_calls_size(device):
     # pairs of some hundred short pieces (jagged rings) and of few long ones,
     # all in one call (a wave each) and 500 at a time (a workgroup each): the
     # path sums have one order, so the areas are the same bytes
-    (sa, sxy), (ta, txy) = datagen.star_pair_set(13, 4400, 4400, 0.0, 148.0)
+    (sa, sxy), (ta, txy) = datagen.star_pair_set(13, 8400, 8400, 0.0, 205.0)
     a = [sxy[sa[i]:sa[i + 1] - 1] for i in range(len(sa) - 1)] + [_wavy(900, 0.0, 0.0, 1.0), _wavy(61, 0.3, 0.2, 0.5)]
     b = [txy[ta[i]:ta[i + 1] - 1] for i in range(len(ta) - 1)] + [_wavy(300, 0.1, 0.0, 0.9), _wavy(700, 0.2, 0.3, 0.8)]
-    w = Workload(rings_from_list(a), rings_from_list(b), vpr=10)
+    w = Workload(rings_from_list(a), rings_from_list(b), vpr=64)
     n = len(w.pa)
-    assert n > 8192 + 500
+    assert n >= 16384
     w.upload(device)
     c, area, _ = device.intersection_area()
     assert (c[:, 1] > 128).any() and (c[:, 1] > 0).sum() > 2000
