@@ -3,6 +3,7 @@ and the reference -a heuristic, bit-exact against the oracle."""
 import numpy as np
 import pytest
 
+import oracle
 from farm_amd import capi
 from tests.helpers import Workload, rings_from_list, star_pairs
 
@@ -113,6 +114,48 @@ def test_groups_of_chunks(device, chunk, vpr):
         st = device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=tile, chunk=chunk).stats
         print(f"  -v {vpr} tile={tile} chunk={chunk}: {st['segment_tests']} run", flush=True)
         assert st["segment_tests"] + st["pruned_tests"] == full["segment_tests"]
+
+
+def _collinear_slivers(seed, n):
+    # pairs of thin triangles one behind the other along a line, their long
+    # sides on it to within an ulp and parallel to within 1e-6: apart, so that
+    # only the rounding of the f32 cross products can make them cross
+    rng = np.random.default_rng(seed)
+    scale = 2.0 ** rng.integers(-6, 6, n)[:, None, None]
+    th = np.where(rng.random(n) < 0.7, rng.uniform(0, np.pi, n), rng.choice([0, 0.25, 0.5, 0.75], n) * np.pi)
+    turn = th + rng.choice([0.0, 1.0], n) * 10 ** rng.uniform(-9, -6, n)
+    o, u, w = rng.uniform(-1, 1, (n, 2)), np.stack([np.cos(th), np.sin(th)], 1), np.stack([np.cos(turn), np.sin(turn)], 1)
+    a = o.astype(np.float32)
+    b = (o + rng.uniform(0.1, 1, n)[:, None] * u).astype(np.float32)
+    ab = b.astype(np.float64) - a
+    nrm = np.stack([-ab[:, 1], ab[:, 0]], 1) / np.linalg.norm(ab, axis=1)[:, None]
+    c = a + (1 + 10 ** rng.uniform(-1.5, 0.5, n))[:, None] * ab + rng.uniform(-1, 1, n)[:, None] * 1e-7 * nrm
+    d = c + rng.uniform(0.1, 1, n)[:, None] * w
+    A = np.stack([a, b, a + 1e-3 * nrm], 1) * scale
+    B = np.stack([c, d, d - 1e-3 * nrm], 1) * scale
+    return A.astype(np.float32), B.astype(np.float32)
+
+
+def test_crossings_that_rounding_makes_up(device):
+    # the direction prune may not drop them (its rule for k_refine, and the
+    # intersection's collection, which has it too); one pixel a triangle, so
+    # every pair of sides is looked at
+    A, B = _collinear_slivers(47, 20000)
+    k = np.arange(len(A))
+    w = Workload(rings_from_list(list(A)), rings_from_list(list(B)), vpr=64, pairs=(k, k))
+    want, _ = w.oracle(0)
+    gap = np.maximum(B.min(1) - A.max(1), A.min(1) - B.max(1)).max(1)
+    reach = (np.maximum(A.max(1), B.max(1)) - np.minimum(A.min(1), B.min(1))).sum(1)
+    made_up = (want == 1) & (gap > reach * 2.0 ** -7)
+    assert made_up.sum() > 300, made_up.sum()
+    w.upload(device)
+    for tile in (1, 2, 4, 8):
+        for flags in (0, capi.FLAG_NO_PRUNE):
+            r = device.intersect(mode=capi.MODE_EXACT_BATCHED, tile_a=tile, chunk=16, flags=flags)
+            diff = np.nonzero(r.bits != (want == 1))[0]
+            assert diff.size == 0, f"tile {tile} flags {flags}: {diff.size} pairs differ, first {diff[:10]}"
+    counts, _, _ = device.intersection_area()
+    assert np.array_equal(counts, oracle.intersection(w.OA, w.OB, w.pa, w.pb)[0])
 
 
 @pytest.mark.parametrize("shape,vpr,tile", [("star", 10, 1), ("star", 48, 2), ("lakes", 10, 2), ("lakes", 32, 4),

@@ -69,6 +69,18 @@ def test_gradients_at_tile_edges(device, m):
         o += n
 
 
+# CRC-32 of farm_mlp_forward's outputs for _rand_problem(500 + m, m)'s first two
+# draws, as one MFMA product a layer over all rows gave them
+FORWARD_CRC = {1: 1113353877, 17: 3338742613, 64: 1524767650, 300: 121737229, 5000: 2536647548, 70000: 1736403895}
+
+
+@pytest.mark.parametrize("m", list(FORWARD_CRC))
+def test_forward_bytes(device, m):
+    p, X, _, _ = _rand_problem(500 + m, m)
+    device.mlp_set_params(p)
+    assert zlib.crc32(np.ascontiguousarray(device.mlp_forward(X)).tobytes()) == FORWARD_CRC[m]
+
+
 # CRC-32 of the gradients (+ 0.0, so that -0 is 0) of _rand_problem(300 + m, m)
 # and of the weights after training on _rand_problem(900 + rows + batch, rows):
 # the sums over a batch's rows have one order (chunks of about 1,024 rows, 16
@@ -204,9 +216,10 @@ def test_learned_queue_order_keeps_exact_results(device, star_model):
 
 
 def test_fused_inference_equals_the_three_launch_forward(device, star_model):
-    # farm_mlp_predict_pairs runs normalisation and the three layers in one
-    # kernel; its logits and cost predictions equal the generic MFMA GEMM
-    # path's (farm_mlp_forward on the same normalised features) bit for bit
+    # farm_mlp_predict_pairs normalises on the device; its logits and cost
+    # predictions are those of farm_mlp_forward on rows normalised on the host,
+    # bit for bit (the same kernel: test_forward_bytes holds its outputs to
+    # those of one product a layer)
     M = star_model
     device.mlp_set_params(M["params"], M["norm"])
     device.upload_polygons(M["test_ps"].both)
