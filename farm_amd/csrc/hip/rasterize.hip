@@ -697,6 +697,12 @@ constexpr uint64_t kShortRing = 8;  // 4,000 complex rings: 15.8 ms at 8, 16.0 a
 // jagged rings of up to 500 vertices (78 per CU), 0 / 2: 1.12, 0.85.
 constexpr uint64_t kWholeRings = 16;
 
+// A column with a point near an axis is marked in its candidate count (a ring of
+// kMarkEdges edges or more, whose count may need the bit, goes as marked): only
+// there does pass 1 keep a list of those points.
+constexpr uint32_t kStripNear = 0x80000000u;
+constexpr int kMarkEdges = 1 << 29;
+
 template <int PASS>
 struct StripLds {
     uint32_t sh[4];
@@ -715,7 +721,7 @@ __device__ __forceinline__ bool strip_columns(const RPoly &g, const float *X, co
                                               int c_begin, int c_end, const double *__restrict__ colx,
                                               uint32_t *__restrict__ stripc, const uint64_t *__restrict__ stripo,
                                               const uint64_t *__restrict__ hasho, float2 *__restrict__ pool,
-                                              float2 *__restrict__ nearpool, unsigned long long *__restrict__ hkeys,
+                                              unsigned long long *__restrict__ hkeys,
                                               uint32_t *__restrict__ hidx, uint32_t *__restrict__ stripn,
                                               float *__restrict__ stripmy, StripLds<PASS> &L) {
     const Bucket bk(g.x0, g.sx, g.dimx + 2, absx);
@@ -726,23 +732,29 @@ __device__ __forceinline__ bool strip_columns(const RPoly &g, const float *X, co
         const double Xi = colx[g.vl + c], Xi1 = colx[g.vl + c + 1];
         if (PASS == 0) {
             uint32_t cnt = 0;
+            bool nr = false;
             for (int e = threadIdx.x; e < ne; e += kRB) {
                 const float ax = Xp[e], bx = Xp[e + 1];
                 if (!bk.reaches(ax, bx, c)) continue;
                 float2 pts[4];
-                cnt += strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, pts);
+                const uint32_t n = strip_points(ax, Yp[e], bx, Yp[e + 1], e == 0, Xi, Xi1, pts);
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++) nr = nr || (j < n && near_axis(pts[j]));
+                cnt += n;
             }
+            nr = __syncthreads_or(nr);
             uint32_t tot;
             block_scan(cnt, L.sh, &tot);
-            if (threadIdx.x == 0) stripc[g.vl + c] = tot;
+            if (threadIdx.x == 0) stripc[g.vl + c] = nr && ne < kMarkEdges ? tot | kStripNear : tot;
             continue;
         }
-        const uint32_t cnt = stripc[g.vl + c];
+        const uint32_t cnt = ne < kMarkEdges ? stripc[g.vl + c] & ~kStripNear : stripc[g.vl + c];
         if (cnt == 0) {
             if (threadIdx.x == 0) stripn[g.vl + c] = 0;
             continue;
         }
-        float2 *pts = pool + stripo[g.vl + c], *nearp = nearpool + stripo[g.vl + c];
+        // (the points near an axis behind the strip's room, in columns that have any)
+        float2 *pts = pool + stripo[g.vl + c], *nearp = pts + cnt + 1;
         if (threadIdx.x == 0) L.nkept = 0;
         const bool lds = cnt <= kLdsCands;
         uint32_t slots = kLdsSlots;
@@ -892,7 +904,6 @@ __global__ __launch_bounds__(kRB) void k_rstrip(const RPoly *__restrict__ P, con
                                                 const uint32_t *__restrict__ colpoly, const uint32_t *__restrict__ items,
                                                 uint32_t *__restrict__ stripc, const uint64_t *__restrict__ stripo,
                                                 const uint64_t *__restrict__ hasho, float2 *__restrict__ pool,
-                                                float2 *__restrict__ nearpool,
                                                 unsigned long long *__restrict__ hkeys, uint32_t *__restrict__ hidx,
                                                 uint32_t *__restrict__ stripn, float *__restrict__ stripmy) {
     const uint32_t item = items[blockIdx.x], cs = item & ~kItemWhole;
@@ -904,7 +915,7 @@ __global__ __launch_bounds__(kRB) void k_rstrip(const RPoly *__restrict__ P, con
     __shared__ StripLds<PASS> L;
     auto columns = [&](auto look) {
         return strip_columns<PASS, decltype(look)::value>(g, X, Y, (double)absx[i], nrow, c_begin, c_end, colx, stripc,
-                                                          stripo, hasho, pool, nearpool, hkeys, hidx, stripn, stripmy,
+                                                          stripo, hasho, pool, hkeys, hidx, stripn, stripmy,
                                                           L);
     };
     const bool ok = PASS == 1 && g.nv > kShortRing * kRB + 1 ? columns(std::true_type()) : columns(std::false_type());
@@ -1596,16 +1607,16 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
         }
         return FARM_OK;
     };
-    auto strips = [&](auto kernel, const uint64_t *so, const uint64_t *hof, float2 *pool, float2 *nearpool,
+    auto strips = [&](auto kernel, const uint64_t *so, const uint64_t *hof, float2 *pool,
                       unsigned long long *hkeys, uint32_t *hidx) {
         return sliced(items.size(), [&](uint64_t s0, dim3 groups) {
             hipLaunchKernelGGL(kernel, groups, dim3(kRB), 0, h->stream, (const RPoly *)d_rp, P<float>(h->x),
                                P<float>(h->y), (const float *)d_absx, d_flag, (const int *)ncols, (const int *)nrows,
                                (const double *)colx, (const uint32_t *)colpoly, (const uint32_t *)d_items + s0, stripc,
-                               so, hof, pool, nearpool, hkeys, hidx, stripn, stripmy);
+                               so, hof, pool, hkeys, hidx, stripn, stripmy);
         });
     };
-    if ((rc = strips(k_rstrip<0>, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr))) return rc;
+    if ((rc = strips(k_rstrip<0>, nullptr, nullptr, nullptr, nullptr, nullptr))) return rc;
     // pool sizes: every candidate plus the closing point; hashes in HBM for
     // strips beyond the LDS table
     {
@@ -1614,25 +1625,30 @@ int rasterize_uploaded(farm_handle h, int64_t np, const std::vector<uint64_t> &v
         HIPCHK(h, hipStreamSynchronize(h->stream));
         std::vector<uint64_t> po(nvl + 1), ho(nvl + 1);
         uint64_t tp = 0, th = 0;
-        for (uint64_t s = 0; s < nvl; s++) {
-            po[s] = tp;
-            ho[s] = th;
-            tp += sc[s] ? sc[s] + 1 : 0;
-            if (sc[s] > kLdsCands) {
-                uint64_t sl = 1;
-                while (sl < 2ull * sc[s]) sl <<= 1;
-                th += sl;
+        for (int64_t i = 0; i < np; i++) {
+            const bool marks = voff[i + 1] - voff[i] - 1 < (uint64_t)kMarkEdges;
+            for (uint64_t s = rp[i].vl; s < rp[i].vl + rp[i].dimx + 2; s++) {
+                const bool nr = !marks || (sc[s] & kStripNear);
+                const uint64_t cnt = marks ? sc[s] & ~kStripNear : sc[s];
+                po[s] = tp;
+                ho[s] = th;
+                tp += cnt ? cnt + 1 + (nr ? cnt : 0) : 0;
+                if (cnt > kLdsCands) {
+                    uint64_t sl = 1;
+                    while (sl < 2 * cnt) sl <<= 1;
+                    th += sl;
+                }
             }
         }
         po[nvl] = tp;
         ho[nvl] = th;
         HIPCHK(h, hipMemcpyAsync(stripo, po.data(), 8 * (nvl + 1), hipMemcpyHostToDevice, h->stream));
         HIPCHK(h, hipMemcpyAsync(hasho, ho.data(), 8 * (nvl + 1), hipMemcpyHostToDevice, h->stream));
-        float2 *pool, *nearpool;
+        float2 *pool;
         unsigned long long *hkeys;
         uint32_t *hidx;
-        if ((rc = T.get(h, &pool, tp)) || (rc = T.get(h, &nearpool, tp)) || (rc = T.get(h, &hkeys, th)) || (rc = T.get(h, &hidx, th))) return rc;
-        if ((rc = strips(k_rstrip<1>, stripo, hasho, pool, nearpool, hkeys, hidx))) return rc;
+        if ((rc = T.get(h, &pool, tp)) || (rc = T.get(h, &hkeys, th)) || (rc = T.get(h, &hidx, th))) return rc;
+        if ((rc = strips(k_rstrip<1>, stripo, hasho, pool, hkeys, hidx))) return rc;
         if (npix) {
             hipLaunchKernelGGL(k_rcells, dim3(grid_for(npix)), dim3(kRB), 0, h->stream, (const RPoly *)d_rp,
                                (const uint32_t *)d_pixpoly, npix, (const uint32_t *)d_flag, (const int *)ncols,
