@@ -373,6 +373,7 @@ int finish_set(farm_handle h) {
     if ((rc = ensure(h, h->pixedges, 4 * h->nstatus))) return rc;
     h->ring_area_ready = false;
     h->set_gen++;
+    h->poly_gen++;
     if (h->npolys > 0) {
         hipLaunchKernelGGL(k_pixedges, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys,
                            P<uint32_t>(h->pixedges));
@@ -464,7 +465,7 @@ int build_chunk_boxes(farm_handle h, uint32_t C) {
 // of another size (else those serve).  Synchronises the stream.
 int build_ix_boxes(farm_handle h) {
     int rc;
-    if (h->chunk == kIxChunk || h->ix_gen == h->set_gen) return FARM_OK;
+    if (h->chunk == kIxChunk || h->ix_gen == h->poly_gen) return FARM_OK;
     const uint64_t nseqs = h->nseqs;
     if ((rc = ensure(h, h->ixcnt, 4 * (nseqs + 1)))) return rc;
     if ((rc = ensure(h, h->ixoff, 4 * (nseqs + 1)))) return rc;
@@ -487,7 +488,7 @@ int build_ix_boxes(farm_handle h) {
         HIPCHK(h, hipGetLastError());
     }
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    h->ix_gen = h->set_gen;
+    h->ix_gen = h->poly_gen;
     return FARM_OK;
 }
 

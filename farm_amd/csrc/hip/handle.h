@@ -49,7 +49,7 @@ struct farm_handle_s {
     int cc = FARM_CATEGORY_COUNT;
     farm::DevBuf hdr, status, pixoff, seqs, x, y, xyd, choff, chcnt, chbox, chseg, cgbox, cgseg, voff, vnodes, pixedges, shape_ctr;
     // 16-segment chunks for the intersection's collection when the
-    // refinement's boxes are of another size (built for set generation ix_gen)
+    // refinement's boxes are of another size (built for polygon generation ix_gen)
     farm::DevBuf ixcnt, ixoff, ixbox, ixseg;
     uint64_t ix_gen = ~0ull;
     uint64_t nstatus = 0;
@@ -67,6 +67,7 @@ struct farm_handle_s {
     uint64_t max_pixel_pairs = 0xffffffffull;     // per-call limit (farm_set_pixel_pair_limit)
     bool use_graphs = true;                        // capture the batch launches in a hipGraph
     uint64_t set_gen = 0;                          // bumped by every upload that moves device arrays
+    uint64_t poly_gen = 0;                         // bumped by every new set of polygons
     struct IsxGraph {
         unsigned char key[128];
         hipGraphExec_t exec;
@@ -106,7 +107,7 @@ struct farm_handle_s {
     uint64_t max_border_pix = 0;  // most BORDER pixels of a finest layer
     farm::DevBuf layers, lstatus, areas;
     bool areas_ready = false;  // areas hold the set's per-pixel clipped areas
-    farm::DevBuf pixbox, pixlen;  // built for set generation pixrec_gen
+    farm::DevBuf pixbox, pixlen;  // built for polygon generation pixrec_gen
     uint64_t pixrec_gen = ~0ull;
     farm::DevBuf wctr, wovf, wslab, wslab_big, wout, wmd;
     // intersection
@@ -188,7 +189,7 @@ inline DevSet devset(farm_handle h) {
         S.ixoff = S.choff;
         S.ixbox = S.chbox;
         S.ixseg = S.chseg;
-    } else if (h->ix_gen == h->set_gen) {
+    } else if (h->ix_gen == h->poly_gen) {
         S.ixoff = P<uint32_t>(h->ixoff);
         S.ixbox = P<float4>(h->ixbox);
         S.ixseg = P<uint4>(h->ixseg);

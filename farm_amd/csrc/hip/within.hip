@@ -1393,13 +1393,13 @@ int within_consts(farm_handle h) {
 int build_pixrec(farm_handle h) {
     int rc;
     if ((rc = build_ix_boxes(h))) return rc;
-    if (h->pixrec_gen == h->set_gen) return FARM_OK;
+    if (h->pixrec_gen == h->poly_gen) return FARM_OK;
     if ((rc = ensure(h, h->pixbox, 16 * h->nstatus))) return rc;
     if ((rc = ensure(h, h->pixlen, 8 * h->nstatus))) return rc;
     hipLaunchKernelGGL(k_pixrec, dim3((unsigned)h->npolys), dim3(256), 0, h->stream, devset(h), h->npolys,
                        P<float4>(h->pixbox), P<uint2>(h->pixlen));
     HIPCHK(h, hipGetLastError());
-    h->pixrec_gen = h->set_gen;
+    h->pixrec_gen = h->poly_gen;
     return FARM_OK;
 }
 

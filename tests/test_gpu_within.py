@@ -45,6 +45,33 @@ def test_lakes_10km(device):
     assert (md != 100000.0).sum() > 1000  # the refinement path is exercised
 
 
+def test_records_follow_the_polygons():
+    # the pixels' and chunks' records are kept over pair lists and chunk sizes
+    # and made anew for another set, larger or smaller, on the same handle
+    dev = capi.Device(0)
+    try:
+        for n, chunk in ((300, 16), (500, 32), (200, 32), (200, 16), (400, 8)):
+            dev.set_tuning(4, chunk)
+            ro, xy = datagen.lake_set(60 + n + chunk, n, hi=0.7)
+            _run(dev, ro, xy)
+            H = capi.HostSet.from_rings(ro, xy)
+            pa, pb = capi.candidates(H, H, expand_km=10.0, skip_self=True)
+            want, wmd, _ = oracle.within(*[_oracle_set(ro, xy)] * 2, pa, pb, 10.0)
+            for part in (slice(1, None, 3), slice(2, None, 5)):
+                dev.upload_pairs(pa[part], pb[part])
+                bits, md, _ = dev.within(10.0)
+                assert np.array_equal(bits, want[part]) and np.array_equal(md.view(np.uint64), wmd[part].view(np.uint64))
+                dev.set_tuning(4, 8)  # (other chunks, the same records)
+    finally:
+        dev.close()
+
+
+def _oracle_set(ro, xy):
+    O = oracle.OracleSet(ro, xy)
+    O.rasterize(10, hierarchy=True, nlow=1)
+    return O
+
+
 @pytest.mark.parametrize("d_km", [0.0, 2.0, 25.0])
 def test_lakes_other_distances(device, d_km):
     ro, xy = datagen.lake_set(5, 500, hi=0.8)
