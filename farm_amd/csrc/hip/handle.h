@@ -31,7 +31,6 @@ constexpr int kW1 = kNFeat * kHidden, kB1 = kHidden, kW2 = kHidden * kHidden, kB
 constexpr int kOffW1 = 0, kOffB1 = kOffW1 + kW1, kOffW2 = kOffB1 + kB1, kOffB2 = kOffW2 + kW2, kOffW3 = kOffB2 + kB2,
               kOffB3 = kOffW3 + kW3, kNParams = kOffB3 + kB3;
 
-
 // HIP takes fewer than 2^32 work items a launch: the most workgroups of 256
 constexpr uint64_t kMaxLaunchGroups = (1ull << 24) - 1;
 

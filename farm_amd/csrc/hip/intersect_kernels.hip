@@ -1057,7 +1057,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 // lane on 400 complex rings x 9,973 lakes (-v 256): 9.2 ms
                 // without groups, 6.4 with groups of 4, 6.1 of 8; with chunks of
                 // 32 segments 7.45, 6.7 and 6.9.  For 4,000 x 100,000 of
-                // them, 16 segments: 110.5, 76.9, 74.5 ms.
+                // them, 16 segments: 110.5, 76.9, 74.5 ms.  (All with the prune
+                // still a switch in the kernel; without it 6.03 and 72.7 with
+                // groups of 4.)
                 const cfloat *cbox = (const cfloat *)(groups ? S.cgbox + g0 / kGroup : vbox);
                 const cuint *cseg = (const cuint *)(groups ? S.cgseg + g0 / kGroup : vseg);
                 const uint32_t nbox = groups ? (nch + kGroup - 1) / kGroup : nch;

@@ -1071,8 +1071,8 @@ __global__ __launch_bounds__(256) void k_ix_heavy(DevSet S, const uint32_t *__re
 // on one pair (records in slabs of kWaves * cap), then, wave by wave, the other
 // pairs of the window (flags; slabs of cap).  BIG: pairs that overflowed the
 // first launch's slabs, all on the list (n = 0).
-// Four waves per SIMD (128 registers, 13 of them spilled): 61.8 ms for 618,000
-// complex x lakes pairs against 66.7 ms at three.
+// Four waves per SIMD (128 registers, 20 of them spilled): 56.0 ms for 618,000
+// complex x lakes pairs against 63.6 ms at three, 4,000 jagged pairs 2.55 and 2.67.
 template <bool BIG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_intersection(DevSet S, const double *__restrict__ ring2a,
                                                       const uint32_t *__restrict__ pa, const uint32_t *__restrict__ pb,
