@@ -132,7 +132,8 @@ typedef struct farm_polyset {
 
 typedef struct farm_opts {
     int32_t mode;
-    int32_t tile_a;        /* source edges per lane of the batched refinement; 0 = autotuned */
+    int32_t tile_a;        /* source edges per lane of the batched refinement; 0 = autotuned, or
+                              with nothing tuned or set by the set's shape */
     int32_t tile_b;        /* target segments per chunk box of the batched refinement (8, 16
                               or 32); 0 = autotuned.  A size other than the one the set's
                               boxes are built for rebuilds them (allocates, synchronises) */
@@ -278,7 +279,9 @@ int farm_intersect_dev(farm_handle h, uint64_t begin, uint64_t end, const farm_o
  * per-call scratch is a fixed device array of the library (about 80 MiB on
  * each GPU the library runs on, held until the process ends): at most
  * 2^18 pairs, 2^20 BORDER x BORDER pixel pairs and 2^20 refinement tiles
- * per call, else FARM_ECAPACITY (out_dev then holds no valid results).
+ * per call, else FARM_ECAPACITY (out_dev then holds no valid results).  A
+ * tile width that neither the caller nor the autotuner chose gives way to 4
+ * edges per lane where its own tiles do not fit.
  * Modes: exact batched, exact plain and the reference -a heuristic (the
  * learned modes need the MLP's buffers: FARM_EINVAL).  Every call on one GPU
  * shares that array, so calls that overlap on one GPU (from several handles
