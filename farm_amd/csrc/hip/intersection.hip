@@ -543,7 +543,7 @@ struct Ring {
 // (0 past the piece's last and for other pieces, which adds nothing; a longer
 // piece's row has its vertices and ends), and one wave adds up the rows.
 constexpr int kRow = 8;
-constexpr int kRowLong = 0x7ff8b17e;  // high word of a longer piece's row: a NaN no sum makes
+constexpr int kRowLong = 0x7ff8b17e;  // high word of a longer piece's row: a NaN no arithmetic makes
 
 // This lane's part of a ring's path sum, from the n rows.  (A call of its own:
 // inlined it spills the kernel's registers.  Both rings' sums by two waves, after
@@ -747,6 +747,9 @@ __device__ double ring_pieces(const DevSet &S, const farm_raster_hdr &hp, const 
 #pragma unroll
                     for (int k = 0; k < kRow; k++)
                         if (k <= nvert) t[k] = ring.term(first, nvert, ax, ay, bx, by, k);
+                    // a NaN vertex keeps its low bits through the arithmetic
+                    // and could read as a longer piece's row
+                    if (!(t[0] == t[0])) t[0] = NAN;
                 } else if (in_area) {
                     t[0] = __hiloint2double(kRowLong, 0);
                     t[1] = __hiloint2double(nvert, first);
